@@ -26,6 +26,7 @@ HIPCC_FLAGS = [
     "-ffp-contract=off",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-fno-slp-vectorize",  # vectors of two FP32 lanes only cost moves without packed FP32
     "-Wall",
     "-Wno-unused-function",
     "-Wno-unused-variable",

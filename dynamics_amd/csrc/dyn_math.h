@@ -291,28 +291,50 @@ DYN_HD void dyn_coul_erfc(float r2, float rinv, float qq, float beta,
   *s = qe * (rinv * rinv) * (gr + two_b_sqrtpi);
 }
 
-// Tabulated erfc Coulomb of the pair kernel.  With x = βr the force scalar
-// is s = qq/r³ · φ(x), φ(x) = erfc(x) + (2/√π) x e^{−x²}, and the energy
-// E = qq/r · erfc(x).  Both functions of x are tabulated on [0, 4] as
-// cubic Hermite pieces (values and derivatives from the closed forms, in
-// double; φ'(x) = −(4/√π) x² e^{−x²}, erfc'(x) = −(2/√π) e^{−x²}) over
-// DYN_COUL_TAB_N intervals: entry i holds φ's cubic on interval i, entry
-// DYN_COUL_TAB_N + i erfc's (so a forces-only evaluation needs the first
-// half only), each as (c0, c1, c2, c3) in the local coordinate t ∈ [0, 1).
-// Interpolation error ≤ h⁴/384·max|f⁗| ≈ 1e-10 (h = 1/128), below f32
-// rounding, so the table reproduces the closed forms to f32 accuracy with
-// one load and three fmas in place of exp(−x²)·erfcx(x).  Evaluation uses
-// only IEEE-exact operations (mul, floor, conversion, fma), so the host
-// replay, given the same table, reproduces it bit for bit.
-#define DYN_COUL_TAB_N 512
+// 1/x for normal positive x: bit-level seed (max rel. error 0.0506), one
+// third-order and one Newton step.  Max relative error 1.3e-7 over the
+// normal range of the pair distances (checked in tests).
+DYN_HD float dyn_rcpf(float x) {
+  float y = dyn_u2f(0x7ef31000u - dyn_f2u(x));
+  float e = dyn_fmaf(-x, y, 1.0f);
+  y = dyn_fmaf(y, dyn_fmaf(e, e, e), y);
+  e = dyn_fmaf(-x, y, 1.0f);
+  return dyn_fmaf(y, e, y);
+}
+
+// Tabulated erfc Coulomb of the pair kernel.  With x = βr and y = x² = β²r²
+// the force scalar is s = qq·β³·Ψ(y), Ψ(y) = φ(x)/x³, φ(x) = erfc(x) +
+// (2/√π) x e^{−x²}, and the energy E = qq·β·Λ(y), Λ(y) = erfc(x)/x.  Ψ and Λ
+// are tabulated over y itself, so a pair inside the table needs no square
+// root, reciprocal or exponential: 16 octaves of y from 2⁻¹¹, 64 intervals
+// each, found from the exponent's low four bits and the mantissa's top six
+// (any bit pattern finds an entry, so a lane outside the cutoff reads inside
+// the table too).  Each entry is the cubic Hermite piece of its interval
+// (values and derivatives from the closed forms, in double) in t = y − the
+// interval's lower end, which is exact.  The interpolation error is below
+// 1e-8 relative for y ≤ 1, 7e-7 at y = 16 (where Ψ and Λ are e⁻¹⁶ of the
+// bare Coulomb terms).  Evaluation uses only IEEE-exact operations (mul,
+// sub, fma, bit masks), so the host replay, given the same table, reproduces
+// it bit for bit.
+//
+// Pairs closer than the table's first octave (r below 0.07 Å at β =
+// 0.3123/Å) take φ(x) and erfc(x) over x = βr on [0, 4]: DYN_COUL_X_N cubic
+// Hermite pieces each (error ≤ h⁴/384·max|f⁗| ≈ 1e-10, h = 1/128).
+//
+// Layout: two halves of DYN_COUL_TAB_N entries, the forces' (φ by x, then Ψ
+// by y) and the energies' (erfc by x, then Λ by y).
+#define DYN_COUL_X_N 512
 #define DYN_COUL_TAB_XMAX 4.0f
 #define DYN_COUL_TAB_SCALE 128.0f  // intervals per unit of x
+#define DYN_COUL_Y_N 1024
+#define DYN_COUL_Y_MIN 0x1p-11f
+#define DYN_COUL_TAB_N (DYN_COUL_X_N + DYN_COUL_Y_N)
 
-// The table's cubic at u = x · DYN_COUL_TAB_SCALE (u given).
+// The cubic of one half (entry_off 0 or 1) at u = x · DYN_COUL_TAB_SCALE.
 DYN_HD float dyn_tab_cubic_u(const float4* tab, int entry_off, float u) {
   const float fl = dyn_floorf(u);
   int i = (int)fl;
-  i = i < 0 ? 0 : (i > DYN_COUL_TAB_N - 1 ? DYN_COUL_TAB_N - 1 : i);
+  i = i < 0 ? 0 : (i > DYN_COUL_X_N - 1 ? DYN_COUL_X_N - 1 : i);
   const float t = u - fl;
   const float4 c = tab[entry_off * DYN_COUL_TAB_N + i];
   return dyn_fmaf(dyn_fmaf(dyn_fmaf(c.w, t, c.z), t, c.y), t, c.x);
@@ -322,36 +344,109 @@ DYN_HD float dyn_tab_cubic(const float4* tab, int entry_off, float x) {
   return dyn_tab_cubic_u(tab, entry_off, x * DYN_COUL_TAB_SCALE);
 }
 
-// u = βr·DYN_COUL_TAB_SCALE in one product: the scale is a power of two, so
-// r·(β·scale) equals (r·β)·scale bit for bit.
+// An entry times a factor (β³ of the forces, β of the energies).
+DYN_HD float4 dyn_tab_scale(float4 c, float f) {
+  c.x *= f;
+  c.y *= f;
+  c.z *= f;
+  c.w *= f;
+  return c;
+}
+
+// f times the piece of ytab (DYN_COUL_Y_N entries, Ψ or Λ) at y ≥
+// DYN_COUL_Y_MIN; SCALED: the entries hold that factor already (the pair
+// kernel's copies in LDS).
+template <bool SCALED>
+DYN_HD float dyn_tab_y(const float4* ytab, float y, float f) {
+  const uint32_t lo = dyn_f2u(y) & 0xFFFE0000u;  // the interval's lower end
+  const float t = y - dyn_u2f(lo);
+  // the entry's byte offset (bits 17 to 26 as an index, times 16)
+#if defined(__HIP_DEVICE_COMPILE__)
+  // one instruction (lo's low 17 bits are clear; the compiler would shift y
+  // and mask the result instead)
+  uint32_t at;
+  asm("v_bfe_u32 %0, %1, 13, 14" : "=v"(at) : "v"(lo));
+#else
+  const uint32_t at = (lo >> 13) & (16u * (DYN_COUL_Y_N - 1));
+#endif
+  float4 c = *(const float4*)((const char*)ytab + at);
+  if (!SCALED) c = dyn_tab_scale(c, f);
+  return dyn_fmaf(dyn_fmaf(dyn_fmaf(c.w, t, c.z), t, c.y), t, c.x);
+}
+
+// r² below which a pair's y = r²β² may lie below the y tables (with room for
+// the product's rounding); never below the r² of coincident sites.
+DYN_HD float dyn_coul_r2_lo(float beta2) {
+  return dyn_maxf(1e-16f, 1.0001f * DYN_COUL_Y_MIN / beta2);
+}
+
+// The x tables' form, for pairs below the y tables.
+DYN_HD void dyn_coul_erfc_close(float r2, float qq, float beta, const float4* tab, float* s,
+                                float* e) {
+  const float rinv = dyn_rsqrtf(r2);
+  const float u = (r2 * rinv) * (beta * DYN_COUL_TAB_SCALE);
+  *s = qq * ((rinv * rinv) * rinv) * dyn_tab_cubic_u(tab, 0, u);
+  *e = qq * rinv * dyn_tab_cubic_u(tab, 1, u);
+}
+
+// The tabulated pair at any r² (both forms; rinv = 1/r is not needed).
 DYN_HD void dyn_coul_erfc_tab(float r2, float rinv, float qq, float beta, const float4* tab,
                               float* s, float* e) {
-  const float u = (r2 * rinv) * (beta * DYN_COUL_TAB_SCALE);
-  const float phi = dyn_tab_cubic_u(tab, 0, u);
-  *s = qq * ((rinv * rinv) * rinv) * phi;
-  *e = qq * rinv * dyn_tab_cubic_u(tab, 1, u);
+  const float beta2 = beta * beta;
+  (void)rinv;
+  if (!(r2 > dyn_coul_r2_lo(beta2))) {
+    dyn_coul_erfc_close(r2, qq, beta, tab, s, e);
+    return;
+  }
+  const float y = r2 * beta2;
+  *s = qq * dyn_tab_y<false>(tab + DYN_COUL_X_N, y, beta2 * beta);
+  *e = qq * dyn_tab_y<false>(tab + DYN_COUL_TAB_N + DYN_COUL_X_N, y, beta);
 }
 
 // The table (2·DYN_COUL_TAB_N float4 as 8·DYN_COUL_TAB_N floats), built on
 // the host in double from the closed forms (a host function).
 static inline void dyn_coul_tab_build(float* out) {
-  const double h = 1.0 / (double)DYN_COUL_TAB_SCALE;
   const double k2 = 1.1283791670955126;  // 2/√π
-  auto phi = [&](double x) { return erfc(x) + k2 * x * exp(-x * x); };
-  auto dphi = [&](double x) { return -2.0 * k2 * x * x * exp(-x * x); };
-  auto ef = [&](double x) { return erfc(x); };
-  auto def = [&](double x) { return -k2 * exp(-x * x); };
-  for (int i = 0; i < DYN_COUL_TAB_N; ++i) {
-    const double x0 = i * h, x1 = (i + 1) * h;
-    for (int which = 0; which < 2; ++which) {
-      const double f0 = which ? ef(x0) : phi(x0), f1 = which ? ef(x1) : phi(x1);
-      const double d0 = h * (which ? def(x0) : dphi(x0)), d1 = h * (which ? def(x1) : dphi(x1));
-      float* c = out + 4 * (which * DYN_COUL_TAB_N + i);
-      c[0] = (float)f0;
-      c[1] = (float)d0;
-      c[2] = (float)(3.0 * (f1 - f0) - 2.0 * d0 - d1);
-      c[3] = (float)(2.0 * (f0 - f1) + d0 + d1);
-    }
+  // the Hermite piece over an interval of width h, in t = argument − lower
+  // end times sc
+  auto piece = [](float* c, double f0, double f1, double d0, double d1, double h, double sc) {
+    d0 *= h;
+    d1 *= h;
+    c[0] = (float)f0;
+    c[1] = (float)(d0 * sc);
+    c[2] = (float)((3.0 * (f1 - f0) - 2.0 * d0 - d1) * sc * sc);
+    c[3] = (float)((2.0 * (f0 - f1) + d0 + d1) * sc * sc * sc);
+  };
+  // one erfc and one exponential a node: the two ends of neighbouring
+  // intervals are one node
+  struct Node { double f, df, e, de; };
+  auto node_x = [&](double x) {
+    const double er = erfc(x), ex = exp(-x * x);
+    return Node{er + k2 * x * ex, -2.0 * k2 * x * x * ex, er, -k2 * ex};
+  };
+  auto node_y = [&](double y) {
+    const double x = sqrt(y), er = erfc(x), ex = exp(-y);
+    const double psi = (er + k2 * x * ex) / (y * x);
+    return Node{psi, (-k2 * ex - 1.5 * psi) / y, er / x, -0.5 * psi};
+  };
+  auto put = [&](int at, const Node& a, const Node& b, double h, double sc) {
+    piece(out + 4 * at, a.f, b.f, a.df, b.df, h, sc);
+    piece(out + 4 * (DYN_COUL_TAB_N + at), a.e, b.e, a.de, b.de, h, sc);
+  };
+  const double h = 1.0 / (double)DYN_COUL_TAB_SCALE;
+  Node a = node_x(0.0);
+  for (int i = 0; i < DYN_COUL_X_N; ++i) {
+    const Node b = node_x((i + 1) * h);
+    put(i, a, b, h, 1.0);
+    a = b;
+  }
+  a = node_y((double)DYN_COUL_Y_MIN);
+  for (int k = 0; k < DYN_COUL_Y_N; ++k) {
+    // octave 0 starts at DYN_COUL_Y_MIN = 2⁻¹¹ (biased exponent 116)
+    const double lo = ldexp(1.0, k / 64 - 11), hy = lo / 64.0;
+    const Node b = node_y(lo + (k % 64 + 1) * hy);
+    put(DYN_COUL_X_N + ((((k / 64 + 116) & 15) << 6) | (k % 64)), a, b, hy, 1.0 / hy);
+    a = b;
   }
 }
 

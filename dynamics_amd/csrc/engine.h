@@ -70,52 +70,94 @@ struct DynPairParams {
   const float4* coul_tab;  // the erfc Coulomb table (dyn_coul_tab_build)
 };
 
-// One lane of an 8×8 tile: the pair (i, j) of the given kind.  Returns the
-// scalar s (F_i = s·d) and energies; s = e = 0 for an inactive lane.
-// `active` already includes the list mask; the cutoff test happens here.
+// The two Coulomb tables a lane reads (dyn_math.h): Ψ and Λ over y = β²r².
+// The pair kernel reads copies in LDS, multiplied by β³ and β (etab is not
+// read by a forces-only evaluation).
+struct DynCoulTabs {
+  const float4 *ftab, *etab;
+};
+DYN_HD DynCoulTabs dyn_coul_tabs(const float4* coul_tab) {
+  return DynCoulTabs{coul_tab + DYN_COUL_X_N, coul_tab + DYN_COUL_TAB_N + DYN_COUL_X_N};
+}
+
+// The pair (i, j) of the given kind at squared distance r2: the scalar s
+// (F_i = s·d) and energies, zero for an inactive lane.  `active` already
+// includes the list mask; the cutoff test happens here.  r2_lo =
+// dyn_coul_r2_lo(β²).  No square root or reciprocal of r² is taken for
+// Coulomb pairs (tabulated over β²r²); LJ takes 1/r² directly.  SCALED: tabs
+// holds the tables multiplied by β³ and β.  Returns whether the pair interacts but lies below
+// the Coulomb tables: then s and the energies are not set, and
+// dyn_tile_close gives them.
+template <int KIND, bool SCALED>
+DYN_HD bool dyn_tile_eval(float r2, float qi, float qj, float c6, float c12, bool active, float r2_lo,
+                          const DynPairParams& P, const DynCoulTabs& tabs, float* s_out, float* e_lj,
+                          float* e_c, int* hit) {
+  constexpr bool kLj = KIND == DYN_KIND_SS || KIND == DYN_KIND_SO || KIND == DYN_KIND_OO;
+  constexpr bool kCoul = KIND == DYN_KIND_SS || KIND == DYN_KIND_SQ || KIND == DYN_KIND_QQ;
+  // (no short-circuits: every lane takes the same path)
+  const bool near_ = active & (r2 < P.rc2);
+  const bool in = near_ & (r2 > (kCoul ? r2_lo : 1e-16f));
+  const bool lj_in = in & (r2 <= P.lj_rc2);
+  float s = 0.f, elj = 0.f, ec = 0.f;
+  if (kLj) dyn_lj(dyn_rcpf(r2), c6, c12, &s, &elj);
+  if (kCoul) {
+    const float y = r2 * P.beta2;
+    const float qq = qi * qj;
+    const float sc = qq * dyn_tab_y<SCALED>(tabs.ftab, y, P.beta2 * P.beta);
+    ec = qq * dyn_tab_y<SCALED>(tabs.etab, y, P.beta);
+    s = kLj ? (r2 <= P.lj_rc2 ? sc + s : sc) : sc;
+    *s_out = in ? s : 0.f;
+    *e_lj = kLj && lj_in ? elj : 0.f;
+    *e_c = in ? ec : 0.f;
+  } else {
+    *s_out = lj_in ? s : 0.f;
+    *e_lj = lj_in ? elj : 0.f;
+    *e_c = 0.f;
+  }
+  *hit = in ? 1 : 0;
+  return kCoul && (near_ & !in);
+}
+
+// A pair dyn_tile_eval returned true for (sites that coincide do not
+// interact).
+template <int KIND>
+DYN_HD void dyn_tile_close(float r2, float qi, float qj, float c6, float c12, const DynPairParams& P,
+                           float* s_out, float* e_lj, float* e_c, int* hit) {
+  *s_out = *e_lj = *e_c = 0.f;
+  *hit = r2 > 1e-16f ? 1 : 0;
+  if (!*hit) return;
+  dyn_coul_erfc_close(r2, qi * qj, P.beta, P.coul_tab, s_out, e_c);
+  if (KIND == DYN_KIND_SS && r2 <= P.lj_rc2) {
+    float sl;
+    dyn_lj(dyn_rcpf(r2), c6, c12, &sl, e_lj);
+    *s_out = *s_out + sl;
+  }
+}
+
+// (c6, c12) of a pair of the given kind.
+template <int KIND>
+DYN_HD float2 dyn_tile_c(int ti, int tj, const DynPairParams& P, const float2* lj_table) {
+  float2 c;
+  c.x = P.c6_oo;
+  c.y = P.c12_oo;
+  if (KIND == DYN_KIND_SS || KIND == DYN_KIND_SO)
+    c = lj_table[(ti & DYN_TYPE_MASK) * P.n_types + (tj & DYN_TYPE_MASK)];
+  return c;
+}
+
+// One lane of an 8×8 tile from the two sites: displacement d (minimum
+// image), scalar s, energies, squared distance (0 for an inactive lane).
 template <int KIND>
 DYN_HD void dyn_tile_pair(const float pi[4], int ti, const float pj[4], int tj, bool active,
                           const DynPairParams& P, const float2* lj_table, float d[3],
                           float* s_out, float* e_lj, float* e_c, float* r2_out, int* hit) {
-  float d0 = pi[0] - pj[0], d1 = pi[1] - pj[1], d2 = pi[2] - pj[2];
-  d0 = dyn_min_image_rint(d0, P.ext[0], P.inv_ext[0]);
-  d1 = dyn_min_image_rint(d1, P.ext[1], P.inv_ext[1]);
-  d2 = dyn_min_image_rint(d2, P.ext[2], P.inv_ext[2]);
-  d[0] = d0;
-  d[1] = d1;
-  d[2] = d2;
-  const float r2 = dyn_fmaf(d2, d2, dyn_fmaf(d1, d1, d0 * d0));
-  const bool in = active && r2 < P.rc2 && r2 > 1e-16f;
-  const float r2s = in ? r2 : 1.0f;
-  const float rinv = dyn_rsqrtf(r2s);
-  float s = 0.f, elj = 0.f, ec = 0.f;
-  if (KIND == DYN_KIND_SS || KIND == DYN_KIND_SO || KIND == DYN_KIND_OO) {
-    float c6, c12;
-    if (KIND == DYN_KIND_OO) {
-      c6 = P.c6_oo;
-      c12 = P.c12_oo;
-    } else {
-      const float2 c = lj_table[(ti & DYN_TYPE_MASK) * P.n_types + (tj & DYN_TYPE_MASK)];
-      c6 = c.x;
-      c12 = c.y;
-    }
-    float sl, el;
-    dyn_lj(rinv * rinv, c6, c12, &sl, &el);
-    const bool lj_in = in && r2 <= P.lj_rc2;
-    s = lj_in ? sl : 0.f;
-    elj = lj_in ? el : 0.f;
-  }
-  if (KIND == DYN_KIND_SS || KIND == DYN_KIND_SQ || KIND == DYN_KIND_QQ) {
-    float sc, ee;
-    dyn_coul_erfc_tab(r2s, rinv, pi[3] * pj[3], P.beta, P.coul_tab, &sc, &ee);
-    s = KIND == DYN_KIND_SS ? s + (in ? sc : 0.f) : (in ? sc : 0.f);
-    ec = in ? ee : 0.f;
-  }
-  *s_out = s;
-  *e_lj = elj;
-  *e_c = ec;
-  *r2_out = in ? r2 : 0.f;
-  *hit = in ? 1 : 0;
+  for (int a = 0; a < 3; ++a) d[a] = dyn_min_image_rint(pi[a] - pj[a], P.ext[a], P.inv_ext[a]);
+  const float r2 = dyn_fmaf(d[2], d[2], dyn_fmaf(d[1], d[1], d[0] * d[0]));
+  const float2 c = dyn_tile_c<KIND>(ti, tj, P, lj_table);
+  if (dyn_tile_eval<KIND, false>(r2, pi[3], pj[3], c.x, c.y, active, dyn_coul_r2_lo(P.beta2), P,
+                                 dyn_coul_tabs(P.coul_tab), s_out, e_lj, e_c, hit))
+    dyn_tile_close<KIND>(r2, pi[3], pj[3], c.x, c.y, P, s_out, e_lj, e_c, hit);
+  *r2_out = *hit ? r2 : 0.f;
 }
 
 // FP64 variant for the precision sweep: the same interactions from the same
@@ -163,21 +205,14 @@ DYN_HD void dyn_tile_pair_f64(const float pi[4], int ti, const float pj[4], int 
   *hit = in ? 1 : 0;
 }
 
-// Alchemical variant (src/cuda/cuda.cu:367-566): a lane whose two sites lie
-// on different sides of the decoupled molecule (exactly one carries
-// DYN_TYPE_ALCH) takes Beutler soft-core LJ at the schedule's LJ λ and
-// Coulomb scaled by the schedule's factor, and returns dH/dλ; every other
-// lane returns dyn_tile_pair's result bit for bit.  lj_se holds the
+// Alchemical pair (src/cuda/cuda.cu:367-566) within the cutoff: two sites on
+// different sides of the decoupled molecule (exactly one carries
+// DYN_TYPE_ALCH) take Beutler soft-core LJ at the schedule's LJ λ and Coulomb
+// scaled by the schedule's factor, and return dH/dλ.  lj_se holds the
 // combined (σ, ε) of each type pair.
 template <int KIND>
-DYN_HD void dyn_tile_pair_alch(const float pi[4], int ti, const float pj[4], int tj, bool active,
-                               const DynPairParams& P, const float2* lj_table,
-                               const float2* lj_se, float d[3], float* s_out, float* e_lj,
-                               float* e_c, float* r2_out, int* hit, float* dh) {
-  dyn_tile_pair<KIND>(pi, ti, pj, tj, active, P, lj_table, d, s_out, e_lj, e_c, r2_out, hit);
-  *dh = 0.f;
-  if (((ti ^ tj) & DYN_TYPE_ALCH) == 0 || !*hit) return;
-  const float r2 = *r2_out;
+DYN_HD void dyn_tile_alch(float r2, float qi, float qj, int ti, int tj, const DynPairParams& P,
+                          const float2* lj_se, float* s_out, float* e_lj, float* e_c, float* dh) {
   const float rinv = dyn_rsqrtf(r2);
   float s = 0.f, elj = 0.f, ec = 0.f, dhh = 0.f;
   if (KIND == DYN_KIND_SS || KIND == DYN_KIND_SO) {
@@ -192,7 +227,7 @@ DYN_HD void dyn_tile_pair_alch(const float pi[4], int ti, const float pj[4], int
   }
   if (KIND == DYN_KIND_SS || KIND == DYN_KIND_SQ) {
     float sc, ee;
-    dyn_coul_erfc(r2, rinv, pi[3] * pj[3], P.beta, P.beta2, P.two_b_sqrtpi, &sc, &ee);
+    dyn_coul_erfc(r2, rinv, qi * qj, P.beta, P.beta2, P.two_b_sqrtpi, &sc, &ee);
     s = s + sc * P.sch.coulomb_scale;
     ec = ee * P.sch.coulomb_scale;
     dhh = dhh + ee * P.sch.coulomb_dscale_dlambda;
@@ -201,4 +236,17 @@ DYN_HD void dyn_tile_pair_alch(const float pi[4], int ti, const float pj[4], int
   *e_lj = elj;
   *e_c = ec;
   *dh = dhh;
+}
+
+// dyn_tile_pair with alchemical pairs (every other lane returns
+// dyn_tile_pair's result bit for bit).
+template <int KIND>
+DYN_HD void dyn_tile_pair_alch(const float pi[4], int ti, const float pj[4], int tj, bool active,
+                               const DynPairParams& P, const float2* lj_table,
+                               const float2* lj_se, float d[3], float* s_out, float* e_lj,
+                               float* e_c, float* r2_out, int* hit, float* dh) {
+  dyn_tile_pair<KIND>(pi, ti, pj, tj, active, P, lj_table, d, s_out, e_lj, e_c, r2_out, hit);
+  *dh = 0.f;
+  if (((ti ^ tj) & DYN_TYPE_ALCH) != 0 && *hit)
+    dyn_tile_alch<KIND>(*r2_out, pi[3], pj[3], ti, tj, P, lj_se, s_out, e_lj, e_c, dh);
 }

@@ -10,13 +10,14 @@
 //              are cut into work items of ≤ item_groups groups; solute–solute
 //              entries get exclusion masks                            (rebuild)
 //   slots      gather current positions into cluster slots       (reuse path)
-//   pairs      8×8 wave tiles over the work items: LJ + erfc Coulomb; each
-//              lane keeps its i-site force in registers and a work item
-//              stores its 8 i-site forces once: no atomics, no j-side sums
+//   pairs      8×8 wave tiles, a workgroup per row, a wave per work item:
+//              LJ + erfc Coulomb; each lane keeps its i-site force in
+//              registers and the row stores its 8 i-site forces once: no
+//              atomics, no j-side sums
 //   corr       1-4 pairs (scaled real space) and reciprocal corrections
 //   pme        spread → FFT → convolve → inverse FFT → gather
-//   finalize   site forces + the work-item rows of each site's slot →
-//              site-order fixed-point forces; fixed-order energy sums
+//   finalize   corrections + pair forces + SPME forces → site-order
+//              fixed-point forces; fixed-order energy sums
 // Capacities are checked on the device; an overflow sets a status bit that
 // the host reads at the next synchronization and reports as an error, after
 // growing the buffers for the next call.
@@ -50,7 +51,8 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kPairBlock = 256;       // 4 waves, one work item each at a time
-constexpr uint64_t kPairGridCap = 6144;  // ~4 × the pair kernel's resident workgroups
+constexpr uint64_t kPairAhead = 16;   // groups of a list the pair kernel may read past its end
+constexpr uint32_t kPairGridCap = 6144;  // a few times the pair kernel's resident workgroups
 constexpr int kColCap = 4096;         // sites per column (LDS sort)
 constexpr int kMaxColsPerClass = 4096;
 constexpr int kNumPart = 9;           // f64 partials per work item of the pair kernel
@@ -933,31 +935,33 @@ struct PairArgs {
   const int32_t* slot_type;
   const int32_t* slot_gid;
   const uint8_t* cl_class;
+  const uint32_t* n_cl;      // rows
   const uint32_t* row_ptr;   // groups
+  const uint32_t* chunk_ptr; // work items
   const uint32_t* cj;        // 8 entries per group (copy 0; cj2: copy 1)
   const unsigned long long* cmask;
-  const uint2* chunks;
   const uint32_t* cj2;
   const unsigned long long* cmask2;
-  const uint2* chunks2;
   const unsigned int* fl;    // the engine's flags: the copy in use, the largest displacement
   int staged;                // staged list builds: a stale current list voids the evaluation
   unsigned int hard_limit;   // half the list buffer, squared (float bits)
-  const uint32_t* n_chunks;
+  const float4* coul_y;      // the Coulomb tables over y, times β³ (Ψ) and β (Λ)
   const float2* lj_table;    // (c6, c12) per type pair
   const float2* lj_se;       // (σ, ε) per type pair, for soft-core
   const double2* lj_table64; // (c6, c12) in double, for the FP64 option
   int64_t* mol_e;            // n_mol² molecule-pair energies (fixed point), or null
   const int32_t* mol_of;     // per solute atom: its molecule
   uint32_t n_mol;
+  uint32_t null_slot;        // the padding j slot
   int64_t* fitem;            // per work item: 3 components × 8 i slots, fixed point
   const int32_t* slot_site;  // per slot: its site (−1: padding)
-  int64_t* fx_site;          // site forces (fixed point, component-major): the i forces are added
+  int64_t* fx_pair;          // pair force of every site (fixed point, component-major): written
   uint32_t n_sites;
   uint32_t keep_items;       // write each item's row of i forces to fitem (for inspection)
   double* partials;          // kNumPart values × cap_chunks (value-major), per work item
   uint64_t cap_chunks;
   uint32_t chunk;            // j groups per work item
+  uint32_t unused;           // no implicit padding: argument packs are compared byte for byte
   unsigned int* status;      // a list-build overflow leaves the list unusable
 };
 
@@ -969,6 +973,11 @@ struct TileAccT {
   T fi[3];
   T e_lj_s, e_lj_w, e_c_s, e_c_w, vir, dh;
   uint32_t n_ss, n_lj, n_c;  // wave-uniform counts (popcounts)
+  __device__ __forceinline__ void clear() {
+    fi[0] = fi[1] = fi[2] = T(0);
+    e_lj_s = e_lj_w = e_c_s = e_c_w = vir = dh = T(0);
+    n_ss = n_lj = n_c = 0;
+  }
 };
 
 __device__ __forceinline__ void wave_add_fx(int64_t* __restrict__ M, int key, double e);
@@ -1010,31 +1019,12 @@ __device__ __forceinline__ void wave_add_fx(int64_t* __restrict__ M, int key, do
   }
 }
 
-// ALCH: the group holds at least one lane across the decoupled molecule's
-// boundary (the alchemical variant returns the plain result on the others).
-// ENERGY: accumulate energies, virial, dH/dλ and pair counts (forces only
+// Adds one evaluated tile lane (scalar s, displacement d, energies) to the
+// wave's sums.  ENERGY: energies, virial and pair counts too (forces only
 // otherwise).
-// F64: FP64 pair arithmetic (precision sweep; no alchemical groups).
-template <int KIND, bool ALCH, bool ENERGY, bool F64>
-__device__ __forceinline__ void tile_entry(const PairArgs& A, const float pi[4], int ti,
-                                           const float4& pjv, int tj, bool active,
-                                           TileAccT<std::conditional_t<F64, double, float>>& T,
-                                           int gi, int gj) {
-  using R = std::conditional_t<F64, double, float>;
-  const float pj[4] = {pjv.x, pjv.y, pjv.z, pjv.w};
-  R d[3], s, elj, ec, r2;
-  int hit;
-  if constexpr (F64) {
-    dyn_tile_pair_f64<KIND>(pi, ti, pj, tj, active, A.P, A.lj_table64, d, &s, &elj, &ec, &r2, &hit);
-  } else if constexpr (ALCH) {
-    float dh;
-    dyn_tile_pair_alch<KIND>(pi, ti, pj, tj, active, A.P, A.lj_table, A.lj_se, d, &s, &elj, &ec,
-                             &r2, &hit, &dh);
-    if (ENERGY) T.dh += dh;
-  } else {
-    dyn_tile_pair<KIND>(pi, ti, pj, tj, active, A.P, A.lj_table, d, &s, &elj, &ec, &r2, &hit);
-  }
-  if constexpr (F64) {
+template <int KIND, bool ENERGY, class R>
+__device__ __forceinline__ void tile_add(TileAccT<R>& T, R s, const R d[3], R elj, R ec, R r2, int hit) {
+  if constexpr (std::is_same<R, double>::value) {
     T.fi[0] += s * d[0];
     T.fi[1] += s * d[1];
     T.fi[2] += s * d[2];
@@ -1054,39 +1044,498 @@ __device__ __forceinline__ void tile_entry(const PairArgs& A, const float pi[4],
     else T.e_c_w += ec;
   }
   T.vir += s * r2;
-  if constexpr (KIND == DYN_KIND_SS)
-    if (A.mol_e) mol_energy_add(A.mol_e, A.mol_of, A.n_mol, gi, gj, (double)elj + (double)ec);
-  const uint32_t h = (uint32_t)__popcll(__ballot(hit != 0));
+  const uint32_t h = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(hit != 0));
   if (KIND == DYN_KIND_SS) T.n_ss += h;
   else if (KIND == DYN_KIND_SO || KIND == DYN_KIND_OO) T.n_lj += h;
   else T.n_c += h;
 }
 
-// LDS of the FP32 pair kernel: the erfc Coulomb table, then the LJ
-// (c6, c12) table of n_types² entries.  Per-lane table reads from LDS are
-// counted apart from the global loads, so the j data prefetched for the next
-// group stays in flight while a group reads its table values (a global table
-// read would make the wave wait for every load issued before it).
-constexpr size_t kPairTabEntries = 2 * DYN_COUL_TAB_N;  // float4
-__host__ __device__ constexpr size_t pair_lds_bytes(int n_types, bool energy) {
-  return (energy ? kPairTabEntries : DYN_COUL_TAB_N) * 16 + (size_t)n_types * (size_t)n_types * 8;
+// The i side of a row, one lane (ia, jb) of a wave.
+struct TileI {
+  float p[4];     // position and charge (a padding slot's x is −kFarX)
+  float r2_lo;
+  int t, g, ci;
+  bool pad;
+  bool any_in, any_out;  // i sites within and outside the decoupled molecule
+};
+
+// How a lane finds the image of its j site.
+//   kImgNone   the wrapped coordinates differ by no box length
+//   kImgShift  by the same multiples for every i slot (taken off per j)
+//   kImgLane   each pair its own minimum image (small boxes, rows across the
+//              box boundary)
+// The displacement is the same to the bit in all three: pi − pj rounded
+// once, then the exact multiple of the box length taken off.
+enum { kImgNone = 0, kImgShift = 1, kImgLane = 2 };
+constexpr float kFarX = 1e18f;  // x of a slot that pairs with nothing (its square stays finite)
+
+// The lanes where p holds (of a compare: no copy of it into a register, as
+// __ballot makes).
+__device__ __forceinline__ unsigned long long lanes(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// Lane `K` of each quad's value, in the quad's four lanes.
+template <int K>
+__device__ __forceinline__ int quad_lane(int v) {
+  return __builtin_amdgcn_mov_dpp(v, K * 0x55, 0xf, 0xf, true);
+}
+template <int K>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(quad_lane<K>(__float_as_int(v)));
 }
 
-// One wave per work item at a time (≤ A.chunk groups of one row); lane
-// ia + 8·jb holds the pair (i slot 8I+ia, j entry jb of the group).  The next
-// group's j data is loaded before the current group is evaluated.  A work
-// item stores its 8 i-slot forces in its own row of fitem (no atomics) and
-// its energies, virial and pair counts as one partial per value, so every
-// sum keeps a fixed order whichever wave runs the item; the grid holds a few
-// times as many workgroups as fit on the device at once, each copying the
-// tables to LDS once and taking items in a grid stride, so the hardware's
-// workgroup dispatch still balances the load.
-template <bool ENERGY, bool F64>
+// The j side of up to four groups: lane (quad, K) holds the quad's entry of
+// group K.
+struct TileJ {
+  float4 p;
+  float sx, sy, sz;  // box lengths between the image seen from the row and p (kImgShift)
+  int t, g;
+};
+
+// dyn_tile_eval for a lane of the fast path, which knows that no pair it
+// keeps lies below the Coulomb tables (tile_quad): r2 is at least rc² for a
+// pair that does not interact.
+template <int KIND>
+__device__ __forceinline__ bool tile_fast(float r2, float qi, float qj, const float2& c,
+                                          const DynPairParams& P, const DynCoulTabs& tabs, float* s_out,
+                                          float* e_lj, float* e_c) {
+  constexpr bool kLj = KIND == DYN_KIND_SS || KIND == DYN_KIND_SO || KIND == DYN_KIND_OO;
+  constexpr bool kCoul = KIND == DYN_KIND_SS || KIND == DYN_KIND_SQ || KIND == DYN_KIND_QQ;
+  const bool in = kCoul ? r2 < P.rc2 : (r2 < P.rc2) & (r2 > 1e-16f);
+  const bool lj_in = in & (r2 <= P.lj_rc2);
+  float s = 0.f, elj = 0.f, ec = 0.f;
+  if (kLj) dyn_lj(dyn_rcpf(r2), c.x, c.y, &s, &elj);
+  if (kCoul) {
+    const float y = r2 * P.beta2, qq = qi * qj;
+    const float sc = qq * dyn_tab_y<true>(tabs.ftab, y, 0.f);
+    ec = qq * dyn_tab_y<true>(tabs.etab, y, 0.f);
+    s = kLj ? (r2 <= P.lj_rc2 ? sc + s : sc) : sc;
+  }
+  *s_out = (kCoul ? in : lj_in) ? s : 0.f;
+  *e_lj = kLj && lj_in ? elj : 0.f;
+  *e_c = kCoul && in ? ec : 0.f;
+  return in;
+}
+
+// Group K of the batch (its j entry is lane K's of each quad; g: its index):
+// one pair per lane.  close: the smallest r² of a Coulomb pair met (at or
+// below I.r2_lo, the pair lies below the tables and what was added is not
+// its force).
+template <int KIND, bool ENERGY, int IMG, int K>
+__device__ __forceinline__ void tile_quad(const PairArgs& A, const TileI& I, const TileJ& J, uint32_t g,
+                                          const DynCoulTabs& tabs, const float2* ljt,
+                                          TileAccT<float>& T, float& close) {
+  constexpr bool kCoul = KIND == DYN_KIND_SS || KIND == DYN_KIND_SQ || KIND == DYN_KIND_QQ;
+  const float jx = quad_lane<K>(J.p.x);
+  float d[3] = {I.p[0] - jx, I.p[1] - quad_lane<K>(J.p.y), I.p[2] - quad_lane<K>(J.p.z)};
+  if (IMG == kImgShift) {
+    d[0] -= quad_lane<K>(J.sx);
+    d[1] -= quad_lane<K>(J.sy);
+    d[2] -= quad_lane<K>(J.sz);
+  } else if (IMG == kImgLane) {
+    for (int a = 0; a < 3; ++a) d[a] = dyn_min_image_rint(d[a], A.P.ext[a], A.P.inv_ext[a]);
+  }
+  float r2 = dyn_fmaf(d[2], d[2], dyn_fmaf(d[1], d[1], d[0] * d[0]));
+  // sites of one water, a solute site with itself (an O with itself: r² = 0),
+  // a listed exclusion, and for kImgLane the slots that pair with nothing
+  // (their far x may come out near by a minimum image)
+  bool off = false;
+  if (KIND == DYN_KIND_QQ || KIND == DYN_KIND_SS) off = I.g == quad_lane<K>(J.g);
+  if (IMG == kImgLane) off = off | I.pad | (jx > 0.5f * kFarX);
+  if (KIND == DYN_KIND_SS) off = off | __builtin_amdgcn_inverse_ballot_w64(~A.cmask[g]);
+  if (off) r2 = kFarX;
+  const int tj = KIND == DYN_KIND_SS || KIND == DYN_KIND_SO ? quad_lane<K>(J.t) : 0;
+  const float2 c = dyn_tile_c<KIND>(I.t, tj, A.P, ljt);
+  if (kCoul) close = fminf(close, r2);
+  float s, elj, ec;
+  const bool hit = tile_fast<KIND>(r2, I.p[3], quad_lane<K>(J.p.w), c, A.P, tabs, &s, &elj, &ec);
+  tile_add<KIND, ENERGY, float>(T, s, d, elj, ec, hit ? r2 : 0.f, hit);
+}
+
+// Four groups of one kind, from group g (a group past the item's last holds
+// far j sites).
+template <int KIND, bool ENERGY, int IMG>
+__device__ __forceinline__ void tile_batch(const PairArgs& A, const TileI& I, const TileJ& J, uint32_t g,
+                                           const DynCoulTabs& tabs, const float2* ljt,
+                                           TileAccT<float>& T, float& close) {
+  tile_quad<KIND, ENERGY, IMG, 0>(A, I, J, g, tabs, ljt, T, close);
+  tile_quad<KIND, ENERGY, IMG, 1>(A, I, J, g + 1, tabs, ljt, T, close);
+  // two groups' values live at a time: registers for more resident waves
+  __builtin_amdgcn_sched_barrier(0);
+  tile_quad<KIND, ENERGY, IMG, 2>(A, I, J, g + 2, tabs, ljt, T, close);
+  tile_quad<KIND, ENERGY, IMG, 3>(A, I, J, g + 3, tabs, ljt, T, close);
+}
+
+// Group K of a batch of two classes.
+template <bool ENERGY, int K>
+__device__ __forceinline__ void tile_mixed(int ci, uint32_t v, const PairArgs& A, const TileI& I,
+                                           const TileJ& J, uint32_t g, const DynCoulTabs& tabs,
+                                           const float2* ljt, TileAccT<float>& T, float& close) {
+  // (readlane returns a signed int: class 2 sets the top bit)
+  switch (dyn_kind(ci, (int)((uint32_t)__builtin_amdgcn_readlane(v, K) >> DYN_JCLS_SHIFT))) {
+    case DYN_KIND_QQ: tile_quad<DYN_KIND_QQ, ENERGY, kImgLane, K>(A, I, J, g + K, tabs, ljt, T, close); break;
+    case DYN_KIND_OO: tile_quad<DYN_KIND_OO, ENERGY, kImgLane, K>(A, I, J, g + K, tabs, ljt, T, close); break;
+    case DYN_KIND_SS: tile_quad<DYN_KIND_SS, ENERGY, kImgLane, K>(A, I, J, g + K, tabs, ljt, T, close); break;
+    case DYN_KIND_SO: tile_quad<DYN_KIND_SO, ENERGY, kImgLane, K>(A, I, J, g + K, tabs, ljt, T, close); break;
+    case DYN_KIND_SQ: tile_quad<DYN_KIND_SQ, ENERGY, kImgLane, K>(A, I, J, g + K, tabs, ljt, T, close); break;
+    default: break;
+  }
+}
+
+// Whether the pairs of a row within the cutoff see every j site in one image
+// whichever i slot they belong to (ok), and whether that image is always the
+// wrapped coordinates themselves (in).  lo, hi: the range of the i
+// slots' wrapped coordinates.  A pair within rc in another image than the one
+// nearest the range's middle would need rc + half the range ≥ half the box;
+// every other image of a pair is at least half a box length away, beyond the
+// cutoff like the minimum image of a pair outside it.
+struct RowImage {
+  float c[3];  // the middle, in box lengths
+  bool ok, in;
+};
+// Smallest and largest of the 8 i slots' coordinates (wrapped: not negative,
+// so ordered like their bit patterns).
+template <bool MAX>
+__device__ __forceinline__ uint32_t ext8(uint32_t v) {
+  auto f = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
+  v = f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true));
+  v = f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true));
+  return f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, true));
+}
+__device__ __forceinline__ RowImage row_image(const DynPairParams& P, const float4& p) {
+  RowImage r;
+  const float rc = __builtin_amdgcn_sqrtf(P.rc2) * 1.0001f + 1e-3f;
+  const float x[3] = {p.x, p.y, p.z};
+  bool ok = true, in = true;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const uint32_t u = __float_as_uint(x[a]);
+    const float lo = __uint_as_float(ext8<false>(u)), hi = __uint_as_float(ext8<true>(u));
+    r.c[a] = 0.5f * (lo + hi) * P.inv_ext[a];
+    ok = ok & (rc + 0.5f * (hi - lo) < 0.4999f * P.ext[a]);
+    in = in & (lo > rc) & (hi + rc < P.ext[a]);
+  }
+  // the same in every lane
+  r.ok = __builtin_amdgcn_ballot_w64(ok) != 0ull;
+  r.in = __builtin_amdgcn_ballot_w64(in) != 0ull;
+  return r;
+}
+
+// Value at byte offset `at` of an array (a 32-bit offset beside a uniform
+// base: one address instruction per load).
+template <class T>
+__device__ __forceinline__ const T& at_bytes(const T* __restrict__ base, uint32_t at) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + at);
+}
+
+// A wave's place in an item of a row: the batch from group g (v: the lane's
+// entry, J: its j site), the entries of the next batch and their byte offset.
+struct TileCur {
+  uint32_t g, at, v, vn;
+  TileJ J;
+};
+constexpr uint32_t kBatchBytes = 4u * 4u * DYN_CL_SIZE;
+
+// The j site of entry v: position and charge, LJ type (TYPE), exclusion
+// group (GID).
+template <bool TYPE, bool GID>
+__device__ __forceinline__ void load_j(const PairArgs& A, uint32_t v, TileJ& J) {
+  const uint32_t js = v & DYN_JSLOT_MASK;
+  J.p = at_bytes(A.xyzq, js * 16u);
+  if (TYPE) J.t = at_bytes(A.slot_type, js * 4u);
+  if (GID) J.g = at_bytes(A.slot_gid, js * 4u);
+}
+
+// Class of the batch's last entry (of `left` groups to the item's end).
+__device__ __forceinline__ uint32_t last_class(uint32_t v, uint32_t left) {
+  // (readlane returns a signed int: class 2 sets the top bit)
+  return (uint32_t)__builtin_amdgcn_readlane(v, min(left, 4u) - 1u) >> DYN_JCLS_SHIFT;
+}
+
+// Whether any pair of the row's i slots and the batch's j sites crosses the
+// decoupled molecule's boundary (a lane holds one of its quad's four j sites).
+__device__ __forceinline__ bool tile_crosses(const TileI& I, const TileJ& J, bool far) {
+  const bool in = (J.t & DYN_TYPE_ALCH) != 0;
+  return (I.any_out & (lanes(!far & in) != 0ull)) | (I.any_in & (lanes(!far & !in) != 0ull));
+}
+
+// The batches of one class (cls) from C on, to the item's end (g1), the first
+// batch that reaches another class or (ALCH) the first with an alchemical
+// pair.
+template <int KIND, bool ENERGY, bool ALCH>
+__device__ __forceinline__ void tile_run(const PairArgs& A, const TileI& I, const RowImage& Im,
+                                         const uint32_t* __restrict__ row, uint32_t g1, uint32_t cls,
+                                         const DynCoulTabs& tabs, const float2* ljt, TileCur& C,
+                                         TileAccT<float>& T, float& close) {
+  constexpr bool kAlch = ALCH && KIND <= DYN_KIND_SQ;
+  constexpr bool kType = KIND == DYN_KIND_SS || KIND == DYN_KIND_SO || kAlch;
+  constexpr bool kGid = KIND == DYN_KIND_SS || KIND == DYN_KIND_QQ;
+  const uint32_t pq = threadIdx.x & 3u;
+  do {
+    const uint32_t left = (uint32_t)__builtin_amdgcn_readfirstlane(g1 - C.g);
+    if (last_class(C.v, left) != cls) return;
+    bool far = (C.v & DYN_JSLOT_MASK) == A.null_slot;
+    if (left < 4u) far = far | (pq >= left);
+    if (kAlch && tile_crosses(I, C.J, far)) return;
+    const uint32_t g = C.g;
+    TileJ J = C.J;
+    C.v = C.vn;
+    load_j<kType, kGid>(A, C.v, C.J);
+    C.at += kBatchBytes;
+    C.vn = at_bytes(row, C.at);
+    C.g += 4;
+    if (Im.ok) {
+      bool shift = false;
+      if (!Im.in) {
+        J.sx = dyn_rintf(dyn_fmaf(-J.p.x, A.P.inv_ext[0], Im.c[0])) * A.P.ext[0];
+        J.sy = dyn_rintf(dyn_fmaf(-J.p.y, A.P.inv_ext[1], Im.c[1])) * A.P.ext[1];
+        J.sz = dyn_rintf(dyn_fmaf(-J.p.z, A.P.inv_ext[2], Im.c[2])) * A.P.ext[2];
+        shift = lanes(fmaxf(fmaxf(fabsf(J.sx), fabsf(J.sy)), fabsf(J.sz)) != 0.f) != 0ull;
+      }
+      if (far) J.p.x = kFarX;
+      if (shift) tile_batch<KIND, ENERGY, kImgShift>(A, I, J, g, tabs, ljt, T, close);
+      else tile_batch<KIND, ENERGY, kImgNone>(A, I, J, g, tabs, ljt, T, close);
+    } else {
+      if (far) J.p.x = kFarX;
+      tile_batch<KIND, ENERGY, kImgLane>(A, I, J, g, tabs, ljt, T, close);
+    }
+  } while (C.g < g1);
+}
+
+// One group (g) with everything a lane may need: each pair's own minimum
+// image, alchemical pairs, pairs below the Coulomb tables, molecule-pair
+// energies.
+template <int KIND, bool ENERGY, bool ALCH>
+__device__ __forceinline__ void tile_any(const PairArgs& A, const TileI& I, const TileJ& J, uint32_t g,
+                                         const DynCoulTabs& tabs, const float2* ljt, TileAccT<float>& T) {
+  bool active = dyn_slot_pair_valid(I.g, J.g);
+  if (KIND == DYN_KIND_SS) active = active & __builtin_amdgcn_inverse_ballot_w64(A.cmask[g]);
+  float d[3] = {I.p[0] - J.p.x, I.p[1] - J.p.y, I.p[2] - J.p.z};
+  for (int a = 0; a < 3; ++a) d[a] = dyn_min_image_rint(d[a], A.P.ext[a], A.P.inv_ext[a]);
+  const float r2 = dyn_fmaf(d[2], d[2], dyn_fmaf(d[1], d[1], d[0] * d[0]));
+  const float2 c = dyn_tile_c<KIND>(I.t, J.t, A.P, ljt);
+  float s, elj, ec, dh = 0.f;
+  int hit;
+  if (dyn_tile_eval<KIND, true>(r2, I.p[3], J.p.w, c.x, c.y, active, I.r2_lo, A.P, tabs, &s, &elj, &ec, &hit))
+    dyn_tile_close<KIND>(r2, I.p[3], J.p.w, c.x, c.y, A.P, &s, &elj, &ec, &hit);
+  if (ALCH && KIND <= DYN_KIND_SQ) {
+    if (((I.t ^ J.t) & DYN_TYPE_ALCH) != 0 && hit)
+      dyn_tile_alch<KIND>(r2, I.p[3], J.p.w, I.t, J.t, A.P, A.lj_se, &s, &elj, &ec, &dh);
+    if (ENERGY) T.dh += dh;
+  }
+  if constexpr (ENERGY && KIND == DYN_KIND_SS)
+    if (A.mol_e) mol_energy_add(A.mol_e, A.mol_of, A.n_mol, I.g, J.g, (double)elj + (double)ec);
+  tile_add<KIND, ENERGY, float>(T, s, d, elj, ec, hit ? r2 : 0.f, hit);
+}
+
+// n ≤ 4 groups from group g, one after another, by tile_any (v, Q: the lane's
+// entry and its j site).
+template <bool ENERGY, bool ALCH>
+__device__ __forceinline__ void tile_batch_any(const PairArgs& A, const TileI& I, uint32_t v, const TileJ& Q,
+                                               uint32_t g, uint32_t n, const DynCoulTabs& tabs,
+                                               const float2* ljt, TileAccT<float>& T) {
+  const int quad = (int)(threadIdx.x & (kWave - 1u) & ~3u);
+  for (uint32_t k = 0; k < n; ++k, ++g) {
+    const int src = quad | (int)k;
+    TileJ J;
+    J.p.x = __shfl(Q.p.x, src, kWave);
+    J.p.y = __shfl(Q.p.y, src, kWave);
+    J.p.z = __shfl(Q.p.z, src, kWave);
+    J.p.w = __shfl(Q.p.w, src, kWave);
+    J.t = __shfl(Q.t, src, kWave);
+    J.g = __shfl(Q.g, src, kWave);
+    // (readlane returns a signed int: class 2 sets the top bit)
+    switch (dyn_kind(I.ci, (int)((uint32_t)__builtin_amdgcn_readlane(v, k) >> DYN_JCLS_SHIFT))) {
+      case DYN_KIND_QQ: tile_any<DYN_KIND_QQ, ENERGY, ALCH>(A, I, J, g, tabs, ljt, T); break;
+      case DYN_KIND_OO: tile_any<DYN_KIND_OO, ENERGY, ALCH>(A, I, J, g, tabs, ljt, T); break;
+      case DYN_KIND_SS: tile_any<DYN_KIND_SS, ENERGY, ALCH>(A, I, J, g, tabs, ljt, T); break;
+      case DYN_KIND_SO: tile_any<DYN_KIND_SO, ENERGY, ALCH>(A, I, J, g, tabs, ljt, T); break;
+      case DYN_KIND_SQ: tile_any<DYN_KIND_SQ, ENERGY, ALCH>(A, I, J, g, tabs, ljt, T); break;
+      default: break;
+    }
+  }
+}
+
+// The j groups [g0, g1) of a row in FP32.  A batch is four groups: the lane
+// with position p in its quad loads the entry of group p (both quads of a jb
+// hold the same four entries), and group K's data reach a quad's lanes by
+// DPP as an operand of the instruction that uses them.  Loads and the
+// image shift are then paid once per four groups, where a lane per pair
+// that loads its own j entry pays 4 loads and 9 instructions of minimum
+// image per group (the kernel is bound by VALU issue, see k_eng_pairs).
+// Batches of one class run in a loop of their own kind (the entries of a row
+// are ordered by class).  While a batch is evaluated, the j data of the next
+// and the entries of the one after are in flight; the entries past the
+// item's end are read (the next row's, or kPairAhead spare ones) and not
+// used.  any: every batch by the general path, tile_batch_any, which
+// otherwise takes those with alchemical pairs.  Returns false when a pair
+// below the Coulomb tables was met: T is then not the item's sum.
+template <bool ENERGY, bool ALCH>
+__device__ __forceinline__ bool tile_item(const PairArgs& A, const TileI& I, const RowImage& Im, bool any,
+                                          uint32_t g0, uint32_t g1, const DynCoulTabs& tabs,
+                                          const float2* ljt, TileAccT<float>& T) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const uint32_t* __restrict__ row = A.cj + (size_t)g0 * DYN_CL_SIZE;
+  TileCur C;
+  C.g = g0;
+  C.at = 4u * (DYN_CL_SIZE * (lane & 3u) + (lane >> 3));  // this lane's entry of a batch, in bytes
+  C.v = at_bytes(row, C.at);
+  C.at += kBatchBytes;
+  C.vn = at_bytes(row, C.at);
+  C.J.sx = C.J.sy = C.J.sz = 0.f;
+  float close = kFarX;
+  do {
+    load_j<true, true>(A, C.v, C.J);
+    const uint32_t left = (uint32_t)__builtin_amdgcn_readfirstlane(g1 - C.g);
+    const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane(C.v) >> DYN_JCLS_SHIFT;
+    const bool far = ((C.v & DYN_JSLOT_MASK) == A.null_slot) | ((lane & 3u) >= left);
+    const bool gen = any || (ALCH && tile_crosses(I, C.J, far));
+    if (!gen && last_class(C.v, left) == c0) {
+      switch (dyn_kind(I.ci, (int)c0)) {
+        case DYN_KIND_QQ: tile_run<DYN_KIND_QQ, ENERGY, ALCH>(A, I, Im, row, g1, c0, tabs, ljt, C, T, close); break;
+        case DYN_KIND_OO: tile_run<DYN_KIND_OO, ENERGY, ALCH>(A, I, Im, row, g1, c0, tabs, ljt, C, T, close); break;
+        case DYN_KIND_SS: tile_run<DYN_KIND_SS, ENERGY, ALCH>(A, I, Im, row, g1, c0, tabs, ljt, C, T, close); break;
+        case DYN_KIND_SO: tile_run<DYN_KIND_SO, ENERGY, ALCH>(A, I, Im, row, g1, c0, tabs, ljt, C, T, close); break;
+        case DYN_KIND_SQ: tile_run<DYN_KIND_SQ, ENERGY, ALCH>(A, I, Im, row, g1, c0, tabs, ljt, C, T, close); break;
+        default: return true;  // never listed
+      }
+      continue;
+    }
+    if (gen) {
+      tile_batch_any<ENERGY, ALCH>(A, I, C.v, C.J, C.g, min(left, 4u), tabs, ljt, T);
+    } else {
+      TileJ J = C.J;
+      if (far) J.p.x = kFarX;
+      tile_mixed<ENERGY, 0>(I.ci, C.v, A, I, J, C.g, tabs, ljt, T, close);
+      tile_mixed<ENERGY, 1>(I.ci, C.v, A, I, J, C.g, tabs, ljt, T, close);
+      if (left > 2u) tile_mixed<ENERGY, 2>(I.ci, C.v, A, I, J, C.g, tabs, ljt, T, close);
+      if (left > 3u) tile_mixed<ENERGY, 3>(I.ci, C.v, A, I, J, C.g, tabs, ljt, T, close);
+    }
+    C.v = C.vn;
+    C.at += kBatchBytes;
+    C.vn = at_bytes(row, C.at);
+    C.g += 4;
+  } while (C.g < g1);
+  return lanes(close <= I.r2_lo) == 0ull;
+}
+
+// The j groups [g0, g1) of a row with FP64 pair arithmetic (the precision
+// option): a lane loads its own j entry.
+template <int KIND, bool ENERGY>
+__device__ __forceinline__ void tile_entry64(const PairArgs& A, const TileI& I, const float4& pjv, int tj,
+                                             int gj, bool active, TileAccT<double>& T) {
+  const float pj[4] = {pjv.x, pjv.y, pjv.z, pjv.w};
+  double d[3], s, elj, ec, r2;
+  int hit;
+  dyn_tile_pair_f64<KIND>(I.p, I.t, pj, tj, active, A.P, A.lj_table64, d, &s, &elj, &ec, &r2, &hit);
+  if constexpr (ENERGY && KIND == DYN_KIND_SS)
+    if (A.mol_e) mol_energy_add(A.mol_e, A.mol_of, A.n_mol, I.g, gj, elj + ec);
+  tile_add<KIND, ENERGY, double>(T, s, d, elj, ec, r2, hit);
+}
+template <bool ENERGY>
+__device__ __forceinline__ void tile_item64(const PairArgs& A, const TileI& I, uint32_t g0, uint32_t g1,
+                                            TileAccT<double>& T) {
+  const int lane = threadIdx.x & (kWave - 1);
+  for (uint32_t g = g0; g < g1; ++g) {
+    const uint32_t v = A.cj[(size_t)g * DYN_CL_SIZE + (lane >> 3)];
+    const uint32_t js = v & DYN_JSLOT_MASK;
+    const float4 pj = A.xyzq[js];
+    const int tj = A.slot_type[js], gj = A.slot_gid[js];
+    // readfirstlane returns a signed int: shift the entry as unsigned (class
+    // 2 sets the top bit)
+    const int kind = dyn_kind(I.ci, (int)((uint32_t)__builtin_amdgcn_readfirstlane(v) >> DYN_JCLS_SHIFT));
+    bool active = dyn_slot_pair_valid(I.g, gj);
+    if (kind == DYN_KIND_SS) active = active && ((A.cmask[g] >> lane) & 1ull);
+    switch (kind) {
+      case DYN_KIND_QQ: tile_entry64<DYN_KIND_QQ, ENERGY>(A, I, pj, tj, gj, active, T); break;
+      case DYN_KIND_OO: tile_entry64<DYN_KIND_OO, ENERGY>(A, I, pj, tj, gj, active, T); break;
+      case DYN_KIND_SS: tile_entry64<DYN_KIND_SS, ENERGY>(A, I, pj, tj, gj, active, T); break;
+      case DYN_KIND_SO: tile_entry64<DYN_KIND_SO, ENERGY>(A, I, pj, tj, gj, active, T); break;
+      case DYN_KIND_SQ: tile_entry64<DYN_KIND_SQ, ENERGY>(A, I, pj, tj, gj, active, T); break;
+      default: break;
+    }
+  }
+}
+
+// Sum over the 8 j lanes of each i slot (lanes ia, ia+8, …, ia+56), in every
+// lane: the xor-8, xor-16, xor-32 tree, by a rotation within rows of 16 lanes
+// and the swaps of row and half-wave pairs.
+__device__ __forceinline__ float sum_jb(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));  // row_ror:8
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ double sum_jb(double v) {
+  v = xor_sum_d(v, 8);
+  v = xor_sum_d(v, 16);
+  return xor_sum_d(v, 32);
+}
+
+// Exchanges a double's halves as permlane swaps do: swap32_sum returns a's
+// sum over lanes l and l ± 32 in the lower half-wave and b's in the upper,
+// swap16_sum a's over two neighbouring rows of 16 lanes in the even row and b's in
+// the odd one.
+__device__ __forceinline__ double swap32_sum(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)__double2loint(a), (uint32_t)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double swap16_sum(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(a), (uint32_t)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// Sum over each row of 16 lanes, in every lane of the row.
+__device__ __forceinline__ double row_sum(double v) {
+  auto ror = [](double x, auto ctrl) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(x), decltype(ctrl)::value, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(x), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v += ror(v, std::integral_constant<int, 0x128>{});
+  v += ror(v, std::integral_constant<int, 0x124>{});
+  v += ror(v, std::integral_constant<int, 0x122>{});
+  return v + ror(v, std::integral_constant<int, 0x121>{});
+}
+
+// A workgroup per row (i cluster) at a time, a wave per work item (≤ A.chunk
+// groups of the row); lane ia + 8·jb holds the pair (i slot 8I+ia, j entry jb
+// of a group).
+//
+// Bound: VALU issue (85% of the cycles at 252,480 sites, 33 instructions a
+// group of 64 pairs in the forces variant; LDS and memory stay below half of
+// theirs).  So what a pair does was cut to the least: the Coulomb force is
+// one table value over β²r² (no square root, no reciprocal), 1/r² of LJ an
+// integer guess and a Newton step, minimum images are taken per j site of a
+// batch instead of per pair, and the j site reaches the lanes as DPP operands
+// (tile_item).  Per-lane table reads from LDS are counted apart from the global
+// loads, so the j data prefetched for the next batch stay in flight while a
+// batch reads its table values.  The row's items are all in one workgroup, so
+// the i forces are summed through LDS and stored once by site, with no
+// atomics.  A work item writes its energies, virial and pair counts as one
+// partial per value, so every sum keeps a fixed order whichever wave runs the
+// item.  The grid holds a few times as many workgroups as fit on the device at
+// once, each copying the tables to LDS once and taking rows in a grid stride,
+// so the hardware's workgroup dispatch still balances the load.
+//
+// One lane a pair with its own loads, a wave per item and atomic force sums
+// took, at 252,480 sites, 395 µs per MD evaluation (median; now 285), 310 with
+// energies (259); 28,000 sites 55 (42) and 54 (54); a batch of 32 boxes 259
+// (186); 16 alchemical windows 340 (329).
+template <bool ENERGY, bool F64, bool ALCH>
 __device__ __forceinline__ void
 k_eng_pairs(PairArgs A) {
   using R = std::conditional_t<F64, double, float>;
+  // the Coulomb tables over y (β³Ψ, and βΛ with energies; at offset 0, so a
+  // lane's table address is its entry's offset) and the row's forces (two
+  // buffers); in FP32 the LJ (c6, c12) table of n_types² entries follows
+  constexpr int kTab = F64 ? 1 : (ENERGY ? 2 : 1) * DYN_COUL_Y_N;
+  __shared__ float4 s_tab[kTab];
+  __shared__ int64_t s_f[2][kPairBlock / kWave][3 * DYN_CL_SIZE];
+  extern __shared__ float2 s_lj[];
   const int lane = threadIdx.x & (kWave - 1);
   const int ia = lane & 7, jb = lane >> 3;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   if (*A.status) return;
   // in staged mode a site may have moved half the list buffer since the
   // current list's build: the list may then miss pairs, and the evaluation
@@ -1098,132 +1547,111 @@ k_eng_pairs(PairArgs A) {
   if ((A.fl[kFlSel] ^ A.fl[kFlCommit]) != 0u) {
     A.cj = A.cj2;
     A.cmask = A.cmask2;
-    A.chunks = A.chunks2;
   }
+  const uint32_t n_cl = *A.n_cl;
+  if (blockIdx.x >= n_cl) return;
+  DynCoulTabs tabs = {nullptr, nullptr};
+  const float2* ljt = nullptr;
   if constexpr (!F64) {
-    extern __shared__ float4 pair_lds[];
-    float4* tab = pair_lds;
-    float2* ljt = reinterpret_cast<float2*>(pair_lds + (ENERGY ? kPairTabEntries : DYN_COUL_TAB_N));
+    for (int k = threadIdx.x; k < kTab; k += kPairBlock) s_tab[k] = A.coul_y[k];
     const int nt2 = A.P.n_types * A.P.n_types;
-    // forces only: the φ half of the Coulomb table (the erfc half serves energies)
-    const int ntab = ENERGY ? (int)kPairTabEntries : DYN_COUL_TAB_N;
-    for (int k = threadIdx.x; k < ntab; k += kPairBlock) tab[k] = A.P.coul_tab[k];
-    for (int k = threadIdx.x; k < nt2; k += kPairBlock) ljt[k] = A.lj_table[k];
+    for (int k = threadIdx.x; k < nt2; k += kPairBlock) s_lj[k] = A.lj_table[k];
     __syncthreads();
-    A.P.coul_tab = tab;
-    A.lj_table = ljt;
+    tabs.ftab = s_tab;
+    tabs.etab = s_tab + (ENERGY ? DYN_COUL_Y_N : 0);
+    ljt = s_lj;
   }
-  const uint32_t n_items = (uint32_t)min((uint64_t)*A.n_chunks, A.cap_chunks);
-  const uint32_t wave0 = blockIdx.x * (kPairBlock / kWave) + (threadIdx.x / kWave);
-  const uint32_t nwaves = gridDim.x * (kPairBlock / kWave);
-  for (uint32_t item = wave0; item < n_items; item += nwaves) {
-    const uint2 ch = A.chunks[item];
-    const uint32_t I = __builtin_amdgcn_readfirstlane(ch.x);
-    const uint32_t g0 = __builtin_amdgcn_readfirstlane(ch.y);
-    const uint32_t g1 = min(g0 + A.chunk, A.row_ptr[I + 1]);
-    const float4 piv = A.xyzq[I * DYN_CL_SIZE + ia];
-    const float pi[4] = {piv.x, piv.y, piv.z, piv.w};
-    const int ti = A.slot_type[I * DYN_CL_SIZE + ia];
-    const int gi = A.slot_gid[I * DYN_CL_SIZE + ia];
-    const int ci = A.cl_class[I];
-    TileAccT<R> T;
-    T.fi[0] = T.fi[1] = T.fi[2] = R(0);
-    T.e_lj_s = T.e_lj_w = T.e_c_s = T.e_c_w = T.vir = T.dh = R(0);
-    T.n_ss = T.n_lj = T.n_c = 0;
-    // two-deep software pipeline: while group g is evaluated, the j data of
-    // group g + 1 and the entry of group g + 2 are in flight.  The loads are
-    // issued on every iteration (the last ones repeat the row's last group)
-    // so the wait counts stay exact.
-    const uint32_t glast = g1 - 1;
-    uint32_t v = A.cj[(size_t)g0 * DYN_CL_SIZE + jb];
-    uint32_t vn = A.cj[(size_t)min(g0 + 1, glast) * DYN_CL_SIZE + jb];
-    float4 pj = A.xyzq[v & DYN_JSLOT_MASK];
-    int tj = A.slot_type[v & DYN_JSLOT_MASK];
-    int gj = A.slot_gid[v & DYN_JSLOT_MASK];
-    for (uint32_t g = g0; g < g1; ++g) {
-      // readfirstlane returns a signed int: shift the entry as unsigned (class
-      // 2 sets the top bit)
-      const int cls = (int)((uint32_t)__builtin_amdgcn_readfirstlane(v) >> DYN_JCLS_SHIFT);
-      const float4 pjc = pj;
-      const int tjc = tj, gjc = gj;
-      {
-        const uint32_t jsn = vn & DYN_JSLOT_MASK;
-        pj = A.xyzq[jsn];
-        tj = A.slot_type[jsn];
-        gj = A.slot_gid[jsn];
-        v = vn;
-        vn = A.cj[(size_t)min(g + 2, glast) * DYN_CL_SIZE + jb];
+  int buf = 0;
+  for (uint32_t row = blockIdx.x; row < n_cl; row += gridDim.x, buf ^= 1) {
+    const uint32_t r0 = A.row_ptr[row], r1 = A.row_ptr[row + 1];
+    const float4 piv = A.xyzq[row * DYN_CL_SIZE + ia];
+    TileI I;
+    I.p[0] = piv.x;
+    I.p[1] = piv.y;
+    I.p[2] = piv.z;
+    I.p[3] = piv.w;
+    I.r2_lo = dyn_coul_r2_lo(A.P.beta2);
+    I.t = A.slot_type[row * DYN_CL_SIZE + ia];
+    I.g = A.slot_gid[row * DYN_CL_SIZE + ia];
+    I.ci = A.cl_class[row];
+    I.pad = I.g == DYN_GID_PAD;
+    I.any_in = ALCH && lanes(!I.pad & ((I.t & DYN_TYPE_ALCH) != 0)) != 0ull;
+    I.any_out = ALCH && lanes(!I.pad & ((I.t & DYN_TYPE_ALCH) == 0)) != 0ull;
+    int64_t acc[3] = {0, 0, 0};
+    uint32_t it = w, g0 = r0 + w * A.chunk;
+    RowImage Im;
+    if constexpr (!F64)
+      if (g0 < r1) {
+        Im = row_image(A.P, piv);
+        if (I.pad) I.p[0] = -kFarX;
       }
-      const int kind = dyn_kind(ci, cls);
-      bool active = dyn_slot_pair_valid(gi, gjc);
-      if (kind == DYN_KIND_SS) active = active && ((A.cmask[g] >> lane) & 1ull);
-      const bool alch = !F64 && A.P.alch_on && kind <= DYN_KIND_SQ &&
-                        __ballot(((ti ^ tjc) & DYN_TYPE_ALCH) != 0) != 0ull;
-      switch (kind) {
-        case DYN_KIND_QQ: tile_entry<DYN_KIND_QQ, false, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc); break;
-        case DYN_KIND_OO: tile_entry<DYN_KIND_OO, false, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc); break;
-        case DYN_KIND_SS:
-          if (alch) tile_entry<DYN_KIND_SS, true, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc);
-          else tile_entry<DYN_KIND_SS, false, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc);
-          break;
-        case DYN_KIND_SO:
-          if (alch) tile_entry<DYN_KIND_SO, true, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc);
-          else tile_entry<DYN_KIND_SO, false, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc);
-          break;
-        case DYN_KIND_SQ:
-          if (alch) tile_entry<DYN_KIND_SQ, true, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc);
-          else tile_entry<DYN_KIND_SQ, false, ENERGY, F64>(A, pi, ti, pjc, tjc, active, T, gi, gjc);
-          break;
-        default: break;
-      }
-    }
-    // i forces: sum over the 8 j lanes of each i slot (lanes ia, ia+8, …, ia+56)
-    for (int c = 0; c < 3; ++c) {
-      R f = T.fi[c];
+    for (; g0 < r1; it += kPairBlock / kWave, g0 += kPairBlock / kWave * A.chunk) {
+      const uint32_t g1 = min(g0 + A.chunk, r1);
+      TileAccT<R> T;
+      T.clear();
       if constexpr (F64) {
-        f = xor_sum_d(f, 8);
-        f = xor_sum_d(f, 16);
-        f = xor_sum_d(f, 32);
+        tile_item64<ENERGY>(A, I, g0, g1, T);
       } else {
-        f = xor_sum(f, 8);
-        f = xor_sum(f, 16);
-        f = xor_sum(f, 32);
+        // molecule-pair energies are added by the general path only
+        bool any = ENERGY && A.mol_e && I.ci == DYN_CLS_SOLUTE;
+        while (!tile_item<ENERGY, ALCH>(A, I, Im, any, g0, g1, tabs, ljt, T)) {
+          any = true;  // (and then it returns true)
+          T.clear();
+        }
       }
-      T.fi[c] = f;
-    }
-    if (jb == 0) {
-      // the i forces in fixed point, added to the sites' sums (integer sums:
-      // the order of the items does not change them) and, for inspection,
-      // kept as the item's row
-      int64_t* o = A.fitem + (size_t)item * (3 * DYN_CL_SIZE);
-      int64_t q[3];
+      for (int c = 0; c < 3; ++c) T.fi[c] = sum_jb(T.fi[c]);
+      const size_t item = (size_t)A.chunk_ptr[row] + it;
       for (int c = 0; c < 3; ++c) {
-        if constexpr (F64) q[c] = dyn_fx64(T.fi[c]);
-        else q[c] = dyn_fx(T.fi[c]);
-        if (A.keep_items) o[c * DYN_CL_SIZE + ia] = q[c];
+        int64_t q;
+        if constexpr (F64) q = dyn_fx64(T.fi[c]);
+        else q = dyn_fx(T.fi[c]);
+        acc[c] += q;
+        if (A.keep_items && jb == 0) A.fitem[item * (3 * DYN_CL_SIZE) + c * DYN_CL_SIZE + ia] = q;
       }
-      const int32_t site = A.slot_site[I * DYN_CL_SIZE + ia];
-      if (site >= 0)
-        for (int c = 0; c < 3; ++c)
-          atomicAdd(reinterpret_cast<unsigned long long*>(A.fx_site + (size_t)c * A.n_sites + site),
-                    (unsigned long long)q[c]);
+      if (!ENERGY) continue;
+      // six sums over the wave at the cost of two: a swap of half-waves
+      // leaves one value in each half, a swap of rows one in each row of 16
+      const double a0 = swap32_sum((double)T.e_lj_w, (double)T.e_c_w);
+      const double a1 = swap32_sum((double)T.e_lj_s, (double)T.e_c_s);
+      const double a2 = swap32_sum((double)T.vir, (double)T.dh);
+      const double b0 = row_sum(swap16_sum(a0, a1)), b1 = row_sum(swap16_sum(a2, a2));
+      double* const out = A.partials + item;
+      // rows of b0: LJ water, LJ solute, Coulomb water, Coulomb solute; of
+      // b1: virial, virial, dH/dλ, dH/dλ
+      if ((lane & 15) == 0) out[(size_t)(lane >> 4) * A.cap_chunks] = b0;
+      if ((lane & 31) == 1) out[(size_t)(lane == 1 ? 4 : 8) * A.cap_chunks] = b1;
+      if (lane < 3) out[(size_t)(5 + lane) * A.cap_chunks] = (double)(lane == 0 ? T.n_ss : lane == 1 ? T.n_lj : T.n_c);
     }
-    if (!ENERGY) continue;
-    double acc[6] = {T.e_lj_w, T.e_lj_s, T.e_c_w, T.e_c_s, T.vir, T.dh};
-    for (int k = 0; k < 6; ++k) {
-      double x = acc[k];
-      for (int m = 1; m < kWave; m <<= 1) x = xor_sum_d(x, m);
-      acc[k] = x;
-    }
-    if (lane == 0) {
-      for (int k = 0; k < 5; ++k) A.partials[(size_t)k * A.cap_chunks + item] = acc[k];
-      A.partials[(size_t)5 * A.cap_chunks + item] = (double)T.n_ss;
-      A.partials[(size_t)6 * A.cap_chunks + item] = (double)T.n_lj;
-      A.partials[(size_t)7 * A.cap_chunks + item] = (double)T.n_c;
-      A.partials[(size_t)8 * A.cap_chunks + item] = acc[5];
+    // the row's forces: the waves' sums (integers: the order of the items
+    // does not change them), stored by site.  Two buffers: the next row's
+    // sums are written while this row's are read.
+    if (jb == 0)
+      for (int c = 0; c < 3; ++c) s_f[buf][w][c * DYN_CL_SIZE + ia] = acc[c];
+    __syncthreads();
+    if (threadIdx.x < 3 * DYN_CL_SIZE) {
+      int64_t f = 0;
+      for (int k = 0; k < kPairBlock / kWave; ++k) f += s_f[buf][k][threadIdx.x];
+      const int32_t site = A.slot_site[row * DYN_CL_SIZE + (threadIdx.x & (DYN_CL_SIZE - 1))];
+      if (site >= 0) A.fx_pair[(size_t)(threadIdx.x / DYN_CL_SIZE) * A.n_sites + site] = f;
     }
   }
 }
+
+}  // namespace
+
+// Registers for five resident waves per SIMD for forces and four with
+// energies.  Forces at 252,480 sites, 3 to 8 waves asked for: 5 was the
+// fastest (6 spills: 3% slower; 4: 4%); energies 4 (5 spills: 6% slower).
+template <>
+struct dyn::MinWavesPerSimd<k_eng_pairs<false, false, false>> {
+  static constexpr int value = 5;
+};
+template <>
+struct dyn::MinWavesPerSimd<k_eng_pairs<true, false, false>> {
+  static constexpr int value = 4;
+};
+
+namespace {
 
 // Correction pairs: kind 1 = 1-4 pair (scaled real-space LJ + Coulomb, plus
 // the reciprocal correction of the mode), kind 0 = excluded pair (standard
@@ -1541,30 +1969,14 @@ __device__ __forceinline__ void k_eng_prep(PrepArgs A) {
 
 
 // Site-order forces: the site accumulators (corrections), the SPME forces
-// (this evaluation's or the kept ones of an earlier one) and the pair
-// kernel's work-item rows of the site's slot (when the pair kernel ran).
-__device__ __forceinline__ void k_eng_finalize(const int64_t* __restrict__ fx_site,
-                               const int64_t* __restrict__ fx_recip,
-                               const int64_t* __restrict__ fitem,
-                               const uint32_t* __restrict__ chunk_ptr, uint64_t cap_chunks,
-                               const uint32_t* __restrict__ slot_of, uint32_t n_sites,
-                               uint32_t n_slots, int64_t* __restrict__ out,
-                               unsigned int* __restrict__ fl, int forced) {
+// (this evaluation's or the kept ones of an earlier one) and the pair forces.
+__device__ __forceinline__ void k_eng_finalize(ForceParts P, int64_t* __restrict__ out) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s == 0) evaluation_flags_end(fl, forced);
-  if (s >= n_sites) return;
-  ForceParts P;
-  P.fx_site = fx_site;
-  P.fx_recip = fx_recip;
-  P.fitem = fitem;
-  P.chunk_ptr = chunk_ptr;
-  P.slot_of = slot_of;
-  P.cap_chunks = cap_chunks;
-  P.n_sites = n_sites;
-  P.n_slots = n_slots;
+  if (s == 0) evaluation_flags_end(P.fl, P.forced);
+  if (s >= P.n_sites) return;
   int64_t f[3];
   site_force_sum(P, s, f);
-  for (int c = 0; c < 3; ++c) out[(size_t)c * n_sites + s] = f[c];
+  for (int c = 0; c < 3; ++c) out[(size_t)c * P.n_sites + s] = f[c];
 }
 
 // Slot-order pair forces (component-major), for inspection.
@@ -1676,7 +2088,8 @@ struct dyn_engine {
   DevBuf<float2> lj_table;   // (c6, c12) per type pair
   DevBuf<float2> lj_se;      // (σ, ε) per type pair (soft-core)
   DevBuf<double2> lj_table64;  // (c6, c12) in double (FP64 pair option)
-  DevBuf<float4> coul_tab;     // erfc Coulomb table of the pair kernel (dyn_coul_tab_build)
+  DevBuf<float4> coul_tab;     // erfc Coulomb tables (dyn_coul_tab_build), then those over y
+                               // times β³ and β (the pair kernel's LDS copies)
   std::vector<int32_t> h_type;  // per-site type words (host copy)
   // decoupled molecule: solute sites [alch0, alch1), λ
   uint32_t alch0 = 0, alch1 = 0;
@@ -1747,7 +2160,7 @@ struct dyn_engine {
   // device flags (kFlWords words, kFl* indices)
   DevBuf<unsigned int> dflags;
   // accumulators
-  DevBuf<int64_t> fitem, fx_site, fx_out, fx_slot;  // fx_slot: inspection only
+  DevBuf<int64_t> fitem, fx_site, fx_pair, fx_out, fx_slot;  // fx_slot: inspection only
   DevBuf<double> pair_part, corr_part, eng_out, red1;
   unsigned corr_blocks = 0;
   // a pass over this engine alone: argument packs of both streams
@@ -1929,10 +2342,14 @@ void dyn_engine::reserve_rows(uint32_t entries) {
 // List capacity in groups of 8 j entries, and work items.
 void dyn_engine::reserve_list(uint64_t groups, uint64_t n_items) {
   if (groups > cap_entries) {
-    cj.reserve(groups * DYN_CL_SIZE);
-    cmask.reserve(groups);
-    cj2.reserve(groups * DYN_CL_SIZE);
-    cmask2.reserve(groups);
+    // the pair kernel reads ahead past a row's end (kPairAhead groups past
+    // the last row's): every entry of the buffers names a slot
+    for (DevBuf<uint32_t>* b : {&cj, &cj2}) {
+      b->reserve((groups + kPairAhead) * DYN_CL_SIZE);
+      DYN_HIP(hipMemsetAsync(b->p, 0, sizeof(uint32_t) * (groups + kPairAhead) * DYN_CL_SIZE, stream));
+    }
+    for (DevBuf<unsigned long long>* b : {&cmask, &cmask2}) b->reserve(groups + kPairAhead);
+    DYN_HIP(hipStreamSynchronize(stream));
     cap_entries = groups;
   }
   if (n_items > cap_chunks) {
@@ -2324,26 +2741,27 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
       A.slot_type = e.slot_type.p;
       A.slot_gid = e.slot_gid.p;
       A.cl_class = e.cl_class.p;
+      A.n_cl = e.counters.p + 0;
       A.row_ptr = e.row_ptr.p;
+      A.chunk_ptr = e.chunk_ptr.p;
       A.cj = e.cj.p;
       A.cmask = e.cmask.p;
-      A.chunks = e.chunks.p;
       A.cj2 = e.cj2.p;
       A.cmask2 = e.cmask2.p;
-      A.chunks2 = e.chunks2.p;
       A.fl = e.dflags.p;
       A.staged = staged_mode && !forced[i] ? 1 : 0;
       A.hard_limit = build_limit(e);
-      A.n_chunks = e.counters.p + 2;
+      A.coul_y = e.coul_tab.p + 2 * DYN_COUL_TAB_N;
       A.lj_table = e.lj_table.p;
       A.lj_se = e.lj_se.p;
       A.lj_table64 = e.lj_table64.p;
       A.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
       A.mol_of = e.mol_of.p;
       A.n_mol = e.n_mol;
+      A.null_slot = e.cap_slots;
       A.fitem = e.fitem.p;
       A.slot_site = e.slot_site.p;
-      A.fx_site = e.fx_site.p;
+      A.fx_pair = e.fx_pair.p;
       A.n_sites = e.n_sites;
       // a fused evaluation's caller reads site sums only
       A.keep_items = (flags & kComputeFusedFinalize) ? 0u : 1u;
@@ -2352,29 +2770,33 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
       A.chunk = e.prm.item_groups;
       A.status = e.status.p;
     }
-    // a wave per work item, up to kPairGridCap workgroups (the item count is
-    // known on the device only; the waves take items in a grid stride)
+    // a workgroup per row, up to kPairGridCap workgroups (the row count is
+    // known on the device only; the workgroups take rows in a grid stride)
     const unsigned gp = max_grid(S, [](dyn_engine& e) {
-      return (unsigned)std::min<uint64_t>(kPairGridCap, std::max<uint64_t>(1, (e.cap_chunks + 3) / 4));
+      return std::min<uint32_t>(kPairGridCap, std::max(1u, e.cap_cl));
     });
     // FP64 pair arithmetic when the first system asks for it (a set shares it)
     const bool f64 = (E[0]->prm.precision & DYN_PREC_PAIR_F64) != 0;
     int nt_max = 0;
     for (dyn_engine* e : E) nt_max = std::max(nt_max, e->n_types);
-    const size_t shm = pair_lds_bytes(nt_max, energy_on);
-    auto pa = [&](uint32_t i) { return PA[i]; };
-    if (energy_on && !f64)
-      launch<k_eng_pairs<true, false>, kPairBlock>(R, "k_eng_pairs<true>", 0, gp, kPairBlock, shm,
-          [&](uint32_t i) { return args<k_eng_pairs<true, false>>(pa(i)); });
-    else if (!f64)
-      launch<k_eng_pairs<false, false>, kPairBlock>(R, "k_eng_pairs<false>", 0, gp, kPairBlock, shm,
-          [&](uint32_t i) { return args<k_eng_pairs<false, false>>(pa(i)); });
-    else if (energy_on)
-      launch<k_eng_pairs<true, true>, kPairBlock>(R, "k_eng_pairs<true, f64>", 0, gp, kPairBlock, 0,
-          [&](uint32_t i) { return args<k_eng_pairs<true, true>>(pa(i)); });
-    else
-      launch<k_eng_pairs<false, true>, kPairBlock>(R, "k_eng_pairs<false, f64>", 0, gp, kPairBlock, 0,
-          [&](uint32_t i) { return args<k_eng_pairs<false, true>>(pa(i)); });
+    const size_t shm = f64 ? 0 : sizeof(float2) * (size_t)nt_max * (size_t)nt_max;  // the LJ table
+    // alchemical pairs exist in a system of the set
+    bool alch = false;
+    for (uint32_t i = 0; i < ns; ++i) alch = alch || PL[i].alch_on;
+    auto go = [&](auto F, const char* name) {
+      launch<decltype(F)::value, kPairBlock>(R, name, 0, gp, kPairBlock, shm, [&](uint32_t i) {
+        return args<decltype(F)::value>(PA[i]);
+      });
+    };
+#define DYN_PAIRS(E, F64, ALCH) \
+  std::integral_constant<decltype(&k_eng_pairs<E, F64, ALCH>), &k_eng_pairs<E, F64, ALCH>> {}
+    if (f64 && energy_on) go(DYN_PAIRS(true, true, false), "k_eng_pairs<true, f64>");
+    else if (f64) go(DYN_PAIRS(false, true, false), "k_eng_pairs<false, f64>");
+    else if (alch && energy_on) go(DYN_PAIRS(true, false, true), "k_eng_pairs<true, alch>");
+    else if (alch) go(DYN_PAIRS(false, false, true), "k_eng_pairs<false, alch>");
+    else if (energy_on) go(DYN_PAIRS(true, false, false), "k_eng_pairs<true>");
+    else go(DYN_PAIRS(false, false, false), "k_eng_pairs<false>");
+#undef DYN_PAIRS
   }
   if (any_staged && one_stream) set_build_lists(S, R, sgate, true);
   stream_order(RS.stream, R.stream, S.ev_join);
@@ -2386,12 +2808,8 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
     std::memset(&P, 0, sizeof P);
     P.fx_site = e.fx_site.p;
     P.fx_recip = (pl.recip_on || pl.reuse) ? e.fx_recip.p : nullptr;
-    P.fitem = nullptr;  // the pair kernel adds its i forces to fx_site
-    P.chunk_ptr = e.chunk_ptr.p;
-    P.slot_of = e.slot_of.p;
-    P.cap_chunks = e.cap_chunks;
+    P.fx_pair = short_on ? e.fx_pair.p : nullptr;
     P.n_sites = e.n_sites;
-    P.n_slots = e.cap_slots;
     P.fl = e.dflags.p;
     P.forced = forced[i] ? 1 : 0;
     e.fx_stale = fused;
@@ -2400,13 +2818,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
     Profiler::Scope ps(prof, "finalize");
     const unsigned gs = max_grid(S, [](dyn_engine& e) { return grid_for(e.n_sites, 256); });
     if (!fused) launch<k_eng_finalize>(R, "k_eng_finalize", 0, gs, 256, 0, [&](uint32_t i) {
-      dyn_engine& e = *E[i];
-      const Plan& pl = PL[i];
-      return args<k_eng_finalize>(e.fx_site.p,
-                                  (pl.recip_on || pl.reuse) ? e.fx_recip.p : (const int64_t*)nullptr,
-                                  (const int64_t*)nullptr, e.chunk_ptr.p,
-                                  e.cap_chunks, e.slot_of.p, e.n_sites, e.cap_slots, e.fx_out.p,
-                                  e.dflags.p, forced[i] ? 1 : 0);
+      return args<k_eng_finalize>(E[i]->parts, E[i]->fx_out.p);
     });
     if (short_on && energy_on)
       launch<k_eng_energy_reduce1, kRed1Block>(R, "k_eng_energy_reduce1", 0, kRed1Grid, kRed1Block,
@@ -2688,6 +3100,7 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->stg_wpos_ref.reserve(ns);
     E->stg_slot_of.reserve(ns);
     E->fx_site.reserve(3 * (size_t)ns);
+    E->fx_pair.reserve(3 * (size_t)ns);
     E->fx_out.reserve(3 * (size_t)ns);
     E->fx_recip.reserve(3 * (size_t)ns);
     E->h_fx.reserve(3 * (size_t)ns);
@@ -2700,10 +3113,16 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->status.reserve(1);
     E->dflags.reserve(kFlWords);
     {
-      std::vector<float> tab(8 * DYN_COUL_TAB_N);
-      dyn_coul_tab_build(tab.data());
-      E->coul_tab.reserve(2 * DYN_COUL_TAB_N);
-      DYN_HIP(hipMemcpyAsync(E->coul_tab.p, tab.data(), sizeof(float) * tab.size(),
+      std::vector<float4> tab(2 * DYN_COUL_TAB_N + 2 * DYN_COUL_Y_N);
+      dyn_coul_tab_build(reinterpret_cast<float*>(tab.data()));
+      const DynCoulTabs src = dyn_coul_tabs(tab.data());
+      float4* const ty = tab.data() + 2 * DYN_COUL_TAB_N;
+      for (int k = 0; k < DYN_COUL_Y_N; ++k) {
+        ty[k] = dyn_tab_scale(src.ftab[k], p.beta * p.beta * p.beta);
+        ty[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], p.beta);
+      }
+      E->coul_tab.reserve(tab.size());
+      DYN_HIP(hipMemcpyAsync(E->coul_tab.p, tab.data(), sizeof(float4) * tab.size(),
                              hipMemcpyHostToDevice, E->stream));
       DYN_HIP(hipStreamSynchronize(E->stream));
     }
@@ -2715,6 +3134,7 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->pme_xyzq.reserve(std::max<uint32_t>(E->n_q, 1));
     E->pme_b.reserve(std::max<uint32_t>(E->n_q, 1));
     E->pme_on = (p.grid[0] > 0 && p.grid[1] > 0 && p.grid[2] > 0) || p.mesh_spacing > 0.f;
+    DYN_HIP(hipMemsetAsync(E->fx_pair.p, 0, 24 * (size_t)ns, E->stream));
     DYN_HIP(hipMemsetAsync(E->counters.p, 0, 32, E->stream));
     DYN_HIP(hipMemsetAsync(E->slot_of.p, 0, 4 * (size_t)ns, E->stream));
     DYN_HIP(hipMemsetAsync(E->status.p, 0, 4, E->stream));

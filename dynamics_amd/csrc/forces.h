@@ -26,17 +26,14 @@ constexpr int kFlWords = 16;
 // The parts of the last evaluation's site forces (fixed point, component-
 // major), as the finalize kernel sums them.
 struct ForceParts {
-  const int64_t* fx_site;     // correction (and compatibility) forces by site
+  const int64_t* fx_site;     // correction forces by site
   const int64_t* fx_recip;    // SPME forces by site, or null
-  const int64_t* fitem;       // pair forces of each work item's 8 i slots, or null
-  const uint32_t* chunk_ptr;  // first work item of each row
-  const uint32_t* slot_of;    // per site: its slot
-  uint64_t cap_chunks;
-  uint32_t n_sites, n_slots;
-  unsigned int* fl;           // the engine's device flags
+  const int64_t* fx_pair;     // pair forces by site, or null
+  uint32_t n_sites;
   int forced;                 // the evaluation's list build was asked for by the host
-  int unused;                 // no implicit padding: argument packs are compared byte for byte
+  unsigned int* fl;           // the engine's device flags
 };
+static_assert(sizeof(ForceParts) == 40, "ForceParts has no padding");
 
 // Pair forces of slot k: the sum over its row's work items (integer sums:
 // the order does not change the result).
@@ -75,15 +72,14 @@ __device__ __forceinline__ void slot_item_forces(const int64_t* __restrict__ fit
 
 // Site s's force (fixed point) from the parts.
 __device__ __forceinline__ void site_force_sum(const ForceParts& P, uint32_t s, int64_t f[3]) {
-  f[0] = P.fx_site[s];
-  f[1] = P.fx_site[(size_t)P.n_sites + s];
-  f[2] = P.fx_site[2 * (size_t)P.n_sites + s];
-  if (P.fx_recip) {
-    f[0] += P.fx_recip[s];
-    f[1] += P.fx_recip[(size_t)P.n_sites + s];
-    f[2] += P.fx_recip[2 * (size_t)P.n_sites + s];
-  }
-  if (P.fitem) slot_item_forces(P.fitem, P.chunk_ptr, P.cap_chunks, min(P.slot_of[s], P.n_slots - 1), f);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) f[c] = P.fx_site[(size_t)c * P.n_sites + s];
+  if (P.fx_recip)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) f[c] += P.fx_recip[(size_t)c * P.n_sites + s];
+  if (P.fx_pair)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) f[c] += P.fx_pair[(size_t)c * P.n_sites + s];
 }
 
 // The end of the evaluation's list bookkeeping (one thread, after the pair

@@ -63,6 +63,28 @@ def test_short_range_vs_fp64_and_replay(gpu, cases, name):
     _check_item_sums(eng, dbg, ie)
 
 
+@pytest.mark.parametrize("cutoff,close", [(3.0, 0.0), (6.5, 0.0), (10.5, 0.0), (12.8, 0.0), (6.5, 0.03),
+                                          (12.8, 1e-9)])
+def test_pair_tile_images_and_remainders(gpu, cases, cutoff, close):
+    """27 Å box at cutoffs where rows have a few groups or many (batches of
+    four with every remainder, batches of two classes) and see their j sites
+    unshifted, shifted by whole boxes or each pair in its own image; a solute
+    atom placed almost (0.03 Å) or fully on a water hydrogen, below the
+    Coulomb tables.  Fixed-point sums equal the host replay's exactly."""
+    s = copy.copy(cases["solvated"])
+    if close:
+        s.pos_dyn = s.pos_dyn.copy()
+        s.pos_dyn[5] = s.pos_h0[11] + np.float32([close, 0.0, 0.0])
+    print(f"pair tiles: cutoff={cutoff} close={close}", flush=True)
+    eng = _engine(s, cutoff=cutoff, lj_cutoff=min(cutoff, 9.0))
+    eng.compute(api.COMPUTE_SHORT)
+    dbg = eng.debug_export()
+    fx, _, ie = replay_engine_tiles(dbg, s, cutoff, min(cutoff, 9.0), BETA, per_item=True)
+    assert np.array_equal(fx, dbg["fx_slot"]), "slot fixed-point sums differ from replay"
+    _check_item_sums(eng, dbg, ie)
+    eng.close()
+
+
 def _check_item_sums(eng, dbg, ie):
     """Per work item energies, virial and dH/dλ against the host replay: a
     sum the replay leaves at zero (e.g. a solute energy of a water-only item)
