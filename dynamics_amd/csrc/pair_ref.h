@@ -36,7 +36,10 @@ struct DynRefParams {
 // Returns false when the pair is skipped (r² < 1e-16, as the kernel does).
 // f: force on tgt (src receives −f when symmetric).  e: pair energy,
 // dhdl: dH/dλ of the pair, vir: d·f accumulated by the caller in f64.
-DYN_HD bool dyn_ref_pair(const float* pos, const DynPairRec& p, const DynRefParams& P,
+// r2_far: a squared distance beyond the Coulomb cutoff; pairs past it that
+// have no LJ are all zeros and skipped too (up to the largest r² whose direction
+// is a number).
+DYN_HD bool dyn_ref_pair(const float* pos, const DynPairRec& p, const DynRefParams& P, float r2_far,
                          float f[3], float* e, float* dhdl, double* vir) {
   const float* a = pos + 3u * p.tgt;
   const float* b = pos + 3u * p.src;
@@ -46,6 +49,7 @@ DYN_HD bool dyn_ref_pair(const float* pos, const DynPairRec& p, const DynRefPara
   d2 = dyn_min_image_rint(d2, P.ext[2], P.inv_ext[2]);
   const float r2 = dyn_fmaf(d2, d2, dyn_fmaf(d1, d1, d0 * d0));
   if (r2 < 1e-16f) return false;
+  if (r2 > r2_far && r2 < 1e30f && (!(p.flags & DYN_PF_LJ) || P.lj_disabled)) return false;
   const float inv_r = dyn_rsqrtf(r2);
   const float r = r2 * inv_r;
   const float dir0 = d0 * inv_r, dir1 = d1 * inv_r, dir2 = d2 * inv_r;
@@ -98,4 +102,10 @@ DYN_HD bool dyn_ref_pair(const float* pos, const DynPairRec& p, const DynRefPara
   *dhdl = dh;
   *vir = (double)d0 * (double)f[0] + (double)d1 * (double)f[1] + (double)d2 * (double)f[2];
   return true;
+}
+
+// Without the short cut: every pair evaluated in full.
+DYN_HD bool dyn_ref_pair(const float* pos, const DynPairRec& p, const DynRefParams& P, float f[3],
+                         float* e, float* dhdl, double* vir) {
+  return dyn_ref_pair(pos, p, P, 1e30f, f, e, dhdl, vir);
 }

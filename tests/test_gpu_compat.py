@@ -159,3 +159,31 @@ def test_compat_errors(gpu, solv):
     ctx.set_pairs(empty)
     f_dyn, f_w, vir, en, _ = _compute(ctx, s)
     assert not f_dyn.any() and not f_w.any() and vir == 0.0
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 262144 + 17, 4_300_000])
+def test_compat_pair_runs(gpu, n):
+    """Random pairs of 4,000 waters (16,000 sites: more than a run's table
+    holds), one-sided and symmetric, with and without LJ, from a single pair to
+    several runs per workgroup: fixed-point sums equal the replay's exactly."""
+    s = systems.small_water(n_water=4000, box=49.6, lattice_n=16, seed=3)
+    rng = np.random.default_rng(n)
+    u8, f4 = np.uint8, np.float32
+    wt, ws = rng.integers(1, 5, n).astype(u8), rng.integers(1, 5, n).astype(u8)
+    tgt = rng.integers(0, 4000, n).astype(np.uint32)
+    src = ((tgt + rng.integers(1, 4000, n)) % 4000).astype(np.uint32)
+    one = np.ones(n, u8)
+    pairs = {"tgt": tgt, "src": src, "sigma": np.full(n, 3.1, f4), "eps": np.full(n, 0.2, f4),
+             "q_tgt": np.full(n, -0.5, f4), "q_src": np.full(n, 0.4, f4), "atom_type_tgt": one,
+             "water_site_tgt": wt, "atom_type_src": one, "water_site_src": ws,
+             "scale14": rng.integers(0, 2, n).astype(u8), "calc_lj": rng.integers(0, 2, n).astype(u8),
+             "calc_coul": rng.integers(0, 2, n).astype(u8), "symmetric": rng.integers(0, 2, n).astype(u8)}
+    print(f"pair runs: n={n}", flush=True)
+    ctx = _ctx(s)
+    ctx.set_pairs(pairs)
+    _, _, vir, en, _ = _compute(ctx, s)
+    fx_r, e_r, w_r, _ = replay_ref_pairs(s, pairs, RC, ALPHA)
+    assert np.array_equal(ctx.fixed_forces(), fx_r)
+    # sums of n double terms in another order: 1e-9 of the terms is ample
+    assert abs(vir - w_r) <= 1e-9 * abs(w_r) + 1e-9
+    ctx.close()
