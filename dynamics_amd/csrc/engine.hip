@@ -51,7 +51,7 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kPairBlock = 256;       // 4 waves, one work item each at a time
-constexpr uint64_t kPairAhead = 16;   // groups of a list the pair kernel may read past its end
+constexpr uint32_t kPairAhead = 16;   // groups of a list the pair kernel may read past its end
 constexpr uint32_t kPairGridCap = 6144;  // a few times the pair kernel's resident workgroups
 constexpr int kColCap = 4096;         // sites per column (LDS sort)
 constexpr int kMaxColsPerClass = 4096;
@@ -865,6 +865,12 @@ k_eng_list_fill(const ListArgs& A, const uint32_t* __restrict__ ent_tmp,
       row_ptr[r0 + threadIdx.x] = s_g[threadIdx.x];
       chunk_ptr[r0 + threadIdx.x] = s_i[threadIdx.x];
     }
+    // the pair kernel reads ahead past a row's end: the groups after the last
+    // row name a slot too
+    if (r0 + nr == n_cl && threadIdx.x < kPairAhead * DYN_CL_SIZE) {
+      const uint64_t end = (uint64_t)s_g[nr - 1] + s_m[nr - 1];
+      if (end <= A.cap_entries) cj[end * DYN_CL_SIZE + threadIdx.x] = A.null_slot;
+    }
     for (uint32_t sgi = (uint32_t)w; sgi < nr * 3u; sgi += kListWaves) {
       const uint32_t I = r0 + sgi / 3u;
       const int cls = (int)(sgi % 3u);
@@ -945,7 +951,6 @@ struct PairArgs {
   const unsigned int* fl;    // the engine's flags: the copy in use, the largest displacement
   int staged;                // staged list builds: a stale current list voids the evaluation
   unsigned int hard_limit;   // half the list buffer, squared (float bits)
-  const float4* coul_y;      // the Coulomb tables over y, times β³ (Ψ) and β (Λ)
   const float2* lj_table;    // (c6, c12) per type pair
   const float2* lj_se;       // (σ, ε) per type pair, for soft-core
   const double2* lj_table64; // (c6, c12) in double, for the FP64 option
@@ -1553,7 +1558,11 @@ k_eng_pairs(PairArgs A) {
   DynCoulTabs tabs = {nullptr, nullptr};
   const float2* ljt = nullptr;
   if constexpr (!F64) {
-    for (int k = threadIdx.x; k < kTab; k += kPairBlock) s_tab[k] = A.coul_y[k];
+    const DynCoulTabs src = dyn_coul_tabs(A.P.coul_tab);
+    for (int k = threadIdx.x; k < DYN_COUL_Y_N; k += kPairBlock) {
+      s_tab[k] = dyn_tab_scale(src.ftab[k], A.P.beta2 * A.P.beta);
+      if (ENERGY) s_tab[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], A.P.beta);
+    }
     const int nt2 = A.P.n_types * A.P.n_types;
     for (int k = threadIdx.x; k < nt2; k += kPairBlock) s_lj[k] = A.lj_table[k];
     __syncthreads();
@@ -2088,8 +2097,7 @@ struct dyn_engine {
   DevBuf<float2> lj_table;   // (c6, c12) per type pair
   DevBuf<float2> lj_se;      // (σ, ε) per type pair (soft-core)
   DevBuf<double2> lj_table64;  // (c6, c12) in double (FP64 pair option)
-  DevBuf<float4> coul_tab;     // erfc Coulomb tables (dyn_coul_tab_build), then those over y
-                               // times β³ and β (the pair kernel's LDS copies)
+  DevBuf<float4> coul_tab;     // erfc Coulomb tables (dyn_coul_tab_build)
   std::vector<int32_t> h_type;  // per-site type words (host copy)
   // decoupled molecule: solute sites [alch0, alch1), λ
   uint32_t alch0 = 0, alch1 = 0;
@@ -2160,7 +2168,8 @@ struct dyn_engine {
   // device flags (kFlWords words, kFl* indices)
   DevBuf<unsigned int> dflags;
   // accumulators
-  DevBuf<int64_t> fitem, fx_site, fx_pair, fx_out, fx_slot;  // fx_slot: inspection only
+  DevBuf<int64_t> fitem, fx_site, fx_out, fx_slot;  // fx_slot: inspection only
+  int64_t* fx_pair = nullptr;                       // after fx_site's 3·n_sites
   DevBuf<double> pair_part, corr_part, eng_out, red1;
   unsigned corr_blocks = 0;
   // a pass over this engine alone: argument packs of both streams
@@ -2342,14 +2351,8 @@ void dyn_engine::reserve_rows(uint32_t entries) {
 // List capacity in groups of 8 j entries, and work items.
 void dyn_engine::reserve_list(uint64_t groups, uint64_t n_items) {
   if (groups > cap_entries) {
-    // the pair kernel reads ahead past a row's end (kPairAhead groups past
-    // the last row's): every entry of the buffers names a slot
-    for (DevBuf<uint32_t>* b : {&cj, &cj2}) {
-      b->reserve((groups + kPairAhead) * DYN_CL_SIZE);
-      DYN_HIP(hipMemsetAsync(b->p, 0, sizeof(uint32_t) * (groups + kPairAhead) * DYN_CL_SIZE, stream));
-    }
+    for (DevBuf<uint32_t>* b : {&cj, &cj2}) b->reserve((groups + kPairAhead) * DYN_CL_SIZE);
     for (DevBuf<unsigned long long>* b : {&cmask, &cmask2}) b->reserve(groups + kPairAhead);
-    DYN_HIP(hipStreamSynchronize(stream));
     cap_entries = groups;
   }
   if (n_items > cap_chunks) {
@@ -2751,7 +2754,6 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
       A.fl = e.dflags.p;
       A.staged = staged_mode && !forced[i] ? 1 : 0;
       A.hard_limit = build_limit(e);
-      A.coul_y = e.coul_tab.p + 2 * DYN_COUL_TAB_N;
       A.lj_table = e.lj_table.p;
       A.lj_se = e.lj_se.p;
       A.lj_table64 = e.lj_table64.p;
@@ -2761,7 +2763,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
       A.null_slot = e.cap_slots;
       A.fitem = e.fitem.p;
       A.slot_site = e.slot_site.p;
-      A.fx_pair = e.fx_pair.p;
+      A.fx_pair = e.fx_pair;
       A.n_sites = e.n_sites;
       // a fused evaluation's caller reads site sums only
       A.keep_items = (flags & kComputeFusedFinalize) ? 0u : 1u;
@@ -2808,7 +2810,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
     std::memset(&P, 0, sizeof P);
     P.fx_site = e.fx_site.p;
     P.fx_recip = (pl.recip_on || pl.reuse) ? e.fx_recip.p : nullptr;
-    P.fx_pair = short_on ? e.fx_pair.p : nullptr;
+    P.fx_pair = short_on ? e.fx_pair : nullptr;
     P.n_sites = e.n_sites;
     P.fl = e.dflags.p;
     P.forced = forced[i] ? 1 : 0;
@@ -3099,8 +3101,8 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->slot_of.reserve(ns);
     E->stg_wpos_ref.reserve(ns);
     E->stg_slot_of.reserve(ns);
-    E->fx_site.reserve(3 * (size_t)ns);
-    E->fx_pair.reserve(3 * (size_t)ns);
+    E->fx_site.reserve(6 * (size_t)ns);
+    E->fx_pair = E->fx_site.p + 3 * (size_t)ns;
     E->fx_out.reserve(3 * (size_t)ns);
     E->fx_recip.reserve(3 * (size_t)ns);
     E->h_fx.reserve(3 * (size_t)ns);
@@ -3113,14 +3115,8 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->status.reserve(1);
     E->dflags.reserve(kFlWords);
     {
-      std::vector<float4> tab(2 * DYN_COUL_TAB_N + 2 * DYN_COUL_Y_N);
+      std::vector<float4> tab(2 * DYN_COUL_TAB_N);
       dyn_coul_tab_build(reinterpret_cast<float*>(tab.data()));
-      const DynCoulTabs src = dyn_coul_tabs(tab.data());
-      float4* const ty = tab.data() + 2 * DYN_COUL_TAB_N;
-      for (int k = 0; k < DYN_COUL_Y_N; ++k) {
-        ty[k] = dyn_tab_scale(src.ftab[k], p.beta * p.beta * p.beta);
-        ty[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], p.beta);
-      }
       E->coul_tab.reserve(tab.size());
       DYN_HIP(hipMemcpyAsync(E->coul_tab.p, tab.data(), sizeof(float4) * tab.size(),
                              hipMemcpyHostToDevice, E->stream));
@@ -3134,7 +3130,6 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->pme_xyzq.reserve(std::max<uint32_t>(E->n_q, 1));
     E->pme_b.reserve(std::max<uint32_t>(E->n_q, 1));
     E->pme_on = (p.grid[0] > 0 && p.grid[1] > 0 && p.grid[2] > 0) || p.mesh_spacing > 0.f;
-    DYN_HIP(hipMemsetAsync(E->fx_pair.p, 0, 24 * (size_t)ns, E->stream));
     DYN_HIP(hipMemsetAsync(E->counters.p, 0, 32, E->stream));
     DYN_HIP(hipMemsetAsync(E->slot_of.p, 0, 4 * (size_t)ns, E->stream));
     DYN_HIP(hipMemsetAsync(E->status.p, 0, 4, E->stream));
