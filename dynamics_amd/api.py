@@ -332,7 +332,12 @@ class ForcesPositsGpu:
         st = None if is_static is None else _c(is_static, np.uint8)
         n_outer = po.shape[0]
         row_ptr = np.zeros(n_outer + 1, np.uint32)
-        cap = max(1024, n_outer * 64)
+        # room for a uniform density and a tenth more, so that dense sets are
+        # built once too (untouched pages of the array cost nothing)
+        ext = _c(extent, np.float32).astype(np.float64).reshape(-1)
+        ball = 4.19 * max(float(skin_sq_w_cutoff), 0.0) ** 1.5 / max(float(np.prod(ext)), 1e-300)
+        row = min(1.1 * pi.shape[0] * min(ball, 1.0) + 16.0, 4096.0)
+        cap = max(1024, n_outer * 64, int(n_outer * row))
         total = C.c_uint64()
         for _ in range(2):
             col = np.zeros(cap, np.uint32)

@@ -69,3 +69,27 @@ def test_neighbor_errors_and_empty(gpu):
         ctx.build_neighbors(p, p[:3], None, ext, True, 100.0)
     rp_g, col_g = ctx.build_neighbors(p, np.zeros((0, 3), np.float32), None, ext, False, 100.0)
     assert not rp_g.any() and col_g.size == 0
+
+
+@pytest.mark.parametrize("n_outer,n_inner,ext,radius,spread", [
+    (1, 1, 20.0, 6.0, 1.0), (70, 2047, 25.0, 6.0, 1.0), (70, 2048, 25.0, 9.0, 3.0),
+    (300, 2049, 18.0, 6.0, 25.0),          # up to 12 boxes out: beyond the approximate test
+    (500, 3000, 300.0, 12.0, 1.0),         # 15,625 cells
+    (40, 140_000, 120.0, 8.0, 1.0),        # two ranges of indices
+    (64, 4000, 11.0, 6.0, 2.0),            # one cell per axis, rows across the whole box
+])
+def test_neighbor_rows_sizes(gpu, n_outer, n_inner, ext, radius, spread):
+    """Rows equal the brute-force lists at the edges of the bitmap's words
+    and ranges, of the cell counts and of the approximate test, with points
+    exactly at the threshold distance."""
+    rng = np.random.default_rng(n_inner)
+    mid, half = 0.5 * ext, 0.5 * ext * spread
+    po = rng.uniform(mid - half, mid + half, (n_outer, 3)).astype(np.float32)
+    pi = rng.uniform(mid - half, mid + half, (n_inner, 3)).astype(np.float32)
+    k = min(n_outer, n_inner)
+    pi[:k:3] = po[:k:3] + np.array([0, radius, 0], np.float32)
+    e = np.full(3, ext, np.float32)
+    print(f"neighbors: {n_outer} x {n_inner}, box {ext}, radius {radius}", flush=True)
+    ctx = api.ForcesPositsGpu(n_outer, 0, 10.0, 0.3)
+    _check(ctx, po, pi, None, e, False, np.float32(radius * radius))
+    _check(ctx, po, po, (np.arange(n_outer) % 3 == 0).astype(np.uint8), e, True, np.float32(radius * radius))
