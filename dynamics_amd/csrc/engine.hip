@@ -56,6 +56,11 @@ constexpr uint32_t kPairGridCap = 6144;  // a few times the pair kernel's reside
 constexpr int kColCap = 4096;         // sites per column (LDS sort)
 constexpr int kMaxColsPerClass = 4096;
 constexpr int kNumPart = 9;           // f64 partials per work item of the pair kernel
+constexpr int kEngOut = 20;           // f64 sums of an evaluation (see k_eng_energy_reduce)
+// words of an engine's report to the host, after those kEngOut doubles
+constexpr uint32_t kRepStatus = 0, kRepCounters = 8, kRepStaging = 16, kRepFlags = 24,
+                   kRepWords = kRepFlags + kFlWords;
+constexpr uint32_t kRepDoubles = kEngOut + kRepWords / 2;
 
 // status bits
 constexpr unsigned kStColumn = 1u, kStRow = 2u, kStEntries = 4u, kStChunks = 8u, kStMask = 16u,
@@ -1260,7 +1265,7 @@ __device__ __forceinline__ uint32_t last_class(uint32_t v, uint32_t left) {
 // decoupled molecule's boundary (a lane holds one of its quad's four j sites).
 __device__ __forceinline__ bool tile_crosses(const TileI& I, const TileJ& J, bool far) {
   const bool in = (J.t & DYN_TYPE_ALCH) != 0;
-  return (I.any_out & (lanes(!far & in) != 0ull)) | (I.any_in & (lanes(!far & !in) != 0ull));
+  return (I.any_out && lanes(!far & in) != 0ull) || (I.any_in && lanes(!far & !in) != 0ull);
 }
 
 // The batches of one class (cls) from C on, to the item's end (g1), the first
@@ -1988,6 +1993,62 @@ __device__ __forceinline__ void k_eng_finalize(ForceParts P, int64_t* __restrict
   for (int c = 0; c < 3; ++c) out[(size_t)c * P.n_sites + s] = f[c];
 }
 
+// Copies a block of doubles to pinned host memory (block b0 of the launch).
+__device__ __forceinline__ void k_eng_report(const double* __restrict__ src, double* __restrict__ dst,
+                                             uint32_t n, uint32_t b0) {
+  if (blockIdx.x == b0)
+    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) dst[k] = src[k];
+}
+
+// The force array as dyn_engine_get_forces returns it — solute sites, then
+// per water O, H0, H1, M — in doubles, and the report, stored straight into
+// pinned host memory: one launch and one wait for a read, where copies of the
+// fixed-point arrays and of each status word took seven, and the host
+// converted and reordered the forces.  252,480 sites (6 MB): 113 µs, the rate of the
+// bus.
+__device__ __forceinline__ void k_eng_forces_out(const int64_t* __restrict__ fx, uint32_t n_dyn,
+                                                 uint32_t n_sites, double* __restrict__ out,
+                                                 const double* __restrict__ rep,
+                                                 double* __restrict__ h_rep) {
+  k_eng_report(rep, h_rep, kRepDoubles, 0);
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t o = k / 3u, c = k - 3u * o;
+  if (o >= n_sites) return;
+  uint32_t s = o;
+  if (o >= n_dyn) {  // a water's sites are O, M, H0, H1
+    const uint32_t f = (o - n_dyn) & 3u;
+    s = o - f + (f == 0u ? 0u : f == 3u ? 1u : f + 1u);
+  }
+  out[k] = (double)fx[(size_t)c * n_sites + s] * DYN_FX_INV_SCALE;
+}
+
+// Positions from pinned host memory — solute, O, M, H0 and H1 arrays one
+// after another, each from a multiple of 16 bytes — into site order: 256
+// sites of one array per workgroup, read once and in 16-byte pieces (host
+// memory is not cached).
+__device__ __forceinline__ void k_eng_positions(const float4* __restrict__ h, uint32_t n_dyn,
+                                                uint32_t n_water, float4* __restrict__ pos) {
+  __shared__ float s_x[4 * 192];
+  const uint32_t bd = (n_dyn + 255u) / 256u, bw = (n_water + 255u) / 256u;
+  uint32_t b = blockIdx.x, part = 0, n = n_dyn;
+  size_t at = 0;
+  if (b >= bd) {
+    b -= bd;
+    part = 1u + b / max(bw, 1u);
+    if (part > 4u) return;
+    b -= (part - 1u) * bw;
+    n = n_water;
+    at = (3 * (size_t)n_dyn + 3) / 4 + (part - 1) * ((3 * (size_t)n_water + 3) / 4);
+  }
+  const uint32_t t = threadIdx.x, k = 192u * b + t;
+  if (t < 192u && 4u * k < 3u * n) *reinterpret_cast<float4*>(s_x + 4 * t) = h[at + k];
+  __syncthreads();
+  const uint32_t i = 256u * b + t;
+  if (i >= n) return;
+  const uint32_t s = part == 0u ? i : n_dyn + 4u * i + (part - 1u);
+  pos[s] = make_float4(s_x[3 * t], s_x[3 * t + 1], s_x[3 * t + 2], 0.f);
+}
+
 // Slot-order pair forces (component-major), for inspection.
 __device__ __forceinline__ void k_eng_slot_forces(const int64_t* __restrict__ fitem,
                                   const uint32_t* __restrict__ chunk_ptr, uint64_t cap_chunks,
@@ -2008,7 +2069,6 @@ __device__ __forceinline__ void k_eng_slot_forces(const int64_t* __restrict__ fi
 // and second SPME evaluation (written by SPME itself); those not evaluated
 // are cleared here.
 constexpr int kRedBlock = 1024;
-constexpr int kEngOut = 20;
 constexpr int kRed1Grid = 128;   // first-stage workgroups (fixed: part of the sum's order)
 constexpr int kRed1Block = 256;
 
@@ -2077,6 +2137,12 @@ k_eng_energy_reduce(const double* __restrict__ red1, const double* __restrict__ 
 // check would, so the error and repeat paths run without a real failure.
 __global__ void k_dbg_or_status(unsigned int* status, unsigned int bits) { atomicOr(status, bits); }
 
+template <class T>
+struct View {  // part of a DevBuf
+  T* p = nullptr;
+};
+constexpr int kFxFixed = 1, kFxDouble = 2;
+
 struct dyn_engine {
   std::string err;
   int device = 0;
@@ -2140,14 +2206,15 @@ struct dyn_engine {
   uint32_t row_cap = 0;                      // j entries per walk-unit slice of ent_tmp
   // device counters: [0] n_cl, [1] n_groups, [2] n_items, [3] max row (groups),
   // [4] longest row that overflowed its slice (entries)
-  DevBuf<uint32_t> counters;
+  View<uint32_t> counters;
   // the staging list of an asynchronous build (slot and row arrays, copied
   // into the ones above by the next evaluation's preparation kernel) and the
   // second copy of the per-group arrays (dflags[kFlSel] names the current)
   DevBuf<float4> stg_wpos_ref, stg_xyzq;
   DevBuf<int32_t> stg_slot_site, stg_slot_type, stg_slot_gid;
   DevBuf<uint8_t> stg_cl_class;
-  DevBuf<uint32_t> stg_slot_of, stg_row_ptr, stg_chunk_ptr, stg_counters;
+  DevBuf<uint32_t> stg_slot_of, stg_row_ptr, stg_chunk_ptr;
+  View<uint32_t> stg_counters;
   DevBuf<uint32_t> cj2;
   DevBuf<unsigned long long> cmask2;
   DevBuf<uint2> chunks2;
@@ -2164,13 +2231,19 @@ struct dyn_engine {
     return ListCopies{cj.p, cj2.p, cmask.p, cmask2.p, chunks.p, chunks2.p, dflags.p,
                       staged ? 1 : 0, 0};
   }
-  DevBuf<unsigned int> status;
+  View<unsigned int> status;
   // device flags (kFlWords words, kFl* indices)
-  DevBuf<unsigned int> dflags;
+  View<unsigned int> dflags;
+  View<double> eng_out;
+  // what the host reads after an evaluation, one block and one copy: eng_out,
+  // then the words of kRep* (status, counters, stg_counters, dflags)
+  DevBuf<double> report;
+  PinnedBuf<double> h_report;
+  const uint32_t* rep_words() const { return reinterpret_cast<const uint32_t*>(h_report.p + kEngOut); }
   // accumulators
   DevBuf<int64_t> fitem, fx_site, fx_out, fx_slot;  // fx_slot: inspection only
   int64_t* fx_pair = nullptr;                       // after fx_site's 3·n_sites
-  DevBuf<double> pair_part, corr_part, eng_out, red1;
+  DevBuf<double> pair_part, corr_part, red1;
   unsigned corr_blocks = 0;
   // a pass over this engine alone: argument packs of both streams
   ArgCache own_cache, side_cache;
@@ -2182,10 +2255,7 @@ struct dyn_engine {
   bool recip_kept = false;         // fx_recip and its energies are those of this box
   // host copies
   PinnedBuf<int64_t> h_fx;
-  PinnedBuf<double> h_eng;
-  // [0] status, [1..5] counters, [6] builds, [7] current copy, [8..12] staging counters
-  PinnedBuf<uint32_t> h_misc;
-  bool fx_fresh = false;
+  int fx_fresh = 0;  // h_fx holds the last evaluation's forces (kFxFixed, kFxDouble)
   // the last evaluation's force parts; fx_stale: enqueued with
   // kComputeFusedFinalize, so fx_out does not hold its forces
   ForceParts parts{};
@@ -2218,6 +2288,7 @@ struct dyn_engine {
   void reserve_rows(uint32_t entries);
   void reserve_list(uint64_t groups, uint64_t items);
   void check_status();
+  void check_report();
   EngineSet self_set() {
     EngineSet S;
     S.e = {this};
@@ -2848,16 +2919,21 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
     e.list_valid = true;  // every later evaluation keeps it valid on the device
     e.energies_valid = energy_on;
     e.mol_valid = energy_on && e.n_mol;
-    e.fx_fresh = false;
+    e.fx_fresh = 0;
   }
 }
 
 void engine_set_check(EngineSet& S) {
+  // every engine's report by one launch, one wait
+  launch<k_eng_report>(S.R, "k_eng_report", 0, 1, 64, 0, [&](uint32_t i) {
+    return args<k_eng_report>((const double*)S.e[i]->report.p, S.e[i]->h_report.p, kRepDoubles, 0u);
+  });
+  DYN_HIP(hipStreamSynchronize(S.R.stream));
   const Error* first = nullptr;
   Error keep(0, "");
   for (dyn_engine* e : S.e) {
     try {
-      e->check_status();
+      e->check_report();
     } catch (const Error& err) {
       if (!first) {
         keep = err;
@@ -2871,13 +2947,15 @@ void engine_set_check(EngineSet& S) {
 }  // namespace dyn
 
 void dyn_engine::check_status() {
-  DYN_HIP(hipMemcpyAsync(h_misc.p, status.p, 4, hipMemcpyDeviceToHost, stream));
-  DYN_HIP(hipMemcpyAsync(h_misc.p + 1, counters.p, 20, hipMemcpyDeviceToHost, stream));
-  DYN_HIP(hipMemcpyAsync(h_misc.p + 6, dflags.p + kFlBuilds, 4, hipMemcpyDeviceToHost, stream));
-  DYN_HIP(hipMemcpyAsync(h_misc.p + 7, dflags.p + kFlSel, 4, hipMemcpyDeviceToHost, stream));
-  DYN_HIP(hipMemcpyAsync(h_misc.p + 8, stg_counters.p, 20, hipMemcpyDeviceToHost, stream));
+  DYN_HIP(hipMemcpyAsync(h_report.p, report.p, sizeof(double) * kRepDoubles, hipMemcpyDeviceToHost, stream));
   DYN_HIP(hipStreamSynchronize(stream));
-  const uint32_t st = h_misc.p[0];
+  check_report();
+}
+
+// The status of the report in h_report.
+void dyn_engine::check_report() {
+  const uint32_t* const rep = rep_words();
+  const uint32_t st = rep[kRepStatus];
   if (!st) return;
   DYN_HIP(hipMemsetAsync(status.p, 0, 4, stream));
   DYN_HIP(hipMemsetAsync(col_count.p, 0, sizeof(uint32_t) * (n_cols + 1), stream));
@@ -2905,17 +2983,30 @@ void dyn_engine::check_status() {
   }
   if (st & kStRow) {
     // the longest row of either list's build (counters [4])
-    const uint32_t longest = std::max(h_misc.p[5], h_misc.p[12]);
+    const uint32_t longest = std::max(rep[kRepCounters + 4], rep[kRepStaging + 4]);
     DYN_HIP(hipMemsetAsync(counters.p + 4, 0, 4, stream));
     DYN_HIP(hipMemsetAsync(stg_counters.p + 4, 0, 4, stream));
     reserve_rows(std::max<uint32_t>(longest + longest / 4, row_cap + row_cap / 2));
   }
-  const uint64_t ne = std::max(h_misc.p[2], h_misc.p[9]), nch = std::max(h_misc.p[3], h_misc.p[10]);
+  const uint64_t ne = std::max(rep[kRepCounters + 1], rep[kRepStaging + 1]),
+                 nch = std::max(rep[kRepCounters + 2], rep[kRepStaging + 2]);
   reserve_list(ne + ne / 4 + 1024, nch + nch / 4 + 256);
   throw Error(DYN_ERR_CAPACITY, fmt("pair list outgrew its buffers (%llu groups, %llu work "
                                     "items, row slices of %u entries); they have been enlarged, "
                                     "call again", (unsigned long long)ne,
                                     (unsigned long long)nch, row_cap));
+}
+
+// Copies n floats; whether one of them is not finite.
+static bool copy_finite(float* __restrict__ dst, const float* __restrict__ src, size_t n) {
+  uint32_t bad = 0;
+  for (size_t k = 0; k < n; ++k) {
+    uint32_t u;
+    memcpy(&u, src + k, 4);
+    bad |= (u & 0x7f800000u) == 0x7f800000u ? 1u : 0u;
+    memcpy(dst + k, &u, 4);
+  }
+  return bad != 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -3106,14 +3197,17 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->fx_out.reserve(3 * (size_t)ns);
     E->fx_recip.reserve(3 * (size_t)ns);
     E->h_fx.reserve(3 * (size_t)ns);
-    E->eng_out.reserve(kEngOut);
     E->red1.reserve((size_t)kRed1Grid * kNumPart);
-    E->h_eng.reserve(kEngOut);
-    E->h_misc.reserve(16);
-    E->counters.reserve(8);
-    E->stg_counters.reserve(8);
-    E->status.reserve(1);
-    E->dflags.reserve(kFlWords);
+    E->h_report.reserve(kRepDoubles);
+    E->report.reserve(kRepDoubles);
+    E->eng_out.p = E->report.p;
+    {
+      uint32_t* const words = reinterpret_cast<uint32_t*>(E->report.p + kEngOut);
+      E->status.p = words + kRepStatus;
+      E->counters.p = words + kRepCounters;
+      E->stg_counters.p = words + kRepStaging;
+      E->dflags.p = words + kRepFlags;
+    }
     {
       std::vector<float4> tab(2 * DYN_COUL_TAB_N);
       dyn_coul_tab_build(reinterpret_cast<float*>(tab.data()));
@@ -3130,11 +3224,8 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     E->pme_xyzq.reserve(std::max<uint32_t>(E->n_q, 1));
     E->pme_b.reserve(std::max<uint32_t>(E->n_q, 1));
     E->pme_on = (p.grid[0] > 0 && p.grid[1] > 0 && p.grid[2] > 0) || p.mesh_spacing > 0.f;
-    DYN_HIP(hipMemsetAsync(E->counters.p, 0, 32, E->stream));
     DYN_HIP(hipMemsetAsync(E->slot_of.p, 0, 4 * (size_t)ns, E->stream));
-    DYN_HIP(hipMemsetAsync(E->status.p, 0, 4, E->stream));
-    DYN_HIP(hipMemsetAsync(E->dflags.p, 0, 4 * kFlWords, E->stream));
-    DYN_HIP(hipMemsetAsync(E->stg_counters.p, 0, 4 * 8, E->stream));
+    DYN_HIP(hipMemsetAsync(E->report.p, 0, E->report.bytes(), E->stream));
     // reference positions are read before the first build writes them (the
     // first evaluation's reading is discarded): keep them defined
     DYN_HIP(hipMemsetAsync(E->wpos_ref.p, 0, sizeof(float4) * ns, E->stream));
@@ -3213,17 +3304,25 @@ extern "C" int dyn_engine_set_positions(dyn_engine* eng, const float* pos_dyn,
     const uint32_t nd = eng->n_dyn, nw = eng->n_water;
     DYN_REQUIRE(nd == 0 || pos_dyn, "pos_dyn is null");
     DYN_REQUIRE(nw == 0 || (pos_w_o && pos_w_m && pos_w_h0 && pos_w_h1), "water positions null");
-    float4* h = eng->h_pos.p;
-    for (uint32_t i = 0; i < nd; ++i) h[i] = make_float4(pos_dyn[3 * i], pos_dyn[3 * i + 1], pos_dyn[3 * i + 2], 0.f);
-    const float* w[4] = {pos_w_o, pos_w_m, pos_w_h0, pos_w_h1};
-    for (uint32_t m = 0; m < nw; ++m)
-      for (int k = 0; k < 4; ++k)
-        h[nd + 4 * m + k] = make_float4(w[k][3 * m], w[k][3 * m + 1], w[k][3 * m + 2], 0.f);
-    for (uint32_t s = 0; s < eng->n_sites; ++s)
-      DYN_REQUIRE(std::isfinite(h[s].x) && std::isfinite(h[s].y) && std::isfinite(h[s].z),
-                  "non-finite position at site %u", s);
-    DYN_HIP(hipMemcpyAsync(eng->pos_own.p, h, sizeof(float4) * eng->n_sites,
-                           hipMemcpyHostToDevice, eng->stream));
+    // the five arrays one after another, each from a multiple of 16 bytes
+    const float* src[5] = {pos_dyn, pos_w_o, pos_w_m, pos_w_h0, pos_w_h1};
+    float* const h = reinterpret_cast<float*>(eng->h_pos.p);
+    bool bad = false;
+    size_t at = 0;
+    for (int k = 0; k < 5; ++k) {
+      const size_t n = 3 * (size_t)(k == 0 ? nd : nw);
+      bad = copy_finite(h + at, src[k], n) || bad;
+      at += (n + 3) & ~(size_t)3;
+    }
+    if (bad)
+      for (uint32_t s = 0; s < eng->n_sites; ++s) {
+        const float* x = s < nd ? pos_dyn + 3 * (size_t)s : src[1 + (s - nd) % 4] + 3 * (size_t)((s - nd) / 4);
+        DYN_REQUIRE(std::isfinite(x[0]) && std::isfinite(x[1]) && std::isfinite(x[2]),
+                    "non-finite position at site %u", s);
+      }
+    const BatchRun R = eng->self_set().R;
+    launch<k_eng_positions>(R, "k_eng_positions", 0, (nd + 255) / 256 + 4 * ((nw + 255) / 256), 256, 0,
+                            [&](uint32_t) { return args<k_eng_positions>((const float4*)h, nd, nw, eng->pos_own.p); });
     DYN_HIP(hipStreamSynchronize(eng->stream));
     eng->pos_dev = eng->pos_own.p;
     eng->pos_set = true;
@@ -3365,37 +3464,40 @@ extern "C" int dyn_engine_sync(dyn_engine* eng) {
   });
 }
 
-static void fetch_fx(dyn_engine* eng) {
+// The last evaluation's forces in h_fx: fixed-point (component-major) or
+// doubles in the order dyn_engine_get_forces returns them.
+static void fetch_fx(dyn_engine* eng, int form) {
   if (!eng->computed) throw Error(DYN_ERR_STATE, "no compute yet");
   if (eng->fx_stale) throw Error(DYN_ERR_STATE, "the last evaluation's forces were summed by its caller");
-  if (eng->fx_fresh) return;
-  eng->check_status();
-  DYN_HIP(hipMemcpyAsync(eng->h_fx.p, eng->fx_out.p, sizeof(int64_t) * 3 * eng->n_sites,
-                         hipMemcpyDeviceToHost, eng->stream));
-  DYN_HIP(hipStreamSynchronize(eng->stream));
-  eng->fx_fresh = true;
+  if (eng->fx_fresh == form) return;
+  eng->fx_fresh = 0;
+  const size_t n = 3 * (size_t)eng->n_sites;
+  if (form == kFxFixed) {
+    DYN_HIP(hipMemcpyAsync(eng->h_fx.p, eng->fx_out.p, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
+                           eng->stream));
+    eng->check_status();
+  } else {
+    const BatchRun R = eng->self_set().R;
+    launch<k_eng_forces_out>(R, "k_eng_forces_out", 0, grid_for(n, 256), 256, 0, [&](uint32_t) {
+      return args<k_eng_forces_out>((const int64_t*)eng->fx_out.p, eng->n_dyn, eng->n_sites,
+                                    reinterpret_cast<double*>(eng->h_fx.p),
+                                    (const double*)eng->report.p, eng->h_report.p);
+    });
+    DYN_HIP(hipStreamSynchronize(eng->stream));
+    eng->check_report();
+  }
+  eng->fx_fresh = form;
 }
 
 extern "C" int dyn_engine_get_forces(dyn_engine* eng, double* f_dyn, double* f_water) {
   ENG_CHECK(eng);
   DYN_API_BODY(eng, {
     DeviceGuard g(eng->device);
-    fetch_fx(eng);
-    const uint32_t ns = eng->n_sites, nd = eng->n_dyn, nw = eng->n_water;
-    const int64_t* F = eng->h_fx.p;
-    if (f_dyn)
-      for (uint32_t i = 0; i < nd; ++i)
-        for (int c = 0; c < 3; ++c) f_dyn[3 * i + c] = (double)F[(size_t)c * ns + i] * DYN_FX_INV_SCALE;
-    if (f_water) {
-      // ForcesOnWaterMol order f_o, f_h0, f_h1, f_m; site order O, M, H0, H1
-      const int site_of_field[4] = {0, 2, 3, 1};
-      for (uint32_t m = 0; m < nw; ++m)
-        for (int fld = 0; fld < 4; ++fld) {
-          const uint32_t s = nd + 4 * m + site_of_field[fld];
-          for (int c = 0; c < 3; ++c)
-            f_water[12 * (size_t)m + 3 * fld + c] = (double)F[(size_t)c * ns + s] * DYN_FX_INV_SCALE;
-        }
-    }
+    fetch_fx(eng, kFxDouble);
+    const double* F = reinterpret_cast<const double*>(eng->h_fx.p);
+    if (f_dyn && eng->n_dyn) memcpy(f_dyn, F, sizeof(double) * 3 * (size_t)eng->n_dyn);
+    if (f_water && eng->n_water)
+      memcpy(f_water, F + 3 * (size_t)eng->n_dyn, sizeof(double) * 12 * (size_t)eng->n_water);
   });
 }
 
@@ -3405,7 +3507,7 @@ extern "C" int dyn_engine_get_fixed_forces(dyn_engine* eng, int64_t* out, uint64
     DeviceGuard g(eng->device);
     DYN_REQUIRE(out && n_values >= 3ull * eng->n_sites, "need %llu values",
                 (unsigned long long)(3ull * eng->n_sites));
-    fetch_fx(eng);
+    fetch_fx(eng, kFxFixed);
     memcpy(out, eng->h_fx.p, sizeof(int64_t) * 3 * eng->n_sites);
   });
 }
@@ -3414,19 +3516,13 @@ extern "C" const int64_t* dyn_engine_forces_device(const dyn_engine* eng) {
   return eng ? eng->fx_out.p : nullptr;
 }
 
-extern "C" int dyn_engine_get_energies(dyn_engine* eng, dyn_energies* out) {
-  ENG_CHECK(eng);
-  DYN_API_BODY(eng, {
-    DeviceGuard g(eng->device);
-    DYN_REQUIRE(out, "out is null");
-    if (!eng->computed) throw Error(DYN_ERR_STATE, "no compute yet");
-    if (!eng->energies_valid)
-      throw Error(DYN_ERR_STATE, "the last compute skipped energies (DYN_COMPUTE_NO_ENERGY)");
-    eng->check_status();
-    DYN_HIP(hipMemcpyAsync(eng->h_eng.p, eng->eng_out.p, kEngOut * sizeof(double),
-                           hipMemcpyDeviceToHost, eng->stream));
-    DYN_HIP(hipStreamSynchronize(eng->stream));
-    const double* v = eng->h_eng.p;
+// The energies in the engine's report (read since its last evaluation).
+static void report_energies(dyn_engine* eng, dyn_energies* out) {
+  if (!eng->computed) throw Error(DYN_ERR_STATE, "no compute yet");
+  if (!eng->energies_valid)
+    throw Error(DYN_ERR_STATE, "the last compute skipped energies (DYN_COMPUTE_NO_ENERGY)");
+  {
+    const double* v = eng->h_report.p;
     // v[0..8]: e_lj_w, e_lj_s, e_c_w, e_c_s, virial_pairs, pair counts by
     // kind, dH/dλ; v[9..15]: e_lj14, e_c14, e_corr, vir_sr14, vir_recip_corr, dH/dλ,
     // 1-4 pairs within the cutoff;
@@ -3461,9 +3557,19 @@ extern "C" int dyn_engine_get_energies(dyn_engine* eng, dyn_energies* out) {
     E.pair_count_kind[2] = (uint64_t)std::llround(v[7]);
     E.pair_count = E.pair_count_kind[0] + E.pair_count_kind[1] + E.pair_count_kind[2] +
                    (uint64_t)std::llround(v[15]);
-    E.list_entries = eng->h_misc.p[2];
-    E.list_builds = eng->h_misc.p[6];
+    E.list_entries = eng->rep_words()[kRepCounters + 1];
+    E.list_builds = eng->rep_words()[kRepFlags + kFlBuilds];
     *out = E;
+  }
+}
+
+extern "C" int dyn_engine_get_energies(dyn_engine* eng, dyn_energies* out) {
+  ENG_CHECK(eng);
+  DYN_API_BODY(eng, {
+    DeviceGuard g(eng->device);
+    DYN_REQUIRE(out, "out is null");
+    if (eng->computed && eng->energies_valid) eng->check_status();
+    report_energies(eng, out);
   });
 }
 
@@ -3477,8 +3583,9 @@ extern "C" int dyn_engine_debug_export(dyn_engine* eng, uint32_t* n_slots, uint3
     DeviceGuard g(eng->device);
     if (!eng->list_valid) throw Error(DYN_ERR_STATE, "no list built yet");
     eng->check_status();
-    const size_t nc = eng->h_misc.p[1], ns = nc * DYN_CL_SIZE, ne = eng->h_misc.p[2],
-                 nit = eng->h_misc.p[3];
+    const uint32_t* const rep = eng->rep_words();
+    const size_t nc = rep[kRepCounters], ns = nc * DYN_CL_SIZE, ne = rep[kRepCounters + 1],
+                 nit = rep[kRepCounters + 2];
     if (n_slots) *n_slots = (uint32_t)ns;
     if (n_clusters) *n_clusters = (uint32_t)nc;
     if (n_entries) *n_entries = ne;
@@ -3490,7 +3597,7 @@ extern "C" int dyn_engine_debug_export(dyn_engine* eng, uint32_t* n_slots, uint3
     if (slot_gid) DYN_HIP(hipMemcpyAsync(slot_gid, eng->slot_gid.p, 4 * ns, hipMemcpyDeviceToHost, s));
     if (cl_class) DYN_HIP(hipMemcpyAsync(cl_class, eng->cl_class.p, nc, hipMemcpyDeviceToHost, s));
     if (row_ptr) DYN_HIP(hipMemcpyAsync(row_ptr, eng->row_ptr.p, 4 * (nc + 1), hipMemcpyDeviceToHost, s));
-    const bool second = eng->h_misc.p[7] != 0;  // the current copy of the per-group arrays
+    const bool second = rep[kRepFlags + kFlSel] != 0;  // the current copy of the per-group arrays
     const uint32_t* cj_d = second ? eng->cj2.p : eng->cj.p;
     const unsigned long long* cm_d = second ? eng->cmask2.p : eng->cmask.p;
     const uint2* ch_d = second ? eng->chunks2.p : eng->chunks.p;
@@ -3521,7 +3628,7 @@ extern "C" int dyn_engine_debug_item_partials(dyn_engine* eng, double* out, uint
     if (!eng->energies_valid)
       throw Error(DYN_ERR_STATE, "the last compute evaluated no pair energies");
     eng->check_status();
-    const uint64_t nit = eng->h_misc.p[3];
+    const uint64_t nit = eng->rep_words()[kRepCounters + 2];
     DYN_REQUIRE(n_items == nit, "n_items %llu, the list has %llu work items",
                 (unsigned long long)n_items, (unsigned long long)nit);
     for (int v = 0; v < kNumPart; ++v)
@@ -3591,6 +3698,12 @@ void engine_set_stream(dyn_engine* eng, hipStream_t s) {
 const int64_t* engine_forces_device(const dyn_engine* eng) { return eng->fx_out.p; }
 ForceParts engine_force_parts(const dyn_engine* eng) { return eng->parts; }
 bool engine_forces_stale(const dyn_engine* eng) { return eng->fx_stale; }
+void engine_check(dyn_engine* eng) { eng->check_status(); }
+void engine_report_energies(dyn_engine* eng, dyn_energies* out) { report_energies(eng, out); }
+void* engine_host_stage(dyn_engine* eng) {
+  eng->fx_fresh = 0;
+  return eng->h_fx.p;
+}
 EngineSet engine_self_set(dyn_engine* eng) { return eng->self_set(); }
 int engine_device(const dyn_engine* eng) { return eng->device; }
 void engine_sizes(const dyn_engine* eng, uint32_t* n_dyn, uint32_t* n_water) {
@@ -3637,7 +3750,7 @@ void engine_restore(dyn_engine* e) {
   e->computed = e->ck.computed;
   e->energies_valid = e->ck.energies_valid;
   e->mol_valid = false;
-  e->fx_fresh = false;
+  e->fx_fresh = 0;
   e->fx_stale = false;
   e->list_valid = false;
 }

@@ -13,6 +13,7 @@
 #include "forces.h"
 
 struct dyn_engine;
+struct dyn_energies;
 
 namespace dyn {
 
@@ -72,6 +73,14 @@ const int64_t* engine_forces_device(const dyn_engine* eng);
 // array is stale (the evaluation was enqueued with kComputeFusedFinalize).
 ForceParts engine_force_parts(const dyn_engine* eng);
 bool engine_forces_stale(const dyn_engine* eng);
+// Wait for the engine's work and check its device status.
+void engine_check(dyn_engine* eng);
+// dyn_engine_get_energies without a wait, after a check (engine_check,
+// engine_set_check) that followed the last evaluation.
+void engine_report_energies(dyn_engine* eng, dyn_energies* out);
+// Pinned host memory of the engine, 24 bytes per site, for the caller's
+// next read.
+void* engine_host_stage(dyn_engine* eng);
 // Keep / put back the last evaluation's forces, SPME forces and energies
 // (enqueued on the engine's stream); a restore also invalidates the list.
 void engine_checkpoint(dyn_engine* eng);

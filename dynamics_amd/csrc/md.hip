@@ -570,27 +570,54 @@ __device__ __forceinline__ void k_md_zero(int64_t* __restrict__ f, size_t n) {
   if (i < n) f[i] = 0;
 }
 
-// Kinetic energies (amu Å²/ps²) and the bonded-energy partials, reduced by
-// one workgroup.  out: [0] kinetic over solute atoms and water O/H site
-// velocities (the reference's measure, src/thermostat.rs:46-63), [1..3]
-// bond, angle, dihedral energy, [4] kinetic of the rigid-body motion (solute
-// atoms as they are; per water the centre-of-mass and rotational part,
-// ½ M v_com² + ½ ω·L with I ω = L about the centre of mass).
+// The state as dyn_md_get_state returns it — solute positions and
+// velocities, water positions (O, M, H0, H1) and velocities (O, H0, H1), packed
+// floats one after another — straight into pinned host memory.  A thread per
+// float, so the stores over the bus are whole lines.  (Copies of the float4
+// arrays that the host then repacked: 2.47 ms at 252,480 sites; now 0.42 ms, 0.10 of it the kernel.)
+__device__ __forceinline__ void k_md_state_out(const float* __restrict__ x, const float* __restrict__ v,
+                                               uint32_t n_dyn, uint32_t n_water,
+                                               float* __restrict__ out) {
+  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t nd3 = 3 * (size_t)n_dyn, nw12 = 12 * (size_t)n_water, nw9 = 9 * (size_t)n_water;
+  if (k < 2 * nd3) {
+    const uint32_t j = (uint32_t)(k < nd3 ? k : k - nd3);
+    out[k] = (k < nd3 ? x : v)[4 * (size_t)(j / 3u) + j % 3u];
+    return;
+  }
+  size_t j = k - 2 * nd3;
+  if (j < nw12) {
+    const uint32_t s = (uint32_t)(j / 3u), c = (uint32_t)j - 3u * s;
+    out[k] = x[4 * ((size_t)n_dyn + s) + c];
+    return;
+  }
+  j -= nw12;
+  if (j >= nw9) return;
+  const uint32_t m = (uint32_t)(j / 9u), r = (uint32_t)j - 9u * m, a = r / 3u, c = r - 3u * a;
+  const uint32_t s = 4u * m + (a == 0u ? 0u : a + 1u);
+  out[k] = v[4 * ((size_t)n_dyn + s) + c];
+}
+
+// Kinetic energies (amu Å²/ps²), one pair of partials per workgroup: over
+// solute atoms and water O/H site velocities (the reference's measure,
+// src/thermostat.rs:46-63), and of the rigid-body motion (solute atoms as they
+// are; per water the centre-of-mass and rotational part, ½ M v_com² + ½ ω·L with
+// I ω = L about the centre of mass).  The host sums the partials in order.
+// Bound: the chain of a water's double-precision arithmetic, so a thread takes
+// one atom or water (one workgroup over all of them took 346 µs at 252,480
+// sites, 6.2 µs now).
 __device__ __forceinline__ void
 k_md_energies(const float4* __restrict__ x, const float4* __restrict__ v,
               const float* __restrict__ mass, uint32_t n_dyn, uint32_t n_water, Box B,
-              const double* __restrict__ bpart, uint32_t n_bblk, double* __restrict__ out) {
-  __shared__ double red[5][1024];
-  const uint32_t t = threadIdx.x;
-  double a[5] = {0, 0, 0, 0, 0};
-  for (uint32_t i = t; i < n_dyn; i += 1024) {
+              double* __restrict__ out) {
+  __shared__ double red[2][kBlock];
+  const uint32_t t = threadIdx.x, i = blockIdx.x * kBlock + t;
+  double a0 = 0.0, a1 = 0.0;
+  if (i < n_dyn) {
     const float4 u = v[i];
-    const double k = 0.5 * (double)mass[i] * ((double)u.x * u.x + (double)u.y * u.y + (double)u.z * u.z);
-    a[0] += k;
-    a[4] += k;
-  }
-  for (uint32_t m = t; m < n_water; m += 1024) {
-    const uint32_t b = n_dyn + 4 * m;
+    a0 = a1 = 0.5 * (double)mass[i] * ((double)u.x * u.x + (double)u.y * u.y + (double)u.z * u.z);
+  } else if (i < n_dyn + n_water) {
+    const uint32_t b = n_dyn + 4 * (i - n_dyn);
     const uint32_t ss[3] = {b, b + 2, b + 3};
     const double ms[3] = {kMassO, kMassH, kMassH};
     double r[3][3], w[3][3], vc[3] = {0, 0, 0}, rc[3] = {0, 0, 0};
@@ -604,7 +631,7 @@ k_md_energies(const float4* __restrict__ x, const float4* __restrict__ v,
       w[k][0] = u.x;
       w[k][1] = u.y;
       w[k][2] = u.z;
-      a[0] += 0.5 * ms[k] * (w[k][0] * w[k][0] + w[k][1] * w[k][1] + w[k][2] * w[k][2]);
+      a0 += 0.5 * ms[k] * (w[k][0] * w[k][0] + w[k][1] * w[k][1] + w[k][2] * w[k][2]);
       for (int c = 0; c < 3; ++c) {
         vc[c] += ms[k] * w[k][c] / (double)kMassW;
         rc[c] += ms[k] * r[k][c] / (double)kMassW;
@@ -641,18 +668,17 @@ k_md_energies(const float4* __restrict__ x, const float4* __restrict__ v,
         krot += 0.5 * om * L[c];
       }
     }
-    a[4] += 0.5 * (double)kMassW * (vc[0] * vc[0] + vc[1] * vc[1] + vc[2] * vc[2]) + krot;
+    a1 = 0.5 * (double)kMassW * (vc[0] * vc[0] + vc[1] * vc[1] + vc[2] * vc[2]) + krot;
   }
-  for (uint32_t r = t; r < n_bblk; r += 1024)
-    for (int c = 0; c < 3; ++c) a[1 + c] += bpart[4 * r + c];
-  for (int c = 0; c < 5; ++c) red[c][t] = a[c];
+  red[0][t] = a0;
+  red[1][t] = a1;
   __syncthreads();
-  for (int s2 = 512; s2 > 0; s2 >>= 1) {
-    if (t < (uint32_t)s2)
-      for (int c = 0; c < 5; ++c) red[c][t] += red[c][t + s2];
+  for (uint32_t s2 = kBlock / 2; s2 > 0; s2 >>= 1) {
+    if (t < s2)
+      for (int c = 0; c < 2; ++c) red[c][t] += red[c][t + s2];
     __syncthreads();
   }
-  if (t < 5) out[t] = red[t][0];
+  if (t < 2) out[2 * blockIdx.x + t] = red[t][0];
 }
 
 // Pressure groups: every water (O, H0, H1; M is a virtual site), every
@@ -721,12 +747,18 @@ __device__ __forceinline__ double group_com(const GroupArgs& G, const float4* __
 // Per group: kinetic energy of the centre of mass ½M|V|² (amu Å²/ps²) and
 // the intra-group virial Σ (r_a − R)·F_a (kcal/mol; a water's M-site force
 // projected onto O and the H sites as the kick does); one partial pair per
-// workgroup.
+// workgroup.  Both go straight to pinned host memory, with the bonded partials
+// (n_bpart doubles): no copies for the host to wait for.
 __device__ __forceinline__ void k_md_press(GroupArgs G, const float4* __restrict__ x,
                                            const float4* __restrict__ v, Fx F,
-                                           double* __restrict__ partials, uint32_t nblk) {
+                                           double* __restrict__ partials,
+                                           const double* __restrict__ bpart,
+                                           double* __restrict__ h_bpart, uint32_t nblk,
+                                           uint32_t n_bpart) {
   __shared__ double red[2][kBlock];
   if (blockIdx.x >= nblk) return;
+  if (blockIdx.x == 0)
+    for (uint32_t k = threadIdx.x; k < n_bpart; k += kBlock) h_bpart[k] = bpart[k];
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   double kin = 0.0, cvir = 0.0;
   if (g < G.n_sgroups + G.n_water) {
@@ -1105,8 +1137,8 @@ struct dyn_md {
   DevBuf<uint32_t> cl_ptr;
   DevBuf<uint2> cons_ij;
   DevBuf<float> cons_r0sq, cons_invm;
-  DevBuf<double> eout;
-  PinnedBuf<double> h_out;
+  unsigned eblocks = 1;     // workgroups of k_md_energies
+  PinnedBuf<double> h_out;  // their partials
   uint64_t step = 0;
   DevBuf<uint64_t> step_dev;  // the step index (the Langevin noise's), a workgroup count
   uint64_t n_eval = 0;  // force evaluations since set_state (SPME cadence)
@@ -1116,7 +1148,6 @@ struct dyn_md {
   uint32_t n_sgroups = 0;
   DevBuf<uint32_t> grp_ptr, grp_atoms;
   unsigned pblocks = 1;
-  DevBuf<double> ppart;
   PinnedBuf<double> h_ppart, h_bpart;
   double pressure = std::nan(""), virial = std::nan(""), kin_com = std::nan("");
   uint64_t n_pcouple = 0;  // barostat rescalings so far
@@ -1277,7 +1308,7 @@ GroupArgs group_args(const dyn_md& M) {
 }
 
 // Enqueue the pressure parts of every MD of the set (the forces of the last
-// evaluation, the current velocities) and their copies to the host.
+// evaluation, the current velocities), which go to the host.
 void md_pressure_enqueue(MdSet& S) {
   Profiler::Scope ps(*S.prof, "md_pressure");
   unsigned g = 1;
@@ -1286,20 +1317,16 @@ void md_pressure_enqueue(MdSet& S) {
     dyn_md& m = *S.m[i];
     const Fx F = force_view(m);
     return args<k_md_press>(group_args(m), (const float4*)m.x.p, (const float4*)m.v.p, F,
-                            m.ppart.p, m.pblocks);
+                            m.h_ppart.p, (const double*)m.bpart.p, m.h_bpart.p, m.pblocks,
+                            4u * m.bblocks);
   });
-  for (dyn_md* m : S.m) {
-    DYN_HIP(hipMemcpyAsync(m->h_ppart.p, m->ppart.p, sizeof(double) * 2 * m->pblocks,
-                           hipMemcpyDeviceToHost, S.R.stream));
-    DYN_HIP(hipMemcpyAsync(m->h_bpart.p, m->bpart.p, sizeof(double) * 4 * m->bblocks,
-                           hipMemcpyDeviceToHost, S.R.stream));
-  }
 }
 
 constexpr double kBarPerKcalMolA3 = 69476.95457055373;  // src/barostat.rs:22
 constexpr double kKbBarA3 = 138.0649;                   // k_B in bar·Å³/K, src/barostat.rs:26
 
-// Pressure (bar) from the copies md_pressure_enqueue made, after the wait:
+// Pressure (bar) from what md_pressure_enqueue left, after the wait and the
+// engine's check:
 // P = (2 K_com + W)/(3V) over the pressure groups (src/barostat.rs:419-431
 // with the group virial W = W_nonbonded + W_bonded − Σ_g Σ_a (r_a − R_g)·F_a).
 double md_pressure_finish(dyn_md& m) {
@@ -1311,7 +1338,7 @@ double md_pressure_finish(dyn_md& m) {
   if (m.n_bond + m.n_angle + m.n_dihe)
     for (unsigned b = 0; b < m.bblocks; ++b) wb += m.h_bpart.p[4 * b + 3];
   dyn_energies E{};
-  engine_call(dyn_engine_get_energies(m.eng, &E), m.eng);
+  engine_report_energies(m.eng, &E);
   const double V = (double)m.box[0] * m.box[1] * m.box[2];
   m.kin_com = kin / (double)kKcalToNative;
   m.virial = E.virial_sr + E.virial_recip + wb - cvir;
@@ -1891,7 +1918,6 @@ extern "C" int dyn_md_create(dyn_md** out, dyn_engine* eng, const dyn_md_params*
       up(M->grp_ptr, gptr.data(), gptr.size(), 4);
       up(M->grp_atoms, gat.data(), gat.size(), 4);
       M->pblocks = grid_for(std::max<uint32_t>(M->n_sgroups + nw, 1), kBlock);
-      M->ppart.reserve(2 * (size_t)M->pblocks);
       M->h_ppart.reserve(2 * (size_t)M->pblocks);
       M->h_bpart.reserve(4 * (size_t)M->bblocks);
     }
@@ -1907,8 +1933,8 @@ extern "C" int dyn_md_create(dyn_md** out, dyn_engine* eng, const dyn_md_params*
     M->v_ck.reserve(ns);
     M->step_dev.reserve(2);  // the step index, the workgroup count of k_md_step_ba
     DYN_HIP(hipMemsetAsync(M->step_dev.p, 0, 16, M->stream));
-    M->eout.reserve(8);
-    M->h_out.reserve(8);
+    M->eblocks = grid_for(std::max<uint32_t>(nd + nw, 1), kBlock);
+    M->h_out.reserve(2 * (size_t)M->eblocks);
     DYN_HIP(hipStreamSynchronize(M->stream));
     *out = M.release();
     return DYN_OK;
@@ -1991,25 +2017,24 @@ extern "C" int dyn_md_get_state(dyn_md* md, float* pos_dyn, float* vel_dyn, floa
   DYN_API_BODY(md, {
     DeviceGuard g(md->device);
     if (!md->state_set) throw Error(DYN_ERR_STATE, "state not set");
-    engine_call(dyn_engine_sync(md->eng), md->eng);
-    const uint32_t nd = md->n_dyn, nw = md->n_water, ns = md->n_sites;
-    std::vector<float4> hx(ns), hv(ns);
-    DYN_HIP(hipMemcpyAsync(hx.data(), md->x.p, 16 * (size_t)ns, hipMemcpyDeviceToHost, md->stream));
-    DYN_HIP(hipMemcpyAsync(hv.data(), md->v.p, 16 * (size_t)ns, hipMemcpyDeviceToHost, md->stream));
-    DYN_HIP(hipStreamSynchronize(md->stream));
-    for (uint32_t i = 0; i < nd; ++i) {
-      if (pos_dyn) memcpy(pos_dyn + 3 * i, &hx[i], 12);
-      if (vel_dyn) memcpy(vel_dyn + 3 * i, &hv[i], 12);
-    }
-    for (uint32_t m = 0; m < nw; ++m) {
-      if (pos_water)
-        for (int k = 0; k < 4; ++k) memcpy(pos_water + 12 * (size_t)m + 3 * k, &hx[nd + 4 * m + k], 12);
-      if (vel_water) {
-        memcpy(vel_water + 9 * (size_t)m, &hv[nd + 4 * m], 12);
-        memcpy(vel_water + 9 * (size_t)m + 3, &hv[nd + 4 * m + 2], 12);
-        memcpy(vel_water + 9 * (size_t)m + 6, &hv[nd + 4 * m + 3], 12);
-      }
-    }
+    const uint32_t nd = md->n_dyn, nw = md->n_water;
+    // (6·nd + 21·nw floats: the stage holds 6 per site)
+    float* const h = static_cast<float*>(engine_host_stage(md->eng));
+    MdSet S = self_set(md);
+    launch<k_md_state_out>(S.R, "k_md_state_out", 0, grid_for(6 * (size_t)nd + 21 * (size_t)nw, kBlock),
+                           kBlock, 0, [&](uint32_t) {
+      return args<k_md_state_out>((const float*)md->x.p, (const float*)md->v.p, nd, nw, h);
+    });
+    engine_check(md->eng);
+    size_t at = 0;
+    auto take = [&](float* out, size_t n) {
+      if (out && n) memcpy(out, h + at, sizeof(float) * n);
+      at += n;
+    };
+    take(pos_dyn, 3 * (size_t)nd);
+    take(vel_dyn, 3 * (size_t)nd);
+    take(pos_water, 12 * (size_t)nw);
+    take(vel_water, 9 * (size_t)nw);
   });
 }
 
@@ -2023,32 +2048,34 @@ extern "C" int dyn_md_get_energies(dyn_md* md, dyn_md_energies* out) {
     if (!md->forces_valid) md_forces(S, true);
     Box B;
     for (int a = 0; a < 3; ++a) B.L[a] = md->box[a];
-    launch<k_md_energies, 1024>(S.R, "k_md_energies", 0, 1, 1024, 0, [&](uint32_t) {
-      return args<k_md_energies>(md->x.p, md->v.p, md->mass.p, md->n_dyn, md->n_water, B,
-                                 md->bpart.p,
-                                 (md->n_bond + md->n_angle + md->n_dihe) ? md->bblocks : 0u,
-                                 md->eout.p);
+    // the kinetic energies, the pressure of the current velocities and the
+    // last evaluation's forces, the engine's report: one wait
+    launch<k_md_energies, kBlock>(S.R, "k_md_energies", 0, md->eblocks, kBlock, 0, [&](uint32_t) {
+      return args<k_md_energies>((const float4*)md->x.p, (const float4*)md->v.p,
+                                 (const float*)md->mass.p, md->n_dyn, md->n_water, B, md->h_out.p);
     });
-    DYN_HIP(hipMemcpyAsync(md->h_out.p, md->eout.p, 5 * sizeof(double), hipMemcpyDeviceToHost,
-                           md->stream));
-    engine_call(dyn_engine_sync(md->eng), md->eng);
-    DYN_HIP(hipStreamSynchronize(md->stream));
+    md_pressure_enqueue(S);
+    engine_check(md->eng);
+    double kin = 0.0, kin_rigid = 0.0, eb[3] = {0.0, 0.0, 0.0};
+    for (unsigned b = 0; b < md->eblocks; ++b) {
+      kin += md->h_out.p[2 * b];
+      kin_rigid += md->h_out.p[2 * b + 1];
+    }
+    if (md->n_bond + md->n_angle + md->n_dihe)
+      for (unsigned b = 0; b < md->bblocks; ++b)
+        for (int c = 0; c < 3; ++c) eb[c] += md->h_bpart.p[4 * b + c];
     dyn_md_energies E{};
-    E.kinetic = md->h_out.p[0] / (double)kKcalToNative;
-    E.kinetic_rigid = md->h_out.p[4] / (double)kKcalToNative;
-    E.bond = md->h_out.p[1];
-    E.angle = md->h_out.p[2];
-    E.dihedral = md->h_out.p[3];
+    E.kinetic = kin / (double)kKcalToNative;
+    E.kinetic_rigid = kin_rigid / (double)kKcalToNative;
+    E.bond = eb[0];
+    E.angle = eb[1];
+    E.dihedral = eb[2];
     // degrees of freedom: 3 per solute atom less one per constraint, 6 per
     // rigid water
     const double dof = 3.0 * md->n_dyn - (double)md->n_cons + 6.0 * md->n_water;
     E.dof = dof;
-    E.temperature = dof > 0 ? 2.0 * md->h_out.p[4] / (dof * (double)kKb) : 0.0;
+    E.temperature = dof > 0 ? 2.0 * kin_rigid / (dof * (double)kKb) : 0.0;
     E.steps = md->step;
-    // pressure of the current velocities and the last evaluation's forces
-    md_pressure_enqueue(S);
-    engine_call(dyn_engine_sync(md->eng), md->eng);
-    DYN_HIP(hipStreamSynchronize(md->stream));
     try {
       E.pressure = md_pressure_finish(*md);
     } catch (const Error& e) {
@@ -2064,14 +2091,13 @@ extern "C" int dyn_md_get_energies(dyn_md* md, dyn_md_energies* out) {
     E.potential_bonded = E.bond + E.angle + E.dihedral;
     {
       dyn_energies EE{};
-      const int rc = dyn_engine_get_energies(md->eng, &EE);
-      if (rc == DYN_OK) {
+      try {
+        engine_report_energies(md->eng, &EE);
         E.potential_nonbonded = md->eng_mode_reference ? EE.reference : EE.total;
         E.dh_dl = EE.dh_dl;
-      } else if (rc == DYN_ERR_STATE) {  // the last evaluation skipped energies
+      } catch (const Error& e) {
+        if (e.code != DYN_ERR_STATE) throw;  // the last evaluation skipped energies
         E.potential_nonbonded = E.dh_dl = std::nan("");
-      } else {
-        engine_call(rc, md->eng);
       }
     }
     E.potential = E.potential_nonbonded + E.potential_bonded;
