@@ -78,13 +78,6 @@ __device__ __forceinline__ void pme_bin_charge(const BinArgs& B, float4 p, bool 
   }
 }
 
-struct FftAxis {
-  int N;
-  int nstages;
-  int radix[16];
-};
-
-FftAxis make_fft_axis(int N);  // throws if N has a prime factor > 5
 bool is_235_smooth(uint32_t n);
 
 // Position/charge input for spreading and gathering: float4 (x, y, z, q).
@@ -95,16 +88,16 @@ struct PmeCore {
   hipStream_t stream = nullptr;
   Profiler* prof = nullptr;
   uint32_t K[3] = {0, 0, 0};
+  uint64_t plan[3] = {0, 0, 0};  // FFT radices per axis (fft_plan)
   float L[3] = {0, 0, 0};
   float beta = 0.f;
   int order = 4;
   size_t ngrid = 0;
-  FftAxis ax[3];
-  DevBuf<FftAxis> ax_dev;       // device copy of ax
+  size_t nspec = 0;  // K0·K1·(K2/2 + 1): points of the half spectrum
   bool f64 = false;             // FP64 option: the *64 buffers replace their f32 twins
   DevBuf<int64_t> grid_fx;      // K0·K1·K2 fixed-point charge grid
-  DevBuf<float2> cgrid;         // complex working grid
-  DevBuf<float> G;              // influence function
+  DevBuf<float2> cgrid;         // half spectrum, then (as floats) the potential
+  DevBuf<float> G;              // influence function on the half spectrum
   DevBuf<double> bsq;           // 1/|b_a(m)|² per axis (K0 + K1 + K2 values)
   DevBuf<float2> tw[3];         // e^{-2πi k/N} tables per axis
   DevBuf<double2> cgrid64;

@@ -1,5 +1,5 @@
 // pme.hip — SPME reciprocal space on gfx950: fixed-point B-spline charge
-// spreading, a mixed-radix (2/3/4/5) Stockham FFT staged through LDS, the
+// spreading, real mixed-radix (8/4/2/9/3/5) Stockham FFTs staged through LDS, the
 // influence-function convolution fused into the x-axis pass with FP64 energy
 // and virial reductions, and the force gather.  Replaces the `ewald` crate's
 // PmeRecip (used at src/non_bonded.rs:681-795, :850-875).
@@ -29,30 +29,26 @@ bool is_235_smooth(uint32_t n) {
   return n == 1;
 }
 
-FftAxis make_fft_axis(int N) {
-  FftAxis a;
-  a.N = N;
-  a.nstages = 0;
-  int n = N;
-  // radix-4 first, then 2, 3, 5
-  while (n % 4 == 0) {
-    a.radix[a.nstages++] = 4;
-    n /= 4;
-  }
-  while (n % 2 == 0) {
-    a.radix[a.nstages++] = 2;
-    n /= 2;
-  }
-  while (n % 3 == 0) {
-    a.radix[a.nstages++] = 3;
-    n /= 3;
-  }
-  while (n % 5 == 0) {
-    a.radix[a.nstages++] = 5;
-    n /= 5;
-  }
-  if (n != 1) throw Error(DYN_ERR_ARG, fmt("grid size %d has a prime factor above 5", N));
-  return a;
+// Radices of an FFT of length N, the first in the lowest four bits (0: no
+// more): few stages — 8 while what is left of the twos is not 2 or 4, then 4s,
+// 2; 9, 3; 5.
+static uint64_t fft_plan(uint32_t N) {
+  uint64_t plan = 0;
+  int at = 0;
+  uint32_t n = N;
+  auto take = [&](uint32_t r) {
+    plan |= (uint64_t)r << at;
+    at += 4;
+    n /= r;
+  };
+  while (n % 8 == 0 && (n % 16 != 0 || n % 32 == 0)) take(8);
+  while (n % 4 == 0) take(4);
+  while (n % 2 == 0) take(2);
+  while (n % 9 == 0) take(9);
+  while (n % 3 == 0) take(3);
+  while (n % 5 == 0) take(5);
+  if (n != 1) throw Error(DYN_ERR_ARG, fmt("grid size %u has a prime factor above 5", N));
+  return plan;
 }
 
 }  // namespace dyn
@@ -62,7 +58,10 @@ using namespace dyn;
 namespace {
 
 constexpr int kFftBlock = 256;
-constexpr int kFftCap = 2048;  // complex elements per workgroup (two LDS buffers: 32 KB)
+constexpr int kFftCap = 4096;      // complex elements of a pass's LDS buffer, at most
+constexpr int kFftLines = 16;      // lines per workgroup where the grid has enough of them
+constexpr size_t kPlaneLds = 64u << 10;  // LDS of a plane launch and its workgroups, at most
+constexpr unsigned kPlaneGroups = 256;
 
 // Complex arithmetic on float2 (the default SPME) or double2 (the FP64
 // option).
@@ -75,6 +74,10 @@ struct CxT<float2> {
   static constexpr float c3 = -0.5f, s3 = 0.866025403784438647f;
   static constexpr float c51 = 0.309016994374947424f, c52 = -0.809016994374947424f;
   static constexpr float s51 = 0.951056516295153572f, s52 = 0.587785252292473129f;
+  static constexpr float h = 0.707106781186547524f;  // √½; cos and sin of 40°, 80°, 160°:
+  static constexpr float c91 = 0.766044443118978035f, s91 = 0.642787609686539327f;
+  static constexpr float c92 = 0.173648177666930349f, s92 = 0.984807753012208059f;
+  static constexpr float c94 = -0.939692620785908384f, s94 = 0.342020143325668733f;
 };
 template <>
 struct CxT<double2> {
@@ -83,12 +86,23 @@ struct CxT<double2> {
   static constexpr double c3 = -0.5, s3 = 0.866025403784438647;
   static constexpr double c51 = 0.309016994374947424, c52 = -0.809016994374947424;
   static constexpr double s51 = 0.951056516295153572, s52 = 0.587785252292473129;
+  static constexpr double h = 0.707106781186547524;
+  static constexpr double c91 = 0.766044443118978035, s91 = 0.642787609686539327;
+  static constexpr double c92 = 0.173648177666930349, s92 = 0.984807753012208059;
+  static constexpr double c94 = -0.939692620785908384, s94 = 0.342020143325668733;
 };
 
 template <class C>
 __device__ __forceinline__ C cadd(C a, C b) { return CxT<C>::mk(a.x + b.x, a.y + b.y); }
 template <class C>
 __device__ __forceinline__ C csub(C a, C b) { return CxT<C>::mk(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ float rfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double rfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// a + b·s
+template <class C>
+__device__ __forceinline__ C cfma(C b, typename CxT<C>::R s, C a) {
+  return CxT<C>::mk(rfma(b.x, s, a.x), rfma(b.y, s, a.y));
+}
 template <class C>
 __device__ __forceinline__ C cscale(C a, typename CxT<C>::R s) { return CxT<C>::mk(a.x * s, a.y * s); }
 // multiply by SIGN·i
@@ -100,7 +114,7 @@ __device__ __forceinline__ C cmul_si(C a) {
 template <int SIGN, class C>
 __device__ __forceinline__ C ctw(C v, C t) {
   const typename CxT<C>::R ti = SIGN < 0 ? t.y : -t.y;
-  return CxT<C>::mk(v.x * t.x - v.y * ti, v.x * ti + v.y * t.x);
+  return CxT<C>::mk(rfma(v.x, t.x, -(v.y * ti)), rfma(v.x, ti, v.y * t.x));
 }
 
 template <int SIGN, class C>
@@ -121,21 +135,21 @@ __device__ __forceinline__ void dft4(C* v) {
 template <int SIGN, class C>
 __device__ __forceinline__ void dft3(C* v) {
   const C t = cadd(v[1], v[2]);
-  const C d = cscale(cmul_si<SIGN>(csub(v[1], v[2])), CxT<C>::s3);
-  const C a = cadd(v[0], cscale(t, CxT<C>::c3));
+  const C d = cmul_si<SIGN>(csub(v[1], v[2]));
+  const C a = cfma(t, CxT<C>::c3, v[0]);
   v[0] = cadd(v[0], t);
-  v[1] = cadd(a, d);
-  v[2] = csub(a, d);
+  v[1] = cfma(d, CxT<C>::s3, a);
+  v[2] = cfma(d, -CxT<C>::s3, a);
 }
 template <int SIGN, class C>
 __device__ __forceinline__ void dft5(C* v) {
   const auto c1 = CxT<C>::c51, c2 = CxT<C>::c52, s1 = CxT<C>::s51, s2 = CxT<C>::s52;
   const C t1 = cadd(v[1], v[4]), t2 = cadd(v[2], v[3]);
   const C d1 = csub(v[1], v[4]), d2 = csub(v[2], v[3]);
-  const C a1 = cadd(v[0], cadd(cscale(t1, c1), cscale(t2, c2)));
-  const C a2 = cadd(v[0], cadd(cscale(t1, c2), cscale(t2, c1)));
-  const C b1 = cmul_si<SIGN>(cadd(cscale(d1, s1), cscale(d2, s2)));
-  const C b2 = cmul_si<SIGN>(csub(cscale(d1, s2), cscale(d2, s1)));
+  const C a1 = cfma(t1, c1, cfma(t2, c2, v[0]));
+  const C a2 = cfma(t1, c2, cfma(t2, c1, v[0]));
+  const C b1 = cmul_si<SIGN>(cfma(d1, s1, cscale(d2, s2)));
+  const C b2 = cmul_si<SIGN>(cfma(d1, s2, cscale(d2, -s1)));
   v[0] = cadd(v[0], cadd(t1, t2));
   v[1] = cadd(a1, b1);
   v[4] = csub(a1, b1);
@@ -143,34 +157,55 @@ __device__ __forceinline__ void dft5(C* v) {
   v[3] = csub(a2, b2);
 }
 
-// One radix-R Stockham stage with compile-time sizes (line length N,
-// sub-transform length NS): the index arithmetic folds to shifts and masks.
-template <int SIGN, int N, int R, int NS, class C>
-__device__ __forceinline__ void fft_stage(const C* __restrict__ a, C* __restrict__ b, int nl,
-                                          const C* __restrict__ tw) {
-  constexpr int NR = N / R, TWS = N / (NS * R);
-  const int total = nl * NR;
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int l = i / NR;
-    const int j = i - l * NR;
-    const int k = j % NS;
-    const C* src = a + l * N;
-    C* dst = b + l * N;
-    C v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      C x = src[j + r * NR];
-      if (r) x = ctw<SIGN>(x, tw[(r * k * TWS) % N]);
-      v[r] = x;
-    }
-    if constexpr (R == 4) dft4<SIGN>(v);
-    else dft2<SIGN>(v);
-    const int d = (j / NS) * NS * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) dst[d + r * NS] = v[r];
-  }
-  __syncthreads();
+template <int SIGN, class C>
+__device__ __forceinline__ void dft8(C* v) {
+  const auto h = CxT<C>::h;
+  C e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
+  dft4<SIGN>(e);
+  dft4<SIGN>(o);
+  const C i1 = cmul_si<SIGN>(o[1]), i3 = cmul_si<SIGN>(o[3]);
+  o[1] = cadd(o[1], i1);  // times √½: · e^{SIGN·iπ/4}
+  o[2] = cmul_si<SIGN>(o[2]);
+  o[3] = csub(i3, o[3]);  // times √½: · e^{SIGN·3iπ/4}
+  v[0] = cadd(e[0], o[0]);
+  v[4] = csub(e[0], o[0]);
+  v[1] = cfma(o[1], h, e[1]);
+  v[5] = cfma(o[1], -h, e[1]);
+  v[2] = cadd(e[2], o[2]);
+  v[6] = csub(e[2], o[2]);
+  v[3] = cfma(o[3], h, e[3]);
+  v[7] = cfma(o[3], -h, e[3]);
 }
+template <int SIGN, class C>
+__device__ __forceinline__ void dft9(C* v) {
+  using R = typename CxT<C>::R;
+  const R sg = SIGN < 0 ? R(-1) : R(1);
+  C c[3][3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    c[q][0] = v[q];
+    c[q][1] = v[q + 3];
+    c[q][2] = v[q + 6];
+    dft3<SIGN>(c[q]);
+  }
+  auto mul = [&](C z, R wc, R ws) { return CxT<C>::mk(rfma(z.x, wc, -(z.y * (sg * ws))), rfma(z.x, sg * ws, z.y * wc)); };
+  c[1][1] = mul(c[1][1], CxT<C>::c91, CxT<C>::s91);
+  c[1][2] = mul(c[1][2], CxT<C>::c92, CxT<C>::s92);
+  c[2][1] = mul(c[2][1], CxT<C>::c92, CxT<C>::s92);
+  c[2][2] = mul(c[2][2], CxT<C>::c94, CxT<C>::s94);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    C o[3] = {c[0][k], c[1][k], c[2][k]};
+    dft3<SIGN>(o);
+    v[k] = o[0];
+    v[k + 3] = o[1];
+    v[k + 6] = o[2];
+  }
+}
+
+// The reciprocal fast_div takes (within an ulp: no correctly rounded
+// division, whose latency a small pass would show).
+__device__ __forceinline__ float fast_rcp(int d) { return __builtin_amdgcn_rcpf((float)d); }
 
 // x / d for 0 ≤ x < 2²² by a float reciprocal and one correction step.
 __device__ __forceinline__ int fast_div(int x, int d, float rd) {
@@ -181,73 +216,60 @@ __device__ __forceinline__ int fast_div(int x, int d, float rd) {
   return q;
 }
 
-// One radix-R Stockham stage with the line length and sub-transform length
-// known at run time (the general grids): the radix is a template parameter so
-// the butterfly stays in registers, and the divisions use fast_div.  The
-// twiddle index r·k·(N/(Ns·R)) stays below N.
+// One radix-R Stockham stage of nl lines of length N in LDS, element n of
+// line l at a[n·S + l]: consecutive threads take consecutive lines, so a
+// wave's LDS accesses are contiguous, and the index arithmetic is paid once
+// per R points.  Ns: length of the sub-transforms so far, M = N/Ns.  The
+// twiddle index r·k·(M/R) stays below N.
 template <int SIGN, int R, class C>
-__device__ __forceinline__ void fft_stage_rt(const C* __restrict__ a, C* __restrict__ b, int nl,
-                                             int N, int Ns, const C* __restrict__ tw) {
-  const int NR = N / R, tws = N / (Ns * R);
-  const float rNR = 1.0f / (float)NR, rNs = 1.0f / (float)Ns;
+__device__ __forceinline__ void fft_stage(const C* __restrict__ a, C* __restrict__ b, int nl, int S,
+                                          int N, int Ns, int M, const C* __restrict__ tw) {
+  const int NR = N / R, tws = M / R;
+  const float rnl = fast_rcp(nl), rNs = fast_rcp(Ns);
   const int total = nl * NR;
   for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int l = fast_div(i, NR, rNR);
-    const int j = i - l * NR;
-    const int q = fast_div(j, Ns, rNs);
-    const int k = j - q * Ns;
-    const C* src = a + l * N;
-    C* dst = b + l * N;
+    const int j = fast_div(i, nl, rnl);
+    const int l = i - j * nl;
+    const C* src = a + j * S + l;
     C v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      C x = src[j + r * NR];
-      if (r) x = ctw<SIGN>(x, tw[r * k * tws]);
-      v[r] = x;
+    for (int r = 0; r < R; ++r) v[r] = src[r * NR * S];
+    int d = j * R;
+    if (Ns > 1) {
+      const int q = fast_div(j, Ns, rNs), k = j - q * Ns;
+      d = q * Ns * R + k;
+#pragma unroll
+      for (int r = 1; r < R; ++r) v[r] = ctw<SIGN>(v[r], tw[r * k * tws]);
     }
-    if constexpr (R == 4) dft4<SIGN>(v);
+    if constexpr (R == 8) dft8<SIGN>(v);
+    else if constexpr (R == 4) dft4<SIGN>(v);
     else if constexpr (R == 2) dft2<SIGN>(v);
+    else if constexpr (R == 9) dft9<SIGN>(v);
     else if constexpr (R == 3) dft3<SIGN>(v);
     else dft5<SIGN>(v);
-    const int d = q * Ns * R + k;
+    C* dst = b + d * S + l;
 #pragma unroll
-    for (int r = 0; r < R; ++r) dst[d + r * Ns] = v[r];
+    for (int r = 0; r < R; ++r) dst[r * Ns * S] = v[r];
   }
   __syncthreads();
 }
 
-// The same transform as lds_fft for the power-of-two lengths of common grids
-// (radix 4 first, then 2, the plan of make_fft_axis).
-template <int SIGN, int N, class C>
-__device__ __forceinline__ C* lds_fft_pow2(C* a, C* b, int nl, const C* __restrict__ tw) {
-  static_assert(N == 32 || N == 64 || N == 128, "fixed plans for 32, 64 and 128 points");
-  fft_stage<SIGN, N, 4, 1>(a, b, nl, tw);
-  fft_stage<SIGN, N, 4, 4>(b, a, nl, tw);
-  if constexpr (N == 32) {
-    fft_stage<SIGN, N, 2, 16>(a, b, nl, tw);
-    return b;
-  } else {
-    fft_stage<SIGN, N, 4, 16>(a, b, nl, tw);
-    if constexpr (N == 64) return b;
-    fft_stage<SIGN, N, 2, 64>(b, a, nl, tw);
-    return a;
-  }
-}
-
-// Stockham autosort FFT of nl lines of length N held in LDS as a[l·N + n].
-// Returns the buffer holding the (natural-order) result.  NF: a line length
-// every system of the launch shares (32, 64 or 128: the fixed plan), or 0.
-template <int SIGN, int NF, class C>
-__device__ C* lds_fft(C* a, C* b, int nl, const FftAxis& ax, const C* __restrict__ tw) {
-  if constexpr (NF != 0) return lds_fft_pow2<SIGN, NF>(a, b, nl, tw);
-  const int N = ax.N;
-  int Ns = 1;
-  for (int s = 0; s < ax.nstages; ++s) {
-    const int R = ax.radix[s];
-    if (R == 4) fft_stage_rt<SIGN, 4>(a, b, nl, N, Ns, tw);
-    else if (R == 2) fft_stage_rt<SIGN, 2>(a, b, nl, N, Ns, tw);
-    else if (R == 3) fft_stage_rt<SIGN, 3>(a, b, nl, N, Ns, tw);
-    else fft_stage_rt<SIGN, 5>(a, b, nl, N, Ns, tw);
+// Stockham autosort FFT of nl lines held in LDS (fft_stage's layout), plan
+// as fft_plan packs it.  Returns the buffer holding the (natural-order)
+// result.  A line sees the same stages and arithmetic in every kernel and
+// grouping.
+template <int SIGN, class C>
+__device__ __forceinline__ C* lds_fft(C* a, C* b, int nl, int S, int N, uint64_t plan,
+                                      const C* __restrict__ tw) {
+  int Ns = 1, M = N;
+  for (; plan != 0; plan >>= 4) {
+    const int R = (int)(plan & 15u);
+    if (R == 8) fft_stage<SIGN, 8>(a, b, nl, S, N, Ns, M, tw), M /= 8;
+    else if (R == 4) fft_stage<SIGN, 4>(a, b, nl, S, N, Ns, M, tw), M /= 4;
+    else if (R == 2) fft_stage<SIGN, 2>(a, b, nl, S, N, Ns, M, tw), M /= 2;
+    else if (R == 9) fft_stage<SIGN, 9>(a, b, nl, S, N, Ns, M, tw), M /= 9;
+    else if (R == 3) fft_stage<SIGN, 3>(a, b, nl, S, N, Ns, M, tw), M /= 3;
+    else fft_stage<SIGN, 5>(a, b, nl, S, N, Ns, M, tw), M /= 5;
     C* t = a;
     a = b;
     b = t;
@@ -256,148 +278,251 @@ __device__ C* lds_fft(C* a, C* b, int nl, const FftAxis& ax, const C* __restrict
   return a;
 }
 
-// The stage of fft_stage on nl lines stored interleaved (element n of line l
-// at a[n·NL + l]): consecutive threads take consecutive lines, so a wave's
-// LDS accesses are contiguous.  Every line sees the arithmetic of fft_stage.
-template <int SIGN, int N, int R, int NS, int NL, class C>
-__device__ __forceinline__ void fft_stage_t(const C* __restrict__ a, C* __restrict__ b,
-                                            const C* __restrict__ tw) {
-  constexpr int NR = N / R, TWS = N / (NS * R);
-  for (int i = threadIdx.x; i < NL * NR; i += blockDim.x) {
-    const int j = i / NL;
-    const int l = i - j * NL;
-    const int k = j % NS;
-    C v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      C x = a[(j + r * NR) * NL + l];
-      if (r) x = ctw<SIGN>(x, tw[(r * k * TWS) % N]);
-      v[r] = x;
-    }
-    if constexpr (R == 4) dft4<SIGN>(v);
-    else dft2<SIGN>(v);
-    const int d = (j / NS) * NS * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) b[(d + r * NS) * NL + l] = v[r];
-  }
-  __syncthreads();
-}
-
-// lds_fft_pow2 on NL interleaved lines.
-template <int SIGN, int N, int NL, class C>
-__device__ __forceinline__ C* lds_fft_pow2_t(C* a, C* b, const C* __restrict__ tw) {
-  static_assert(N == 32 || N == 64, "plane passes for 32 and 64 points");
-  fft_stage_t<SIGN, N, 4, 1, NL>(a, b, tw);
-  fft_stage_t<SIGN, N, 4, 4, NL>(b, a, tw);
-  if constexpr (N == 32) {
-    fft_stage_t<SIGN, N, 2, 16, NL>(a, b, tw);
-  } else {
-    fft_stage_t<SIGN, N, 4, 16, NL>(a, b, tw);
-  }
-  return b;
-}
-
-struct PassGeom {
+// The transforms.  The charge grid and the potential are real, so the
+// spectrum holds only kz = 0 … Kz/2 (nh values a line), which halves the y
+// and x passes: two z lines (y = 2p and 2p + 1 of an x plane, a pair) are the
+// real and imaginary parts of one complex transform, taken apart after it
+// and put together before the inverse one.  Spectrum element (x, y, kz) lies
+// at (x·Ky + y)·nh + kz.
+//
+// Bound: memory and LDS traffic, and launch latency on small grids.  A
+// workgroup of a y or x pass takes about 16 consecutive kz (128 bytes) of
+// every element of its lines: whole cache lines, which with 4 consecutive
+// values were fetched by four workgroups on different XCDs.  Radix 8 and 9
+// stages halve the LDS exchanges of radix 4 and 3.  128³ alone: z pass 12 µs, y 14,
+// x with the convolution 19 (complex radix-4 passes of 4 lines: 12 to 28, and 37).
+struct FftGeom {
   int K[3];
-  int lines;      // total lines in this pass
-  int L;          // lines per workgroup
+  int nh;  // kz values of the spectrum: K[2]/2 + 1
+  int np;  // z-line pairs per x plane
+  int L;   // lines (pairs, kz columns) per workgroup
+  uint64_t plan[3];
 };
+static_assert(sizeof(FftGeom) == 48, "FftGeom has no padding");
 
-// Address of element n of line `line` for the axis pass AXIS (0 = x, 1 = y, 2 = z).
-template <int AXIS>
-__device__ __forceinline__ size_t pass_addr(const PassGeom& g, int line, int n) {
-  if (AXIS == 2) return (size_t)line * g.K[2] + n;
-  if (AXIS == 1) {
-    const int x = line / g.K[2], z = line - x * g.K[2];
-    return ((size_t)x * g.K[1] + n) * g.K[2] + z;
-  }
-  const int y = line / g.K[2], z = line - y * g.K[2];
-  return ((size_t)n * g.K[1] + y) * g.K[2] + z;
+// Sizes known to be the same in every lane (an argument pack in memory would
+// keep them, and all index arithmetic on them, in vector registers).
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ FftGeom uni(const FftGeom& g) {
+  FftGeom u;
+  for (int a = 0; a < 3; ++a) u.K[a] = uni(g.K[a]);
+  u.nh = uni(g.nh);
+  u.np = uni(g.np);
+  u.L = uni(g.L);
+  for (int a = 0; a < 3; ++a)
+    u.plan[a] = (uint64_t)(uint32_t)uni((int)(g.plan[a] >> 32)) << 32 | (uint32_t)uni((int)g.plan[a]);
+  return u;
 }
 
-// LDS element e of a group ↔ (line l, point n).  z lines are contiguous in
-// memory so n runs fastest; for y and x lines, consecutive lines are
-// consecutive in z, so l runs fastest and loads stay coalesced.
-template <int AXIS>
-__device__ __forceinline__ void split_e(int e, int L, int N, int& l, int& n) {
-  if (AXIS == 2) {
-    l = e / N;
-    n = e - l * N;
-  } else {
-    n = e / L;
-    l = e - n * L;
-  }
-}
-
-// One FFT pass along AXIS over complex data in place.  FROM_FX: the input is
-// the int64 fixed-point charge grid (z pass only).
-template <int AXIS, int SIGN, bool FROM_FX, class C, int NF>
-__device__ __forceinline__ void
-k_fft_pass(C* __restrict__ data, const int64_t* __restrict__ grid_fx, PassGeom g,
-           const FftAxis* __restrict__ axp, const C* __restrict__ tw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  C* smem = reinterpret_cast<C*>(smem_raw);
+// A pair's line spectra from the transform X of its combination: A = (X(k) +
+// conj X(−k))/2, B = (X(k) − conj X(−k))/2i.
+template <class C>
+__device__ __forceinline__ void pair_split(C x, C y, C& A, C& B) {
   using R = typename CxT<C>::R;
-  const FftAxis& ax = *axp;  // device copy: uniform loads, no private copy
-  const int N = ax.N;
-  const int line0 = blockIdx.x * g.L;
-  if (line0 >= g.lines) return;  // beyond this system's lines
-  const int nl = min(g.L, g.lines - line0);
-  C* A = smem;
-  C* B = smem + g.L * N;
-  const int tot = nl * N;
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, n;
-    split_e<AXIS>(e, nl, N, l, n);
-    const size_t addr = pass_addr<AXIS>(g, line0 + l, n);
-    C v;
-    if (FROM_FX) v = CxT<C>::mk((R)((double)grid_fx[addr] * (1.0 / DYN_GRID_FX_SCALE)), R(0));
-    else v = data[addr];
-    A[l * N + n] = v;
+  A = CxT<C>::mk(R(0.5) * (x.x + y.x), R(0.5) * (x.y - y.y));
+  B = CxT<C>::mk(R(0.5) * (x.y + y.y), R(0.5) * (y.x - x.x));
+}
+
+// Puts A(k) + iB(k) of a pair into column l of the LDS lines, at k and, from
+// the conjugates, at N − k (the values at k = 0 and N/2 are real).
+template <class C>
+__device__ __forceinline__ void pair_join(C* __restrict__ a, int S, int l, int k, int N, C A, C B) {
+  if (k == 0 || 2 * k == N) {
+    a[k * S + l] = CxT<C>::mk(A.x, B.x);
+    return;
   }
-  __syncthreads();
-  C* Rs = lds_fft<SIGN, NF>(A, B, nl, ax, tw);
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, n;
-    split_e<AXIS>(e, nl, N, l, n);
-    data[pass_addr<AXIS>(g, line0 + l, n)] = Rs[l * N + n];
+  a[k * S + l] = CxT<C>::mk(A.x - B.y, A.y + B.x);
+  a[(N - k) * S + l] = CxT<C>::mk(A.x + B.y, B.x - A.y);
+}
+
+// put(e, load(e)) for the workgroup's e in [0, n), a thread's next kAhead
+// loads in flight together (one after another they cost a memory latency
+// each: most of a pass on the smaller grids).
+constexpr int kAhead = 8;
+template <class Load, class Put>
+__device__ __forceinline__ void for_loaded(int n, Load&& load, Put&& put) {
+  for (int e0 = threadIdx.x; e0 < n; e0 += kAhead * blockDim.x) {
+    decltype(load(0)) v[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int e = e0 + u * blockDim.x;
+      if (e < n) v[u] = load(e);
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int e = e0 + u * blockDim.x;
+      if (e < n) put(e, v[u]);
+    }
   }
 }
 
-// The z and y passes of one direction in one launch (single precision,
-// fixed plans, NY·NZ ≤ kPlaneCap): a workgroup holds the x plane of its
-// block index in LDS and transforms its z lines then its y lines (forward,
-// from the fixed-point charge grid) or its y lines then its z lines
-// (inverse).  Every line sees the stages, twiddles and order of the
-// separate passes, so the result is the same to the bit.
-constexpr int kPlaneCap = 4096;
-constexpr int kPlaneBlock = 512;
-template <int SIGN, bool FROM_FX, int NY, int NZ>
-__device__ __forceinline__ void k_fft_plane(float2* __restrict__ data,
-                                            const int64_t* __restrict__ grid_fx, int nx,
-                                            const float2* __restrict__ twy,
-                                            const float2* __restrict__ twz) {
-  static_assert(NY * NZ <= kPlaneCap, "plane exceeds the LDS buffers");
+template <class C>
+__device__ __forceinline__ void load_tw(C* __restrict__ dst, const C* __restrict__ src, int n) {
+  for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = src[k];
+}
+
+// Fixed-point charges of nl z-line pairs from pair q0 on into LDS lines.
+template <class C>
+__device__ __forceinline__ void load_pairs(C* __restrict__ a, int S, const int64_t* __restrict__ grid_fx,
+                                           const FftGeom& g, int q0, int nl) {
+  using R = typename CxT<C>::R;
+  const int N = g.K[2];
+  const float rN = fast_rcp(N), rnp = fast_rcp(g.np);
+  for_loaded(2 * nl * N, [&](int e) -> int64_t {
+    const int l2 = fast_div(e, N, rN), n = e - l2 * N;
+    const int q = q0 + (l2 >> 1), x = fast_div(q, g.np, rnp), y = 2 * (q - x * g.np) + (l2 & 1);
+    return y < g.K[1] ? grid_fx[((size_t)x * g.K[1] + y) * N + n] : 0;
+  }, [&](int e, int64_t v) {
+    const int l2 = fast_div(e, N, rN), n = e - l2 * N;
+    reinterpret_cast<R*>(a)[2 * (n * S + (l2 >> 1)) + (l2 & 1)] = (R)((double)v * (1.0 / DYN_GRID_FX_SCALE));
+  });
+}
+template <class C>
+__device__ __forceinline__ void store_pairs(const C* __restrict__ a, int S,
+                                            typename CxT<C>::R* __restrict__ phi, const FftGeom& g,
+                                            int q0, int nl) {
+  using R = typename CxT<C>::R;
+  const int N = g.K[2];
+  const float rN = fast_rcp(N), rnp = fast_rcp(g.np);
+  for (int e = threadIdx.x; e < 2 * nl * N; e += blockDim.x) {
+    const int l2 = fast_div(e, N, rN), n = e - l2 * N, l = l2 >> 1;
+    const int q = q0 + l, x = fast_div(q, g.np, rnp), y = 2 * (q - x * g.np) + (l2 & 1);
+    if (y < g.K[1])
+      phi[((size_t)x * g.K[1] + y) * N + n] = reinterpret_cast<const R*>(a)[2 * (n * S + l) + (l2 & 1)];
+  }
+}
+
+// LDS row stride of nl z-line pairs (odd: the loads along z write down a
+// column of LDS).
+__host__ __device__ inline int pair_stride(int nl) { return nl | 1; }
+
+// z pass of g.L pairs per workgroup: charges to spectrum (FWD) or spectrum
+// to potential.
+template <bool FWD, class C>
+__device__ __forceinline__ void
+k_fft_z(C* __restrict__ spec, const int64_t* __restrict__ grid_fx, typename CxT<C>::R* __restrict__ phi,
+        FftGeom geom, const C* __restrict__ tw) {
+  const FftGeom g = uni(geom);
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  float2* A = reinterpret_cast<float2*>(smem_raw);
-  float2* B = A + NY * NZ;
-  const int x = blockIdx.x;
-  if (x >= nx) return;  // beyond this system's planes
-  const size_t base = (size_t)x * NY * NZ;
-  for (int e = threadIdx.x; e < NY * NZ; e += blockDim.x) {
-    if (FROM_FX) A[e] = make_float2((float)((double)grid_fx[base + e] * (1.0 / DYN_GRID_FX_SCALE)), 0.0f);
-    else A[e] = data[base + e];
-  }
-  __syncthreads();
-  float2* out;
-  if (SIGN < 0) {
-    float2* rz = lds_fft_pow2<SIGN, NZ>(A, B, NY, twz);  // NY contiguous z lines
-    out = lds_fft_pow2_t<SIGN, NY, NZ>(rz, rz == A ? B : A, twy);
+  const int q0 = blockIdx.x * g.L, pairs = g.K[0] * g.np;
+  if (q0 >= pairs) return;  // beyond this system's lines
+  const int N = g.K[2], nl = min(g.L, pairs - q0), S = pair_stride(g.L);
+  C* A = reinterpret_cast<C*>(smem_raw);
+  C* B = A + N * S;
+  C* s_tw = B + N * S;
+  load_tw(s_tw, tw, N);
+  const float rnh = fast_rcp(g.nh), rnp = fast_rcp(g.np);
+  if (FWD) {
+    load_pairs(A, S, grid_fx, g, q0, nl);
+    __syncthreads();
+    const C* X = lds_fft<-1>(A, B, nl, S, N, g.plan[2], s_tw);
+    for (int e = threadIdx.x; e < nl * g.nh; e += blockDim.x) {
+      const int l = fast_div(e, g.nh, rnh), k = e - l * g.nh;
+      const int q = q0 + l, x = fast_div(q, g.np, rnp), y = 2 * (q - x * g.np);
+      C a, b;
+      pair_split(X[k * S + l], X[(k ? N - k : 0) * S + l], a, b);
+      C* out = spec + ((size_t)x * g.K[1] + y) * g.nh + k;
+      out[0] = a;
+      if (y + 1 < g.K[1]) out[g.nh] = b;
+    }
   } else {
-    float2* ry = lds_fft_pow2_t<SIGN, NY, NZ>(A, B, twy);
-    out = lds_fft_pow2<SIGN, NZ>(ry, ry == A ? B : A, NY, twz);
+    struct Two { C a, b; };
+    for_loaded(nl * g.nh, [&](int e) {
+      const int l = fast_div(e, g.nh, rnh), k = e - l * g.nh;
+      const int q = q0 + l, x = fast_div(q, g.np, rnp), y = 2 * (q - x * g.np);
+      const C* in = spec + ((size_t)x * g.K[1] + y) * g.nh + k;
+      return Two{in[0], y + 1 < g.K[1] ? in[g.nh] : CxT<C>::mk(0, 0)};
+    }, [&](int e, const Two& v) {
+      const int l = fast_div(e, g.nh, rnh);
+      pair_join(A, S, l, e - l * g.nh, N, v.a, v.b);
+    });
+    __syncthreads();
+    const C* X = lds_fft<+1>(A, B, nl, S, N, g.plan[2], s_tw);
+    store_pairs(X, S, phi, g, q0, nl);
   }
-  for (int e = threadIdx.x; e < NY * NZ; e += blockDim.x) data[base + e] = out[e];
+}
+
+// y pass of g.L consecutive kz of an x plane per workgroup, in place.
+template <int SIGN, class C>
+__device__ __forceinline__ void
+k_fft_y(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw) {
+  const FftGeom g = uni(geom);
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int tiles = (g.nh + g.L - 1) / g.L;
+  const int x = blockIdx.x / tiles, k0 = (blockIdx.x - x * tiles) * g.L;
+  if (x >= g.K[0]) return;  // beyond this system's lines
+  const int N = g.K[1], nl = min(g.L, g.nh - k0);
+  C* A = reinterpret_cast<C*>(smem_raw);
+  C* B = A + N * g.L;
+  C* s_tw = B + N * g.L;
+  load_tw(s_tw, tw, N);
+  C* base = spec + (size_t)x * N * g.nh + k0;
+  const float rnl = fast_rcp(nl);
+  for_loaded(N * nl, [&](int e) {
+    const int n = fast_div(e, nl, rnl), l = e - n * nl;
+    return base[(size_t)n * g.nh + l];
+  }, [&](int e, C v) { A[e] = v; });
+  __syncthreads();
+  const C* X = lds_fft<SIGN>(A, B, nl, nl, N, g.plan[1], s_tw);
+  for (int e = threadIdx.x; e < N * nl; e += blockDim.x) {
+    const int n = fast_div(e, nl, rnl), l = e - n * nl;
+    base[(size_t)n * g.nh + l] = X[e];
+  }
+}
+
+// The z and y passes of one direction in one launch, a workgroup per x
+// plane in LDS: the same arithmetic as the separate passes, a launch and a
+// round trip of the spectrum less (pme_run says where).
+constexpr int kPlaneBlock = 512;  // (1024: 3% faster alone, but 28,000-site MD steps, which run it beside
+                                  // the pair kernel, 7% slower)
+template <bool FWD>
+__device__ __forceinline__ void
+k_fft_plane(float2* __restrict__ spec, const int64_t* __restrict__ grid_fx, float* __restrict__ phi,
+            FftGeom geom, const float2* __restrict__ twy,
+            const float2* __restrict__ twz) {
+  const FftGeom g = uni(geom);
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int x = blockIdx.x;
+  if (x >= g.K[0]) return;  // beyond this system's planes
+  const int NY = g.K[1], NZ = g.K[2], nh = g.nh, S = pair_stride(g.np);
+  const int cap = max(NZ * S, NY * nh);
+  float2* A = reinterpret_cast<float2*>(smem_raw);
+  float2* B = A + cap;
+  float2* s_twy = B + cap;
+  float2* s_twz = s_twy + NY;
+  load_tw(s_twy, twy, NY);
+  load_tw(s_twz, twz, NZ);
+  const float rnh = fast_rcp(nh);
+  float2* plane = spec + (size_t)x * NY * nh;
+  if (FWD) {
+    load_pairs(A, S, grid_fx, g, x * g.np, g.np);
+    __syncthreads();
+    float2* X = lds_fft<-1>(A, B, g.np, S, NZ, g.plan[2], s_twz);
+    float2* Y = X == A ? B : A;
+    for (int e = threadIdx.x; e < g.np * nh; e += blockDim.x) {
+      const int l = fast_div(e, nh, rnh), k = e - l * nh;
+      float2 a, b;
+      pair_split(X[k * S + l], X[(k ? NZ - k : 0) * S + l], a, b);
+      Y[2 * l * nh + k] = a;
+      if (2 * l + 1 < NY) Y[(2 * l + 1) * nh + k] = b;
+    }
+    __syncthreads();
+    const float2* Z = lds_fft<-1>(Y, X, nh, nh, NY, g.plan[1], s_twy);
+    for (int e = threadIdx.x; e < NY * nh; e += blockDim.x) plane[e] = Z[e];
+  } else {
+    for_loaded(NY * nh, [&](int e) { return plane[e]; }, [&](int e, float2 v) { A[e] = v; });
+    __syncthreads();
+    float2* Y = lds_fft<+1>(A, B, nh, nh, NY, g.plan[1], s_twy);
+    float2* X = Y == A ? B : A;
+    for (int e = threadIdx.x; e < g.np * nh; e += blockDim.x) {
+      const int l = fast_div(e, nh, rnh), k = e - l * nh;
+      pair_join(X, S, l, k, NZ, Y[2 * l * nh + k],
+                2 * l + 1 < NY ? Y[(2 * l + 1) * nh + k] : make_float2(0.f, 0.f));
+    }
+    __syncthreads();
+    const float2* Z = lds_fft<+1>(X, Y, g.np, S, NZ, g.plan[2], s_twz);
+    store_pairs(Z, S, phi, g, x * g.np, g.np);
+  }
 }
 
 struct ConvArgs {
@@ -405,104 +530,72 @@ struct ConvArgs {
   double pi2_over_b2;  // π²/β²
 };
 
-// x pass fused with the convolution: forward FFT along x, multiply by G(m)
-// (accumulating ½G|F[Q]|² and its virial weight in f64), inverse FFT along x.
-template <class CX, int NF>
+// x pass fused with the convolution, g.L consecutive (y, kz) columns per
+// workgroup: forward FFT along x, multiply by G(m) (accumulating ½G|F[Q]|² and
+// its virial weight), inverse FFT along x.  A kz inside the half spectrum
+// stands for −kz too.  Each point's energy is computed in f64 and rounded to
+// 2⁻³² fixed point, so the sums do not depend on the grouping of the lines.
+template <class C>
 __device__ __forceinline__ void
-k_fft_conv_x(CX* __restrict__ data, PassGeom g, const FftAxis* __restrict__ axp,
-             const CX* __restrict__ tw, const typename CxT<CX>::R* __restrict__ G, ConvArgs C,
-             int64_t* __restrict__ partials) {
+k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
+             const typename CxT<C>::R* __restrict__ G, ConvArgs V, int64_t* __restrict__ partials) {
+  const FftGeom g = uni(geom);
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  CX* smem = reinterpret_cast<CX*>(smem_raw);
-  const FftAxis& ax = *axp;
-  const int N = ax.N;
-  const int line0 = blockIdx.x * g.L;
-  if (line0 >= g.lines) return;  // beyond this system's lines
-  const int nl = min(g.L, g.lines - line0);
-  CX* A = smem;
-  CX* B = smem + g.L * N;
-  const int tot = nl * N;
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, n;
-    split_e<0>(e, nl, N, l, n);
-    A[l * N + n] = data[pass_addr<0>(g, line0 + l, n)];
-  }
+  __shared__ long long red[2][kFftBlock / 64];
+  const int N = g.K[0], cols = g.K[1] * g.nh, c0 = blockIdx.x * g.L;
+  if (c0 >= cols) return;  // beyond this system's lines
+  const int nl = min(g.L, cols - c0);
+  C* A = reinterpret_cast<C*>(smem_raw);
+  C* B = A + N * g.L;
+  C* s_tw = B + N * g.L;
+  load_tw(s_tw, tw, N);
+  const float rnl = fast_rcp(nl), rnh = fast_rcp(g.nh);
+  for_loaded(N * nl, [&](int e) {
+    const int n = fast_div(e, nl, rnl), l = e - n * nl;
+    return spec[(size_t)n * cols + c0 + l];
+  }, [&](int e, C v) { A[e] = v; });
   __syncthreads();
-  CX* R = lds_fft<-1, NF>(A, B, nl, ax, tw);
-  CX* O = (R == A) ? B : A;
-  // the influence function of the block's points into the free LDS buffer
-  // (coalesced reads), for the energy sums and the product
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, n;
-    split_e<0>(e, nl, N, l, n);
-    O[l * N + n].x = G[pass_addr<0>(g, line0 + l, n)];
-  }
-  __syncthreads();
-  // energy and virial weight per line (a wave per line, lanes over its
-  // points, shuffle sums), each line's pair rounded to 2^-32 fixed point and
-  // summed as integers: the workgroup's partial does not depend on how many
-  // lines it holds, so the total is the same for any grouping of the lines
-  {
-    __shared__ long long red[2][kFftBlock / 64];
-    long long qe = 0, qw = 0;
-    const int wv = threadIdx.x / 64, lane = threadIdx.x & 63;
-    for (int l = wv; l < nl; l += kFftBlock / 64) {
-      const int line = line0 + l;
-      const int my = line / g.K[2], mz = line - my * g.K[2];
-      const int myp = my <= g.K[1] / 2 ? my : my - g.K[1];
-      const int mzp = mz <= g.K[2] / 2 ? mz : mz - g.K[2];
-      const double fy = myp * (double)C.invL[1], fz = mzp * (double)C.invL[2];
-      double e_acc = 0.0, w_acc = 0.0;
-      for (int n = lane; n < N; n += 64) {
-        const auto gv = O[l * N + n].x;
-        const CX v = R[l * N + n];
-        const double en = 0.5 * (double)gv * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
-        const int mxp = n <= g.K[0] / 2 ? n : n - g.K[0];
-        const double fx = mxp * (double)C.invL[0];
-        const double msq = fx * fx + fy * fy + fz * fz;
-        e_acc += en;
-        w_acc += en * (1.0 - 2.0 * C.pi2_over_b2 * msq);
-      }
-      for (int m = 32; m >= 1; m >>= 1) {
-        e_acc += __shfl_xor(e_acc, m, 64);
-        w_acc += __shfl_xor(w_acc, m, 64);
-      }
-      qe += (long long)dyn_fx64(e_acc);
-      qw += (long long)dyn_fx64(w_acc);
-    }
-    if (lane == 0) {
-      red[0][wv] = qe;
-      red[1][wv] = qw;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      long long te = 0, tw2 = 0;
-      for (int k = 0; k < kFftBlock / 64; ++k) {
-        te += red[0][k];
-        tw2 += red[1][k];
-      }
-      partials[2 * blockIdx.x] = te;
-      partials[2 * blockIdx.x + 1] = tw2;
-    }
-  }
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, n;
-    split_e<0>(e, nl, N, l, n);
-    const auto gv = O[l * N + n].x;
-    CX v = R[l * N + n];
+  C* X = lds_fft<-1>(A, B, nl, nl, N, g.plan[0], s_tw);
+  long long qe = 0, qw = 0;
+  for_loaded(N * nl, [&](int e) {
+    const int n = fast_div(e, nl, rnl);
+    return G[(size_t)n * cols + c0 + e - n * nl];
+  }, [&](int e, typename CxT<C>::R gv) {
+    const int n = fast_div(e, nl, rnl), c = c0 + e - n * nl;
+    C v = X[e];
+    const int my = fast_div(c, g.nh, rnh), mz = c - my * g.nh;
+    const double fx = (n <= N / 2 ? n : n - N) * (double)V.invL[0];
+    const double fy = (my <= g.K[1] / 2 ? my : my - g.K[1]) * (double)V.invL[1];
+    const double fz = mz * (double)V.invL[2];
+    const double msq = fx * fx + fy * fy + fz * fz;
+    const double wz = mz == 0 || 2 * mz == g.K[2] ? 0.5 : 1.0;
+    const double en = wz * (double)gv * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
+    qe += (long long)dyn_fx64(en);
+    qw += (long long)dyn_fx64(en * (1.0 - 2.0 * V.pi2_over_b2 * msq));
     v.x *= gv;
     v.y *= gv;
-    R[l * N + n] = v;
+    X[e] = v;
+  });
+  for (int m = 32; m >= 1; m >>= 1) {
+    qe += __shfl_xor(qe, m, 64);
+    qw += __shfl_xor(qw, m, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x / 64] = qe;
+    red[1][threadIdx.x / 64] = qw;
   }
   __syncthreads();
-  CX* R2 = lds_fft<+1, NF>(R, O, nl, ax, tw);
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, n;
-    split_e<0>(e, nl, N, l, n);
-    data[pass_addr<0>(g, line0 + l, n)] = R2[l * N + n];
+  if (threadIdx.x < 2) {
+    long long s = 0;
+    for (int k = 0; k < kFftBlock / 64; ++k) s += red[threadIdx.x][k];
+    partials[2 * blockIdx.x + threadIdx.x] = s;
+  }
+  const C* Z = lds_fft<+1>(X, X == A ? B : A, nl, nl, N, g.plan[0], s_tw);
+  for (int e = threadIdx.x; e < N * nl; e += blockDim.x) {
+    const int n = fast_div(e, nl, rnl), l = e - n * nl;
+    spec[(size_t)n * cols + c0 + l] = Z[e];
   }
 }
-
 
 struct SplineArgs {
   int K[3];
@@ -630,9 +723,9 @@ __device__ __forceinline__ int64_t fx_of(R f) {
 }
 
 constexpr int kGatherBlock = 128;
-template <int ORDER, class C>
+template <int ORDER, class R>
 __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, uint32_t n, SplineArgs S,
-                             const C* __restrict__ phi, const uint32_t* __restrict__ site,
+                             const R* __restrict__ phi, const uint32_t* __restrict__ site,
                              int64_t* __restrict__ fx, int comp_major, uint32_t nsites,
                              float* __restrict__ fout, float fscale,
                              const int64_t* __restrict__ partials, int nbp,
@@ -640,7 +733,6 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
                              uint32_t nbk) {
   // partials: the convolution's per-workgroup energy and virial sums in
   // 2^-32 fixed point (nbp workgroups)
-  using R = typename CxT<C>::R;
   constexpr bool F32 = std::is_same<R, float>::value;
   // the spread has read the brick counts: clear them for the next binning
   if (brick_count)
@@ -694,13 +786,13 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
       const int gx = (k0[0] + S.K[0] - ORDER + 1 + jx) % S.K[0];
       for (int jy = 0; jy < ORDER; ++jy) {
         const int gy = (k0[1] + S.K[1] - ORDER + 1 + jy) % S.K[1];
-        const C* row = phi + ((size_t)gx * S.K[1] + gy) * S.K[2];
+        const R* row = phi + ((size_t)gx * S.K[1] + gy) * S.K[2];
         const R txy = th[0][jx] * th[1][jy];
         const R dxy = dth[0][jx] * th[1][jy];
         const R tdy = th[0][jx] * dth[1][jy];
         for (int jz = 0; jz < ORDER; ++jz) {
           const int gz = (k0[2] + S.K[2] - ORDER + 1 + jz) % S.K[2];
-          const R ph = row[gz].x;
+          const R ph = row[gz];
           if constexpr (F32) {
             sx = dyn_fmaf(ph, dxy * th[2][jz], sx);
             sy = dyn_fmaf(ph, tdy * th[2][jz], sy);
@@ -741,21 +833,41 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
   }
 }
 
-// Lines per workgroup of an FFT pass: about 512 points per workgroup (two
-// per thread), at most kFftCap/N lines, and few enough lines that the pass
-// over all nsys systems of a launch still has ≥ 512 workgroups.
-PassGeom pass_geom(const uint32_t K[3], int axis, uint32_t nsys) {
-  PassGeom g;
+// Geometry of the pass along an axis over nsys systems: kFftLines lines per
+// workgroup (128 bytes of consecutive kz), fewer where the lines are long or
+// the launch would have fewer than 256 workgroups; kz tiles of a y pass of
+// about equal width.
+FftGeom pass_geom(const PmeCore& c, int axis, uint32_t nsys, size_t elem) {
+  const uint32_t* K = c.K;
+  FftGeom g;
   for (int a = 0; a < 3; ++a) g.K[a] = (int)K[a];
-  const int N = (int)K[axis];
-  g.lines = (int)(K[0] * K[1] * K[2] / K[axis]);
-  const int l_work = std::max(1, 512 / N);
-  const int l_par = (int)std::max<int64_t>(1, (int64_t)g.lines * std::max<uint32_t>(nsys, 1) / 512);
-  int L = std::max(1, std::min(kFftCap / N, std::min(l_work, l_par)));
-  int p2 = 1;
-  while (p2 * 2 <= L) p2 *= 2;
-  g.L = p2;
+  g.nh = (int)K[2] / 2 + 1;
+  g.np = ((int)K[1] + 1) / 2;
+  const int N = g.K[axis];
+  const int64_t lines = axis == 2 ? (int64_t)g.K[0] * g.np : (int64_t)(axis == 1 ? g.K[0] : g.K[1]) * g.nh;
+  const int fit = std::max(1, (int)(kFftCap * sizeof(float2) / elem) / N);
+  int L = std::min(kFftLines, fit);
+  while (L > 4 && lines * std::max<uint32_t>(nsys, 1) / L < 256) L /= 2;
+  if (axis == 1) {
+    const int tiles = std::max(1, (g.nh + L / 4) / L);
+    L = std::min((g.nh + tiles - 1) / tiles, fit);
+  }
+  g.L = L;
+  for (int a = 0; a < 3; ++a) g.plan[a] = c.plan[a];
   return g;
+}
+unsigned pass_groups(const FftGeom& g, int axis) {
+  if (axis == 1) return (unsigned)(g.K[0] * ((g.nh + g.L - 1) / g.L));
+  const int lines = axis == 2 ? g.K[0] * g.np : g.K[1] * g.nh;
+  return (unsigned)((lines + g.L - 1) / g.L);
+}
+size_t pass_lds(const FftGeom& g, int axis, size_t elem) {
+  const size_t N = (size_t)g.K[axis], S = (size_t)(axis == 2 ? pair_stride(g.L) : g.L);
+  return (2 * N * S + N) * elem;
+}
+size_t plane_lds(const FftGeom& g) {
+  const size_t cap = std::max((size_t)g.K[2] * pair_stride(g.np), (size_t)g.K[1] * g.nh);
+  return (2 * cap + g.K[1] + g.K[2]) * sizeof(float2);
 }
 
 }  // namespace
@@ -773,15 +885,14 @@ void PmeCore::init(int dev, hipStream_t s, Profiler* p, const uint32_t k[3], con
                 k[a], ord);
     DYN_REQUIRE(is_235_smooth(k[a]), "grid size %u must factor into 2, 3 and 5", k[a]);
     K[a] = k[a];
-    ax[a] = make_fft_axis((int)k[a]);
+    plan[a] = fft_plan(k[a]);
   }
-  ax_dev.reserve(3);
-  DYN_HIP(hipMemcpyAsync(ax_dev.p, ax, sizeof ax, hipMemcpyHostToDevice, s));
   DYN_REQUIRE(ord == 4 || ord == 5, "B-spline order must be 4 or 5 (got %d)", ord);
   DYN_REQUIRE(b > 0.f && std::isfinite(b), "beta must be > 0");
   order = ord;
   beta = b;
   ngrid = (size_t)K[0] * K[1] * K[2];
+  nspec = (size_t)K[0] * K[1] * (K[2] / 2 + 1);
   grid_fx.reserve(ngrid);
   for (int a = 0; a < 3; ++a) nbk[a] = (K[a] + kBrick - 1) / kBrick;
   const size_t nb = (size_t)nbk[0] * nbk[1] * nbk[2];
@@ -792,11 +903,11 @@ void PmeCore::init(int dev, hipStream_t s, Profiler* p, const uint32_t k[3], con
   DYN_HIP(hipMemsetAsync(brick_count.p, 0, sizeof(uint32_t) * (nb + 1), stream));
   DYN_HIP(hipMemsetAsync(status.p, 0, sizeof(unsigned int), stream));
   if (f64) {
-    cgrid64.reserve(ngrid);
-    G64.reserve(ngrid);
+    cgrid64.reserve(nspec + (ngrid + 1) / 2);
+    G64.reserve(nspec);
   } else {
-    cgrid.reserve(ngrid);
-    G.reserve(ngrid);
+    cgrid.reserve(nspec + (ngrid + 1) / 2);
+    G.reserve(nspec);
   }
   for (int a = 0; a < 3; ++a) {
     std::vector<float2> t(K[a]);
@@ -819,13 +930,13 @@ void PmeCore::init(int dev, hipStream_t s, Profiler* p, const uint32_t k[3], con
   }
   // energy and virial partials: one fixed-point pair per x-pass workgroup
   // (at most one per line)
-  partials.reserve(2 * (size_t)K[1] * K[2]);
+  partials.reserve(2 * (size_t)K[1] * (K[2] / 2 + 1));
   res_dev.reserve(2);
   set_moduli();
   set_box(l);
 }
 
-// Influence function at every grid point (set_box), in double:
+// Influence function at every point of the half spectrum (set_box), in double:
 // G(m) = exp(−π²|m|²/β²)/(π V |m|²) · Π_a |b_a(m_a)|², m_a = m'_a/L_a with
 // m'_a the signed index; G(0) = 0.  bsq: 1/|b_a|² per axis, axes concatenated.
 template <class R>
@@ -833,13 +944,14 @@ __global__ void __launch_bounds__(256)
 k_pme_influence(R* __restrict__ G, const double* __restrict__ bsq, uint32_t K0, uint32_t K1,
                 uint32_t K2, double il0, double il1, double il2, double inv_piv, double pi2_b2) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)K0 * K1 * K2) return;
-  const uint32_t mz = (uint32_t)(i % K2);
-  const size_t r = i / K2;
+  const uint32_t nh = K2 / 2 + 1;
+  if (i >= (size_t)K0 * K1 * nh) return;
+  const uint32_t mz = (uint32_t)(i % nh);
+  const size_t r = i / nh;
   const uint32_t my = (uint32_t)(r % K1), mx = (uint32_t)(r / K1);
   const double fx = (mx <= K0 / 2 ? (double)mx : (double)mx - K0) * il0;
   const double fy = (my <= K1 / 2 ? (double)my : (double)my - K1) * il1;
-  const double fz = (mz <= K2 / 2 ? (double)mz : (double)mz - K2) * il2;
+  const double fz = (double)mz * il2;
   const double msq = fx * fx + fy * fy + fz * fz;
   double val = 0.0;
   if (msq > 0)
@@ -895,7 +1007,7 @@ void PmeCore::set_box(const float l[3]) {
   }
   const double V = (double)L[0] * L[1] * L[2];
   const double b2 = (double)beta * beta;
-  const unsigned grid = (unsigned)((ngrid + 255) / 256);
+  const unsigned grid = (unsigned)((nspec + 255) / 256);
   const double il0 = 1.0 / (double)L[0], il1 = 1.0 / (double)L[1], il2 = 1.0 / (double)L[2];
   if (f64)
     hipLaunchKernelGGL((k_pme_influence<double>), dim3(grid), dim3(256), 0, stream, G64.p, bsq.p,
@@ -975,11 +1087,10 @@ void PmeCore::run(uint32_t n, const float4* xyzq, const uint32_t* site, int64_t*
 void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
   const uint32_t ns = R.n;
   std::vector<SplineArgs> S(ns);
-  std::vector<PassGeom> gz(ns), gy(ns), gx(ns);
+  std::vector<FftGeom> gz(ns), gy(ns), gx(ns);
   unsigned g_n = 1, g_b = 1, bz = 1, by = 1, bx = 1;
   size_t shz = 0, shy = 0, shx = 0;
   bool any = false, ord[2][2] = {{false, false}, {false, false}}, prec[2] = {false, false};
-  auto shm = [](const PassGeom& g, int N, size_t elem) { return (size_t)2 * g.L * N * elem; };
   for (uint32_t i = 0; i < ns; ++i) {
     const PmeRun& r = runs[i];
     std::memset(&S[i], 0, sizeof S[i]);
@@ -996,18 +1107,18 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
       S[i].scd[a] = (double)c.K[a] / (double)c.L[a];
     }
     r.core->ensure_cap(r.n);
-    gz[i] = pass_geom(c.K, 2, ns);
-    gy[i] = pass_geom(c.K, 1, ns);
-    gx[i] = pass_geom(c.K, 0, ns);
     const size_t el = c.f64 ? sizeof(double2) : sizeof(float2);
+    gz[i] = pass_geom(c, 2, ns, el);
+    gy[i] = pass_geom(c, 1, ns, el);
+    gx[i] = pass_geom(c, 0, ns, el);
     g_n = std::max(g_n, grid_for(r.n, 256));
     g_b = std::max(g_b, c.nbk[0] * c.nbk[1] * c.nbk[2]);
-    bz = std::max(bz, (unsigned)((gz[i].lines + gz[i].L - 1) / gz[i].L));
-    by = std::max(by, (unsigned)((gy[i].lines + gy[i].L - 1) / gy[i].L));
-    bx = std::max(bx, (unsigned)((gx[i].lines + gx[i].L - 1) / gx[i].L));
-    shz = std::max(shz, shm(gz[i], (int)c.K[2], el));
-    shy = std::max(shy, shm(gy[i], (int)c.K[1], el));
-    shx = std::max(shx, shm(gx[i], (int)c.K[0], el));
+    bz = std::max(bz, pass_groups(gz[i], 2));
+    by = std::max(by, pass_groups(gy[i], 1));
+    bx = std::max(bx, pass_groups(gx[i], 0));
+    shz = std::max(shz, pass_lds(gz[i], 2, el));
+    shy = std::max(shy, pass_lds(gy[i], 1, el));
+    shx = std::max(shx, pass_lds(gx[i], 0, el));
   }
   if (!any) return;
   auto on = [&](uint32_t i) { return runs[i].core != nullptr; };
@@ -1053,28 +1164,48 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
     DYN_SPREAD(5, double, 1)
 #undef DYN_SPREAD
   }
-  // FFT stage over the systems of one precision: C = float2 or double2
-  auto fft = [&](auto F, auto Ctag, const char* name, const std::vector<PassGeom>& g, int axis,
-                 unsigned gx_, size_t shm_, bool from_fx) {
+#define DYN_IC(F) std::integral_constant<decltype(&F), &F>{}
+  struct TF {
+    using type = float2;
+  };
+  struct TD {
+    using type = double2;
+  };
+  // an FFT pass over the systems of one precision: C = float2 or double2
+  auto spec_of = [&](uint32_t i, auto Ctag) -> typename decltype(Ctag)::type* {
+    if constexpr (std::is_same<typename decltype(Ctag)::type, double2>::value) return cp(i)->cgrid64.p;
+    else return cp(i)->cgrid.p;
+  };
+  auto phi_of = [&](uint32_t i, auto Ctag) {
+    using Rt = typename CxT<typename decltype(Ctag)::type>::R;
+    return reinterpret_cast<Rt*>(spec_of(i, Ctag) + cp(i)->nspec);
+  };
+  auto tw_of = [&](uint32_t i, int axis, auto Ctag) -> const typename decltype(Ctag)::type* {
+    if constexpr (std::is_same<typename decltype(Ctag)::type, double2>::value) return cp(i)->tw64[axis].p;
+    else return cp(i)->tw[axis].p;
+  };
+  auto none = [](FftGeom g) {  // no lines in any pass
+    g.K[0] = g.K[1] = 0;
+    g.L = std::max(g.L, 1);
+    return g;
+  };
+  auto fft_z = [&](auto F, auto Ctag, const char* name) {
     using C = typename decltype(Ctag)::type;
-    constexpr bool F64 = std::is_same<C, double2>::value;
-    launch<decltype(F)::value, kFftBlock>(R, name, tag, gx_, kFftBlock, shm_, [&](uint32_t i) {
-      const bool m = mine(i, F64, 0);
-      C* grid = nullptr;
-      const C* tw = nullptr;
-      if (m) {
-        if constexpr (F64) {
-          grid = cp(i)->cgrid64.p;
-          tw = cp(i)->tw64[axis].p;
-        } else {
-          grid = cp(i)->cgrid.p;
-          tw = cp(i)->tw[axis].p;
-        }
-      }
-      PassGeom ge = g[i];
-      if (!m) ge.lines = 0;
-      return args<decltype(F)::value>(grid, from_fx && m ? cp(i)->grid_fx.p : nullptr, ge,
-                                      m ? cp(i)->ax_dev.p + axis : nullptr, tw);
+    using Rt = typename CxT<C>::R;
+    launch<decltype(F)::value, kFftBlock>(R, name, tag, bz, kFftBlock, shz, [&](uint32_t i) {
+      const bool m = mine(i, std::is_same<C, double2>::value, 0);
+      return args<decltype(F)::value>(m ? spec_of(i, Ctag) : (C*)nullptr,
+                                      m ? (const int64_t*)cp(i)->grid_fx.p : nullptr,
+                                      m ? phi_of(i, Ctag) : (Rt*)nullptr, m ? gz[i] : none(gz[i]),
+                                      m ? tw_of(i, 2, Ctag) : (const C*)nullptr);
+    });
+  };
+  auto fft_y = [&](auto F, auto Ctag, const char* name) {
+    using C = typename decltype(Ctag)::type;
+    launch<decltype(F)::value, kFftBlock>(R, name, tag, by, kFftBlock, shy, [&](uint32_t i) {
+      const bool m = mine(i, std::is_same<C, double2>::value, 0);
+      return args<decltype(F)::value>(m ? spec_of(i, Ctag) : (C*)nullptr, m ? gy[i] : none(gy[i]),
+                                      m ? tw_of(i, 1, Ctag) : (const C*)nullptr);
     });
   };
   auto conv = [&](auto F, auto Ctag, const char* name) {
@@ -1084,122 +1215,79 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
       const bool m = mine(i, F64, 0);
       ConvArgs Cv;
       std::memset(&Cv, 0, sizeof Cv);
-      C* grid = nullptr;
-      const C* tw = nullptr;
       const typename CxT<C>::R* G = nullptr;
-      PassGeom ge = gx[i];
       if (m) {
         for (int a = 0; a < 3; ++a) Cv.invL[a] = 1.0f / cp(i)->L[a];
         Cv.pi2_over_b2 = M_PI * M_PI / ((double)cp(i)->beta * cp(i)->beta);
-        if constexpr (F64) {
-          grid = cp(i)->cgrid64.p;
-          tw = cp(i)->tw64[0].p;
-          G = cp(i)->G64.p;
-        } else {
-          grid = cp(i)->cgrid.p;
-          tw = cp(i)->tw[0].p;
-          G = cp(i)->G.p;
-        }
-      } else {
-        ge.lines = 0;
+        if constexpr (F64) G = cp(i)->G64.p;
+        else G = cp(i)->G.p;
       }
-      return args<decltype(F)::value>(grid, ge, m ? cp(i)->ax_dev.p : nullptr, tw, G, Cv,
+      return args<decltype(F)::value>(m ? spec_of(i, Ctag) : (C*)nullptr, m ? gx[i] : none(gx[i]),
+                                      m ? tw_of(i, 0, Ctag) : (const C*)nullptr, G, Cv,
                                       m ? cp(i)->partials.p : nullptr);
     });
   };
-#define DYN_IC(F) std::integral_constant<decltype(&F), &F>{}
-  struct TF {
-    using type = float2;
-  };
-  struct TD {
-    using type = double2;
-  };
-  // a line length shared by every single-precision system of the pass
-  // along an axis (32, 64, 128) selects the fixed-plan FFT kernels
-  auto shared_n = [&](int axis) {
-    int n = -1;
-    for (uint32_t i = 0; i < ns; ++i) {
-      if (!mine(i, false, 0)) continue;
-      const int k = (int)cp(i)->K[axis];
-      if (n < 0) n = k;
-      else if (n != k) return 0;
-    }
-    return (n == 32 || n == 64 || n == 128) ? n : 0;
-  };
-#define DYN_FFT_F32(AXIS, SIGN, FX, NAME, G, B, SH)                                               \
-  switch (shared_n(AXIS)) {                                                                       \
-    case 32: fft(DYN_IC((k_fft_pass<AXIS, SIGN, FX, float2, 32>)), TF{}, NAME, G, AXIS, B, SH, FX); break; \
-    case 64: fft(DYN_IC((k_fft_pass<AXIS, SIGN, FX, float2, 64>)), TF{}, NAME, G, AXIS, B, SH, FX); break; \
-    case 128: fft(DYN_IC((k_fft_pass<AXIS, SIGN, FX, float2, 128>)), TF{}, NAME, G, AXIS, B, SH, FX); break; \
-    default: fft(DYN_IC((k_fft_pass<AXIS, SIGN, FX, float2, 0>)), TF{}, NAME, G, AXIS, B, SH, FX); \
+  // the z and y passes of each direction as one plane launch, where the
+  // planes are few (a launch saved: 64³ 10 µs against 13 and a launch gap,
+  // 80³ 14.3 against 15.3) and their LDS leaves room for other kernels' workgroups;
+  // many or large planes are as fast or faster as two passes (16 grids of
+  // 45³: 18.6 against 16.6; 128³: 26 against 28 alone, 102 against 52 beside the pair
+  // kernel)
+  bool planes = prec[0];
+  size_t shp = 0;
+  unsigned bp = 1, groups = 0;
+  for (uint32_t i = 0; i < ns; ++i) {
+    if (!mine(i, false, 0)) continue;
+    const size_t s = plane_lds(gz[i]);
+    groups += cp(i)->K[0];
+    planes = planes && s <= kPlaneLds && groups <= kPlaneGroups;
+    shp = std::max(shp, s);
+    bp = std::max(bp, cp(i)->K[0]);
   }
-  // the z and y passes of each direction as one plane launch when every
-  // single-precision system shares fixed-plan y and z lengths
-  auto plane = [&](auto F, const char* name, bool from_fx, int ny, int nz) {
-    unsigned gp = 1;
-    for (uint32_t i = 0; i < ns; ++i)
-      if (mine(i, false, 0)) gp = std::max(gp, cp(i)->K[0]);
-    launch<decltype(F)::value, kPlaneBlock>(R, name, tag, gp, kPlaneBlock,
-                                            (size_t)2 * ny * nz * sizeof(float2), [&](uint32_t i) {
+  auto plane = [&](auto F, const char* name) {
+    launch<decltype(F)::value, kPlaneBlock>(R, name, tag, bp, kPlaneBlock, shp, [&](uint32_t i) {
       const bool m = mine(i, false, 0);
-      return args<decltype(F)::value>(m ? cp(i)->cgrid.p : nullptr,
-                                      from_fx && m ? cp(i)->grid_fx.p : nullptr,
-                                      m ? (int)cp(i)->K[0] : 0, m ? cp(i)->tw[1].p : nullptr,
-                                      m ? cp(i)->tw[2].p : nullptr);
+      return args<decltype(F)::value>(m ? spec_of(i, TF{}) : (float2*)nullptr,
+                                      m ? (const int64_t*)cp(i)->grid_fx.p : nullptr,
+                                      m ? phi_of(i, TF{}) : (float*)nullptr, m ? gz[i] : none(gz[i]),
+                                      m ? tw_of(i, 1, TF{}) : (const float2*)nullptr,
+                                      m ? tw_of(i, 2, TF{}) : (const float2*)nullptr);
     });
   };
-#define DYN_PLANE(SIGN, FX, NAME)                                                                  \
-  switch (ny * 1000 + nz) {                                                                       \
-    case 32032: plane(DYN_IC((k_fft_plane<SIGN, FX, 32, 32>)), NAME, FX, 32, 32); break;           \
-    case 32064: plane(DYN_IC((k_fft_plane<SIGN, FX, 32, 64>)), NAME, FX, 32, 64); break;           \
-    case 64032: plane(DYN_IC((k_fft_plane<SIGN, FX, 64, 32>)), NAME, FX, 64, 32); break;           \
-    default: plane(DYN_IC((k_fft_plane<SIGN, FX, 64, 64>)), NAME, FX, 64, 64);                     \
-  }
-  for (int pr = 0; pr < 2; ++pr) {
-    if (!prec[pr]) continue;
-    if (pr == 0) {
-      const int ny = shared_n(1), nz = shared_n(2);
-      const bool planes = ny > 0 && nz > 0 && ny <= 64 && nz <= 64;
-      if (planes) {
-        Profiler::Scope ps(prof, "pme_fft_zy_fwd");
-        DYN_PLANE(-1, true, "k_fft_plane fwd")
-      } else {
-        { Profiler::Scope ps(prof, "pme_fft_z_fwd");
-          DYN_FFT_F32(2, -1, true, "k_fft_pass z fwd", gz, bz, shz) }
-        { Profiler::Scope ps(prof, "pme_fft_y_fwd");
-          DYN_FFT_F32(1, -1, false, "k_fft_pass y fwd", gy, by, shy) }
-      }
-      { Profiler::Scope ps(prof, "pme_fft_x_conv");
-        switch (shared_n(0)) {
-          case 32: conv(DYN_IC((k_fft_conv_x<float2, 32>)), TF{}, "k_fft_conv_x"); break;
-          case 64: conv(DYN_IC((k_fft_conv_x<float2, 64>)), TF{}, "k_fft_conv_x"); break;
-          case 128: conv(DYN_IC((k_fft_conv_x<float2, 128>)), TF{}, "k_fft_conv_x"); break;
-          default: conv(DYN_IC((k_fft_conv_x<float2, 0>)), TF{}, "k_fft_conv_x");
-        } }
-      if (planes) {
-        Profiler::Scope ps(prof, "pme_fft_yz_inv");
-        DYN_PLANE(1, false, "k_fft_plane inv")
-      } else {
-        { Profiler::Scope ps(prof, "pme_fft_y_inv");
-          DYN_FFT_F32(1, 1, false, "k_fft_pass y inv", gy, by, shy) }
-        { Profiler::Scope ps(prof, "pme_fft_z_inv");
-          DYN_FFT_F32(2, 1, false, "k_fft_pass z inv", gz, bz, shz) }
-      }
+  if (prec[0]) {
+    if (planes) {
+      Profiler::Scope ps(prof, "pme_fft_zy_fwd");
+      plane(DYN_IC((k_fft_plane<true>)), "k_fft_plane fwd");
     } else {
       { Profiler::Scope ps(prof, "pme_fft_z_fwd");
-        fft(DYN_IC((k_fft_pass<2, -1, true, double2, 0>)), TD{}, "k_fft_pass z fwd f64", gz, 2, bz, shz, true); }
+        fft_z(DYN_IC((k_fft_z<true, float2>)), TF{}, "k_fft_z fwd"); }
       { Profiler::Scope ps(prof, "pme_fft_y_fwd");
-        fft(DYN_IC((k_fft_pass<1, -1, false, double2, 0>)), TD{}, "k_fft_pass y fwd f64", gy, 1, by, shy, false); }
-      { Profiler::Scope ps(prof, "pme_fft_x_conv");
-        conv(DYN_IC((k_fft_conv_x<double2, 0>)), TD{}, "k_fft_conv_x f64"); }
+        fft_y(DYN_IC((k_fft_y<-1, float2>)), TF{}, "k_fft_y fwd"); }
+    }
+    { Profiler::Scope ps(prof, "pme_fft_x_conv");
+      conv(DYN_IC((k_fft_conv_x<float2>)), TF{}, "k_fft_conv_x"); }
+    if (planes) {
+      Profiler::Scope ps(prof, "pme_fft_yz_inv");
+      plane(DYN_IC((k_fft_plane<false>)), "k_fft_plane inv");
+    } else {
       { Profiler::Scope ps(prof, "pme_fft_y_inv");
-        fft(DYN_IC((k_fft_pass<1, 1, false, double2, 0>)), TD{}, "k_fft_pass y inv f64", gy, 1, by, shy, false); }
+        fft_y(DYN_IC((k_fft_y<1, float2>)), TF{}, "k_fft_y inv"); }
       { Profiler::Scope ps(prof, "pme_fft_z_inv");
-        fft(DYN_IC((k_fft_pass<2, 1, false, double2, 0>)), TD{}, "k_fft_pass z inv f64", gz, 2, bz, shz, false); }
+        fft_z(DYN_IC((k_fft_z<false, float2>)), TF{}, "k_fft_z inv"); }
     }
   }
-#undef DYN_FFT_F32
-#undef DYN_PLANE
+  if (prec[1]) {
+    { Profiler::Scope ps(prof, "pme_fft_z_fwd");
+      fft_z(DYN_IC((k_fft_z<true, double2>)), TD{}, "k_fft_z fwd f64"); }
+    { Profiler::Scope ps(prof, "pme_fft_y_fwd");
+      fft_y(DYN_IC((k_fft_y<-1, double2>)), TD{}, "k_fft_y fwd f64"); }
+    { Profiler::Scope ps(prof, "pme_fft_x_conv");
+      conv(DYN_IC((k_fft_conv_x<double2>)), TD{}, "k_fft_conv_x f64"); }
+    { Profiler::Scope ps(prof, "pme_fft_y_inv");
+      fft_y(DYN_IC((k_fft_y<1, double2>)), TD{}, "k_fft_y inv f64"); }
+    { Profiler::Scope ps(prof, "pme_fft_z_inv");
+      fft_z(DYN_IC((k_fft_z<false, double2>)), TD{}, "k_fft_z inv f64"); }
+  }
   {
     Profiler::Scope ps(prof, "pme_gather");
     const unsigned gg = std::max(1u, (g_n * 256 + kGatherBlock - 1) / kGatherBlock);
@@ -1210,25 +1298,22 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
                                                tag * 4 + (F64 ? 2 : 0) + (order == 5), gg,
                                                kGatherBlock, 0, [&](uint32_t i) {
         const bool m = mine(i, F64, order);
-        const C* phi = nullptr;
-        if (m) {
-          if constexpr (F64) phi = cp(i)->cgrid64.p;
-          else phi = cp(i)->cgrid.p;
-        }
+        const typename CxT<C>::R* phi = nullptr;
+        if (m) phi = phi_of(i, Ctag);
         return args<decltype(F)::value>(runs[i].xyzq, m ? nq(i) : 0u, S[i], phi, runs[i].site,
                                         runs[i].fx, runs[i].comp_major, runs[i].nsites,
                                         runs[i].f_out, runs[i].fscale,
                                         m ? (const int64_t*)cp(i)->partials.p : nullptr,
-                                        m ? (gx[i].lines + gx[i].L - 1) / gx[i].L : 0,
+                                        m ? (int)pass_groups(gx[i], 0) : 0,
                                         m ? runs[i].res : nullptr,
                                         m ? cp(i)->brick_count.p : nullptr,
                                         m ? nb(i, 0) * nb(i, 1) * nb(i, 2) : 0u);
       });
     };
-    if (ord[0][0]) gather(DYN_IC((k_pme_gather<4, float2>)), TF{}, 4);
-    if (ord[0][1]) gather(DYN_IC((k_pme_gather<5, float2>)), TF{}, 5);
-    if (ord[1][0]) gather(DYN_IC((k_pme_gather<4, double2>)), TD{}, 4);
-    if (ord[1][1]) gather(DYN_IC((k_pme_gather<5, double2>)), TD{}, 5);
+    if (ord[0][0]) gather(DYN_IC((k_pme_gather<4, float>)), TF{}, 4);
+    if (ord[0][1]) gather(DYN_IC((k_pme_gather<5, float>)), TF{}, 5);
+    if (ord[1][0]) gather(DYN_IC((k_pme_gather<4, double>)), TD{}, 4);
+    if (ord[1][1]) gather(DYN_IC((k_pme_gather<5, double>)), TD{}, 5);
   }
 #undef DYN_IC
 }

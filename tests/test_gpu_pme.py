@@ -45,6 +45,26 @@ def test_pme_matches_fp64(gpu, order, K):
     assert np.array_equal(grid, replay_pme_spread(xyzq, K, box, order))
 
 
+@pytest.mark.parametrize("K", [(5, 6, 8), (9, 15, 25), (27, 27, 27), (16, 45, 54), (10, 81, 32), (64, 36, 75),
+                               (128, 64, 6), (6, 250, 9), (1024, 8, 12), (8, 1024, 5), (5, 9, 1024),
+                               (100, 96, 120)])
+def test_pme_grid_sizes(gpu, K):
+    """Every radix of the FFT plans, odd and even lengths (a pair of z lines
+    with one line, a half spectrum with and without its last real value), tiles
+    with a remainder, plane and separate passes, the longest lines."""
+    box = np.array([30.0, 33.0, 37.0], np.float32)
+    pos, q = _random_system(700, box, sum(K))
+    print(f"SPME grid {K}", flush=True)
+    pme = api.PmeRecip(K, box, 0.3123, order=5)
+    f, e, w = pme.forces_and_virial(pos, q)
+    f64, e64, w64 = fp64.spme_fp64(pos, q, box, K, 5, 0.3123)
+    self64 = fp64.self_energy(q, 0.3123)
+    # the f32 coordinate x·K/L is off by up to K·2⁻²⁴ grid cells
+    assert rel_rms(f, f64) <= 1e-5 + max(K) * 2.0 ** -24
+    assert abs(e - (e64 + self64)) <= 1e-6 * (abs(e64) + abs(self64))
+    assert abs(w - w64) <= 1e-5 * (abs(w64) + abs(e64))
+
+
 def test_pme_water_config0(gpu):
     s = systems.config0()
     pos, qs, *_ = s.site_arrays()
