@@ -1899,7 +1899,7 @@ __device__ __forceinline__ void k_eng_pme_prep(PmePrepArgs A) {
     if (A.pme_b)
       A.pme_b[t] = make_float4(p.x, p.y, p.z, site >= A.alch0 && site < A.alch1 ? -p.w : p.w);
   }
-  pme_bin_charge(A.bin, p, qv, t);
+  pme_bin_charge(A.bin, p, qv);
 }
 
 // Copies n values of a staging array into the current list's (grid stride).

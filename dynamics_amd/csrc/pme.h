@@ -30,8 +30,11 @@ __device__ __forceinline__ void frac_coord(R x, R sc, int K, int& k0, R& w) {
   const R u = x * sc;
   const R fl = floor(u);
   w = u - fl;
-  int k = (int)fl % K;
-  if (k < 0) k += K;
+  int k = (int)fl;
+  if ((unsigned)k >= (unsigned)K) {  // (not wrapped into the box, or rounded up to its end)
+    k %= K;
+    if (k < 0) k += K;
+  }
   k0 = k;
 }
 
@@ -45,7 +48,7 @@ __device__ __forceinline__ uint32_t brick_of(const int k0[3], const uint32_t nbk
 // and where an overflow is flagged.
 struct BinArgs {
   uint32_t* count;
-  uint32_t* items;
+  float4* items;
   unsigned int* status;
   int K[3];
   float sc[3];
@@ -56,11 +59,10 @@ struct BinArgs {
 };
 static_assert(sizeof(BinArgs) == 72, "BinArgs has no padding");
 
-// Lists charge i (position p) under its home brick.  Every lane of the wave
+// Lists charge p under its home brick.  Every lane of the wave
 // must call it (valid marks the lanes with a charge): one atomic per
 // distinct brick of the wave.
-__device__ __forceinline__ void pme_bin_charge(const BinArgs& B, float4 p, bool valid,
-                                               uint32_t i) {
+__device__ __forceinline__ void pme_bin_charge(const BinArgs& B, float4 p, bool valid) {
   uint32_t b = 0xFFFFFFFFu;  // no brick
   if (valid) {
     const float xs[3] = {p.x, p.y, p.z};
@@ -73,7 +75,7 @@ __device__ __forceinline__ void pme_bin_charge(const BinArgs& B, float4 p, bool 
   }
   const uint32_t rank = wave_rank(b, valid, B.count);
   if (valid) {
-    if (rank < B.cap) B.items[(size_t)b * B.cap + rank] = i;
+    if (rank < B.cap) B.items[(size_t)b * B.cap + rank] = p;
     else atomicOr(B.status, B.status_bit);
   }
 }
@@ -112,7 +114,7 @@ struct PmeCore {
   // reach it.
   uint32_t nbk[3] = {0, 0, 0};  // bricks per axis
   DevBuf<uint32_t> brick_count;  // per brick: charges listed (zeroed after use)
-  DevBuf<uint32_t> brick_items;  // cap_brick slots per brick
+  DevBuf<float4> brick_items;    // cap_brick slots (charges) per brick
   uint32_t cap_brick = 0;
   DevBuf<unsigned int> status;   // standalone runs: 1 = a brick list overflowed
   void ensure_cap(uint32_t n);

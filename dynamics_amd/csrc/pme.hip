@@ -604,6 +604,7 @@ struct SplineArgs {
 };
 
 constexpr int kBrickBlock = 256;
+constexpr int kRowY = kBrick + 1, kRowX = kBrick * kRowY + 1;  // LDS strides of a brick (bank spread)
 
 // Per charge: its home brick (the brick of its base grid point) and a rank
 // in it; the charge goes to slot rank of the brick's fixed-capacity list
@@ -612,7 +613,7 @@ constexpr int kBrickBlock = 256;
 // timing; the brick sums are integers, so the spread grid does not.
 __device__ __forceinline__ void k_pme_bin(const float4* __restrict__ xyzq, uint32_t n, BinArgs B) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  pme_bin_charge(B, i < n ? xyzq[i] : make_float4(0.f, 0.f, 0.f, 0.f), i < n, i);
+  pme_bin_charge(B, i < n ? xyzq[i] : make_float4(0.f, 0.f, 0.f, 0.f), i < n);
 }
 
 // Home bricks along one axis whose charges can reach the points [lo, hi]
@@ -636,50 +637,68 @@ __device__ __forceinline__ HomeRange home_bricks(int lo, int hi, int K) {
   return r;
 }
 
+// Grid point j of the ORDER points that end at base point k0 (mod K): one
+// conditional addition (an integer remainder, 84 a charge, was most of the
+// spread's and the gather's instructions).
+template <int ORDER>
+__device__ __forceinline__ int stencil_point(int k0, int j, int K) {
+  const int g = k0 - ORDER + 1 + j;
+  return g < 0 ? g + K : g;
+}
+
 // One workgroup per brick: every charge of the reaching home bricks adds its
 // stencil points inside the brick to an LDS brick (int64 LDS adds of the
 // same fixed-point values the replay sums), which is then stored once.  The
 // home bricks' charge lists are walked as one flattened index space.
+//
+// Bound: the latency of the dependent loads (counts, then charges) on small
+// grids, instruction issue on large ones.  So a lane per home brick reads the
+// counts, the lists hold the charges themselves and no integer remainder is
+// taken per point: 24,000 charges, order 5, on 80³ 28.9 -> 12.4 µs; order 4
+// keeps its time (21,000 on 64³ 12.4 µs, 192,000 on 128³ 39).  Tried and slower: a thread
+// per charge and x point (order 5 18.6 µs), or per charge, x and y with the
+// weights in LDS (17.1); two 32-bit LDS adds for each 64-bit one (13.7, 43 at
+// 128³).
 template <int ORDER, class R>
 __device__ __forceinline__ void
-k_pme_spread(const float4* __restrict__ xyzq, uint32_t n, SplineArgs S, uint32_t nbx,
-             uint32_t nby, uint32_t nbz, const uint32_t* __restrict__ count,
-             const uint32_t* __restrict__ items, uint32_t cap, int64_t* __restrict__ grid) {
-  __shared__ unsigned long long acc[kBrick * kBrick * kBrick];
-  __shared__ uint32_t s_c0[27], s_beg[28];
+k_pme_spread(SplineArgs S, uint32_t nbx, uint32_t nby, uint32_t nbz, const uint32_t* __restrict__ count,
+             const float4* __restrict__ items, uint32_t cap, int64_t* __restrict__ grid) {
+  __shared__ unsigned long long acc[kBrick * kRowX];
+  __shared__ uint32_t s_c0[32], s_end[32];
   const uint32_t b = blockIdx.x;
   if (b >= nbx * nby * nbz) return;  // beyond this system's bricks
   const int bz = (int)(b % nbz), by = (int)((b / nbz) % nby), bx = (int)(b / (nbz * nby));
   const int lo[3] = {bx * kBrick, by * kBrick, bz * kBrick};
   const int hi[3] = {min(lo[0] + kBrick, S.K[0]) - 1, min(lo[1] + kBrick, S.K[1]) - 1,
                      min(lo[2] + kBrick, S.K[2]) - 1};
-  for (int k = threadIdx.x; k < kBrick * kBrick * kBrick; k += kBrickBlock) acc[k] = 0ull;
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 32) {
+    // at most 27 home bricks; the rest of the 32 entries are empty
     const HomeRange hx = home_bricks<ORDER>(lo[0], hi[0], S.K[0]);
     const HomeRange hy = home_bricks<ORDER>(lo[1], hi[1], S.K[1]);
     const HomeRange hz = home_bricks<ORDER>(lo[2], hi[2], S.K[2]);
-    uint32_t tot = 0;
-    int q = 0;
-    for (int ix = 0; ix < hx.n; ++ix)
-      for (int iy = 0; iy < hy.n; ++iy)
-        for (int iz = 0; iz < hz.n; ++iz) {
-          const uint32_t h = ((uint32_t)hx.brick(ix) * nby + (uint32_t)hy.brick(iy)) * nbz +
-                             (uint32_t)hz.brick(iz);
-          s_c0[q] = h * cap;
-          s_beg[q] = tot;
-          tot += min(count[h], cap);
-          ++q;
-        }
-    for (; q < 28; ++q) s_beg[q] = tot;
+    const int q = threadIdx.x, ix = q / 9, iy = q / 3 - 3 * ix, iz = q - 3 * (q / 3);
+    uint32_t h = 0, c = 0;
+    if (ix < hx.n && iy < hy.n && iz < hz.n) {
+      h = ((uint32_t)hx.brick(ix) * nby + (uint32_t)hy.brick(iy)) * nbz + (uint32_t)hz.brick(iz);
+      c = min(count[h], cap);
+    }
+    uint32_t end = c;
+    for (int off = 1; off < 32; off <<= 1) {
+      const uint32_t u = __shfl_up(end, off, 32);
+      if (q >= off) end += u;
+    }
+    s_end[q] = end;
+    s_c0[q] = h * cap + c - end;  // (mod 2³²: entry t of the whole lies at s_c0 + t)
   }
+  for (int k = threadIdx.x; k < kBrick * kRowX; k += kBrickBlock) acc[k] = 0ull;
   __syncthreads();
-  const uint32_t total = s_beg[27];
+  const uint32_t total = s_end[31];
   for (uint32_t t = threadIdx.x; t < total; t += kBrickBlock) {
-    int q = 0;
-    while (q < 26 && s_beg[q + 1] <= t) ++q;
-    const uint32_t ci = items[s_c0[q] + (t - s_beg[q])];
-    if (ci >= n) continue;
-    const float4 p = xyzq[ci];
+    uint32_t q = 0;  // the first list that ends beyond t
+#pragma unroll
+    for (uint32_t step = 16; step >= 1; step >>= 1)
+      if (s_end[q + step - 1] <= t) q += step;
+    const float4 p = items[(size_t)(uint32_t)(s_c0[q] + t)];
     if (p.w == 0.0f) continue;
     int k0[3];
     R th[3][ORDER], dth[ORDER];
@@ -690,19 +709,20 @@ k_pme_spread(const float4* __restrict__ xyzq, uint32_t n, SplineArgs S, uint32_t
       dyn_bspline<ORDER, R>(w, th[a], dth);
     }
     for (int jx = 0; jx < ORDER; ++jx) {
-      const int gx = (k0[0] + S.K[0] - ORDER + 1 + jx) % S.K[0];
+      const int gx = stencil_point<ORDER>(k0[0], jx, S.K[0]);
       if (gx < lo[0] || gx > hi[0]) continue;
       const R qx = (R)p.w * th[0][jx];
+      unsigned long long* const row = acc + (gx - lo[0]) * kRowX;
       for (int jy = 0; jy < ORDER; ++jy) {
-        const int gy = (k0[1] + S.K[1] - ORDER + 1 + jy) % S.K[1];
+        const int gy = stencil_point<ORDER>(k0[1], jy, S.K[1]);
         if (gy < lo[1] || gy > hi[1]) continue;
         const R qxy = qx * th[1][jy];
         for (int jz = 0; jz < ORDER; ++jz) {
-          const int gz = (k0[2] + S.K[2] - ORDER + 1 + jz) % S.K[2];
+          const int gz = stencil_point<ORDER>(k0[2], jz, S.K[2]);
           if (gz < lo[2] || gz > hi[2]) continue;
           const R v = qxy * th[2][jz];
-          const int li = ((gx - lo[0]) * kBrick + (gy - lo[1])) * kBrick + (gz - lo[2]);
-          atomicAdd(&acc[li], (unsigned long long)dyn_fx_d((double)v, DYN_GRID_FX_SCALE));
+          atomicAdd(row + (gy - lo[1]) * kRowY + (gz - lo[2]),
+                    (unsigned long long)dyn_fx_d((double)v, DYN_GRID_FX_SCALE));
         }
       }
     }
@@ -712,7 +732,7 @@ k_pme_spread(const float4* __restrict__ xyzq, uint32_t n, SplineArgs S, uint32_t
     const int x = lo[0] + k / (kBrick * kBrick), y = lo[1] + (k / kBrick) % kBrick,
               z = lo[2] + k % kBrick;
     if (x <= hi[0] && y <= hi[1] && z <= hi[2])
-      grid[((size_t)x * S.K[1] + y) * S.K[2] + z] = (int64_t)acc[k];
+      grid[((size_t)x * S.K[1] + y) * S.K[2] + z] = (int64_t)acc[(x - lo[0]) * kRowX + (y - lo[1]) * kRowY + (z - lo[2])];
   }
 }
 
@@ -722,7 +742,27 @@ __device__ __forceinline__ int64_t fx_of(R f) {
   else return dyn_fx64(f);
 }
 
-constexpr int kGatherBlock = 128;
+// Order 4: four lanes per charge (a quad), lane g its x point g; the quad's
+// sums are added by DPP and lane c stores component c.  Bound: the
+// latency of a charge's dependent loads (charge, its grid points, its force
+// row), so that small systems gain from more and shorter chains: 1,500
+// charges 7.0 -> 4.7 µs, 21,000 8.9 -> 7.2, 32 systems of 100,000 together
+// 20.9 -> 14.4.  Order 5 takes a thread per charge: five x points leave a quad
+// uneven (24,000 charges: 13.1 µs, one thread each 10.0).
+constexpr int gather_lanes(int order) { return order == 4 ? 4 : 1; }
+constexpr int kGatherBlock = 256;
+template <class R>
+__device__ __forceinline__ R quad_sum(R v);
+template <>
+__device__ __forceinline__ float quad_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));
+}
+template <>
+__device__ __forceinline__ double quad_sum(double v) {
+  v += __shfl_xor(v, 1, 64);
+  return v + __shfl_xor(v, 2, 64);
+}
 template <int ORDER, class R>
 __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, uint32_t n, SplineArgs S,
                              const R* __restrict__ phi, const uint32_t* __restrict__ site,
@@ -766,10 +806,13 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
       res[1] = (double)tw * DYN_FX_INV_SCALE;
     }
   }
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  constexpr int kLanes = gather_lanes(ORDER);
+  const uint32_t i = (blockIdx.x * kGatherBlock + threadIdx.x) / kLanes;
+  const int g = kLanes == 1 ? 0 : (int)(threadIdx.x & 3u);
+  if (i >= n) return;  // (whole quads)
   const float4 p = xyzq[i];
-  R f0 = R(0), f1 = R(0), f2 = R(0);
+  const uint32_t s = site ? site[i] : 0u;
+  R f[3] = {R(0), R(0), R(0)};
   if (p.w != 0.0f) {
     int k0[3];
     R th[3][ORDER], dth[3][ORDER];
@@ -782,16 +825,24 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
       dyn_bspline<ORDER, R>(w, th[a], dth[a]);
     }
     R sx = R(0), sy = R(0), sz = R(0);
-    for (int jx = 0; jx < ORDER; ++jx) {
-      const int gx = (k0[0] + S.K[0] - ORDER + 1 + jx) % S.K[0];
+#pragma unroll
+    for (int j0 = 0; j0 < ORDER; j0 += kLanes) {
+      const int jx = j0 + g;
+      R tx = th[0][j0], dx = dth[0][j0];
+#pragma unroll
+      for (int j = 1; j < kLanes; ++j) {
+        tx = g == j ? th[0][j0 + j] : tx;
+        dx = g == j ? dth[0][j0 + j] : dx;
+      }
+      const int gx = stencil_point<ORDER>(k0[0], jx, S.K[0]);
       for (int jy = 0; jy < ORDER; ++jy) {
-        const int gy = (k0[1] + S.K[1] - ORDER + 1 + jy) % S.K[1];
+        const int gy = stencil_point<ORDER>(k0[1], jy, S.K[1]);
         const R* row = phi + ((size_t)gx * S.K[1] + gy) * S.K[2];
-        const R txy = th[0][jx] * th[1][jy];
-        const R dxy = dth[0][jx] * th[1][jy];
-        const R tdy = th[0][jx] * dth[1][jy];
+        const R txy = tx * th[1][jy];
+        const R dxy = dx * th[1][jy];
+        const R tdy = tx * dth[1][jy];
         for (int jz = 0; jz < ORDER; ++jz) {
-          const int gz = (k0[2] + S.K[2] - ORDER + 1 + jz) % S.K[2];
+          const int gz = stencil_point<ORDER>(k0[2], jz, S.K[2]);
           const R ph = row[gz];
           if constexpr (F32) {
             sx = dyn_fmaf(ph, dxy * th[2][jz], sx);
@@ -805,31 +856,28 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
         }
       }
     }
-    f0 = -(R)p.w * sc[0] * sx * (R)fscale;
-    f1 = -(R)p.w * sc[1] * sy * (R)fscale;
-    f2 = -(R)p.w * sc[2] * sz * (R)fscale;
+    if (kLanes == 4) {
+      sx = quad_sum(sx);
+      sy = quad_sum(sy);
+      sz = quad_sum(sz);
+    }
+    f[0] = -(R)p.w * sc[0] * sx * (R)fscale;
+    f[1] = -(R)p.w * sc[1] * sy * (R)fscale;
+    f[2] = -(R)p.w * sc[2] * sz * (R)fscale;
   }
-  if (site) {
-    const uint32_t s = site[i];
-    if (comp_major & 2) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (kLanes == 4 && g != c) continue;
+    if (!site) {
+      fout[3 * (size_t)i + c] = (float)f[c];
+    } else if (comp_major & 2) {
       // every site has one charge: no other thread of this pass touches it
       // (a second pass over the same sites is a later launch)
-      fx[s] += fx_of(f0);
-      fx[nsites + s] += fx_of(f1);
-      fx[2 * (size_t)nsites + s] += fx_of(f2);
-    } else if (comp_major) {
-      atomicAdd(reinterpret_cast<unsigned long long*>(fx + s), (unsigned long long)fx_of(f0));
-      atomicAdd(reinterpret_cast<unsigned long long*>(fx + nsites + s), (unsigned long long)fx_of(f1));
-      atomicAdd(reinterpret_cast<unsigned long long*>(fx + 2 * (size_t)nsites + s), (unsigned long long)fx_of(f2));
+      fx[(size_t)c * nsites + s] += fx_of(f[c]);
     } else {
-      atomicAdd(reinterpret_cast<unsigned long long*>(fx + 3 * (size_t)s), (unsigned long long)fx_of(f0));
-      atomicAdd(reinterpret_cast<unsigned long long*>(fx + 3 * (size_t)s + 1), (unsigned long long)fx_of(f1));
-      atomicAdd(reinterpret_cast<unsigned long long*>(fx + 3 * (size_t)s + 2), (unsigned long long)fx_of(f2));
+      atomicAdd(reinterpret_cast<unsigned long long*>(fx + (comp_major ? (size_t)c * nsites + s : 3 * (size_t)s + c)),
+                (unsigned long long)fx_of(f[c]));
     }
-  } else {
-    fout[3 * i] = (float)f0;
-    fout[3 * i + 1] = (float)f1;
-    fout[3 * i + 2] = (float)f2;
   }
 }
 
@@ -1146,10 +1194,10 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
     auto spread = [&](auto F, const char* name, bool f64, int order) {
       launch<decltype(F)::value, kBrickBlock>(R, name, tag, g_b, kBrickBlock, 0, [&](uint32_t i) {
         const bool m = mine(i, f64, order);
-        return args<decltype(F)::value>(runs[i].xyzq, m ? nq(i) : 0u, S[i], m ? nb(i, 0) : 0u,
-                                        m ? nb(i, 1) : 0u, m ? nb(i, 2) : 0u,
-                                        m ? cp(i)->brick_count.p : nullptr,
-                                        m ? cp(i)->brick_items.p : nullptr,
+        return args<decltype(F)::value>(S[i], m ? nb(i, 0) : 0u, m ? nb(i, 1) : 0u,
+                                        m ? nb(i, 2) : 0u,
+                                        m ? (const uint32_t*)cp(i)->brick_count.p : nullptr,
+                                        m ? (const float4*)cp(i)->brick_items.p : nullptr,
                                         m ? cp(i)->cap_brick : 0u,
                                         m ? cp(i)->grid_fx.p : nullptr);
       });
@@ -1290,8 +1338,8 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag) {
   }
   {
     Profiler::Scope ps(prof, "pme_gather");
-    const unsigned gg = std::max(1u, (g_n * 256 + kGatherBlock - 1) / kGatherBlock);
     auto gather = [&](auto F, auto Ctag, int order) {
+      const unsigned gg = g_n * (256 / kGatherBlock) * (unsigned)gather_lanes(order);
       using C = typename decltype(Ctag)::type;
       constexpr bool F64 = std::is_same<C, double2>::value;
       launch<decltype(F)::value, kGatherBlock>(R, "k_pme_gather",
