@@ -1693,17 +1693,16 @@ struct CorrArgs {
 
 constexpr int kCorrBlock = 256;
 constexpr int kCorrVals = 7;  // per-block sums of the correction kernel
-__device__ __forceinline__ void
-k_eng_corr(CorrArgs A) {
+__device__ __forceinline__ void corr_terms(const CorrArgs& A, uint32_t block) {
   __shared__ double red[kCorrBlock];
-  if (blockIdx.x >= A.nblk) return;  // partials exist for the system's own blocks
+  if (block >= A.nblk) return;  // partials exist for the system's own blocks
   // e_lj14, e_c14, e_corr, vir_sr, vir_recip, dH/dλ, 1-4 pairs within the cutoff
   double acc[kCorrVals] = {0, 0, 0, 0, 0, 0, 0};
   // molecule-pair matrix: a running entry per thread (1-4 pairs lie within
   // one molecule), flushed when the entry changes and once at the end
   int mkey = -1;
   double me = 0.0;
-  for (uint32_t k = blockIdx.x * kCorrBlock + threadIdx.x; k < A.n; k += A.nblk * kCorrBlock) {
+  for (uint32_t k = block * kCorrBlock + threadIdx.x; k < A.n; k += A.nblk * kCorrBlock) {
     if (A.kind[k] == 0 && !A.recip_on) continue;
     const uint32_t i = A.ci[k], j = A.cj[k];
     const float4 a = A.wpos[i], b = A.wpos[j];
@@ -1808,7 +1807,7 @@ k_eng_corr(CorrArgs A) {
   if (threadIdx.x < kCorrVals) {
     double t = 0.0;
     for (int w = 0; w < kCorrBlock / kWave; ++w) t += red[threadIdx.x * (kCorrBlock / kWave) + w];
-    A.partials[kCorrVals * blockIdx.x + threadIdx.x] = t;
+    A.partials[kCorrVals * block + threadIdx.x] = t;
   }
 }
 
@@ -1879,8 +1878,8 @@ struct PmePrepArgs {
   int64_t* fx_recip;
   BinArgs bin;
 };
-__device__ __forceinline__ void k_eng_pme_prep(PmePrepArgs A) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void pme_prep(const PmePrepArgs& A, uint32_t block) {
+  const uint32_t t = block * 256u + threadIdx.x;
   const uint32_t n = A.g.n_dyn + 4u * A.g.n_water;
   if (t < n) {
     A.fx_recip[t] = 0;
@@ -1900,6 +1899,20 @@ __device__ __forceinline__ void k_eng_pme_prep(PmePrepArgs A) {
       A.pme_b[t] = make_float4(p.x, p.y, p.z, site >= A.alch0 && site < A.alch1 ? -p.w : p.w);
   }
   pme_bin_charge(A.bin, p, qv);
+}
+
+// The short independent pieces of an evaluation in one launch, block ranges
+// one after another: SPME preparation (n_prep blocks), exclusion and 1-4
+// corrections (n_corr), bonded terms.  Each is a few dependent memory latencies
+// and little else, so together they take the time of the longest: 28,000 sites
+// 5.2 + 5.6 + 10.5 µs and two launch gaps before, 11.5 now.
+__device__ __forceinline__ void k_eng_side(const PmePrepArgs& P, const CorrArgs& C, const BondedArgs& B,
+                                           uint32_t n_prep, uint32_t n_corr) {
+  static_assert(kCorrBlock == 256 && kBondedBlock == 256, "one block size");
+  const uint32_t b = blockIdx.x;
+  if (b < n_prep) pme_prep(P, b);
+  else if (b < n_prep + n_corr) corr_terms(C, b - n_prep);
+  else bonded_terms(B, b - n_prep - n_corr);
 }
 
 // Copies n values of a staging array into the current list's (grid stride).
@@ -2099,32 +2112,25 @@ k_eng_energy_reduce1(const double* __restrict__ pp, const uint32_t* __restrict__
   }
 }
 
+// A wave per value (a workgroup of as many waves as values), lanes over the
+// partials.  (Every thread summing every value, then sixteen wave reductions in
+// turn: 10.7 µs; now 4.5.)
 __device__ __forceinline__ void
 k_eng_energy_reduce(const double* __restrict__ red1, const double* __restrict__ cp,
                     uint32_t n_cblk, int pme_runs, double* __restrict__ out) {
   // pme_runs < 0: the SPME sum was kept from an earlier evaluation, with its
   // energies, virials and the reciprocal correction virial (out[13])
-  constexpr int kVals = kNumPart + kCorrVals;
-  __shared__ double red[kVals][kRedBlock / kWave];
-  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  double a[kVals];
-  for (int v = 0; v < kVals; ++v) a[v] = 0.0;
-  if (red1)
-    for (uint32_t r = t; r < (uint32_t)kRed1Grid; r += kRedBlock)
-      for (int v = 0; v < kNumPart; ++v) a[v] += red1[(size_t)r * kNumPart + v];
-  for (uint32_t r = t; r < n_cblk; r += kRedBlock)
-    for (int v = 0; v < kCorrVals; ++v) a[kNumPart + v] += cp[(size_t)r * kCorrVals + v];
-  for (int v = 0; v < kVals; ++v) {
-    double x = a[v];
-    for (int m = 1; m < kWave; m <<= 1) x += __shfl_xor(x, m, kWave);
-    if (lane == 0) red[v][w] = x;
-  }
-  __syncthreads();
-  if (t < kVals) {
-    double x = 0.0;
-    for (int k = 0; k < kRedBlock / kWave; ++k) x += red[t][k];
-    if (!(pme_runs < 0 && t == 13)) out[t] = t < kNumPart ? 0.5 * x : x;
-  }
+  static_assert(kNumPart + kCorrVals == kRedBlock / kWave, "a wave per value");
+  const int t = threadIdx.x, lane = t & (kWave - 1), v = t / kWave;
+  const bool pair = v < kNumPart;
+  const double* __restrict__ p = pair ? red1 : cp;
+  const uint32_t n = pair ? (red1 ? (uint32_t)kRed1Grid : 0u) : n_cblk;
+  const uint32_t stride = pair ? kNumPart : kCorrVals, at = pair ? v : v - kNumPart;
+  double x = 0.0;
+#pragma unroll 4
+  for (uint32_t r = lane; r < n; r += kWave) x += p[(size_t)r * stride + at];
+  for (int m = 1; m < kWave; m <<= 1) x += __shfl_xor(x, m, kWave);
+  if (lane == 0 && !(pme_runs < 0 && v == 13)) out[v] = pair ? 0.5 * x : x;
   if (pme_runs >= 0 && t >= 16 && t < kEngOut && (t - 16) / 2 >= pme_runs) out[t] = 0.0;
 }
 
@@ -2575,8 +2581,7 @@ static void set_build_lists(EngineSet& S, const BatchRun& R, const std::vector<B
   }
 }
 
-void engine_set_enqueue(EngineSet& S, uint32_t flags,
-                        const std::function<void(const BatchRun&)>& side_work) {
+void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
   auto& E = S.e;
   const uint32_t ns = (uint32_t)E.size();
   const BatchRun& R = S.R;
@@ -2683,8 +2688,8 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
       return args<k_eng_prep>(A);
     });
   }
-  // the second stream: SPME (spread → FFT → convolution → inverse FFT →
-  // gather), the exclusion and 1-4 corrections and the caller's side work,
+  // the second stream: the exclusion and 1-4 corrections, the caller's bonded
+  // terms and SPME (spread → FFT → convolution → inverse FFT → gather),
   // overlapping the list build and the pair kernel on the main stream (a
   // fork later in the step delays the side work more than it gains: an
   // event wait between streams takes 10–40 µs to release)
@@ -2694,17 +2699,22 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
   // kernel at once and would take the compute units the FFT planes need —
   // before the pair kernel on the main stream
   const BatchRun& RP = staged_mode ? R : RS;
-  if (any_recip) {
-    {
-      Profiler::Scope ps(prof, "pme_prep");
-      const unsigned gq = max_grid(S, [](dyn_engine& e) {
-        return std::max(grid_for(e.n_sites, 256), grid_for(e.n_q, 256));
-      });
-      launch<k_eng_pme_prep>(RP, "k_eng_pme_prep", 0, gq, 256, 0, [&](uint32_t i) {
-        dyn_engine& e = *E[i];
-        const Plan& pl = PL[i];
-        PmePrepArgs A;
-        std::memset(&A, 0, sizeof A);
+  // the SPME preparation, the exclusion and 1-4 corrections (site
+  // accumulators; finalize reads them) and the caller's bonded terms: one
+  // launch where they share a stream
+  const unsigned n_prep = !any_recip ? 0u : max_grid(S, [](dyn_engine& e) {
+    return std::max(grid_for(e.n_sites, 256), grid_for(e.n_q, 256));
+  });
+  const unsigned n_corr = any_corr ? max_grid(S, [](dyn_engine& e) { return e.corr_blocks; }) : 0u;
+  const unsigned n_bond = side ? side->blocks : 0u;
+  auto side_launch = [&](const BatchRun& RL, int tag, unsigned np, unsigned nc, unsigned nb) {
+    if (np + nc + nb == 0) return;
+    launch<k_eng_side>(RL, "k_eng_side", tag, np + nc + nb, 256, 0, [&](uint32_t i) {
+      dyn_engine& e = *E[i];
+      const Plan& pl = PL[i];
+      PmePrepArgs A;
+      std::memset(&A, 0, sizeof A);
+      if (np) {
         A.pos = e.pos_dev;
         A.q = e.q.p;
         A.g = e.geom;
@@ -2723,9 +2733,45 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
           A.g.n_dyn = 0;
           A.g.n_water = 0;
         }
-        return args<k_eng_pme_prep>(A);
-      });
+      }
+      CorrArgs C;
+      std::memset(&C, 0, sizeof C);
+      if (nc) {
+        C.P = pl.P;
+        C.wpos = e.wpos.p;
+        C.ltype = e.ltype.p;
+        C.lj_table = e.lj_table.p;
+        C.lj_se = e.lj_se.p;
+        C.ci = e.corr_i.p;
+        C.cj = e.corr_j.p;
+        C.kind = e.corr_kind.p;
+        C.n = pl.corr_on ? e.n_corr : 0u;
+        C.mode = (int)e.prm.mode;
+        C.recip_on = pl.recip_on ? 1 : 0;
+        C.nblk = e.corr_blocks;
+        C.fx = e.fx_site.p;
+        C.n_sites = e.n_sites;
+        C.partials = energy_on ? e.corr_part.p : nullptr;
+        C.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
+        C.mol_of = e.mol_of.p;
+        C.n_mol = e.n_mol;
+      }
+      BondedArgs B;
+      std::memset(&B, 0, sizeof B);
+      if (nb) B = side->args(i);
+      return args<k_eng_side>(A, C, B, np, nc);
+    });
+  };
+  {
+    Profiler::Scope ps(prof, "side");
+    if (RP.stream == RS.stream) {
+      side_launch(RS, 0, n_prep, n_corr, n_bond);
+    } else {
+      side_launch(RP, 1, n_prep, 0u, 0u);
+      side_launch(RS, 2, 0u, n_corr, n_bond);
     }
+  }
+  if (any_recip) {
     std::vector<PmeRun> ra(ns), rb(ns);
     for (uint32_t i = 0; i < ns; ++i) {
       dyn_engine& e = *E[i];
@@ -2744,7 +2790,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
       r.res = e.eng_out.p + 16;
       r.status = e.status.p;
       r.status_bit = kStPme;
-      r.binned = true;  // k_eng_pme_prep has listed the charges
+      r.binned = true;  // the side launch has listed the charges
       ra[i] = r;
       r.binned = false;
       if (pl.recip_b) {
@@ -2757,36 +2803,6 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags,
     pme_run(RP, prof, ra.data(), 0);
     if (any_b) pme_run(RP, prof, rb.data(), 1);
   }
-  // the exclusion and 1-4 corrections (site accumulators; finalize reads them)
-  if (any_corr) {
-    Profiler::Scope ps(prof, "corr");
-    const unsigned gc = max_grid(S, [](dyn_engine& e) { return e.corr_blocks; });
-    launch<k_eng_corr, kCorrBlock>(RS, "k_eng_corr", 0, gc, kCorrBlock, 0, [&](uint32_t i) {
-      dyn_engine& e = *E[i];
-      CorrArgs C;
-      std::memset(&C, 0, sizeof C);
-      C.P = PL[i].P;
-      C.wpos = e.wpos.p;
-      C.ltype = e.ltype.p;
-      C.lj_table = e.lj_table.p;
-      C.lj_se = e.lj_se.p;
-      C.ci = e.corr_i.p;
-      C.cj = e.corr_j.p;
-      C.kind = e.corr_kind.p;
-      C.n = PL[i].corr_on ? e.n_corr : 0u;
-      C.mode = (int)e.prm.mode;
-      C.recip_on = PL[i].recip_on ? 1 : 0;
-      C.nblk = e.corr_blocks;
-      C.fx = e.fx_site.p;
-      C.n_sites = e.n_sites;
-      C.partials = energy_on ? e.corr_part.p : nullptr;
-      C.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
-      C.mol_of = e.mol_of.p;
-      C.n_mol = e.n_mol;
-      return args<k_eng_corr>(C);
-    });
-  }
-  if (side_work) side_work(RS);
   // a staged build on the second stream, beside the pair kernel (after it
   // when there is one stream)
   const bool one_stream = RS.stream == R.stream;
@@ -3718,17 +3734,16 @@ int engine_mode(const dyn_engine* eng) { return (int)eng->prm.mode; }
 // Keep the last evaluation's outputs (site forces, SPME forces, energies)
 // on the engine's stream; engine_restore puts them back and marks the list
 // for a rebuild (it was built for positions the caller is discarding).
-void engine_checkpoint(dyn_engine* e) {
+void engine_checkpoint(dyn_engine* e, CopySegs& seg) {
   if (e->fx_stale) throw Error(DYN_ERR_STATE, "the last evaluation's forces were summed by its caller");
   const size_t nf = 3 * (size_t)e->n_sites;
   e->fx_out_ck.reserve(nf);
   e->eng_ck.reserve(kEngOut);
-  DYN_HIP(hipMemcpyAsync(e->fx_out_ck.p, e->fx_out.p, 8 * nf, hipMemcpyDeviceToDevice, e->stream));
-  DYN_HIP(hipMemcpyAsync(e->eng_ck.p, e->eng_out.p, 8 * kEngOut, hipMemcpyDeviceToDevice, e->stream));
+  seg.add(e->fx_out_ck.p, e->fx_out.p, 8 * nf);
+  seg.add(e->eng_ck.p, e->eng_out.p, 8 * kEngOut);
   if (e->pme_on) {
     e->fx_recip_ck.reserve(nf);
-    DYN_HIP(hipMemcpyAsync(e->fx_recip_ck.p, e->fx_recip.p, 8 * nf, hipMemcpyDeviceToDevice,
-                           e->stream));
+    seg.add(e->fx_recip_ck.p, e->fx_recip.p, 8 * nf);
   }
   e->ck.recip_kept = e->recip_kept;
   e->ck.last_recip_b = e->last_recip_b;

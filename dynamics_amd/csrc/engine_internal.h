@@ -5,10 +5,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <functional>
 #include <vector>
 
 #include "batch.h"
+#include "bonded.h"
 #include "common.h"
 #include "forces.h"
 
@@ -34,8 +36,8 @@ struct EngineSet {
 // Enqueue one evaluation of every engine in the set (DYN_COMPUTE_* flags,
 // the same for all).  Each engine decides on the device whether it rebuilds
 // its pair list (DYN_COMPUTE_REBUILD, or a list never built, forces it).
-// side_work, when given, enqueues further work on the side stream (or the
-// main one) after the SPME chain; it must not read the nonbonded forces.
+// side, when given, are bonded terms to evaluate in the same pass (they read
+// no nonbonded forces).
 // Internal compute flag (beside the public DYN_COMPUTE_* bits): list builds
 // the device decides on go to the staging list on the second stream, beside
 // the pair kernel, and become current at the next evaluation; an evaluation
@@ -46,8 +48,11 @@ constexpr uint32_t kComputeStagedBuild = 1u << 30;
 // and the engine's force array stays stale until a later evaluation
 // finalizes.
 constexpr uint32_t kComputeFusedFinalize = 1u << 29;
-void engine_set_enqueue(EngineSet& S, uint32_t flags,
-                        const std::function<void(const BatchRun&)>& side_work = nullptr);
+struct SideWork {
+  unsigned blocks = 0;  // workgroups of the system that needs most
+  std::function<BondedArgs(uint32_t)> args;
+};
+void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side = nullptr);
 // Wait for the set's work and check each engine's device status (throws the
 // first engine's error; buffers that overflowed have been enlarged).
 void engine_set_check(EngineSet& S);
@@ -81,8 +86,27 @@ void engine_report_energies(dyn_engine* eng, dyn_energies* out);
 // Pinned host memory of the engine, 24 bytes per site, for the caller's
 // next read.
 void* engine_host_stage(dyn_engine* eng);
-// Keep / put back the last evaluation's forces, SPME forces and energies
-// (enqueued on the engine's stream); a restore also invalidates the list.
-void engine_checkpoint(dyn_engine* eng);
+// Device arrays to copy, in words of 8 bytes.
+struct CopySegs {
+  static constexpr uint32_t kMax = 8;
+  const uint2* src[kMax];
+  uint2* dst[kMax];
+  uint64_t words_of[kMax];
+  uint64_t n;
+  void add(void* to, const void* from, size_t bytes) {
+    src[n] = static_cast<const uint2*>(from);
+    dst[n] = static_cast<uint2*>(to);
+    words_of[n++] = bytes / 8;
+  }
+  size_t words() const {
+    size_t m = 0;
+    for (uint64_t k = 0; k < n; ++k) m = std::max(m, (size_t)words_of[k]);
+    return m;
+  }
+};
+// Keep / put back the last evaluation's forces, SPME forces and energies (a
+// checkpoint adds the copies its caller makes on the engine's stream); a
+// restore also invalidates the list.
+void engine_checkpoint(dyn_engine* eng, CopySegs& seg);
 void engine_restore(dyn_engine* eng);
 }  // namespace dyn

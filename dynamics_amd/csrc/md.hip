@@ -26,6 +26,7 @@
 #include <numeric>
 #include <vector>
 
+#include "bonded.h"
 #include "common.h"
 #include "dyn_math.h"
 #include "engine_internal.h"
@@ -48,34 +49,7 @@ constexpr int kShakeMaxIt = 100;                   // src/bonded.rs:16
 constexpr int kMaxClusterCons = 16;                // constraints of one cluster
 constexpr int kBlock = 256;
 
-struct V3 {
-  float x, y, z;
-};
-__device__ __forceinline__ V3 v3(float x, float y, float z) { return {x, y, z}; }
-__device__ __forceinline__ V3 operator+(V3 a, V3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ V3 operator-(V3 a, V3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-__device__ __forceinline__ V3 operator*(V3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
-__device__ __forceinline__ float dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ V3 cross(V3 a, V3 b) {
-  return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
-}
-__device__ __forceinline__ V3 ld(const float4& p) { return {p.x, p.y, p.z}; }
-
-struct Box {
-  float L[3];
-};
-// src/barostat.rs:141-170: dv − round(dv/ext)·ext, and rem_euclid wrap into [0, L).
-// Reciprocal, square root and reciprocal square root by the hardware
-// instructions (about 1 ulp): the integrator's constraint, rigid-body and
-// bonded arithmetic needs no correctly rounded division.
-__device__ __forceinline__ float hw_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ float hw_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ float hw_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
-
-__device__ __forceinline__ V3 min_image(V3 d, const Box& b) {
-  return {dyn_min_image_ref(d.x, b.L[0]), dyn_min_image_ref(d.y, b.L[1]),
-          dyn_min_image_ref(d.z, b.L[2])};
-}
+// rem_euclid wrap into [0, L) (src/barostat.rs:141-170).
 __device__ __forceinline__ float wrap_coord(float x, float L) {
   // a coordinate within one box length of the box: one exact add or
   // subtract (the same result as fmod); anything farther takes fmod
@@ -438,130 +412,15 @@ __device__ __forceinline__ float4 langevin_value(float4 vv, uint32_t s, float c,
   return vv;
 }
 
-struct BondedArgs {
-  const float4* x;
-  Box B;
-  uint32_t n_dyn;
-  uint32_t n_bond, n_angle, n_dihe;
-  const uint32_t* bond;   // 2 per term
-  const float2* bond_p;   // k, r0
-  const uint32_t* angle;  // 3 per term (vertex in the middle)
-  const float2* angle_p;  // k, θ0
-  const uint32_t* dihe;   // 4 per term
-  const float4* dihe_p;   // k, periodicity (an integer 0..6), cos(phase), sin(phase)
-  int64_t* f;             // fixed point, component-major over solute atoms
-  double* partials;       // 4 per block: bond, angle, dihedral energy, virial
-  uint32_t nblk;          // workgroups of the system (one partial each)
-};
+__device__ __forceinline__ void k_md_bonded(BondedArgs A) { bonded_terms(A, blockIdx.x); }
 
-__device__ __forceinline__ void add_f(int64_t* f, uint32_t nd, uint32_t i, V3 v) {
-  atomicAdd(reinterpret_cast<unsigned long long*>(f + i), (unsigned long long)dyn_fx(v.x));
-  atomicAdd(reinterpret_cast<unsigned long long*>(f + nd + i), (unsigned long long)dyn_fx(v.y));
-  atomicAdd(reinterpret_cast<unsigned long long*>(f + 2 * (size_t)nd + i), (unsigned long long)dyn_fx(v.z));
-}
-
-// Harmonic bonds and angles (U = k(r − r0)², k(θ − θ0)²) and periodic
-// dihedrals (U = k(1 + cos(nφ − γ)), φ the IUPAC torsion angle); one
-// thread per term, fixed-point force sums.  The virial Σ r_a·F_a of each
-// term is taken relative to one of its atoms (src/bonded.rs:41-46, :79-83,
-// :124-130; the same sign convention for every term).
-__device__ __forceinline__ void k_md_bonded(BondedArgs A) {
-  __shared__ double red[4][kBlock / 64];
-  if (blockIdx.x >= A.nblk) return;  // partials exist for the system's own blocks
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  double e[4] = {0.0, 0.0, 0.0, 0.0};
-  const uint32_t nd = A.n_dyn;
-  if (t < A.n_bond) {
-    const uint32_t i = A.bond[2 * t], j = A.bond[2 * t + 1];
-    const V3 d = min_image(ld(A.x[j]) - ld(A.x[i]), A.B);
-    const float r = hw_sqrt(dot(d, d));
-    const float2 p = A.bond_p[t];
-    const float dr = r - p.y;
-    const V3 fi = d * (2.0f * p.x * dr * hw_rcp(fmaxf(r, 1e-8f)));
-    add_f(A.f, nd, i, fi);
-    add_f(A.f, nd, j, fi * -1.0f);
-    e[0] = (double)(p.x * dr * dr);
-    e[3] = -(double)dot(d, fi);  // (r_i − r_j)·F_i
-  } else if (t - A.n_bond < A.n_angle) {
-    const uint32_t q = t - A.n_bond;
-    const uint32_t i = A.angle[3 * q], j = A.angle[3 * q + 1], k = A.angle[3 * q + 2];
-    const V3 b0 = min_image(ld(A.x[i]) - ld(A.x[j]), A.B);
-    const V3 b2 = min_image(ld(A.x[k]) - ld(A.x[j]), A.B);
-    const float l0s = dot(b0, b0), l2s = dot(b2, b2);
-    if (l0s >= 1e-8f && l2s >= 1e-8f) {
-      const float il0 = hw_rsqrt(l0s), il2 = hw_rsqrt(l2s);
-      const V3 u0 = b0 * il0, u2 = b2 * il2;
-      const float ct = fminf(1.0f, fmaxf(-1.0f, dot(u0, u2)));
-      const float th = acosf(ct);
-      const float ist = hw_rcp(fmaxf(hw_sqrt(1.0f - ct * ct), 1e-8f));
-      const float2 p = A.angle_p[q];
-      const float dth = th - p.y;
-      const float dedt = 2.0f * p.x * dth;
-      const V3 g0 = (u0 * ct - u2) * (il0 * ist);
-      const V3 g2 = (u2 * ct - u0) * (il2 * ist);
-      const V3 f0 = g0 * -dedt, f2 = g2 * -dedt;
-      add_f(A.f, nd, i, f0);
-      add_f(A.f, nd, k, f2);
-      add_f(A.f, nd, j, (f0 + f2) * -1.0f);
-      e[1] = (double)(p.x * dth * dth);
-      e[3] = (double)dot(b0, f0) + (double)dot(b2, f2);
-    }
-  } else if (t - A.n_bond - A.n_angle < A.n_dihe) {
-    const uint32_t q = t - A.n_bond - A.n_angle;
-    const uint32_t i = A.dihe[4 * q], j = A.dihe[4 * q + 1], k = A.dihe[4 * q + 2],
-                   l = A.dihe[4 * q + 3];
-    const V3 b1 = min_image(ld(A.x[j]) - ld(A.x[i]), A.B);
-    const V3 b2 = min_image(ld(A.x[k]) - ld(A.x[j]), A.B);
-    const V3 b3 = min_image(ld(A.x[l]) - ld(A.x[k]), A.B);
-    const V3 n1 = cross(b1, b2), n2 = cross(b2, b3);
-    const float n1s = dot(n1, n1), n2s = dot(n2, n2), b2s = dot(b2, b2);
-    const float b2l = hw_sqrt(b2s);
-    if (n1s >= 1e-6f && n2s >= 1e-6f && b2l >= 1e-6f) {
-      // cos φ, sin φ of the IUPAC torsion φ = atan2(|b2| b1·n2, n1·n2); then
-      // cos nφ, sin nφ by the angle-addition recurrence and the phase by one
-      // more rotation: cos(nφ − γ), sin(nφ − γ) without trigonometric calls
-      const float4 p = A.dihe_p[q];
-      const float y = b2l * dot(b1, n2), x = dot(n1, n2);
-      const float rinv = hw_rsqrt(x * x + y * y);
-      const float c1 = x * rinv, s1 = y * rinv;
-      float cn = 1.0f, sn = 0.0f;
-      const int nper = (int)p.y;
-      for (int k = 0; k < nper; ++k) {
-        const float c2 = cn * c1 - sn * s1;
-        sn = sn * c1 + cn * s1;
-        cn = c2;
-      }
-      const float cos_arg = cn * p.z + sn * p.w;   // cos(nφ − γ)
-      const float sin_arg = sn * p.z - cn * p.w;   // sin(nφ − γ)
-      const float dedphi = -p.x * p.y * sin_arg;
-      // ∂φ/∂x_i = −|b2|/|n1|² n1, ∂φ/∂x_l = |b2|/|n2|² n2; the inner atoms
-      // take the lever-arm split of the two
-      const V3 gi = n1 * (-b2l * hw_rcp(n1s)), gl = n2 * (b2l * hw_rcp(n2s));
-      const float ib2s = hw_rcp(b2s);
-      const float ta = dot(b1, b2) * ib2s, tb = dot(b3, b2) * ib2s;
-      const V3 gj = gl * tb - gi * (1.0f + ta);
-      const V3 gk = gi * ta - gl * (1.0f + tb);
-      add_f(A.f, nd, i, gi * -dedphi);
-      add_f(A.f, nd, j, gj * -dedphi);
-      add_f(A.f, nd, k, gk * -dedphi);
-      add_f(A.f, nd, l, gl * -dedphi);
-      e[2] = (double)(p.x * (1.0f + cos_arg));
-      // relative to atom j: r_i − r_j = −b1, r_k − r_j = b2, r_l − r_j = b2 + b3
-      e[3] = -(double)dot(b1, gi * -dedphi) + (double)dot(b2, gk * -dedphi) +
-             (double)dot(b2 + b3, gl * -dedphi);
-    }
-  }
-  if (!A.partials) return;  // forces only
-  // wave sums by shuffles, then the block's waves in a fixed order
-  for (int c = 0; c < 4; ++c)
-    for (int m = 32; m >= 1; m >>= 1) e[c] += __shfl_xor(e[c], m, 64);
-  if ((threadIdx.x & 63) == 0)
-    for (int c = 0; c < 4; ++c) red[c][threadIdx.x / 64] = e[c];
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    double t = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w) t += red[threadIdx.x][w];
-    A.partials[4 * blockIdx.x + threadIdx.x] = t;
+__device__ __forceinline__ void k_copy_segs(const CopySegs& A) {
+  for (uint32_t k = 0; k < A.n; ++k) {
+    const uint2* __restrict__ src = A.src[k];
+    uint2* __restrict__ dst = A.dst[k];
+    const uint64_t n = A.words_of[k];
+    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock)
+      dst[i] = src[i];
   }
 }
 
@@ -1226,41 +1085,43 @@ void md_forces(MdSet& S, bool energies, bool fb_clear = true, bool fuse = false)
     any = any || (m->n_bond + m->n_angle + m->n_dihe) > 0;
     gb = std::max(gb, m->bblocks);
   }
-  // bonded forces on the engines' second stream, beside the pair kernel
-  auto bonded = [&](const BatchRun& RS) {
-    if (!any) return;
-    const BatchRun& RB = RS.stream == S.side.stream ? S.side : S.R;
-    Profiler::Scope ps(*S.prof, "md_bonded");
-    launch<k_md_bonded, kBlock>(RB, "k_md_bonded", 0, gb, kBlock, 0, [&](uint32_t i) {
-      dyn_md& m = *S.m[i];
-      BondedArgs A;
-      std::memset(&A, 0, sizeof A);
-      A.x = m.x.p;
-      for (int a = 0; a < 3; ++a) A.B.L[a] = m.box[a];
-      A.n_dyn = m.n_dyn;
-      A.n_bond = m.n_bond;
-      A.n_angle = m.n_angle;
-      A.n_dihe = m.n_dihe;
-      A.bond = m.bond.p;
-      A.bond_p = m.bond_p.p;
-      A.angle = m.angle.p;
-      A.angle_p = m.angle_p.p;
-      A.dihe = m.dihe.p;
-      A.dihe_p = m.dihe_p.p;
-      A.f = m.fb.p;
-      A.partials = energies ? m.bpart.p : nullptr;
-      A.nblk = m.bblocks;
-      return args<k_md_bonded>(A);
-    });
+  // bonded forces beside the engines' own work on the second stream
+  SideWork bonded;
+  bonded.blocks = any ? gb : 0u;
+  bonded.args = [&](uint32_t i) {
+    dyn_md& m = *S.m[i];
+    BondedArgs A;
+    std::memset(&A, 0, sizeof A);
+    A.x = m.x.p;
+    for (int a = 0; a < 3; ++a) A.B.L[a] = m.box[a];
+    A.n_dyn = m.n_dyn;
+    A.n_bond = m.n_bond;
+    A.n_angle = m.n_angle;
+    A.n_dihe = m.n_dihe;
+    A.bond = m.bond.p;
+    A.bond_p = m.bond_p.p;
+    A.angle = m.angle.p;
+    A.angle_p = m.angle_p.p;
+    A.dihe = m.dihe.p;
+    A.dihe_p = m.dihe_p.p;
+    A.f = m.fb.p;
+    A.partials = energies ? m.bpart.p : nullptr;
+    A.nblk = m.bblocks;
+    return A;
   };
   if (first) {
     engine_set_compute_sync(S.es, flags);
-    bonded(S.R);
+    if (any) {
+      Profiler::Scope ps(*S.prof, "md_bonded");
+      launch<k_md_bonded, kBlock>(S.R, "k_md_bonded", 0, gb, kBlock, 0, [&](uint32_t i) {
+        return args<k_md_bonded>(bonded.args(i));
+      });
+    }
   } else {
     engine_set_enqueue(S.es,
                        flags | DYN_COMPUTE_ASYNC | (S.staged_builds ? kComputeStagedBuild : 0u) |
                            (fuse ? kComputeFusedFinalize : 0u),
-                       bonded);
+                       &bonded);
   }
   for (dyn_md* m : S.m) m->forces_valid = true;
 }
@@ -1494,22 +1355,28 @@ struct MdCk {
   bool forces_valid;
 };
 
+// One launch copies every array of every MD of the set (7 copies per MD were
+// 200 calls of about 5 µs for a set of 32).
 void md_checkpoint(MdSet& S, std::vector<MdCk>& ck) {
   ck.resize(S.m.size());
+  std::vector<CopySegs> seg(S.m.size());
+  size_t most = 1;
   for (size_t i = 0; i < S.m.size(); ++i) {
     dyn_md& m = *S.m[i];
     const size_t bytes = 16 * (size_t)m.n_sites;
-    DYN_HIP(hipMemcpyAsync(m.x_ck.p, m.x.p, bytes, hipMemcpyDeviceToDevice, S.R.stream));
-    DYN_HIP(hipMemcpyAsync(m.v_ck.p, m.v.p, bytes, hipMemcpyDeviceToDevice, S.R.stream));
+    std::memset(&seg[i], 0, sizeof seg[i]);
+    seg[i].add(m.x_ck.p, m.x.p, bytes);
+    seg[i].add(m.v_ck.p, m.v.p, bytes);
     ck[i] = {m.step, m.n_eval, m.n_pcouple, {m.box[0], m.box[1], m.box[2]}, m.forces_valid};
     if (m.forces_valid) {
-      DYN_HIP(hipMemcpyAsync(m.fb_ck.p, m.fb.p, 24 * (size_t)std::max(m.n_dyn, 1u),
-                             hipMemcpyDeviceToDevice, S.R.stream));
-      DYN_HIP(hipMemcpyAsync(m.bpart_ck.p, m.bpart.p, 32 * (size_t)m.bblocks,
-                             hipMemcpyDeviceToDevice, S.R.stream));
-      engine_checkpoint(m.eng);  // on the same stream as the set's work
+      seg[i].add(m.fb_ck.p, m.fb.p, 24 * (size_t)std::max(m.n_dyn, 1u));
+      seg[i].add(m.bpart_ck.p, m.bpart.p, 32 * (size_t)m.bblocks);
+      engine_checkpoint(m.eng, seg[i]);  // on the same stream as the set's work
     }
+    most = std::max(most, seg[i].words());
   }
+  launch<k_copy_segs>(S.R, "k_copy_segs", 0, grid_for(most, 1024, 1024), kBlock, 0,
+                      [&](uint32_t i) { return args<k_copy_segs>(seg[i]); });
 }
 
 // Waits for whatever the failed attempt left in flight, then puts every MD
