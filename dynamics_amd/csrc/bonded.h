@@ -35,9 +35,12 @@ __device__ __forceinline__ float hw_sqrt(float x) { return __builtin_amdgcn_sqrt
 __device__ __forceinline__ float hw_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // src/barostat.rs:141-170: dv − round(dv/ext)·ext.
+// A displacement within half a box (most are) is its own image; the three
+// correctly rounded divisions are passed over unless a lane needs them.
 __device__ __forceinline__ V3 min_image(V3 d, const Box& b) {
-  return {dyn_min_image_ref(d.x, b.L[0]), dyn_min_image_ref(d.y, b.L[1]),
-          dyn_min_image_ref(d.z, b.L[2])};
+  if (!(fabsf(d.x) < 0.49f * b.L[0] && fabsf(d.y) < 0.49f * b.L[1] && fabsf(d.z) < 0.49f * b.L[2]))
+    d = {dyn_min_image_ref(d.x, b.L[0]), dyn_min_image_ref(d.y, b.L[1]), dyn_min_image_ref(d.z, b.L[2])};
+  return d;
 }
 
 constexpr int kBondedBlock = 256;

@@ -1857,6 +1857,7 @@ struct PrepArgs {
   int force;          // the host asks for a build before the pair kernel: a staged one is dropped
   int64_t* fx_site;
   int64_t* mol_e;
+  uint64_t* step;     // the caller's count of evaluations to advance, or null
   uint32_t n_mol2;
   uint32_t unused;    // no implicit padding: argument packs are compared byte for byte
 };
@@ -1943,6 +1944,7 @@ __device__ __forceinline__ void k_eng_prep(PrepArgs A) {
   // finalize kernel clears them
   const bool commit = !A.force && A.fl[kFlReady] != 0u;
   if (t == 0) A.fl[kFlCommit] = commit ? 1u : 0u;
+  if (t == 0 && A.step) ++*A.step;
   const ListSlots& L = commit ? A.stg : A.cur;
   unsigned int v = 0u;
   if (t < n) {
@@ -2685,6 +2687,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
       A.fx_site = e.fx_site.p;
       A.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
       A.n_mol2 = e.n_mol * e.n_mol;
+      A.step = side && side->step ? side->step(i) : nullptr;
       return args<k_eng_prep>(A);
     });
   }

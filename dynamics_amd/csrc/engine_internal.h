@@ -51,6 +51,7 @@ constexpr uint32_t kComputeFusedFinalize = 1u << 29;
 struct SideWork {
   unsigned blocks = 0;  // workgroups of the system that needs most
   std::function<BondedArgs(uint32_t)> args;
+  std::function<uint64_t*(uint32_t)> step;  // a count to advance by one before them, or none
 };
 void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side = nullptr);
 // Wait for the set's work and check each engine's device status (throws the

@@ -82,6 +82,28 @@ __device__ __forceinline__ void site_force_sum(const ForceParts& P, uint32_t s, 
     for (int c = 0; c < 3; ++c) f[c] += P.fx_pair[(size_t)c * P.n_sites + s];
 }
 
+// Adds a[at .. at + 3], two values per load.
+__device__ __forceinline__ void add4(const int64_t* __restrict__ a, size_t at, int64_t f[4]) {
+  typedef long long pair_t __attribute__((ext_vector_type(2), aligned(8)));
+  const pair_t* p = reinterpret_cast<const pair_t*>(a + at);
+  const pair_t u = p[0], v = p[1];
+  f[0] += u.x;
+  f[1] += u.y;
+  f[2] += v.x;
+  f[3] += v.y;
+}
+// Forces of the four consecutive sites from s on, f[component][site].
+__device__ __forceinline__ void site_force_sum4(const ForceParts& P, uint32_t s, int64_t f[3][4]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const size_t at = (size_t)c * P.n_sites + s;
+    for (int k = 0; k < 4; ++k) f[c][k] = 0;
+    add4(P.fx_site, at, f[c]);
+    if (P.fx_recip) add4(P.fx_recip, at, f[c]);
+    if (P.fx_pair) add4(P.fx_pair, at, f[c]);
+  }
+}
+
 // The end of the evaluation's list bookkeeping (one thread, after the pair
 // kernel): a staged list taken by the preparation kernel is the current one
 // from now on; the growth of the largest displacement (a decaying maximum of

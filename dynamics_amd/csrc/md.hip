@@ -48,6 +48,7 @@ constexpr float kEpsConstr = 1.0e-8f;              // src/bonded.rs:10
 constexpr int kShakeMaxIt = 100;                   // src/bonded.rs:16
 constexpr int kMaxClusterCons = 16;                // constraints of one cluster
 constexpr int kBlock = 256;
+constexpr int kStepBlock = 64;                     // of the step kernels (k_md_step_ba)
 
 // rem_euclid wrap into [0, L) (src/barostat.rs:141-170).
 __device__ __forceinline__ float wrap_coord(float x, float L) {
@@ -246,10 +247,23 @@ struct WaterAcc {
   V3 a[3];  // O, H0, H1
 };
 __device__ __forceinline__ WaterAcc water_accel(const Fx& F, uint32_t base) {
-  const V3 fm = force_of(F, base + 1);
-  const V3 fo = force_of(F, base) + fm * kCO;
-  const V3 f0 = force_of(F, base + 2) + fm * kCH;
-  const V3 f1 = force_of(F, base + 3) + fm * kCH;
+  int64_t q[3][4];
+  if (F.parts) {
+    site_force_sum4(F.P, base, q);
+  } else {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      for (int k = 0; k < 4; ++k) q[c][k] = 0;
+      add4(F.nb, (size_t)c * F.n_sites + base, q[c]);
+    }
+  }
+  V3 f[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    f[k] = {(float)((double)q[0][k] * DYN_FX_INV_SCALE), (float)((double)q[1][k] * DYN_FX_INV_SCALE),
+            (float)((double)q[2][k] * DYN_FX_INV_SCALE)};
+  const V3 fm = f[1];
+  const V3 fo = f[0] + fm * kCO, f0 = f[2] + fm * kCH, f1 = f[3] + fm * kCH;
   const float co = kKcalToNative / kMassO, ch = kKcalToNative / kMassH;
   return {{fo * co, f0 * ch, f1 * ch}};
 }
@@ -734,8 +748,8 @@ struct StepArgs {
 // bonded force sums.  PREV: the group first finishes the previous step
 // (k_md_step_b's kick ½ and RATTLE, with the same forces) in registers, so
 // two steps meet in one launch; the operations and their order are those of
-// the two separate launches.  The index of the step that begins here (it
-// seeds the Langevin noise) is *step_dev + PREV.  Thread g < n_sgroups
+// the two separate launches.  *step_dev is the index of the step that begins
+// here (it seeds the Langevin noise).  Thread g < n_sgroups
 // holds a solute group, thread water0 + w water w (water0 rounds n_sgroups
 // up to a whole wave, so no wave runs both paths).
 template <bool PREV>
@@ -774,7 +788,7 @@ __device__ __forceinline__ void step_group(const StepArgs& A, float4* __restrict
       rattle_star(A.C, g, D, im, X, V);
     }
     if (A.langevin) {
-      const uint64_t step = *step_dev + PREV;
+      const uint64_t step = *step_dev;
 #pragma unroll
       for (int k = 0; k <= kStarMax; ++k)
         if (k <= (int)D.n) V[k] = langevin_value(V[k], D.atom[k], A.lang_c, sg[k], A.seed, step);
@@ -813,7 +827,7 @@ __device__ __forceinline__ void step_group(const StepArgs& A, float4* __restrict
       rattle_cluster(A.C, g, x, v);
     }
     if (A.langevin) {
-      const uint64_t step = *step_dev + PREV;
+      const uint64_t step = *step_dev;
       for (uint32_t a = a0; a < a1; ++a) {
         const uint32_t t = A.G.grp_atoms[a];
         langevin_site(v, t, A.lang_c, A.sigma_dyn[t], A.seed, step);
@@ -844,7 +858,7 @@ __device__ __forceinline__ void step_group(const StepArgs& A, float4* __restrict
   kick_water(wa, A.h, W);
   rigid_drift(W, hd, A.G.B);
   if (A.langevin) {
-    const uint64_t step = *step_dev + PREV;
+    const uint64_t step = *step_dev;
     W.v[0] = langevin_value(W.v[0], base, A.lang_c, A.sigma_o, A.seed, step);
     W.v[2] = langevin_value(W.v[2], base + 2, A.lang_c, A.sigma_h, A.seed, step);
     W.v[3] = langevin_value(W.v[3], base + 3, A.lang_c, A.sigma_h, A.seed, step);
@@ -866,41 +880,33 @@ __device__ __forceinline__ void k_md_step_a(StepArgs A, float4* __restrict__ x,
 }
 
 // The end of one step and the beginning of the next in one launch (no
-// energies or pressure are observed between them).  step_dev[0] is the
-// index of the step that ends here; the launch advances it once every
-// workgroup has used it: each workgroup counts itself in step_dev[1] when
-// its threads are done, and the last one stores the new index and clears
-// the count.  No fence precedes the count: a workgroup's reads of the
-// index have completed (their values are used before the barrier), and the
-// positions and velocities it wrote are read by later launches only, which
-// the end of this launch makes visible (a device-scope fence per workgroup
-// would write back the L2 each time).
+// energies or pressure are observed between them).  The step index is
+// advanced by the preparation launch of every step's evaluation, so that
+// here it is that of the step that begins.
+//
+// Bound: one thread's chain — the forces' loads, two rigid drifts, nine
+// deviates — so a workgroup is one wave (the waters of a small system on as many
+// compute units as there are), the four sites' forces come two to a load, a
+// water within half a box takes no divisions, and no workgroup counts itself
+// (an atomic on one word takes about 0.1 µs per workgroup).  28,000 sites
+// 18.9 µs with workgroups of 256, 8-byte loads, divisions and the count; now
+// 15.5 (252,480 sites 19.6, now 15.4).
 __device__ __forceinline__ void k_md_step_ba(StepArgs A, float4* __restrict__ x,
                                              float4* __restrict__ v,
-                                             uint64_t* __restrict__ step_dev) {
+                                             const uint64_t* __restrict__ step_dev) {
   // in place of the engine's finalize launch: the evaluation's bookkeeping
   if (A.F.parts && blockIdx.x == 0 && threadIdx.x == 0) evaluation_flags_end(A.F.P.fl, A.F.P.forced);
-  if (*A.status) return;  // every workgroup reads the same word: none counts itself
+  if (*A.status) return;
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g < A.water0 + A.G.n_water) step_group<true>(A, x, v, g, step_dev);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned* done = reinterpret_cast<unsigned*>(step_dev + 1);
-    if (atomicAdd(done, 1u) == gridDim.x - 1) {
-      step_dev[0] = step_dev[0] + 1;
-      *done = 0u;
-    }
-  }
 }
 
 // After the force evaluation: kick ½ with the new forces, RATTLE; the step's
 // last launch advances the device step index.
 __device__ __forceinline__ void k_md_step_b(StepArgs A, float4* __restrict__ x,
-                                            float4* __restrict__ v,
-                                            uint64_t* __restrict__ step_inc) {
+                                            float4* __restrict__ v) {
   if (*A.status) return;
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g == 0) ++*step_inc;
   if (g >= A.water0 + A.G.n_water) return;
   if (g < A.G.n_sgroups && A.stars[g].natoms) {
     const StarDesc D = A.stars[g];
@@ -999,7 +1005,7 @@ struct dyn_md {
   unsigned eblocks = 1;     // workgroups of k_md_energies
   PinnedBuf<double> h_out;  // their partials
   uint64_t step = 0;
-  DevBuf<uint64_t> step_dev;  // the step index (the Langevin noise's), a workgroup count
+  DevBuf<uint64_t> step_dev;  // the step index (the Langevin noise's)
   uint64_t n_eval = 0;  // force evaluations since set_state (SPME cadence)
   bool state_set = false, forces_valid = false;
   // pressure groups (solute constraint clusters and lone atoms; waters
@@ -1109,6 +1115,8 @@ void md_forces(MdSet& S, bool energies, bool fb_clear = true, bool fuse = false)
     A.nblk = m.bblocks;
     return A;
   };
+  // a step's evaluation (not one of a state on its own) ends with the next index
+  if (!fb_clear) bonded.step = [&](uint32_t i) { return S.m[i]->step_dev.p; };
   if (first) {
     engine_set_compute_sync(S.es, flags);
     if (any) {
@@ -1228,7 +1236,7 @@ uint32_t step_water0(const dyn_md& m) { return (m.n_sgroups + 63u) / 64u * 64u; 
 
 unsigned step_grid(const MdSet& S) {
   unsigned g = 1;
-  for (dyn_md* m : S.m) g = std::max(g, grid_for(step_water0(*m) + m->n_water, kBlock));
+  for (dyn_md* m : S.m) g = std::max(g, grid_for(step_water0(*m) + m->n_water, kStepBlock));
   return g;
 }
 
@@ -1312,7 +1320,7 @@ bool md_one_step(MdSet& S, bool energies, bool begun, bool may_join) {
   energies = energies || couple;
   if (!begun) {
     Profiler::Scope ps(*S.prof, "md_step_a");
-    launch<k_md_step_a>(S.R, "k_md_step_a", 0, step_grid(S), kBlock, 0, [&](uint32_t i) {
+    launch<k_md_step_a, kStepBlock>(S.R, "k_md_step_a", 0, step_grid(S), kStepBlock, 0, [&](uint32_t i) {
       dyn_md& m = *S.m[i];
       return args<k_md_step_a>(step_args(m), m.x.p, m.v.p, (const uint64_t*)m.step_dev.p);
     });
@@ -1324,15 +1332,15 @@ bool md_one_step(MdSet& S, bool energies, bool begun, bool may_join) {
   const bool join = may_join && !(couple && !langevin);
   if (join) {
     Profiler::Scope ps(*S.prof, "md_step_ba");
-    launch<k_md_step_ba>(S.R, "k_md_step_ba", 0, step_grid(S), kBlock, 0, [&](uint32_t i) {
+    launch<k_md_step_ba, kStepBlock>(S.R, "k_md_step_ba", 0, step_grid(S), kStepBlock, 0, [&](uint32_t i) {
       dyn_md& m = *S.m[i];
-      return args<k_md_step_ba>(step_args(m), m.x.p, m.v.p, m.step_dev.p);
+      return args<k_md_step_ba>(step_args(m), m.x.p, m.v.p, (const uint64_t*)m.step_dev.p);
     });
   } else {
     Profiler::Scope ps(*S.prof, "md_step_b");
-    launch<k_md_step_b>(S.R, "k_md_step_b", 0, step_grid(S), kBlock, 0, [&](uint32_t i) {
+    launch<k_md_step_b, kStepBlock>(S.R, "k_md_step_b", 0, step_grid(S), kStepBlock, 0, [&](uint32_t i) {
       dyn_md& m = *S.m[i];
-      return args<k_md_step_b>(step_args(m), m.x.p, m.v.p, m.step_dev.p);
+      return args<k_md_step_b>(step_args(m), m.x.p, m.v.p);
     });
   }
   if (couple && !langevin) md_barostat(S);  // at the end of the step (src/integrate.rs:241-310)
@@ -1798,8 +1806,8 @@ extern "C" int dyn_md_create(dyn_md** out, dyn_engine* eng, const dyn_md_params*
     M->fb_ck.reserve(3 * (size_t)std::max(nd, 1u));
     M->bpart_ck.reserve(4 * (size_t)M->bblocks);
     M->v_ck.reserve(ns);
-    M->step_dev.reserve(2);  // the step index, the workgroup count of k_md_step_ba
-    DYN_HIP(hipMemsetAsync(M->step_dev.p, 0, 16, M->stream));
+    M->step_dev.reserve(1);
+    DYN_HIP(hipMemsetAsync(M->step_dev.p, 0, 8, M->stream));
     M->eblocks = grid_for(std::max<uint32_t>(nd + nw, 1), kBlock);
     M->h_out.reserve(2 * (size_t)M->eblocks);
     DYN_HIP(hipStreamSynchronize(M->stream));
