@@ -244,20 +244,104 @@ __device__ __forceinline__ int32_t site_gid(const int32_t* wmol, int32_t s) {
 
 // One column, by one workgroup: sort the column's sites by (z, site) and cut
 // them into clusters of 8 (the last padded), writing the slot arrays and each
-// cluster's bounding box.  The column's count is cleared for the next
-// binning pass (the binning kernel counts with atomics into zeroed counts).
+// cluster's bounding box.
+//
+// Bound: latency (a column is some 100 sites).  Up to kRankSites sites a
+// site's place is the number of smaller keys, counted from LDS without a
+// barrier, and its thread still holds everything its slot needs; a bitonic
+// sort takes 28 barriers for 128 keys and loads the sites again.  Longer
+// columns (thin boxes) keep the bitonic sort, which grows more slowly.  28,000
+// sites 26 µs with the bitonic sort only, now 20; 256,000 sites 57, now 40; 2,000
+// sites 14, now 8.2.
+constexpr uint32_t kRankSites = 512;
+constexpr uint32_t kRankPer = 2;  // sites per thread
 constexpr int kSortBlock = 256;
 constexpr unsigned kBuildGrid = 1024;  // workgroups of the grid-stride build kernels
 __device__ __forceinline__ void
 colsort_one(uint32_t c, uint32_t n, uint32_t cl0, const uint32_t* __restrict__ items,
             uint32_t col_slice, const int* __restrict__ col_class, const SlotArgs& S,
             uint8_t* __restrict__ cl_class, float4* __restrict__ bb_c, float4* __restrict__ bb_h,
-            unsigned int* __restrict__ status, unsigned long long* key) {
+            unsigned int* __restrict__ status, unsigned long long* key, const uint32_t (&first)[kRankPer]) {
   const size_t b = (size_t)c * col_slice;
   const uint32_t ncl = (n + DYN_CL_SIZE - 1) / DYN_CL_SIZE;
   if (ncl == 0) return;
   if (n > col_slice) {
     if (threadIdx.x == 0) atomicOr(status, kStColumn);
+    return;
+  }
+  if (n <= kRankSites) {
+    static_assert(kRankPer * kSortBlock == kRankSites, "kRankPer sites per thread");
+    static_assert(kColCap * 8 >= kRankSites * 8 + kRankSites * 16, "keys and sites share key[]");
+    float4* const sp = reinterpret_cast<float4*>(key + kRankSites);  // sites in order
+    float4 p[kRankPer];
+    int32_t type[kRankPer], gid[kRankPer];
+    uint32_t site[kRankPer];
+    unsigned long long mine[kRankPer];
+#pragma unroll
+    for (uint32_t r = 0; r < kRankPer; ++r) {
+      const uint32_t k = threadIdx.x + r * kSortBlock;
+      mine[r] = ~0ull;
+      if (k < n) {
+        const uint32_t s = first[r];
+        site[r] = s;
+        p[r] = S.wpos[s];
+        type[r] = S.ltype[s];
+        gid[r] = site_gid(S.wmol, (int32_t)s);
+        mine[r] = ((unsigned long long)__float_as_uint(p[r].z) << 32) | s;
+      }
+      key[k] = mine[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kRankPer; ++r) {
+      if (r * kSortBlock >= n) break;
+      uint32_t at = 0;
+      // (keys past n are larger than any)
+      for (uint32_t m = 0; m < n; m += 16) {
+        ulonglong2 u[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) u[q] = *reinterpret_cast<const ulonglong2*>(key + m + 2 * q);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) at += (u[q].x < mine[r]) + (u[q].y < mine[r]);
+      }
+      if (threadIdx.x + r * kSortBlock < n) {
+        const size_t slot = (size_t)cl0 * DYN_CL_SIZE + at;
+        S.slot_site[slot] = (int32_t)site[r];
+        S.xyzq[slot] = p[r];
+        S.slot_type[slot] = type[r];
+        S.slot_gid[slot] = gid[r];
+        S.slot_of[site[r]] = (uint32_t)slot;
+        sp[at] = p[r];
+      }
+    }
+    __syncthreads();
+    // eight lanes per cluster: padding slots (at its first site) and the box
+    for (uint32_t k = threadIdx.x; k < ((ncl * DYN_CL_SIZE + kWave - 1) & ~(uint32_t)(kWave - 1)); k += kSortBlock) {
+      const uint32_t cl = k / DYN_CL_SIZE, first = cl * DYN_CL_SIZE;
+      float4 q = sp[min(k < n ? k : first, n - 1u)];
+      float lo[3] = {q.x, q.y, q.z}, hi[3] = {q.x, q.y, q.z};
+      for (int m = 1; m < DYN_CL_SIZE; m <<= 1)
+        for (int a = 0; a < 3; ++a) {
+          lo[a] = fminf(lo[a], __shfl_xor(lo[a], m, kWave));
+          hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], m, kWave));
+        }
+      if (cl >= ncl) continue;
+      if (k >= n) {
+        const size_t slot = (size_t)cl0 * DYN_CL_SIZE + k;
+        q.w = 0.0f;
+        S.slot_site[slot] = -1;
+        S.xyzq[slot] = q;
+        S.slot_type[slot] = S.none_type;
+        S.slot_gid[slot] = DYN_GID_PAD;
+      }
+      if (k == first) {
+        cl_class[cl0 + cl] = (uint8_t)col_class[c];
+        bb_c[cl0 + cl] = make_float4(0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]), 0.5f * (lo[2] + hi[2]), 0.f);
+        // w: the cluster's sites (its first slots; the rest are padding)
+        bb_h[cl0 + cl] = make_float4(0.5f * (hi[0] - lo[0]), 0.5f * (hi[1] - lo[1]), 0.5f * (hi[2] - lo[2]),
+                                     __uint_as_float(min(n - first, (uint32_t)DYN_CL_SIZE)));
+      }
+    }
     return;
   }
   uint32_t np2 = 1;
@@ -333,9 +417,20 @@ k_eng_colsort(BuildGate G, const uint32_t* __restrict__ col_count, const uint32_
               const int* __restrict__ col_class, SlotArgs S, uint8_t* __restrict__ cl_class,
               float4* __restrict__ bb_c, float4* __restrict__ bb_h,
               unsigned int* __restrict__ status, uint32_t n_cols, uint32_t* __restrict__ n_cl) {
-  __shared__ unsigned long long key[kColCap];
+  __shared__ __align__(16) unsigned long long key[kColCap];
   __shared__ uint32_t wsum[kSortBlock / kWave];
   __shared__ uint32_t s_start;
+  // the sites of the workgroup's first column, loaded beside the gate and the
+  // counts (those past the column's count are not used)
+  uint32_t first[kRankPer];
+  auto load_first = [&](uint32_t c) {
+#pragma unroll
+    for (uint32_t r = 0; r < kRankPer; ++r) {
+      const uint32_t k = threadIdx.x + r * kSortBlock;
+      first[r] = c < n_cols && k < col_slice ? items[(size_t)c * col_slice + k] : 0u;
+    }
+  };
+  load_first(blockIdx.x);
   if (!build_on(G)) return;
   // every workgroup scans the columns' cluster counts itself (a scan launch
   // of its own would cost a dependent launch; one inside the binning launch
@@ -375,8 +470,9 @@ k_eng_colsort(BuildGate G, const uint32_t* __restrict__ col_count, const uint32_
     }
     __syncthreads();
     const uint32_t cl0 = s_start;
+    if (c != blockIdx.x) load_first(c);
     colsort_one(c, col_count[c], cl0, items, col_slice, col_class, S, cl_class, bb_c, bb_h, status,
-                key);
+                key, first);
     __syncthreads();  // key[] and s_start are reused by the next column
   }
 }
@@ -590,6 +686,7 @@ k_eng_list_walk(const ListArgs& A, uint32_t* __restrict__ ent_tmp) {
       }
       const bool full_xy = full_x || full_y;
       const int ny = y1 - y0 + 1, n_colc = (x1 - x0 + 1) * ny;
+      const float inv_ny = __builtin_amdgcn_rcpf((float)ny);
       // this unit's half of the window's columns (in walk order)
       const int kmid = (n_colc + 1) / 2;
       const int kbeg = half ? kmid : 0, kend = half ? n_colc : kmid;
@@ -597,17 +694,23 @@ k_eng_list_walk(const ListArgs& A, uint32_t* __restrict__ ent_tmp) {
         const int k = cb + lane;
         uint32_t js = 0, cnt = 0, img = 0;
         if (k < kend) {
-          const int xx = x0 + k / ny, yy = y0 + k % ny;
+          // (k / ny by a reciprocal: exact to within one)
+          int q = (int)((float)k * inv_ny);
+          int r = k - q * ny;
+          if (r < 0) --q, r += ny;
+          else if (r >= ny) ++q, r -= ny;
+          const int xx = x0 + q, yy = y0 + r;
           float dx = 0.f, dy = 0.f;
           if (!full_x) dx = fmaxf(0.f, fmaxf(xx * cg.wx - (c.x + h.x), (c.x - h.x) - (xx + 1) * cg.wx));
           if (!full_y) dy = fmaxf(0.f, fmaxf(yy * cg.wy - (c.y + h.y), (c.y - h.y) - (yy + 1) * cg.wy));
           if (dx * dx + dy * dy < col_r2) {
-            const int cx = ((xx % cg.ncx) + cg.ncx) % cg.ncx;
-            const int cy = ((yy % cg.ncy) + cg.ncy) % cg.ncy;
-            const int col = cg.col_off + cx * cg.ncy + cy;
+            // one period at most: the window is shorter than the grid and
+            // reaches from a wrapped position by less than one box
+            const int px = xx < 0 ? -1 : (xx >= cg.ncx ? 1 : 0), py = yy < 0 ? -1 : (yy >= cg.ncy ? 1 : 0);
+            const int col = cg.col_off + (xx - px * cg.ncx) * cg.ncy + (yy - py * cg.ncy);
             js = A.col_cl_start[col];
             cnt = A.col_cl_start[col + 1] - js;
-            img = (uint32_t)((xx - cx) / cg.ncx + 1) << 21 | (uint32_t)((yy - cy) / cg.ncy + 1) << 23;
+            img = (uint32_t)(px + 1) << 21 | (uint32_t)(py + 1) << 23;
           }
         }
         const uint32_t incl = wave_incl_sum(cnt);
@@ -785,6 +888,13 @@ static_assert(sizeof(ListCopies) == 64, "ListCopies has no padding");
 // sites of i slot ia and of the group's entry jb are a 1-2, 1-3 or 1-4 pair
 // (entry jb's exclusion byte, shifted into place).  One wave per class
 // segment of a row; the segment's entries move four per lane at a time.
+//
+// Every workgroup needs the groups and work items of the rows before its own.
+// Above kScanRows rows they come as sums per kScanSeg rows from a launch of its
+// own (k_eng_row_sums): summed by every workgroup itself, 33,000 rows took
+// 170 µs, now 43 and 4.7.  Below, each workgroup sums the rows themselves: a launch more
+// costs every MD step 3 µs, built or not.
+constexpr uint32_t kScanRows = 8192, kScanSeg = 256;
 constexpr int kFillUnroll = 4;
 constexpr uint32_t kFillRows = 4;  // rows per workgroup of the fill (3 class segments each)
 
@@ -802,10 +912,32 @@ __device__ __forceinline__ uint32_t row_groups(const uint32_t* __restrict__ unit
   return m;
 }
 
+// Groups and work items of each kScanSeg rows (a workgroup each).
+__device__ __forceinline__ void k_eng_row_sums(const ListArgs& A, uint2* __restrict__ seg) {
+  __shared__ uint32_t red[2][kListWaves];
+  static_assert(kScanSeg == kListBlock, "a thread per row");
+  if (!build_on(A.gate)) return;
+  const uint32_t n_cl = *A.n_cl, I = blockIdx.x * kScanSeg + threadIdx.x;
+  if (blockIdx.x * kScanSeg >= n_cl) return;
+  const uint32_t m = I < n_cl ? row_groups(A.unit_cnt, I) : 0u;
+  const uint32_t sg = wave_incl_sum(m), si = wave_incl_sum((m + A.chunk - 1) / A.chunk);
+  if ((threadIdx.x & (kWave - 1)) == kWave - 1) {
+    red[0][threadIdx.x / kWave] = sg;
+    red[1][threadIdx.x / kWave] = si;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint2 s = make_uint2(0u, 0u);
+    for (int w = 0; w < kListWaves; ++w) s = make_uint2(s.x + red[0][w], s.y + red[1][w]);
+    seg[blockIdx.x] = s;
+  }
+}
+
+// seg: the sums of k_eng_row_sums, or null.
 __device__ __forceinline__ void
 k_eng_list_fill(const ListArgs& A, const uint32_t* __restrict__ ent_tmp,
                 uint32_t* __restrict__ row_cnt, uint32_t* __restrict__ row_ptr,
-                uint32_t* __restrict__ chunk_ptr, ListCopies C) {
+                uint32_t* __restrict__ chunk_ptr, const uint2* __restrict__ seg, ListCopies C) {
   __shared__ uint32_t s_m[kFillRows], s_g[kFillRows], s_i[kFillRows];
   __shared__ uint32_t s_red[2][kListWaves];
   if (!build_on(A.gate)) return;
@@ -827,12 +959,19 @@ k_eng_list_fill(const ListArgs& A, const uint32_t* __restrict__ ent_tmp,
   }
   for (uint32_t blk = blockIdx.x; blk * kFillRows < n_cl; blk += gridDim.x) {
     const uint32_t r0 = blk * kFillRows, nr = min(kFillRows, n_cl - r0);
-    // the groups and work items of the rows before this block (every
-    // workgroup sums them itself: a scan launch of its own would cost a
-    // dependent launch on every step, and a scan inside the walk a
-    // device-scope fence per workgroup)
-    uint32_t sg = 0, si = 0;
-    for (uint32_t I = threadIdx.x; I < r0; I += kListBlock) {
+    // the groups and work items of the rows before this block (a scan inside
+    // the walk would cost a device-scope fence per workgroup)
+    uint32_t sg = 0, si = 0, first = 0;
+    if (seg) {
+      const uint32_t ns = r0 / kScanSeg;
+      first = ns * kScanSeg;
+      for (uint32_t k = threadIdx.x; k < ns; k += kListBlock) {
+        const uint2 s = seg[k];
+        sg += s.x;
+        si += s.y;
+      }
+    }
+    for (uint32_t I = first + threadIdx.x; I < r0; I += kListBlock) {
       const uint32_t m = row_groups(A.unit_cnt, I);
       sg += m;
       si += (m + A.chunk - 1) / A.chunk;
@@ -2208,6 +2347,7 @@ struct dyn_engine {
   DevBuf<float4> xyzq, bb_c, bb_h;
   DevBuf<uint32_t> row_cnt, row_ptr, chunk_ptr, cj, ent_tmp, unit_cnt;
   DevBuf<uint8_t> xb_tmp;  // exclusion byte of each ent_tmp entry
+  DevBuf<uint2> seg_sum;   // groups and work items per kScanSeg rows
   DevBuf<unsigned long long> cmask;
   DevBuf<uint2> chunks;
   uint64_t cap_entries = 0, cap_chunks = 0;  // groups of 8 j entries, work items
@@ -2379,6 +2519,7 @@ void dyn_engine::set_geometry() {
   bb_h.reserve(cap_cl);
   row_cnt.reserve(cap_cl + 1);
   unit_cnt.reserve((size_t)cap_cl * kUnits);
+  seg_sum.reserve((cap_cl + kScanSeg - 1) / kScanSeg);  // (a step call allocates nothing)
   row_ptr.reserve(cap_cl + 1);
   chunk_ptr.reserve(cap_cl + 1);
   stg_slot_site.reserve(cap_slots + DYN_CL_SIZE);
@@ -2572,13 +2713,23 @@ static void set_build_lists(EngineSet& S, const BatchRun& R, const std::vector<B
       return args<k_eng_list_walk>(LA[i], e.ent_tmp.p);
     });
   }
+  // (a rule on the largest system: the others' sums are there too)
+  const unsigned seg_grid = max_grid(S, [](dyn_engine& e) { return (e.cap_cl + kScanSeg - 1) / kScanSeg; });
+  const bool scan = seg_grid * kScanSeg > kScanRows;
+  if (scan) {
+    Profiler::Scope ps(prof, "nbl_row_sums");
+    launch<k_eng_row_sums, kListBlock>(R, "k_eng_row_sums", 0, seg_grid, kListBlock, 0, [&](uint32_t i) {
+      return args<k_eng_row_sums>(LA[i], E[i]->seg_sum.p);
+    });
+  }
   {
     Profiler::Scope ps(prof, "nbl_list_fill");
     launch<k_eng_list_fill, kListBlock>(R, "k_eng_list_fill", 0, list_grid, kListBlock, 0,
                                         [&](uint32_t i) {
       dyn_engine& e = *E[i];
-      return args<k_eng_list_fill>(LA[i], e.ent_tmp.p, e.row_cnt.p, T[i].row_ptr,
-                                   T[i].chunk_ptr, e.copies(staged));
+      return args<k_eng_list_fill>(LA[i], e.ent_tmp.p, e.row_cnt.p, T[i].row_ptr, T[i].chunk_ptr,
+                                   scan ? (const uint2*)e.seg_sum.p : (const uint2*)nullptr,
+                                   e.copies(staged));
     });
   }
 }

@@ -63,6 +63,30 @@ def test_short_range_vs_fp64_and_replay(gpu, cases, name):
     _check_item_sums(eng, dbg, ie)
 
 
+@pytest.mark.parametrize("times", [3, 5, 6, 12])
+def test_list_long_columns(gpu, cases, times):
+    """A 24.8 Å wide box 3 to 12 times as long: columns of about 300 to 1,200
+    sites, on both sides of the two column sorts' limit (512), and rows whose
+    candidates reach round the box.  The list equals the host restatement."""
+    s0 = cases["water512"]
+    s = copy.copy(s0)
+    L = float(s0.box[2])
+    s.box = np.array([L, L, L * times], s0.box.dtype)
+    for k in ("pos_o", "pos_m", "pos_h0", "pos_h1"):
+        p = getattr(s0, k)
+        setattr(s, k, np.concatenate([p + np.array([0, 0, L * i], p.dtype) for i in range(times)]))
+    print(f"long columns: {s.n_water} waters", flush=True)
+    eng = _engine(s)
+    eng.compute(api.COMPUTE_SHORT)
+    dbg = eng.debug_export()
+    n, slot_site, cl_class, row_ptr, cj, cm = replay_engine_list(s, RC, 0.0)
+    assert np.array_equal(dbg["slot_site"], slot_site)
+    assert np.array_equal(dbg["cl_class"], cl_class)
+    assert np.array_equal(dbg["row_ptr"], row_ptr)
+    assert np.array_equal(normalize_null_entries(dbg["cj"], 8 * n), cj)
+    eng.close()
+
+
 @pytest.mark.parametrize("cutoff,close", [(3.0, 0.0), (6.5, 0.0), (10.5, 0.0), (12.8, 0.0), (6.5, 0.03),
                                           (12.8, 1e-9)])
 def test_pair_tile_images_and_remainders(gpu, cases, cutoff, close):
