@@ -2147,12 +2147,7 @@ __device__ __forceinline__ void k_eng_finalize(ForceParts P, int64_t* __restrict
   for (int c = 0; c < 3; ++c) out[(size_t)c * P.n_sites + s] = f[c];
 }
 
-// Copies a block of doubles to pinned host memory (block b0 of the launch).
-__device__ __forceinline__ void k_eng_report(const double* __restrict__ src, double* __restrict__ dst,
-                                             uint32_t n, uint32_t b0) {
-  if (blockIdx.x == b0)
-    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) dst[k] = src[k];
-}
+__device__ __forceinline__ void k_eng_report(const ReportView& V) { report_out(V); }
 
 // The force array as dyn_engine_get_forces returns it — solute sites, then
 // per water O, H0, H1, M — in doubles, and the report, stored straight into
@@ -2162,9 +2157,8 @@ __device__ __forceinline__ void k_eng_report(const double* __restrict__ src, dou
 // bus.
 __device__ __forceinline__ void k_eng_forces_out(const int64_t* __restrict__ fx, uint32_t n_dyn,
                                                  uint32_t n_sites, double* __restrict__ out,
-                                                 const double* __restrict__ rep,
-                                                 double* __restrict__ h_rep) {
-  k_eng_report(rep, h_rep, kRepDoubles, 0);
+                                                 const ReportView& V) {
+  if (blockIdx.x == 0) report_out(V);
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t o = k / 3u, c = k - 3u * o;
   if (o >= n_sites) return;
@@ -2387,6 +2381,7 @@ struct dyn_engine {
   // then the words of kRep* (status, counters, stg_counters, dflags)
   DevBuf<double> report;
   PinnedBuf<double> h_report;
+  ReportView report_view() const { return ReportView{report.p, h_report.p, kRepDoubles}; }
   const uint32_t* rep_words() const { return reinterpret_cast<const uint32_t*>(h_report.p + kEngOut); }
   // accumulators
   DevBuf<int64_t> fitem, fx_site, fx_out, fx_slot;  // fx_slot: inspection only
@@ -3096,7 +3091,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
 void engine_set_check(EngineSet& S) {
   // every engine's report by one launch, one wait
   launch<k_eng_report>(S.R, "k_eng_report", 0, 1, 64, 0, [&](uint32_t i) {
-    return args<k_eng_report>((const double*)S.e[i]->report.p, S.e[i]->h_report.p, kRepDoubles, 0u);
+    return args<k_eng_report>(S.e[i]->report_view());
   });
   DYN_HIP(hipStreamSynchronize(S.R.stream));
   const Error* first = nullptr;
@@ -3117,7 +3112,11 @@ void engine_set_check(EngineSet& S) {
 }  // namespace dyn
 
 void dyn_engine::check_status() {
-  DYN_HIP(hipMemcpyAsync(h_report.p, report.p, sizeof(double) * kRepDoubles, hipMemcpyDeviceToHost, stream));
+  BatchRun R;  // (a kernel's stores cost the host less than a copy call)
+  R.stream = stream;
+  R.n = 1;
+  launch<k_eng_report>(R, "k_eng_report", 0, 1, 64, 0,
+                       [&](uint32_t) { return args<k_eng_report>(report_view()); });
   DYN_HIP(hipStreamSynchronize(stream));
   check_report();
 }
@@ -3650,8 +3649,7 @@ static void fetch_fx(dyn_engine* eng, int form) {
     const BatchRun R = eng->self_set().R;
     launch<k_eng_forces_out>(R, "k_eng_forces_out", 0, grid_for(n, 256), 256, 0, [&](uint32_t) {
       return args<k_eng_forces_out>((const int64_t*)eng->fx_out.p, eng->n_dyn, eng->n_sites,
-                                    reinterpret_cast<double*>(eng->h_fx.p),
-                                    (const double*)eng->report.p, eng->h_report.p);
+                                    reinterpret_cast<double*>(eng->h_fx.p), eng->report_view());
     });
     DYN_HIP(hipStreamSynchronize(eng->stream));
     eng->check_report();
@@ -3868,7 +3866,8 @@ void engine_set_stream(dyn_engine* eng, hipStream_t s) {
 const int64_t* engine_forces_device(const dyn_engine* eng) { return eng->fx_out.p; }
 ForceParts engine_force_parts(const dyn_engine* eng) { return eng->parts; }
 bool engine_forces_stale(const dyn_engine* eng) { return eng->fx_stale; }
-void engine_check(dyn_engine* eng) { eng->check_status(); }
+ReportView engine_report_view(const dyn_engine* eng) { return eng->report_view(); }
+void engine_check_report(dyn_engine* eng) { eng->check_report(); }
 void engine_report_energies(dyn_engine* eng, dyn_energies* out) { report_energies(eng, out); }
 void* engine_host_stage(dyn_engine* eng) {
   eng->fx_fresh = 0;

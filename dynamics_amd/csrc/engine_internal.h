@@ -79,9 +79,20 @@ const int64_t* engine_forces_device(const dyn_engine* eng);
 // array is stale (the evaluation was enqueued with kComputeFusedFinalize).
 ForceParts engine_force_parts(const dyn_engine* eng);
 bool engine_forces_stale(const dyn_engine* eng);
-// Wait for the engine's work and check its device status.
-void engine_check(dyn_engine* eng);
-// dyn_engine_get_energies without a wait, after a check (engine_check,
+// The engine's report (status, counters, energy sums) and its place in pinned
+// host memory; a kernel of the caller's read stores it there (report_out, one
+// workgroup), and after the wait engine_check_report looks at the status.
+struct ReportView {
+  const double* src;
+  double* dst;
+  uint64_t n;
+};
+__device__ __forceinline__ void report_out(const ReportView& V) {
+  for (uint32_t k = threadIdx.x; k < (uint32_t)V.n; k += blockDim.x) V.dst[k] = V.src[k];
+}
+ReportView engine_report_view(const dyn_engine* eng);
+void engine_check_report(dyn_engine* eng);
+// dyn_engine_get_energies without a wait, after a check (engine_check_report,
 // engine_set_check) that followed the last evaluation.
 void engine_report_energies(dyn_engine* eng, dyn_energies* out);
 // Pinned host memory of the engine, 24 bytes per site, for the caller's

@@ -450,7 +450,8 @@ __device__ __forceinline__ void k_md_zero(int64_t* __restrict__ f, size_t n) {
 // arrays that the host then repacked: 2.47 ms at 252,480 sites; now 0.42 ms, 0.10 of it the kernel.)
 __device__ __forceinline__ void k_md_state_out(const float* __restrict__ x, const float* __restrict__ v,
                                                uint32_t n_dyn, uint32_t n_water,
-                                               float* __restrict__ out) {
+                                               float* __restrict__ out, const ReportView& V) {
+  if (blockIdx.x == 0) report_out(V);
   const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t nd3 = 3 * (size_t)n_dyn, nw12 = 12 * (size_t)n_water, nw9 = 9 * (size_t)n_water;
   if (k < 2 * nd3) {
@@ -482,7 +483,8 @@ __device__ __forceinline__ void k_md_state_out(const float* __restrict__ x, cons
 __device__ __forceinline__ void
 k_md_energies(const float4* __restrict__ x, const float4* __restrict__ v,
               const float* __restrict__ mass, uint32_t n_dyn, uint32_t n_water, Box B,
-              double* __restrict__ out) {
+              double* __restrict__ out, const ReportView& V) {
+  if (blockIdx.x == 0) report_out(V);
   __shared__ double red[2][kBlock];
   const uint32_t t = threadIdx.x, i = blockIdx.x * kBlock + t;
   double a0 = 0.0, a1 = 0.0;
@@ -1898,9 +1900,11 @@ extern "C" int dyn_md_get_state(dyn_md* md, float* pos_dyn, float* vel_dyn, floa
     MdSet S = self_set(md);
     launch<k_md_state_out>(S.R, "k_md_state_out", 0, grid_for(6 * (size_t)nd + 21 * (size_t)nw, kBlock),
                            kBlock, 0, [&](uint32_t) {
-      return args<k_md_state_out>((const float*)md->x.p, (const float*)md->v.p, nd, nw, h);
+      return args<k_md_state_out>((const float*)md->x.p, (const float*)md->v.p, nd, nw, h,
+                                  engine_report_view(md->eng));
     });
-    engine_check(md->eng);
+    DYN_HIP(hipStreamSynchronize(S.R.stream));
+    engine_check_report(md->eng);
     size_t at = 0;
     auto take = [&](float* out, size_t n) {
       if (out && n) memcpy(out, h + at, sizeof(float) * n);
@@ -1927,10 +1931,12 @@ extern "C" int dyn_md_get_energies(dyn_md* md, dyn_md_energies* out) {
     // last evaluation's forces, the engine's report: one wait
     launch<k_md_energies, kBlock>(S.R, "k_md_energies", 0, md->eblocks, kBlock, 0, [&](uint32_t) {
       return args<k_md_energies>((const float4*)md->x.p, (const float4*)md->v.p,
-                                 (const float*)md->mass.p, md->n_dyn, md->n_water, B, md->h_out.p);
+                                 (const float*)md->mass.p, md->n_dyn, md->n_water, B, md->h_out.p,
+                                 engine_report_view(md->eng));
     });
     md_pressure_enqueue(S);
-    engine_check(md->eng);
+    DYN_HIP(hipStreamSynchronize(S.R.stream));
+    engine_check_report(md->eng);
     double kin = 0.0, kin_rigid = 0.0, eb[3] = {0.0, 0.0, 0.0};
     for (unsigned b = 0; b < md->eblocks; ++b) {
       kin += md->h_out.p[2 * b];
