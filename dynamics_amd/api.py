@@ -334,10 +334,12 @@ class ForcesPositsGpu:
         row_ptr = np.zeros(n_outer + 1, np.uint32)
         # room for a uniform density and a tenth more, so that dense sets are
         # built once too (untouched pages of the array cost nothing)
-        ext = _c(extent, np.float32).astype(np.float64).reshape(-1)
-        ball = 4.19 * max(float(skin_sq_w_cutoff), 0.0) ** 1.5 / max(float(np.prod(ext)), 1e-300)
-        row = min(1.1 * pi.shape[0] * min(ball, 1.0) + 16.0, 4096.0)
-        cap = max(1024, n_outer * 64, int(n_outer * row))
+        cap = max(1024, n_outer * 64)
+        vol = float(np.prod(_c(extent, np.float32), dtype=np.float64))
+        r2 = float(skin_sq_w_cutoff)
+        if 0.0 < vol < 1e300 and 0.0 < r2 < 1e12:
+            row = min(1.1 * pi.shape[0] * min(4.19 * r2 ** 1.5 / vol, 1.0) + 16.0, 4096.0)
+            cap = max(cap, int(n_outer * row))
         total = C.c_uint64()
         for _ in range(2):
             col = np.zeros(cap, np.uint32)
