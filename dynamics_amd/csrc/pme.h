@@ -126,22 +126,15 @@ struct PmeCore {
             float beta, int order, bool fp64 = false);
   void set_box(const float l[3]);  // recomputes G (on the device, asynchronously)
   void set_moduli();                // bsq for the current K and order
-  // Enqueue spread → FFT → convolve → inverse FFT → gather for n charges.
-  // xyzq: device float4 array (positions wrapped or not; wrapped internally).
-  // If site != null, forces are atomically added (fixed point, 2^32) into
-  // fx_sites[3·site[i] + c] (component-interleaved); else written as floats
-  // into f_out[3i + c].  Energy and virial (without self energy) end up in
-  // res_dev[0], res_dev[1] after the final reduction kernel (or in res[0],
-  // res[1] when res is given).  Forces are multiplied by fscale (exactly 1
-  // leaves them unchanged).
-  void run(uint32_t n, const float4* xyzq, const uint32_t* site, int64_t* fx_sites,
-           int fx_component_major, uint32_t fx_nsites, float* f_out, float fscale = 1.0f,
-           double* res = nullptr);
-  ArgCache cache;  // device argument packs of run()
+  ArgCache cache;  // device argument packs of a standalone evaluation
 };
 
-// One system's part of a batched SPME pass (the arguments of PmeCore::run;
-// core == nullptr: the system takes no part).
+// One system's part of a batched SPME pass, spread → FFT → convolve → inverse
+// FFT → gather for n charges (core == nullptr: the system takes no part).
+// xyzq: device float4 array (positions wrapped internally).  If site is set,
+// forces are added (fixed point, 2^32) to fx's row site[i]; else they are written
+// as floats to f_out[3i + c].  Energy and virial (without self energy) end up
+// in res.  Forces are multiplied by fscale (exactly 1 leaves them unchanged).
 struct PmeRun {
   PmeCore* core = nullptr;
   uint32_t n = 0;

@@ -616,6 +616,26 @@ __device__ __forceinline__ void k_pme_bin(const float4* __restrict__ xyzq, uint3
   pme_bin_charge(B, i < n ? xyzq[i] : make_float4(0.f, 0.f, 0.f, 0.f), i < n);
 }
 
+// k_pme_bin from pinned host memory, leaving the charges on the device too.
+__device__ __forceinline__ void k_pme_take(const float4* __restrict__ h, uint32_t n,
+                                           float4* __restrict__ xyzq, BinArgs B) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const float4 p = i < n ? h[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  if (i < n) xyzq[i] = p;
+  pme_bin_charge(B, p, i < n);
+}
+
+// Forces (n floats), energy, virial and the list status to pinned host memory.
+__device__ __forceinline__ void k_pme_out(const float* __restrict__ f, uint32_t n,
+                                          const double* __restrict__ res,
+                                          const unsigned int* __restrict__ status,
+                                          float* __restrict__ h_f, double* __restrict__ h_rep) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) h_f[i] = f[i];
+  if (i < 2u) h_rep[i] = res[i];
+  if (i == 2u) h_rep[2] = (double)*status;
+}
+
 // Home bricks along one axis whose charges can reach the points [lo, hi]
 // (lo a brick start): a charge with base point k0 covers k0 − ORDER + 1 … k0
 // (mod K), so k0 runs over lo … hi + ORDER − 1 (mod K): the bricks of
@@ -1097,36 +1117,6 @@ void PmeCore::grow() {
   brick_items.reserve((size_t)nbk[0] * nbk[1] * nbk[2] * cap_brick);
 }
 
-void PmeCore::run(uint32_t n, const float4* xyzq, const uint32_t* site, int64_t* fx_sites,
-                  int comp_major, uint32_t nsites, float* f_out, float fscale, double* res) {
-  PmeRun r;
-  r.core = this;
-  r.n = n;
-  r.xyzq = xyzq;
-  r.site = site;
-  r.fx = fx_sites;
-  r.comp_major = comp_major;
-  r.nsites = nsites;
-  r.f_out = f_out;
-  r.fscale = fscale;
-  r.res = res ? res : res_dev.p;
-  BatchRun R;
-  R.stream = stream;
-  R.cache = &cache;
-  R.n = 1;
-  // a brick list that overflowed: enlarge and evaluate again
-  for (int attempt = 0;; ++attempt) {
-    pme_run(R, *prof, &r, 0);
-    unsigned int st = 0;
-    DYN_HIP(hipMemcpyAsync(&st, status.p, sizeof st, hipMemcpyDeviceToHost, stream));
-    DYN_HIP(hipStreamSynchronize(stream));
-    if (!st) break;
-    DYN_HIP(hipMemsetAsync(status.p, 0, sizeof st, stream));
-    if (attempt >= 4) throw Error(DYN_ERR_CAPACITY, "SPME brick lists keep overflowing");
-    grow();
-  }
-}
-
 // One SPME evaluation per system of the pass, each stage one launch for all
 // of them (per precision and B-spline order present).  A system with a null
 // core takes part in no stage (its packs describe empty work: no charges, no
@@ -1439,26 +1429,65 @@ extern "C" int dyn_pme_forces_and_virial(dyn_pme* pme, uint32_t n, const float* 
     const size_t nn = std::max<uint32_t>(n, 1);
     pme->xyzq.reserve(nn);
     pme->fout.reserve(3 * nn);
-    pme->h_xyzq.reserve(nn);
-    double q2 = 0.0;
+    pme->h_xyzq.reserve(nn + 2);
+    // four running sums of q²: one would be a chain of additions
+    double qs[4] = {0.0, 0.0, 0.0, 0.0};
+    int bad = 0;
     for (uint32_t i = 0; i < n; ++i) {
-      DYN_REQUIRE(std::isfinite(pos[3 * i]) && std::isfinite(pos[3 * i + 1]) &&
-                      std::isfinite(pos[3 * i + 2]) && std::isfinite(q[i]),
-                  "non-finite input at charge %u", i);
-      pme->h_xyzq.p[i] = make_float4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], q[i]);
-      q2 += (double)q[i] * (double)q[i];
+      const float x = pos[3 * (size_t)i], y = pos[3 * (size_t)i + 1], z = pos[3 * (size_t)i + 2], c = q[i];
+      // (a product with zero is zero unless a factor is not finite)
+      bad |= (x * 0.0f + y * 0.0f) + (z * 0.0f + c * 0.0f) != 0.0f;
+      pme->h_xyzq.p[i] = make_float4(x, y, z, c);
+      qs[i & 3] += (double)c * (double)c;
     }
-    if (n)
-      DYN_HIP(hipMemcpyAsync(pme->xyzq.p, pme->h_xyzq.p, sizeof(float4) * n,
-                             hipMemcpyHostToDevice, pme->stream));
-    pme->core.run(n, pme->xyzq.p, nullptr, nullptr, 0, 0, pme->fout.p);
-    double res[2] = {0, 0};
-    DYN_HIP(hipMemcpyAsync(res, pme->core.res_dev.p, sizeof(res), hipMemcpyDeviceToHost,
-                           pme->stream));
-    if (n && f_out)
-      DYN_HIP(hipMemcpyAsync(f_out, pme->fout.p, sizeof(float) * 3 * n, hipMemcpyDeviceToHost,
-                             pme->stream));
-    DYN_HIP(hipStreamSynchronize(pme->stream));
+    if (bad)
+      for (uint32_t i = 0; i < n; ++i)
+        DYN_REQUIRE(std::isfinite(pos[3 * (size_t)i]) && std::isfinite(pos[3 * (size_t)i + 1]) &&
+                        std::isfinite(pos[3 * (size_t)i + 2]) && std::isfinite(q[i]),
+                    "non-finite input at charge %u", i);
+    const double q2 = (qs[0] + qs[1]) + (qs[2] + qs[3]);
+    // the charges from pinned host memory, the results into it (over the
+    // charges, read by then; energy, virial and status after them): no copies,
+    // one wait
+    PmeCore& core = pme->core;
+    PmeRun r;
+    r.core = &core;
+    r.n = n;
+    r.xyzq = pme->xyzq.p;
+    r.f_out = pme->fout.p;
+    r.fscale = 1.0f;
+    r.res = core.res_dev.p;
+    r.binned = true;
+    BatchRun R;
+    R.stream = pme->stream;
+    R.cache = &core.cache;
+    R.n = 1;
+    float* const h_f = reinterpret_cast<float*>(pme->h_xyzq.p);
+    double* const rep = reinterpret_cast<double*>(pme->h_xyzq.p + nn);
+    const float4* src = pme->h_xyzq.p;
+    // a brick list that overflowed: enlarge and evaluate again
+    for (int attempt = 0;; ++attempt) {
+      core.ensure_cap(n);
+      if (src)
+        launch<k_pme_take>(R, "k_pme_take", 0, grid_for(nn, 256), 256, 0, [&](uint32_t) {
+          return args<k_pme_take>(src, n, pme->xyzq.p, core.bin_args(nullptr, 0));
+        });
+      else
+        r.binned = false;  // from the device's copy
+      pme_run(R, pme->prof, &r, 0);
+      launch<k_pme_out>(R, "k_pme_out", 0, grid_for(3 * nn, 256), 256, 0, [&](uint32_t) {
+        return args<k_pme_out>((const float*)pme->fout.p, 3u * n, (const double*)core.res_dev.p,
+                               (const unsigned int*)core.status.p, h_f, rep);
+      });
+      DYN_HIP(hipStreamSynchronize(pme->stream));
+      if (rep[2] == 0.0) break;
+      src = nullptr;
+      DYN_HIP(hipMemsetAsync(core.status.p, 0, sizeof(unsigned int), pme->stream));
+      if (attempt >= 4) throw Error(DYN_ERR_CAPACITY, "SPME brick lists keep overflowing");
+      core.grow();
+    }
+    const double res[2] = {rep[0], rep[1]};
+    if (n && f_out) memcpy(f_out, h_f, sizeof(float) * 3 * (size_t)n);
     const double e_self = (double)pme->core.beta / std::sqrt(M_PI) * q2;
     if (energy) *energy = res[0] - e_self;
     if (virial) *virial = res[1];
