@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
+
 #include "dyn_math.h"
 
 namespace dyn {
@@ -172,5 +174,12 @@ __device__ __forceinline__ void bonded_terms(const BondedArgs& A, uint32_t block
     A.partials[4 * block + threadIdx.x] = t;
   }
 }
+
+// Bonded terms an MD step hands to its engines' evaluation.
+struct SideWork {
+  unsigned blocks = 0;  // workgroups of the system that needs most
+  std::function<BondedArgs(uint32_t)> args;
+  std::function<uint64_t*(uint32_t)> step;  // a count to advance by one before them, or none
+};
 
 }  // namespace dyn

@@ -2043,9 +2043,10 @@ __device__ __forceinline__ void pme_prep(const PmePrepArgs& A, uint32_t block) {
 
 // The short independent pieces of an evaluation in one launch, block ranges
 // one after another: SPME preparation (n_prep blocks), exclusion and 1-4
-// corrections (n_corr), bonded terms.  Each is a few dependent memory latencies
-// and little else, so together they take the time of the longest: 28,000 sites
-// 5.2 + 5.6 + 10.5 µs and two launch gaps before, 11.5 now.
+// corrections (n_corr), bonded terms (without SPME on the same stream, whose
+// spread takes them otherwise).  Each is a few dependent memory latencies and
+// little else, so together they take the time of the longest: 28,000 sites
+// 5.2 + 5.6 µs and a launch gap before, 6.4 now.
 __device__ __forceinline__ void k_eng_side(const PmePrepArgs& P, const CorrArgs& C, const BondedArgs& B,
                                            uint32_t n_prep, uint32_t n_corr) {
   static_assert(kCorrBlock == 256 && kBondedBlock == 256, "one block size");
@@ -2855,7 +2856,9 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
     return std::max(grid_for(e.n_sites, 256), grid_for(e.n_q, 256));
   });
   const unsigned n_corr = any_corr ? max_grid(S, [](dyn_engine& e) { return e.corr_blocks; }) : 0u;
-  const unsigned n_bond = side ? side->blocks : 0u;
+  // (with SPME on the same stream the bonded terms ride in its spread launch)
+  const bool bond_spread = any_recip && RP.stream == RS.stream;
+  const unsigned n_bond = side && !bond_spread ? side->blocks : 0u;
   auto side_launch = [&](const BatchRun& RL, int tag, unsigned np, unsigned nc, unsigned nb) {
     if (np + nc + nb == 0) return;
     launch<k_eng_side>(RL, "k_eng_side", tag, np + nc + nb, 256, 0, [&](uint32_t i) {
@@ -2949,7 +2952,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
         rb[i] = r;
       }
     }
-    pme_run(RP, prof, ra.data(), 0);
+    pme_run(RP, prof, ra.data(), 0, bond_spread ? side : nullptr);
     if (any_b) pme_run(RP, prof, rb.data(), 1);
   }
   // a staged build on the second stream, beside the pair kernel (after it

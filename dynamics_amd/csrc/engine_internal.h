@@ -48,11 +48,6 @@ constexpr uint32_t kComputeStagedBuild = 1u << 30;
 // and the engine's force array stays stale until a later evaluation
 // finalizes.
 constexpr uint32_t kComputeFusedFinalize = 1u << 29;
-struct SideWork {
-  unsigned blocks = 0;  // workgroups of the system that needs most
-  std::function<BondedArgs(uint32_t)> args;
-  std::function<uint64_t*(uint32_t)> step;  // a count to advance by one before them, or none
-};
 void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side = nullptr);
 // Wait for the set's work and check each engine's device status (throws the
 // first engine's error; buffers that overflowed have been enlarged).

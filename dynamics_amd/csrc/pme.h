@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "batch.h"
+#include "bonded.h"
 #include "common.h"
 #include "wave.h"
 
@@ -154,6 +155,8 @@ struct PmeRun {
 
 // runs[0 .. R.n): one per system of the pass; tag separates passes that run
 // more than once per evaluation (their launch sites keep separate packs).
-void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag);
+// side: bonded terms to evaluate in the same pass, or null.
+void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag,
+             const SideWork* side = nullptr);
 
 }  // namespace dyn
