@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "common.h"
+#include "corr.h"
 #include "wave.h"
 #include "dyn_math.h"
 #include "engine.h"
@@ -1129,8 +1130,6 @@ struct TileAccT {
   }
 };
 
-__device__ __forceinline__ void wave_add_fx(int64_t* __restrict__ M, int key, double e);
-
 // Molecule-pair energy of one tile entry (src/non_bonded.rs:350-361): the
 // pair energy of every solute–solute lane goes to M[m_i·n + m_j] in 2⁻³²
 // kcal/mol fixed point.  The full list visits each pair from both rows, so
@@ -1147,25 +1146,6 @@ __device__ __forceinline__ void mol_energy_add(int64_t* __restrict__ M,
     if (mi == mj) e *= 0.5;
   }
   wave_add_fx(M, key, e);
-}
-
-// Adds e to M[key] (2⁻³² fixed point) for every lane with key ≥ 0: one
-// atomic for the wave when all such lanes share the key.  All lanes of the
-// wave must be active.
-__device__ __forceinline__ void wave_add_fx(int64_t* __restrict__ M, int key, double e) {
-  const unsigned long long live = __ballot(key >= 0);
-  if (!live) return;
-  const int kf = __shfl(key, __ffsll((long long)live) - 1, kWave);
-  if (__ballot(key >= 0 && key != kf) == 0ull) {
-    double x = key >= 0 ? e : 0.0;
-    for (int m = 1; m < kWave; m <<= 1) x += __shfl_xor(x, m, kWave);
-    if ((threadIdx.x & (kWave - 1)) == 0)
-      atomicAdd(reinterpret_cast<unsigned long long*>(M + kf),
-                (unsigned long long)dyn_fx64(x));
-  } else if (key >= 0) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(M + key),
-              (unsigned long long)dyn_fx64(e));
-  }
 }
 
 // Adds one evaluated tile lane (scalar s, displacement d, energies) to the
@@ -1806,162 +1786,7 @@ struct dyn::MinWavesPerSimd<k_eng_pairs<true, false, false>> {
 
 namespace {
 
-// Correction pairs: kind 1 = 1-4 pair (scaled real-space LJ + Coulomb, plus
-// the reciprocal correction of the mode), kind 0 = excluded pair (standard
-// mode: remove qq·erf(βr)/r from the reciprocal sum).
-struct CorrArgs {
-  DynPairParams P;
-  const float4* wpos;      // per site (x, y, z, q)
-  const int32_t* ltype;    // per site type word (DYN_TYPE_ALCH marks the decoupled molecule)
-  const float2* lj_table;
-  const float2* lj_se;     // (σ, ε) per type pair, for soft-core
-  const uint32_t* ci;
-  const uint32_t* cj;
-  const uint8_t* kind;
-  uint32_t n;
-  int mode;
-  int recip_on;            // reciprocal corrections only accompany the SPME sum
-  uint32_t nblk;           // workgroups (one partial each)
-  int64_t* mol_e;          // n_mol² molecule-pair energies, or null
-  const int32_t* mol_of;
-  uint32_t n_mol;
-  int64_t* fx;             // site forces, component-major
-  uint32_t n_sites;
-  double* partials;        // 6 per block: e_lj14, e_c14, e_corr, vir_sr, vir_recip, dH/dλ
-};
-
-constexpr int kCorrBlock = 256;
-constexpr int kCorrVals = 7;  // per-block sums of the correction kernel
-__device__ __forceinline__ void corr_terms(const CorrArgs& A, uint32_t block) {
-  __shared__ double red[kCorrBlock];
-  if (block >= A.nblk) return;  // partials exist for the system's own blocks
-  // e_lj14, e_c14, e_corr, vir_sr, vir_recip, dH/dλ, 1-4 pairs within the cutoff
-  double acc[kCorrVals] = {0, 0, 0, 0, 0, 0, 0};
-  // molecule-pair matrix: a running entry per thread (1-4 pairs lie within
-  // one molecule), flushed when the entry changes and once at the end
-  int mkey = -1;
-  double me = 0.0;
-  for (uint32_t k = block * kCorrBlock + threadIdx.x; k < A.n; k += A.nblk * kCorrBlock) {
-    if (A.kind[k] == 0 && !A.recip_on) continue;
-    const uint32_t i = A.ci[k], j = A.cj[k];
-    const float4 a = A.wpos[i], b = A.wpos[j];
-    float d0 = dyn_min_image_rint(a.x - b.x, A.P.ext[0], A.P.inv_ext[0]);
-    float d1 = dyn_min_image_rint(a.y - b.y, A.P.ext[1], A.P.inv_ext[1]);
-    float d2 = dyn_min_image_rint(a.z - b.z, A.P.ext[2], A.P.inv_ext[2]);
-    const float r2 = dyn_fmaf(d2, d2, dyn_fmaf(d1, d1, d0 * d0));
-    if (!(r2 > 1e-12f)) continue;
-    const float rinv = dyn_rsqrtf(r2);
-    const float qq = a.w * b.w;
-    float s_sr = 0.f, s_rc = 0.f;
-    double e_pair = 0.0;  // the 1-4 pair's energy (molecule-pair matrix)
-    if (A.kind[k] == 1) {
-      if (r2 < A.P.rc2) acc[6] += 1.0;
-      // a 1-4 pair across the decoupled molecule's boundary is also an
-      // alchemical pair (src/non_bonded.rs:581-599)
-      const bool cross = A.P.alch_on && ((A.ltype[i] ^ A.ltype[j]) & DYN_TYPE_ALCH) != 0;
-      const int tab = (A.ltype[i] & DYN_TYPE_MASK) * A.P.n_types + (A.ltype[j] & DYN_TYPE_MASK);
-      if (r2 <= A.P.lj_rc2) {
-        float sl, el;
-        if (cross) {
-          const float2 se = A.lj_se[tab];
-          float dd;
-          dyn_lj_soft_core(r2, se.x, se.y, A.P.sch.lj_lambda, &sl, &el, &dd);
-          acc[5] += (double)(DYN_SCALE_LJ_14 * (dd * A.P.sch.lj_dlambda_dlambda));
-        } else {
-          const float2 c = A.lj_table[tab];
-          dyn_lj(rinv * rinv, c.x, c.y, &sl, &el);
-        }
-        s_sr += DYN_SCALE_LJ_14 * sl;
-        acc[0] += (double)(DYN_SCALE_LJ_14 * el);
-        e_pair += (double)(DYN_SCALE_LJ_14 * el);
-      }
-      if (r2 < A.P.rc2) {
-        float sc, ec;
-        dyn_coul_erfc(r2, rinv, qq, A.P.beta, A.P.beta2, A.P.two_b_sqrtpi, &sc, &ec);
-        sc = 0.833333333f * sc;
-        ec = 0.833333333f * ec;
-        if (cross) {
-          acc[5] += (double)(ec * A.P.sch.coulomb_dscale_dlambda);
-          sc = sc * A.P.sch.coulomb_scale;
-          ec = ec * A.P.sch.coulomb_scale;
-        }
-        s_sr += sc;
-        acc[1] += (double)ec;
-        e_pair += (double)ec;
-      }
-      if (!A.recip_on) {
-        // no reciprocal sum, nothing to correct
-      } else if (A.mode == DYN_MODE_REFERENCE) {
-        // vacuum correction (1/1.2 − 1)·qq/r² along r̂, force only
-        s_rc = (DYN_SCALE_COUL_14 - 1.0f) * qq * (rinv * rinv * rinv);
-      } else {
-        float se, ee;
-        dyn_coul_erf(r2, rinv, qq, A.P.beta, A.P.beta2, A.P.two_b_sqrtpi, &se, &ee);
-        s_rc = -(1.0f - DYN_SCALE_COUL_14) * se;
-        acc[2] += (double)(-(1.0f - DYN_SCALE_COUL_14) * ee);
-      }
-    } else {
-      float se, ee;
-      dyn_coul_erf(r2, rinv, qq, A.P.beta, A.P.beta2, A.P.two_b_sqrtpi, &se, &ee);
-      s_rc = -se;
-      acc[2] += (double)(-ee);
-    }
-    acc[3] += (double)(s_sr * r2);
-    acc[4] += (double)(s_rc * r2);
-    if (A.mol_e && e_pair != 0.0) {
-      const int mi = A.mol_of[i], mj = A.mol_of[j];
-      if (mi != mj) {  // both orders (src/non_bonded.rs:350-361)
-        const uint64_t v = (uint64_t)dyn_fx64(e_pair);
-        atomicAdd(reinterpret_cast<unsigned long long*>(A.mol_e + mi * (int)A.n_mol + mj), v);
-        atomicAdd(reinterpret_cast<unsigned long long*>(A.mol_e + mj * (int)A.n_mol + mi), v);
-      } else {
-        const int key = mi * (int)A.n_mol + mi;
-        if (key != mkey) {
-          if (mkey >= 0)
-            atomicAdd(reinterpret_cast<unsigned long long*>(A.mol_e + mkey),
-                      (unsigned long long)dyn_fx64(me));
-          mkey = key;
-          me = 0.0;
-        }
-        me += e_pair;
-      }
-    }
-    const float s = s_sr + s_rc;
-    const int64_t q0 = dyn_fx(s * d0), q1 = dyn_fx(s * d1), q2 = dyn_fx(s * d2);
-    atomicAdd(reinterpret_cast<unsigned long long*>(A.fx + i), (unsigned long long)q0);
-    atomicAdd(reinterpret_cast<unsigned long long*>(A.fx + A.n_sites + i), (unsigned long long)q1);
-    atomicAdd(reinterpret_cast<unsigned long long*>(A.fx + 2 * (size_t)A.n_sites + i), (unsigned long long)q2);
-    atomicAdd(reinterpret_cast<unsigned long long*>(A.fx + j), (unsigned long long)(-q0));
-    atomicAdd(reinterpret_cast<unsigned long long*>(A.fx + A.n_sites + j), (unsigned long long)(-q1));
-    atomicAdd(reinterpret_cast<unsigned long long*>(A.fx + 2 * (size_t)A.n_sites + j), (unsigned long long)(-q2));
-  }
-  if (A.mol_e) wave_add_fx(A.mol_e, mkey, me);
-  if (!A.partials) return;  // forces only
-  // wave sums by shuffles, then the block's waves in a fixed order
-  for (int v = 0; v < kCorrVals; ++v)
-    for (int m = kWave / 2; m >= 1; m >>= 1) acc[v] += __shfl_xor(acc[v], m, kWave);
-  if ((threadIdx.x & (kWave - 1)) == 0)
-    for (int v = 0; v < kCorrVals; ++v) red[v * (kCorrBlock / kWave) + threadIdx.x / kWave] = acc[v];
-  __syncthreads();
-  if (threadIdx.x < kCorrVals) {
-    double t = 0.0;
-    for (int w = 0; w < kCorrBlock / kWave; ++w) t += red[threadIdx.x * (kCorrBlock / kWave) + w];
-    A.partials[kCorrVals * block + threadIdx.x] = t;
-  }
-}
-
-// Per-site set-up of an evaluation: clear the site force accumulators and
-// gather the charged sites' (x, y, z, q) for the SPME spread.
-// With a decoupled molecule (sites [alch0, alch1)), pme_b receives a second
-// charge set with that molecule's charges negated.
-// The first launch of every evaluation: wrapping, the displacement reading
-// that decides on a list build (the largest squared displacement of any
-// site since the last build, one atomic per workgroup; squared distances
-// are non-negative floats, ordered like their bit patterns), the slot
-// positions of the current list (a build rewrites them), the SPME charges
-// and their binning, and clearing of the accumulators.  Slots and charges
-// take their wrapped positions from pos directly (the same wrap1 of the
-// same input as wpos).
+// A site's wrapped position and charge.
 __device__ __forceinline__ float4 wrapped(const float4* __restrict__ pos,
                                           const float* __restrict__ q, const EngGeom& g,
                                           uint32_t s) {
@@ -1998,11 +1823,12 @@ struct PrepArgs {
   int64_t* mol_e;
   uint64_t* step;     // the caller's count of evaluations to advance, or null
   uint32_t n_mol2;
+  uint32_t blocks;    // workgroups of k_eng_prep before the first that reads these
+  uint32_t stride;    // threads of the workgroups that read these
   uint32_t unused;    // no implicit padding: argument packs are compared byte for byte
 };
 
-// The SPME charges of an evaluation that runs SPME, by the first launch of
-// the second stream (off the main stream's path): their wrapped positions
+// The SPME charges of an evaluation that runs SPME: their wrapped positions
 // (and the second evaluation's charges), their listing under the grid
 // bricks, and the cleared SPME force sums.
 struct PmePrepArgs {
@@ -2041,27 +1867,23 @@ __device__ __forceinline__ void pme_prep(const PmePrepArgs& A, uint32_t block) {
   pme_bin_charge(A.bin, p, qv);
 }
 
-// The short independent pieces of an evaluation in one launch, block ranges
-// one after another: SPME preparation (n_prep blocks), exclusion and 1-4
-// corrections (n_corr), bonded terms (without SPME on the same stream, whose
-// spread takes them otherwise).  Each is a few dependent memory latencies and
-// little else, so together they take the time of the longest: 28,000 sites
-// 5.2 + 5.6 µs and a launch gap before, 6.4 now.
-__device__ __forceinline__ void k_eng_side(const PmePrepArgs& P, const CorrArgs& C, const BondedArgs& B,
-                                           uint32_t n_prep, uint32_t n_corr) {
+// The exclusion and 1-4 corrections (n_corr blocks) and the bonded terms of an
+// evaluation without SPME on their stream (its spread launch takes them
+// otherwise).  Both are a few dependent memory latencies and little else, so
+// together they take the time of the longer.
+__device__ __forceinline__ void k_eng_side(const CorrArgs& C, const BondedArgs& B, uint32_t n_corr) {
   static_assert(kCorrBlock == 256 && kBondedBlock == 256, "one block size");
   const uint32_t b = blockIdx.x;
-  if (b < n_prep) pme_prep(P, b);
-  else if (b < n_prep + n_corr) corr_terms(C, b - n_prep);
-  else bonded_terms(B, b - n_prep - n_corr);
+  if (b < n_corr) corr_terms(C, b);
+  else bonded_terms(B, b - n_corr);
 }
 
-// Copies n values of a staging array into the current list's (grid stride).
+// Copies n values of a staging array into the current list's (thread t of
+// stride).
 template <class T>
-__device__ __forceinline__ void copy_grid(T* __restrict__ dst, const T* __restrict__ src, size_t n) {
-  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-       k += (size_t)gridDim.x * blockDim.x)
-    dst[k] = src[k];
+__device__ __forceinline__ void copy_grid(T* __restrict__ dst, const T* __restrict__ src, size_t n,
+                                          size_t t, size_t stride) {
+  for (size_t k = t; k < n; k += stride) dst[k] = src[k];
 }
 
 // The first launch of every evaluation.  A finished staged build (from the
@@ -2070,15 +1892,26 @@ __device__ __forceinline__ void copy_grid(T* __restrict__ dst, const T* __restri
 // chunks becomes current.  Then: wrapping, the displacement of every site
 // from the current list's build positions (block max, one atomic per
 // workgroup; squared distances are non-negative floats, ordered like their
-// bit patterns), the slot positions of the current list, the SPME charges
-// and their binning, and clearing of the accumulators.  Slots and charges
+// bit patterns), the slot positions of the current list and clearing of the
+// accumulators.  Slots and charges
 // take their wrapped positions from pos directly (the same wrap1 of the same
 // input as wpos).  The build kernels and the pair kernel decide from the
 // largest displacement (BuildGate, k_eng_pairs); the finalize kernel makes
 // the taken staged list the current one for good.
-__device__ __forceinline__ void k_eng_prep(PrepArgs A) {
+//
+// Its first A.blocks workgroups prepare the SPME charges beside this: both are
+// chains of a few memory latencies, and the second stream, the longer one of
+// a small system's step, then starts with the spread.  With the charges and
+// the corrections in a launch of their own before the spread, 20 MD steps took
+// 1564 µs at 2,000 sites, 2466 at 28,000 and 9118 at 252,480; now 1464, 2350
+// and 9048.
+__device__ __forceinline__ void k_eng_prep(const PrepArgs& A, const PmePrepArgs& Q) {
   __shared__ unsigned int red[256 / kWave];
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x < A.blocks) {
+    pme_prep(Q, blockIdx.x);
+    return;
+  }
+  const uint32_t t = (blockIdx.x - A.blocks) * blockDim.x + threadIdx.x;
   const uint32_t n = A.g.n_dyn + 4u * A.g.n_water;
   // every workgroup reads the same words and writes the same decision; the
   // finalize kernel clears them
@@ -2101,9 +1934,9 @@ __device__ __forceinline__ void k_eng_prep(PrepArgs A) {
     A.fx_site[2 * (size_t)n + t] = 0;
   }
   if (A.mol_e)
-    for (uint32_t k = t; k < A.n_mol2; k += gridDim.x * blockDim.x) A.mol_e[k] = 0;
+    for (uint32_t k = t; k < A.n_mol2; k += A.stride) A.mol_e[k] = 0;
   const uint32_t n_cl = L.counters[0];
-  for (uint32_t k = t; k < n_cl * DYN_CL_SIZE; k += gridDim.x * blockDim.x) {
+  for (uint32_t k = t; k < n_cl * DYN_CL_SIZE; k += A.stride) {
     const int32_t s = L.slot_site[k];
     if (s >= 0) {
       A.cur.xyzq[k] = wrapped(A.pos, A.q, A.g, (uint32_t)s);
@@ -2116,15 +1949,15 @@ __device__ __forceinline__ void k_eng_prep(PrepArgs A) {
   }
   if (commit) {
     const size_t ns = (size_t)n_cl * DYN_CL_SIZE;
-    copy_grid(A.cur.slot_site, A.stg.slot_site, ns);
-    copy_grid(A.cur.slot_type, A.stg.slot_type, ns);
-    copy_grid(A.cur.slot_gid, A.stg.slot_gid, ns);
-    copy_grid(A.cur.cl_class, A.stg.cl_class, n_cl);
-    copy_grid(A.cur.slot_of, A.stg.slot_of, n);
-    copy_grid(A.cur.wpos_ref, A.stg.wpos_ref, n);
-    copy_grid(A.cur.row_ptr, A.stg.row_ptr, (size_t)n_cl + 1);
-    copy_grid(A.cur.chunk_ptr, A.stg.chunk_ptr, (size_t)n_cl + 1);
-    copy_grid(A.cur.counters, A.stg.counters, 4);
+    copy_grid(A.cur.slot_site, A.stg.slot_site, ns, t, A.stride);
+    copy_grid(A.cur.slot_type, A.stg.slot_type, ns, t, A.stride);
+    copy_grid(A.cur.slot_gid, A.stg.slot_gid, ns, t, A.stride);
+    copy_grid(A.cur.cl_class, A.stg.cl_class, n_cl, t, A.stride);
+    copy_grid(A.cur.slot_of, A.stg.slot_of, n, t, A.stride);
+    copy_grid(A.cur.wpos_ref, A.stg.wpos_ref, n, t, A.stride);
+    copy_grid(A.cur.row_ptr, A.stg.row_ptr, (size_t)n_cl + 1, t, A.stride);
+    copy_grid(A.cur.chunk_ptr, A.stg.chunk_ptr, (size_t)n_cl + 1, t, A.stride);
+    copy_grid(A.cur.counters, A.stg.counters, 4, t, A.stride);
   }
   for (int m = kWave / 2; m >= 1; m >>= 1) v = max(v, (unsigned int)__shfl_xor((int)v, m, kWave));
   if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = v;
@@ -2818,7 +2651,10 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
     const unsigned gp = max_grid(S, [](dyn_engine& e) {
       return std::max(grid_for(e.n_sites, 256), grid_for(e.cap_slots, 256));
     });
-    launch<k_eng_prep>(R, "k_eng_prep", 0, gp, 256, 0, [&](uint32_t i) {
+    const unsigned np = !any_recip ? 0u : max_grid(S, [](dyn_engine& e) {
+      return std::max(grid_for(e.n_sites, 256), grid_for(e.n_q, 256));
+    });
+    launch<k_eng_prep>(R, "k_eng_prep", 0, np + gp, 256, 0, [&](uint32_t i) {
       dyn_engine& e = *E[i];
       const Plan& pl = PL[i];
       PrepArgs A;
@@ -2835,7 +2671,25 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
       A.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
       A.n_mol2 = e.n_mol * e.n_mol;
       A.step = side && side->step ? side->step(i) : nullptr;
-      return args<k_eng_prep>(A);
+      A.blocks = np;
+      A.stride = gp * 256u;
+      PmePrepArgs Q;
+      std::memset(&Q, 0, sizeof Q);
+      if (pl.recip_on) {  // (a system without SPME this evaluation: nothing to do)
+        Q.pos = e.pos_dev;
+        Q.q = e.q.p;
+        Q.g = e.geom;
+        Q.qsite = e.qsite.p;
+        Q.nq = e.n_q;
+        Q.alch0 = e.alch0;
+        Q.alch1 = e.alch1;
+        Q.pme_xyzq = e.pme_xyzq.p;
+        Q.pme_b = pl.recip_b ? e.pme_b.p : nullptr;
+        Q.fx_recip = e.fx_recip.p;
+        e.pme.ensure_cap(e.n_q);
+        Q.bin = e.pme.bin_args(e.status.p, kStPme);
+      }
+      return args<k_eng_prep>(A, Q);
     });
   }
   // the second stream: the exclusion and 1-4 corrections, the caller's bonded
@@ -2849,79 +2703,49 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
   // kernel at once and would take the compute units the FFT planes need —
   // before the pair kernel on the main stream
   const BatchRun& RP = staged_mode ? R : RS;
-  // the SPME preparation, the exclusion and 1-4 corrections (site
-  // accumulators; finalize reads them) and the caller's bonded terms: one
-  // launch where they share a stream
-  const unsigned n_prep = !any_recip ? 0u : max_grid(S, [](dyn_engine& e) {
-    return std::max(grid_for(e.n_sites, 256), grid_for(e.n_q, 256));
-  });
-  const unsigned n_corr = any_corr ? max_grid(S, [](dyn_engine& e) { return e.corr_blocks; }) : 0u;
-  // (with SPME on the same stream the bonded terms ride in its spread launch)
-  const bool bond_spread = any_recip && RP.stream == RS.stream;
-  const unsigned n_bond = side && !bond_spread ? side->blocks : 0u;
-  auto side_launch = [&](const BatchRun& RL, int tag, unsigned np, unsigned nc, unsigned nb) {
-    if (np + nc + nb == 0) return;
-    launch<k_eng_side>(RL, "k_eng_side", tag, np + nc + nb, 256, 0, [&](uint32_t i) {
-      dyn_engine& e = *E[i];
-      const Plan& pl = PL[i];
-      PmePrepArgs A;
-      std::memset(&A, 0, sizeof A);
-      if (np) {
-        A.pos = e.pos_dev;
-        A.q = e.q.p;
-        A.g = e.geom;
-        A.qsite = e.qsite.p;
-        A.alch0 = e.alch0;
-        A.alch1 = e.alch1;
-        A.pme_xyzq = e.pme_xyzq.p;
-        A.pme_b = pl.recip_b ? e.pme_b.p : nullptr;
-        A.fx_recip = e.fx_recip.p;
-        if (pl.recip_on) {  // the SPME charges are listed under their bricks here
-          e.pme.ensure_cap(e.n_q);
-          A.nq = e.n_q;
-          A.bin = e.pme.bin_args(e.status.p, kStPme);
-        } else {
-          // a system of the batch without SPME this evaluation: nothing to do
-          A.g.n_dyn = 0;
-          A.g.n_water = 0;
-        }
-      }
+  // the exclusion and 1-4 corrections (site accumulators; finalize reads
+  // them) and the caller's bonded terms ride in the spread launch of an SPME
+  // sum on the same stream; without one they are a launch of their own
+  CorrWork corr;
+  if (any_corr) corr.blocks = max_grid(S, [](dyn_engine& e) { return e.corr_blocks; });
+  corr.args = [&](uint32_t i) {
+    dyn_engine& e = *E[i];
+    const Plan& pl = PL[i];
+    CorrArgs C;
+    std::memset(&C, 0, sizeof C);
+    C.P = pl.P;
+    C.wpos = e.wpos.p;
+    C.ltype = e.ltype.p;
+    C.lj_table = e.lj_table.p;
+    C.lj_se = e.lj_se.p;
+    C.ci = e.corr_i.p;
+    C.cj = e.corr_j.p;
+    C.kind = e.corr_kind.p;
+    C.n = pl.corr_on ? e.n_corr : 0u;
+    C.mode = (int)e.prm.mode;
+    C.recip_on = pl.recip_on ? 1 : 0;
+    C.nblk = e.corr_blocks;
+    C.fx = e.fx_site.p;
+    C.n_sites = e.n_sites;
+    C.partials = energy_on ? e.corr_part.p : nullptr;
+    C.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
+    C.mol_of = e.mol_of.p;
+    C.n_mol = e.n_mol;
+    return C;
+  };
+  const bool in_spread = any_recip && RP.stream == RS.stream;
+  const unsigned n_bond = side ? side->blocks : 0u;
+  if (!in_spread && corr.blocks + n_bond) {
+    Profiler::Scope ps(prof, "side");
+    launch<k_eng_side>(RS, "k_eng_side", 0, corr.blocks + n_bond, 256, 0, [&](uint32_t i) {
       CorrArgs C;
       std::memset(&C, 0, sizeof C);
-      if (nc) {
-        C.P = pl.P;
-        C.wpos = e.wpos.p;
-        C.ltype = e.ltype.p;
-        C.lj_table = e.lj_table.p;
-        C.lj_se = e.lj_se.p;
-        C.ci = e.corr_i.p;
-        C.cj = e.corr_j.p;
-        C.kind = e.corr_kind.p;
-        C.n = pl.corr_on ? e.n_corr : 0u;
-        C.mode = (int)e.prm.mode;
-        C.recip_on = pl.recip_on ? 1 : 0;
-        C.nblk = e.corr_blocks;
-        C.fx = e.fx_site.p;
-        C.n_sites = e.n_sites;
-        C.partials = energy_on ? e.corr_part.p : nullptr;
-        C.mol_e = energy_on && e.n_mol ? e.mol_e.p : nullptr;
-        C.mol_of = e.mol_of.p;
-        C.n_mol = e.n_mol;
-      }
+      if (corr.blocks) C = corr.args(i);
       BondedArgs B;
       std::memset(&B, 0, sizeof B);
-      if (nb) B = side->args(i);
-      return args<k_eng_side>(A, C, B, np, nc);
+      if (n_bond) B = side->args(i);
+      return args<k_eng_side>(C, B, corr.blocks);
     });
-  };
-  {
-    Profiler::Scope ps(prof, "side");
-    if (RP.stream == RS.stream) {
-      side_launch(RS, 0, n_prep, n_corr, n_bond);
-    } else {
-      side_launch(RP, 1, n_prep, 0u, 0u);
-      side_launch(RS, 2, 0u, n_corr, n_bond);
-    }
   }
   if (any_recip) {
     std::vector<PmeRun> ra(ns), rb(ns);
@@ -2942,7 +2766,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
       r.res = e.eng_out.p + 16;
       r.status = e.status.p;
       r.status_bit = kStPme;
-      r.binned = true;  // the side launch has listed the charges
+      r.binned = true;  // the preparation kernel has listed the charges
       ra[i] = r;
       r.binned = false;
       if (pl.recip_b) {
@@ -2952,7 +2776,7 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
         rb[i] = r;
       }
     }
-    pme_run(RP, prof, ra.data(), 0, bond_spread ? side : nullptr);
+    pme_run(RP, prof, ra.data(), 0, in_spread ? &corr : nullptr, in_spread ? side : nullptr);
     if (any_b) pme_run(RP, prof, rb.data(), 1);
   }
   // a staged build on the second stream, beside the pair kernel (after it

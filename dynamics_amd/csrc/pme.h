@@ -19,6 +19,7 @@
 #include "batch.h"
 #include "bonded.h"
 #include "common.h"
+#include "corr.h"
 #include "wave.h"
 
 namespace dyn {
@@ -155,8 +156,9 @@ struct PmeRun {
 
 // runs[0 .. R.n): one per system of the pass; tag separates passes that run
 // more than once per evaluation (their launch sites keep separate packs).
-// side: bonded terms to evaluate in the same pass, or null.
+// corr, side: corrections and bonded terms to evaluate in the same pass, or
+// null.
 void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag,
-             const SideWork* side = nullptr);
+             const CorrWork* corr = nullptr, const SideWork* side = nullptr);
 
 }  // namespace dyn

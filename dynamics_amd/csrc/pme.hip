@@ -15,6 +15,7 @@
 
 #include "bonded.h"
 #include "common.h"
+#include "corr.h"
 #include "wave.h"
 #include "dyn_math.h"
 #include "pme.h"
@@ -681,18 +682,21 @@ __device__ __forceinline__ int stencil_point(int k0, int j, int K) {
 // weights in LDS (17.1); two 32-bit LDS adds for each 64-bit one (13.7, 43 at
 // 128³).
 //
-// Bonded terms (B; n_brick: workgroups of bricks before theirs) ride in the same
-// launch: both are chains of memory latencies.  28,000 sites: 16.2 µs, where
-// the launch before this one took 5.1 µs longer with them and this one 12.4 (MD
-// steps 3% faster).
+// The corrections (C, n_corr workgroups after the n_brick of the bricks) and
+// the bonded terms (B, the workgroups after them) of the evaluation ride in the
+// same launch: all three are chains of memory latencies.  28,000 sites: 12.4 µs
+// alone, 16.2 with the bonded terms, which made the launch before this one
+// 5.1 µs longer.
 template <int ORDER, class R>
 __device__ __forceinline__ void
 k_pme_spread(SplineArgs S, uint32_t nbx, uint32_t nby, uint32_t nbz, const uint32_t* __restrict__ count,
              const float4* __restrict__ items, uint32_t cap, int64_t* __restrict__ grid,
-             const BondedArgs& B, uint32_t n_brick) {
-  static_assert(kBrickBlock == kBondedBlock, "one block size");
+             const CorrArgs& C, const BondedArgs& B, uint32_t n_brick, uint32_t n_corr) {
+  static_assert(kBrickBlock == kBondedBlock && kBrickBlock == kCorrBlock, "one block size");
   if (blockIdx.x >= n_brick) {
-    bonded_terms(B, blockIdx.x - n_brick);
+    const uint32_t k = blockIdx.x - n_brick;
+    if (k < n_corr) corr_terms(C, k);
+    else bonded_terms(B, k - n_corr);
     return;
   }
   __shared__ unsigned long long acc[kBrick * kRowX];
@@ -1134,7 +1138,8 @@ void PmeCore::grow() {
 // core takes part in no stage (its packs describe empty work: no charges, no
 // bricks, no lines, no result); neither does it in the launches of the other
 // precision or order.
-void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag, const SideWork* side) {
+void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag, const CorrWork* corr,
+             const SideWork* side) {
   const uint32_t ns = R.n;
   std::vector<SplineArgs> S(ns);
   std::vector<FftGeom> gz(ns), gy(ns), gx(ns);
@@ -1193,23 +1198,27 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag, con
         if (o) B = cp(i)->bin_args(runs[i].status, runs[i].status_bit);
         return args<k_pme_bin>(runs[i].xyzq, o ? nq(i) : 0u, B);
       });
-    // (the first of the pass's spread launches takes the bonded terms)
-    bool with_side = side && side->blocks;
+    // (the first of the pass's spread launches takes the corrections and the
+    // bonded terms)
+    unsigned n_corr = corr ? corr->blocks : 0u, n_bond = side ? side->blocks : 0u;
     auto spread = [&](auto F, const char* name, bool f64, int order) {
-      const bool bonds = with_side;
-      with_side = false;
-      const unsigned g = g_b + (bonds ? side->blocks : 0u);
+      const unsigned nc = n_corr, nt = n_bond;
+      n_corr = n_bond = 0u;
+      const unsigned g = g_b + nc + nt;
       launch<decltype(F)::value, kBrickBlock>(R, name, tag, g, kBrickBlock, 0, [&](uint32_t i) {
         const bool m = mine(i, f64, order);
+        CorrArgs Cr;
+        std::memset(&Cr, 0, sizeof Cr);
+        if (nc) Cr = corr->args(i);
         BondedArgs B;
         std::memset(&B, 0, sizeof B);
-        if (bonds) B = side->args(i);
+        if (nt) B = side->args(i);
         return args<decltype(F)::value>(S[i], m ? nb(i, 0) : 0u, m ? nb(i, 1) : 0u,
                                         m ? nb(i, 2) : 0u,
                                         m ? (const uint32_t*)cp(i)->brick_count.p : nullptr,
                                         m ? (const float4*)cp(i)->brick_items.p : nullptr,
                                         m ? cp(i)->cap_brick : 0u,
-                                        m ? cp(i)->grid_fx.p : nullptr, B, g_b);
+                                        m ? cp(i)->grid_fx.p : nullptr, Cr, B, g_b, nc);
       });
     };
 #define DYN_SPREAD(O, T, F64)                                                                    \
