@@ -1548,7 +1548,10 @@ __device__ __forceinline__ bool tile_item(const PairArgs& A, const TileI& I, con
 }
 
 // The j groups [g0, g1) of a row with FP64 pair arithmetic (the precision
-// option): a lane loads its own j entry.
+// option): a lane loads its own j entry.  Three or four waves a SIMD are too few
+// to hide the loads, so while a group is evaluated the j data of the next and
+// the entry of the one after it are in flight (the last loads repeat the last
+// group): 279,600 sites with energies 1.97 ms, without that 2.23.
 template <int KIND, bool ENERGY>
 __device__ __forceinline__ void tile_entry64(const PairArgs& A, const TileI& I, const float4& pjv, int tj,
                                              int gj, bool active, TileAccT<double>& T) {
@@ -1563,12 +1566,21 @@ __device__ __forceinline__ void tile_entry64(const PairArgs& A, const TileI& I, 
 template <bool ENERGY>
 __device__ __forceinline__ void tile_item64(const PairArgs& A, const TileI& I, uint32_t g0, uint32_t g1,
                                             TileAccT<double>& T) {
-  const int lane = threadIdx.x & (kWave - 1);
+  const int lane = threadIdx.x & (kWave - 1), jb = lane >> 3;
+  const uint32_t glast = g1 - 1;
+  uint32_t vn = A.cj[(size_t)g0 * DYN_CL_SIZE + jb];
+  float4 pn = A.xyzq[vn & DYN_JSLOT_MASK];
+  int tn = A.slot_type[vn & DYN_JSLOT_MASK], gn = A.slot_gid[vn & DYN_JSLOT_MASK];
+  uint32_t v2 = A.cj[(size_t)min(g0 + 1, glast) * DYN_CL_SIZE + jb];
   for (uint32_t g = g0; g < g1; ++g) {
-    const uint32_t v = A.cj[(size_t)g * DYN_CL_SIZE + (lane >> 3)];
-    const uint32_t js = v & DYN_JSLOT_MASK;
-    const float4 pj = A.xyzq[js];
-    const int tj = A.slot_type[js], gj = A.slot_gid[js];
+    const uint32_t v = vn;
+    const float4 pj = pn;
+    const int tj = tn, gj = gn;
+    vn = v2;
+    pn = A.xyzq[vn & DYN_JSLOT_MASK];
+    tn = A.slot_type[vn & DYN_JSLOT_MASK];
+    gn = A.slot_gid[vn & DYN_JSLOT_MASK];
+    v2 = A.cj[(size_t)min(g + 2, glast) * DYN_CL_SIZE + jb];
     // readfirstlane returns a signed int: shift the entry as unsigned (class
     // 2 sets the top bit)
     const int kind = dyn_kind(I.ci, (int)((uint32_t)__builtin_amdgcn_readfirstlane(v) >> DYN_JCLS_SHIFT));
@@ -1781,6 +1793,19 @@ struct dyn::MinWavesPerSimd<k_eng_pairs<false, false, false>> {
 };
 template <>
 struct dyn::MinWavesPerSimd<k_eng_pairs<true, false, false>> {
+  static constexpr int value = 4;
+};
+
+// FP64 arithmetic: a wave more than the registers it would take by itself (193
+// and 150; some go to scratch) hides more than that costs: 279,600 sites with
+// energies 1.97 ms -> 1.65; forces, 56,000 sites, 20 MD steps 11.2 ms -> 10.9 (5
+// waves: 19.6).
+template <>
+struct dyn::MinWavesPerSimd<k_eng_pairs<true, true, false>> {
+  static constexpr int value = 3;
+};
+template <>
+struct dyn::MinWavesPerSimd<k_eng_pairs<false, true, false>> {
   static constexpr int value = 4;
 };
 
