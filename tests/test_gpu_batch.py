@@ -116,6 +116,27 @@ def test_batch_with_list_buffer(gpu, staged):
     assert all(m["graph_steps"] == 0 for _, m, _ in c)
 
 
+def test_batch_medium_total(gpu):
+    """Five boxes of 6,912 sites: the batch (34,560 sites) prepares its SPME
+    charges by a launch of its own, a member alone in the evaluation's first
+    launch; states and energies are the same bit for bit."""
+    s = systems.small_water(n_water=1728, box=39.4, lattice_n=12, seed=3)
+    made = [_make(s, None, 0.0, 1.0, seed=21 + k) for k in range(5)]
+    alone = [_make(s, None, 0.0, 1.0, seed=21 + k) for k in (0, 4)]
+    b = api.Batch([m for _, m in made])
+    for n in (20, 20, 20):
+        b.step(n)
+        for _, m in alone:
+            m.step(n)
+    b.close()
+    out = [[(m.state(), m.energies(), e.energies()) for e, m in r]
+           for r in (alone, (made[0], made[4]))]
+    _same_states(*out)
+    for e, m in made + alone:
+        m.close()
+        e.close()
+
+
 def test_batch_errors(gpu):
     s = systems.small_water()
     e1, m1 = _make(s, None, 0.0, 1.0, 1)
