@@ -450,6 +450,7 @@ __device__ __forceinline__ void
 k_fft_y(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw) {
   const FftGeom g = uni(geom);
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  if (g.K[0] == 0) return;  // takes no part: no tiles to divide by either
   const int tiles = (g.nh + g.L - 1) / g.L;
   const int x = blockIdx.x / tiles, k0 = (blockIdx.x - x * tiles) * g.L;
   if (x >= g.K[0]) return;  // beyond this system's lines

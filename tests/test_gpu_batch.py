@@ -116,6 +116,41 @@ def test_batch_with_list_buffer(gpu, staged):
     assert all(m["graph_steps"] == 0 for _, m, _ in c)
 
 
+def test_batch_mixed_separate_passes(gpu):
+    """A plain box beside two λ-windows whose x planes are too large for one
+    launch of y and z: the separate passes of the windows' second SPME
+    sum run with a member that takes no part in them.  Each member's
+    state and energies are those of its own run, bit for bit."""
+    solv = systems.small_solvated()
+
+    def made():
+        out = []
+        for k, (s, lam) in enumerate([(systems.small_water(), None), (solv, 0.3), (solv, 0.8)]):
+            ff = systems.chain_force_field(s) if s.n_dyn else systems.water_force_field(s)
+            eng = api.Engine(s, cutoff=10.0, beta=BETA, grid=(32, 96, 100), order=4, list_buffer=1.0)
+            pd, pw = api.relax(eng, ff, s.pos_dyn, systems.water_positions(s), steps=200)
+            if lam is not None:
+                eng.set_alchemical(4, 12, lam)
+            m = api.Md(eng, ff, dt=0.002, temperature=300.0, gamma=1.0, seed=31 + k)
+            v, vw = systems.initial_velocities(s, ff)
+            m.set_state(pd, v, pw, vw)
+            out.append((eng, m))
+        return out
+
+    print("plain box and two windows on 32 x 96 x 100 grids", flush=True)
+    alone, batch = made(), made()
+    b = api.Batch([m for _, m in batch])
+    for n in (3, 20):
+        b.step(n)
+        for _, m in alone:
+            m.step(n)
+    b.close()
+    _same_states(*[[(m.state(), m.energies(), e.energies()) for e, m in r] for r in (alone, batch)])
+    for e, m in alone + batch:
+        m.close()
+        e.close()
+
+
 def test_batch_medium_total(gpu):
     """Five boxes of 6,912 sites: the batch (34,560 sites) prepares its SPME
     charges by a launch of its own, a member alone in the evaluation's first
