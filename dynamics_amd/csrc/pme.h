@@ -107,7 +107,7 @@ struct PmeCore {
   DevBuf<double2> cgrid64;
   DevBuf<double> G64;
   DevBuf<double2> tw64[3];
-  DevBuf<int64_t> partials;     // energy/virial partials of the convolution pass (2^-32 fixed point)
+  DevBuf<int64_t> partials;     // energy/virial partials of the convolution pass (fixed point)
   PinnedBuf<double> h_part;
   DevBuf<double> res_dev;       // [energy, virial] reduced on the device
   // Spreading by grid brick (8³ points): each charge is listed under its

@@ -528,6 +528,8 @@ k_fft_plane(float2* __restrict__ spec, const int64_t* __restrict__ grid_fx, floa
   }
 }
 
+// Energy and virial in units of 2⁻³², then what each leaves in units of 2⁻⁶⁴.
+constexpr int kConvSums = 4;
 struct ConvArgs {
   float invL[3];
   double pi2_over_b2;  // π²/β²
@@ -536,15 +538,18 @@ struct ConvArgs {
 // x pass fused with the convolution, g.L consecutive (y, kz) columns per
 // workgroup: forward FFT along x, multiply by G(m) (accumulating ½G|F[Q]|² and
 // its virial weight), inverse FFT along x.  A kz inside the half spectrum
-// stands for −kz too.  Each point's energy is computed in f64 and rounded to
-// 2⁻³² fixed point, so the sums do not depend on the grouping of the lines.
+// stands for −kz too.  Each point's energy is computed in f64 and summed in
+// fixed point, so the sums do not depend on the grouping of the lines; two
+// words (2⁻³² and what that rounds away, 2⁻⁶⁴), since most of a fine grid's points
+// are smaller than 2⁻³³ (with one word two charges of 0.1 on 64³ lost 1.8e-5 of
+// their energy; the second costs 0.6 µs of 8.8 on 64³, 1.0 of 18.6 on 128³).
 template <class C>
 __device__ __forceinline__ void
 k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
              const typename CxT<C>::R* __restrict__ G, ConvArgs V, int64_t* __restrict__ partials) {
   const FftGeom g = uni(geom);
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ long long red[2][kFftBlock / 64];
+  __shared__ long long red[kConvSums][kFftBlock / 64];
   const int N = g.K[0], cols = g.K[1] * g.nh, c0 = blockIdx.x * g.L;
   if (c0 >= cols) return;  // beyond this system's lines
   const int nl = min(g.L, cols - c0);
@@ -559,7 +564,7 @@ k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
   }, [&](int e, C v) { A[e] = v; });
   __syncthreads();
   C* X = lds_fft<-1>(A, B, nl, nl, N, g.plan[0], s_tw);
-  long long qe = 0, qw = 0;
+  long long sum[kConvSums] = {0, 0, 0, 0};
   for_loaded(N * nl, [&](int e) {
     const int n = fast_div(e, nl, rnl);
     return G[(size_t)n * cols + c0 + e - n * nl];
@@ -573,25 +578,27 @@ k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
     const double msq = fx * fx + fy * fy + fz * fz;
     const double wz = mz == 0 || 2 * mz == g.K[2] ? 0.5 : 1.0;
     const double en = wz * (double)gv * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
-    qe += (long long)dyn_fx64(en);
-    qw += (long long)dyn_fx64(en * (1.0 - 2.0 * V.pi2_over_b2 * msq));
+    int64_t hi, lo;
+    dyn_fx128(en, &hi, &lo);
+    sum[0] += hi;
+    sum[2] += lo;
+    dyn_fx128(en * (1.0 - 2.0 * V.pi2_over_b2 * msq), &hi, &lo);
+    sum[1] += hi;
+    sum[3] += lo;
     v.x *= gv;
     v.y *= gv;
     X[e] = v;
   });
-  for (int m = 32; m >= 1; m >>= 1) {
-    qe += __shfl_xor(qe, m, 64);
-    qw += __shfl_xor(qw, m, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x / 64] = qe;
-    red[1][threadIdx.x / 64] = qw;
+#pragma unroll
+  for (int v = 0; v < kConvSums; ++v) {
+    for (int m = 32; m >= 1; m >>= 1) sum[v] += __shfl_xor(sum[v], m, 64);
+    if ((threadIdx.x & 63) == 0) red[v][threadIdx.x / 64] = sum[v];
   }
   __syncthreads();
-  if (threadIdx.x < 2) {
+  if (threadIdx.x < kConvSums) {
     long long s = 0;
     for (int k = 0; k < kFftBlock / 64; ++k) s += red[threadIdx.x][k];
-    partials[2 * blockIdx.x + threadIdx.x] = s;
+    partials[kConvSums * blockIdx.x + threadIdx.x] = s;
   }
   const C* Z = lds_fft<+1>(X, X == A ? B : A, nl, nl, N, g.plan[0], s_tw);
   for (int e = threadIdx.x; e < N * nl; e += blockDim.x) {
@@ -809,7 +816,7 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
                              double* __restrict__ res, uint32_t* __restrict__ brick_count,
                              uint32_t nbk) {
   // partials: the convolution's per-workgroup energy and virial sums in
-  // 2^-32 fixed point (nbp workgroups)
+  // fixed point (nbp workgroups, kConvSums words each)
   constexpr bool F32 = std::is_same<R, float>::value;
   // the spread has read the brick counts: clear them for the next binning
   if (brick_count)
@@ -817,30 +824,24 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
       brick_count[k] = 0u;
   if (res && blockIdx.x == 0) {
     // the first workgroup also sums the convolution's energy and virial
-    // partials (fixed order: strided per thread, then waves, then lanes)
-    __shared__ long long red[2][kGatherBlock / 64];
-    long long e = 0, w = 0;
-    for (int b = threadIdx.x; b < nbp; b += kGatherBlock) {
-      e += (long long)partials[2 * b];
-      w += (long long)partials[2 * b + 1];
-    }
-    for (int m = 32; m >= 1; m >>= 1) {
-      e += __shfl_xor(e, m, 64);
-      w += __shfl_xor(w, m, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-      red[0][threadIdx.x / 64] = e;
-      red[1][threadIdx.x / 64] = w;
+    // partials
+    __shared__ long long red[kConvSums][kGatherBlock / 64];
+    long long sum[kConvSums] = {0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nbp; b += kGatherBlock)
+      for (int v = 0; v < kConvSums; ++v) sum[v] += (long long)partials[kConvSums * b + v];
+#pragma unroll
+    for (int v = 0; v < kConvSums; ++v) {
+      for (int m = 32; m >= 1; m >>= 1) sum[v] += __shfl_xor(sum[v], m, 64);
+      if ((threadIdx.x & 63) == 0) red[v][threadIdx.x / 64] = sum[v];
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      long long te = 0, tw = 0;
+    if (threadIdx.x < 2) {
+      long long hi = 0, lo = 0;
       for (int k = 0; k < kGatherBlock / 64; ++k) {
-        te += red[0][k];
-        tw += red[1][k];
+        hi += red[threadIdx.x][k];
+        lo += red[threadIdx.x + 2][k];
       }
-      res[0] = (double)te * DYN_FX_INV_SCALE;
-      res[1] = (double)tw * DYN_FX_INV_SCALE;
+      res[threadIdx.x] = ((double)hi + (double)lo * DYN_FX_INV_SCALE) * DYN_FX_INV_SCALE;
     }
   }
   constexpr int kLanes = gather_lanes(ORDER);
@@ -1013,9 +1014,8 @@ void PmeCore::init(int dev, hipStream_t s, Profiler* p, const uint32_t k[3], con
     }
     DYN_HIP(hipStreamSynchronize(stream));
   }
-  // energy and virial partials: one fixed-point pair per x-pass workgroup
-  // (at most one per line)
-  partials.reserve(2 * (size_t)K[1] * (K[2] / 2 + 1));
+  // energy and virial partials of every x-pass workgroup (at most one per line)
+  partials.reserve(kConvSums * (size_t)K[1] * (K[2] / 2 + 1));
   res_dev.reserve(2);
   set_moduli();
   set_box(l);

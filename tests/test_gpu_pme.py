@@ -65,6 +65,29 @@ def test_pme_grid_sizes(gpu, K):
     assert abs(w - w64) <= 1e-5 * (abs(w64) + abs(e64))
 
 
+@pytest.mark.parametrize("n,scale,K", [(2, 0.1, (64, 64, 64)), (2, 1.0, (64, 64, 64)),
+                                       (300, 0.02, (45, 40, 36)), (2, 0.5, (8, 9, 10))])
+def test_pme_energy_of_small_terms(gpu, n, scale, K):
+    """Energy and virial whose spectrum points lie near or below 2⁻³² kcal/mol
+    each: nothing of their sum is lost."""
+    beta = float(np.float32(0.3123))
+    box = np.array([40.0, 41.0, 43.0], np.float32)
+    pos, q = _random_system(n, box, 7)
+    q = (q / np.abs(q).max() * scale).astype(np.float32)
+    print(f"SPME small terms: {n} charges up to {scale}, grid {K}", flush=True)
+    pme = api.PmeRecip(K, box, beta, order=4)
+    _, e, w = pme.forces_and_virial(pos, q)
+    _, e64, w64 = fp64.spme_fp64(pos, q, box, K, 4, beta)
+    e_rec = e - fp64.self_energy(q, beta)
+    # Relative errors: the charge grid's 2⁻³³ against weights of q·(1/6)³ at
+    # a charge's own points, 2⁻³³/(0.1/216) = 2.5e-7 at 0.1 and less above;
+    # f32 splines, transforms and influence function a few 2⁻²⁴ each.
+    tol = 2e-6 if scale >= 0.1 else 1e-5
+    assert abs(e_rec - e64) <= tol * abs(e64), (e_rec, e64)
+    assert abs(w - w64) <= tol * (abs(w64) + abs(e64)), (w, w64)
+    pme.close()
+
+
 def test_pme_water_config0(gpu):
     s = systems.config0()
     pos, qs, *_ = s.site_arrays()
