@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -123,6 +124,12 @@ inline unsigned grid_for(size_t n, unsigned block, unsigned max_blocks = 65535u 
   if (g < 1) g = 1;
   if (g > max_blocks) g = max_blocks;
   return (unsigned)g;
+}
+
+// Workgroups for a thread per item, without a limit (a kernel that does not
+// stride over its grid).
+inline unsigned grid_all(size_t n, unsigned block) {
+  return (unsigned)std::max<size_t>((n + block - 1) / block, 1);
 }
 
 // What enqueueing does with work on this thread: kLaunchDirect launches it;

@@ -1898,8 +1898,8 @@ extern "C" int dyn_md_get_state(dyn_md* md, float* pos_dyn, float* vel_dyn, floa
     // (6·nd + 21·nw floats: the stage holds 6 per site)
     float* const h = static_cast<float*>(engine_host_stage(md->eng));
     MdSet S = self_set(md);
-    launch<k_md_state_out>(S.R, "k_md_state_out", 0, grid_for(6 * (size_t)nd + 21 * (size_t)nw, kBlock),
-                           kBlock, 0, [&](uint32_t) {
+    const size_t n_out = 6 * (size_t)nd + 21 * (size_t)nw;
+    launch<k_md_state_out>(S.R, "k_md_state_out", 0, grid_all(n_out, kBlock), kBlock, 0, [&](uint32_t) {
       return args<k_md_state_out>((const float*)md->x.p, (const float*)md->v.p, nd, nw, h,
                                   engine_report_view(md->eng));
     });

@@ -4,6 +4,8 @@ of the solvated chain (bonded terms, SHAKE/RATTLE on bonds to hydrogen,
 rigid water); rigid geometry and constraints over many steps; energy
 conservation of the γ = 0 step; the Langevin temperature."""
 
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -271,4 +273,26 @@ def test_staged_lists_cover_cutoff(gpu):
               f"unlisted {len(miss)} {miss[:4]}", flush=True)
         assert not miss
     m.close()
+    eng.close()
+
+
+def test_state_of_a_very_large_system(gpu):
+    """Every float of the state is read back, also beyond 2¹⁸ workgroups of
+    the kernel that packs it (13 million sites)."""
+    nw = 3_250_000
+    zeros = np.zeros((nw, 3), np.float32)
+    s = dataclasses.replace(systems.small_water(), box=np.full(3, 464.0, np.float32), pos_o=zeros,
+                            pos_m=zeros, pos_h0=zeros, pos_h1=zeros)
+    print(f"state of {4 * nw} sites", flush=True)
+    eng = api.Engine(s, cutoff=3.0, beta=0.3)
+    md = api.Md(eng, systems.water_force_field(s))
+    rng = np.random.default_rng(2)
+    x = rng.random((nw, 4, 3), np.float32)
+    v = rng.random((nw, 3, 3), np.float32)
+    none = np.zeros((0, 3), np.float32)
+    md.set_state(none, none, x, v)
+    _, _, x1, v1 = md.state()
+    same = np.array_equal(x1, x), np.array_equal(v1, v)
+    assert same == (True, True)
+    md.close()
     eng.close()
