@@ -1505,7 +1505,7 @@ extern "C" int dyn_pme_forces_and_virial(dyn_pme* pme, uint32_t n, const float* 
       else
         r.binned = false;  // from the device's copy
       pme_run(R, pme->prof, &r, 0);
-      launch<k_pme_out>(R, "k_pme_out", 0, grid_for(3 * nn, 256), 256, 0, [&](uint32_t) {
+      launch<k_pme_out>(R, "k_pme_out", 0, grid_all(3 * nn, 256), 256, 0, [&](uint32_t) {
         return args<k_pme_out>((const float*)pme->fout.p, 3u * n, (const double*)core.res_dev.p,
                                (const unsigned int*)core.status.p, h_f, rep);
       });

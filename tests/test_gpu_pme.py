@@ -88,6 +88,23 @@ def test_pme_energy_of_small_terms(gpu, n, scale, K):
     pme.close()
 
 
+def test_pme_very_many_charges(gpu):
+    """Forces of 22.5 million charges are all read back (beyond 2¹⁸
+    workgroups of the kernel that stores them): the last charge, at the first one's place
+    and with its value, has its force."""
+    n = 22_500_000
+    rng = np.random.default_rng(4)
+    box = np.full(3, 60.0, np.float32)
+    pos = rng.random((n, 3), np.float32) * box
+    q = rng.random(n, np.float32) - np.float32(0.5)
+    pos[-1], q[-1] = pos[0], q[0]
+    print(f"SPME of {n} charges", flush=True)
+    pme = api.PmeRecip((64, 64, 64), box, 0.3123, order=4)
+    f, _, _ = pme.forces_and_virial(pos, q)
+    assert f[0].any() and np.array_equal(f[0], f[-1])
+    pme.close()
+
+
 def test_pme_water_config0(gpu):
     s = systems.config0()
     pos, qs, *_ = s.site_arrays()
