@@ -1113,7 +1113,30 @@ struct PairArgs {
   uint32_t chunk;            // j groups per work item
   uint32_t unused;           // no implicit padding: argument packs are compared byte for byte
   unsigned int* status;      // a list-build overflow leaves the list unusable
+  const uint2* chunks;       // work items: row, first group (FP64; copy 0; chunks2: copy 1)
+  const uint2* chunks2;
+  const uint32_t* n_chunks;
+  int64_t* fx_site;          // site sums the FP64 kernel's i forces are added to
 };
+
+// Whether the evaluation can go ahead (the same for every workgroup); A's
+// list pointers become those of the copy in use.
+__device__ __forceinline__ bool pairs_begin(PairArgs& A) {
+  if (*A.status) return false;
+  // in staged mode a site may have moved half the list buffer since the
+  // current list's build: the list may then miss pairs, and the evaluation
+  // is void
+  if (A.staged && A.fl[kFlDisp] >= A.hard_limit) {
+    if (threadIdx.x == 0) atomicOr(A.status, kStDisp);
+    return false;
+  }
+  if ((A.fl[kFlSel] ^ A.fl[kFlCommit]) != 0u) {
+    A.cj = A.cj2;
+    A.cmask = A.cmask2;
+    A.chunks = A.chunks2;
+  }
+  return true;
+}
 
 __device__ __forceinline__ float xor_sum(float v, int m) { return v + __shfl_xor(v, m, kWave); }
 __device__ __forceinline__ double xor_sum_d(double v, int m) { return v + __shfl_xor(v, m, kWave); }
@@ -1330,10 +1353,9 @@ __device__ __forceinline__ uint32_t ext8(uint32_t v) {
   v = f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true));
   return f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, true));
 }
-__device__ __forceinline__ RowImage row_image(const DynPairParams& P, const float4& p) {
+__device__ __forceinline__ RowImage row_image(const DynPairParams& P, const float x[4]) {
   RowImage r;
   const float rc = __builtin_amdgcn_sqrtf(P.rc2) * 1.0001f + 1e-3f;
-  const float x[3] = {p.x, p.y, p.z};
   bool ok = true, in = true;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
@@ -1639,6 +1661,40 @@ __device__ __forceinline__ double row_sum(double v) {
   return v + ror(v, std::integral_constant<int, 0x121>{});
 }
 
+// A work item's energies, virial and pair counts.  Six sums over the wave at
+// the cost of two: a swap of half-waves leaves one value in each half, a swap
+// of rows one in each row of 16.
+template <class R>
+__device__ __forceinline__ void item_partials(const PairArgs& A, const TileAccT<R>& T, size_t item, int lane) {
+  const double a0 = swap32_sum((double)T.e_lj_w, (double)T.e_c_w);
+  const double a1 = swap32_sum((double)T.e_lj_s, (double)T.e_c_s);
+  const double a2 = swap32_sum((double)T.vir, (double)T.dh);
+  const double b0 = row_sum(swap16_sum(a0, a1)), b1 = row_sum(swap16_sum(a2, a2));
+  double* const out = A.partials + item;
+  // rows of b0: LJ water, LJ solute, Coulomb water, Coulomb solute; of
+  // b1: virial, virial, dH/dλ, dH/dλ
+  if ((lane & 15) == 0) out[(size_t)(lane >> 4) * A.cap_chunks] = b0;
+  if ((lane & 31) == 1) out[(size_t)(lane == 1 ? 4 : 8) * A.cap_chunks] = b1;
+  if (lane < 3) out[(size_t)(5 + lane) * A.cap_chunks] = (double)(lane == 0 ? T.n_ss : lane == 1 ? T.n_lj : T.n_c);
+}
+
+// The i side of a row for lane (ia, ·).
+__device__ __forceinline__ TileI tile_i(const PairArgs& A, uint32_t row, int ia) {
+  const uint32_t slot = row * DYN_CL_SIZE + ia;
+  const float4 p = A.xyzq[slot];
+  TileI I;
+  I.p[0] = p.x;
+  I.p[1] = p.y;
+  I.p[2] = p.z;
+  I.p[3] = p.w;
+  I.r2_lo = dyn_coul_r2_lo(A.P.beta2);
+  I.t = A.slot_type[slot];
+  I.g = A.slot_gid[slot];
+  I.ci = A.cl_class[row];
+  I.pad = I.g == DYN_GID_PAD;
+  return I;
+}
+
 // A workgroup per row (i cluster) at a time, a wave per work item (≤ A.chunk
 // groups of the row); lane ia + 8·jb holds the pair (i slot 8I+ia, j entry jb
 // of a group).
@@ -1663,109 +1719,61 @@ __device__ __forceinline__ double row_sum(double v) {
 // took, at 252,480 sites, 395 µs per MD evaluation (median; now 285), 310 with
 // energies (259); 28,000 sites 55 (42) and 54 (54); a batch of 32 boxes 259
 // (186); 16 alchemical windows 340 (329).
-template <bool ENERGY, bool F64, bool ALCH>
+template <bool ENERGY, bool ALCH>
 __device__ __forceinline__ void
 k_eng_pairs(PairArgs A) {
-  using R = std::conditional_t<F64, double, float>;
   // the Coulomb tables over y (β³Ψ, and βΛ with energies; at offset 0, so a
   // lane's table address is its entry's offset) and the row's forces (two
   // buffers); in FP32 the LJ (c6, c12) table of n_types² entries follows
-  constexpr int kTab = F64 ? 1 : (ENERGY ? 2 : 1) * DYN_COUL_Y_N;
-  __shared__ float4 s_tab[kTab];
+  __shared__ float4 s_tab[(ENERGY ? 2 : 1) * DYN_COUL_Y_N];
   __shared__ int64_t s_f[2][kPairBlock / kWave][3 * DYN_CL_SIZE];
   extern __shared__ float2 s_lj[];
   const int lane = threadIdx.x & (kWave - 1);
   const int ia = lane & 7, jb = lane >> 3;
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  if (*A.status) return;
-  // in staged mode a site may have moved half the list buffer since the
-  // current list's build: the list may then miss pairs, and the evaluation
-  // is void (every workgroup reads the same words)
-  if (A.staged && A.fl[kFlDisp] >= A.hard_limit) {
-    if (threadIdx.x == 0) atomicOr(A.status, kStDisp);
-    return;
-  }
-  if ((A.fl[kFlSel] ^ A.fl[kFlCommit]) != 0u) {
-    A.cj = A.cj2;
-    A.cmask = A.cmask2;
-  }
+  if (!pairs_begin(A)) return;
   const uint32_t n_cl = *A.n_cl;
   if (blockIdx.x >= n_cl) return;
-  DynCoulTabs tabs = {nullptr, nullptr};
-  const float2* ljt = nullptr;
-  if constexpr (!F64) {
-    const DynCoulTabs src = dyn_coul_tabs(A.P.coul_tab);
-    for (int k = threadIdx.x; k < DYN_COUL_Y_N; k += kPairBlock) {
-      s_tab[k] = dyn_tab_scale(src.ftab[k], A.P.beta2 * A.P.beta);
-      if (ENERGY) s_tab[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], A.P.beta);
-    }
-    const int nt2 = A.P.n_types * A.P.n_types;
-    for (int k = threadIdx.x; k < nt2; k += kPairBlock) s_lj[k] = A.lj_table[k];
-    __syncthreads();
-    tabs.ftab = s_tab;
-    tabs.etab = s_tab + (ENERGY ? DYN_COUL_Y_N : 0);
-    ljt = s_lj;
+  const DynCoulTabs src = dyn_coul_tabs(A.P.coul_tab);
+  for (int k = threadIdx.x; k < DYN_COUL_Y_N; k += kPairBlock) {
+    s_tab[k] = dyn_tab_scale(src.ftab[k], A.P.beta2 * A.P.beta);
+    if (ENERGY) s_tab[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], A.P.beta);
   }
+  const int nt2 = A.P.n_types * A.P.n_types;
+  for (int k = threadIdx.x; k < nt2; k += kPairBlock) s_lj[k] = A.lj_table[k];
+  __syncthreads();
+  const DynCoulTabs tabs = {s_tab, s_tab + (ENERGY ? DYN_COUL_Y_N : 0)};
   int buf = 0;
   for (uint32_t row = blockIdx.x; row < n_cl; row += gridDim.x, buf ^= 1) {
     const uint32_t r0 = A.row_ptr[row], r1 = A.row_ptr[row + 1];
-    const float4 piv = A.xyzq[row * DYN_CL_SIZE + ia];
-    TileI I;
-    I.p[0] = piv.x;
-    I.p[1] = piv.y;
-    I.p[2] = piv.z;
-    I.p[3] = piv.w;
-    I.r2_lo = dyn_coul_r2_lo(A.P.beta2);
-    I.t = A.slot_type[row * DYN_CL_SIZE + ia];
-    I.g = A.slot_gid[row * DYN_CL_SIZE + ia];
-    I.ci = A.cl_class[row];
-    I.pad = I.g == DYN_GID_PAD;
+    TileI I = tile_i(A, row, ia);
     I.any_in = ALCH && lanes(!I.pad & ((I.t & DYN_TYPE_ALCH) != 0)) != 0ull;
     I.any_out = ALCH && lanes(!I.pad & ((I.t & DYN_TYPE_ALCH) == 0)) != 0ull;
     int64_t acc[3] = {0, 0, 0};
     uint32_t it = w, g0 = r0 + w * A.chunk;
     RowImage Im;
-    if constexpr (!F64)
-      if (g0 < r1) {
-        Im = row_image(A.P, piv);
-        if (I.pad) I.p[0] = -kFarX;
-      }
+    if (g0 < r1) {
+      Im = row_image(A.P, I.p);
+      if (I.pad) I.p[0] = -kFarX;
+    }
     for (; g0 < r1; it += kPairBlock / kWave, g0 += kPairBlock / kWave * A.chunk) {
       const uint32_t g1 = min(g0 + A.chunk, r1);
-      TileAccT<R> T;
+      TileAccT<float> T;
       T.clear();
-      if constexpr (F64) {
-        tile_item64<ENERGY>(A, I, g0, g1, T);
-      } else {
-        // molecule-pair energies are added by the general path only
-        bool any = ENERGY && A.mol_e && I.ci == DYN_CLS_SOLUTE;
-        while (!tile_item<ENERGY, ALCH>(A, I, Im, any, g0, g1, tabs, ljt, T)) {
-          any = true;  // (and then it returns true)
-          T.clear();
-        }
+      // molecule-pair energies are added by the general path only
+      bool any = ENERGY && A.mol_e && I.ci == DYN_CLS_SOLUTE;
+      while (!tile_item<ENERGY, ALCH>(A, I, Im, any, g0, g1, tabs, s_lj, T)) {
+        any = true;  // (and then it returns true)
+        T.clear();
       }
       for (int c = 0; c < 3; ++c) T.fi[c] = sum_jb(T.fi[c]);
       const size_t item = (size_t)A.chunk_ptr[row] + it;
       for (int c = 0; c < 3; ++c) {
-        int64_t q;
-        if constexpr (F64) q = dyn_fx64(T.fi[c]);
-        else q = dyn_fx(T.fi[c]);
+        const int64_t q = dyn_fx(T.fi[c]);
         acc[c] += q;
         if (A.keep_items && jb == 0) A.fitem[item * (3 * DYN_CL_SIZE) + c * DYN_CL_SIZE + ia] = q;
       }
-      if (!ENERGY) continue;
-      // six sums over the wave at the cost of two: a swap of half-waves
-      // leaves one value in each half, a swap of rows one in each row of 16
-      const double a0 = swap32_sum((double)T.e_lj_w, (double)T.e_c_w);
-      const double a1 = swap32_sum((double)T.e_lj_s, (double)T.e_c_s);
-      const double a2 = swap32_sum((double)T.vir, (double)T.dh);
-      const double b0 = row_sum(swap16_sum(a0, a1)), b1 = row_sum(swap16_sum(a2, a2));
-      double* const out = A.partials + item;
-      // rows of b0: LJ water, LJ solute, Coulomb water, Coulomb solute; of
-      // b1: virial, virial, dH/dλ, dH/dλ
-      if ((lane & 15) == 0) out[(size_t)(lane >> 4) * A.cap_chunks] = b0;
-      if ((lane & 31) == 1) out[(size_t)(lane == 1 ? 4 : 8) * A.cap_chunks] = b1;
-      if (lane < 3) out[(size_t)(5 + lane) * A.cap_chunks] = (double)(lane == 0 ? T.n_ss : lane == 1 ? T.n_lj : T.n_c);
+      if (ENERGY) item_partials(A, T, item, lane);
     }
     // the row's forces: the waves' sums (integers: the order of the items
     // does not change them), stored by site.  Two buffers: the next row's
@@ -1782,30 +1790,68 @@ k_eng_pairs(PairArgs A) {
   }
 }
 
+// The pairs with FP64 arithmetic (the precision option): a wave per work item,
+// items in a grid stride, i forces added to the sites' sums with atomics.
+//
+// Bound: FP64 issue with three or four waves a SIMD.  With so few a workgroup
+// per row, as in FP32, leaves waves idle at rows of one to three items and in the
+// last round of workgroups.  20 MD steps of 2,000, 28,000 and 252,480 sites, a
+// workgroup per row 1.96, 5.77 and 41.7 ms; a wave per item 1.70, 5.51 and 39.0.
+template <bool ENERGY>
+__device__ __forceinline__ void
+k_eng_pairs64(PairArgs A) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int ia = lane & 7, jb = lane >> 3;
+  if (!pairs_begin(A)) return;
+  const uint32_t n_items = (uint32_t)min((uint64_t)*A.n_chunks, A.cap_chunks);
+  const uint32_t waves = gridDim.x * (kPairBlock / kWave);
+  for (uint32_t item = blockIdx.x * (kPairBlock / kWave) + threadIdx.x / kWave; item < n_items; item += waves) {
+    const uint2 ch = A.chunks[item];
+    const uint32_t row = (uint32_t)__builtin_amdgcn_readfirstlane(ch.x);
+    const uint32_t g0 = (uint32_t)__builtin_amdgcn_readfirstlane(ch.y);
+    const uint32_t g1 = min(g0 + A.chunk, A.row_ptr[row + 1]);
+    const TileI I = tile_i(A, row, ia);
+    TileAccT<double> T;
+    T.clear();
+    tile_item64<ENERGY>(A, I, g0, g1, T);
+    const int32_t site = A.slot_site[row * DYN_CL_SIZE + ia];
+    for (int c = 0; c < 3; ++c) {
+      const int64_t q = dyn_fx64(sum_jb(T.fi[c]));
+      if (jb != 0) continue;
+      if (A.keep_items) A.fitem[(size_t)item * (3 * DYN_CL_SIZE) + c * DYN_CL_SIZE + ia] = q;
+      if (site >= 0)
+        atomicAdd(reinterpret_cast<unsigned long long*>(A.fx_site + (size_t)c * A.n_sites + site),
+                  (unsigned long long)q);
+    }
+    if (ENERGY) item_partials(A, T, item, lane);
+  }
+}
+
 }  // namespace
 
 // Registers for five resident waves per SIMD for forces and four with
 // energies.  Forces at 252,480 sites, 3 to 8 waves asked for: 5 was the
 // fastest (6 spills: 3% slower; 4: 4%); energies 4 (5 spills: 6% slower).
 template <>
-struct dyn::MinWavesPerSimd<k_eng_pairs<false, false, false>> {
+struct dyn::MinWavesPerSimd<k_eng_pairs<false, false>> {
   static constexpr int value = 5;
 };
 template <>
-struct dyn::MinWavesPerSimd<k_eng_pairs<true, false, false>> {
+struct dyn::MinWavesPerSimd<k_eng_pairs<true, false>> {
   static constexpr int value = 4;
 };
 
-// FP64 arithmetic: a wave more than the registers it would take by itself (193
-// and 150; some go to scratch) hides more than that costs: 279,600 sites with
-// energies 1.97 ms -> 1.65; forces, 56,000 sites, 20 MD steps 11.2 ms -> 10.9 (5
-// waves: 19.6).
+// FP64 arithmetic: a wave more than the registers it would take by itself (some
+// go to scratch) hides more than that costs.  Energies 2 -> 3 waves: 252,480
+// sites, an evaluation 2,806 -> 2,780 µs.  Forces 3 -> 4: 20 MD steps of 56,000
+// sites 11.20 -> 10.97 ms, of 252,480 39.7 -> 39.0 (of 14,000 3.94 -> 4.13, still
+// below any other form).
 template <>
-struct dyn::MinWavesPerSimd<k_eng_pairs<true, true, false>> {
+struct dyn::MinWavesPerSimd<k_eng_pairs64<true>> {
   static constexpr int value = 3;
 };
 template <>
-struct dyn::MinWavesPerSimd<k_eng_pairs<false, true, false>> {
+struct dyn::MinWavesPerSimd<k_eng_pairs64<false>> {
   static constexpr int value = 4;
 };
 
@@ -2880,6 +2926,10 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
       A.fitem = e.fitem.p;
       A.slot_site = e.slot_site.p;
       A.fx_pair = e.fx_pair;
+      A.chunks = e.chunks.p;
+      A.chunks2 = e.chunks2.p;
+      A.n_chunks = e.counters.p + 2;
+      A.fx_site = e.fx_site.p;
       A.n_sites = e.n_sites;
       // a fused evaluation's caller reads site sums only
       A.keep_items = (flags & kComputeFusedFinalize) ? 0u : 1u;
@@ -2888,13 +2938,15 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
       A.chunk = e.prm.item_groups;
       A.status = e.status.p;
     }
-    // a workgroup per row, up to kPairGridCap workgroups (the row count is
-    // known on the device only; the workgroups take rows in a grid stride)
-    const unsigned gp = max_grid(S, [](dyn_engine& e) {
-      return std::min<uint32_t>(kPairGridCap, std::max(1u, e.cap_cl));
-    });
     // FP64 pair arithmetic when the first system asks for it (a set shares it)
     const bool f64 = (E[0]->prm.precision & DYN_PREC_PAIR_F64) != 0;
+    // a workgroup per row (FP64: a wave per work item), up to kPairGridCap
+    // workgroups (the counts are known on the device only; the workgroups
+    // stride over their grid)
+    const unsigned gp = max_grid(S, [&](dyn_engine& e) {
+      const uint64_t need = f64 ? (e.cap_chunks + 3) / 4 : e.cap_cl;
+      return (unsigned)std::min<uint64_t>(kPairGridCap, std::max<uint64_t>(1, need));
+    });
     int nt_max = 0;
     for (dyn_engine* e : E) nt_max = std::max(nt_max, e->n_types);
     const size_t shm = f64 ? 0 : sizeof(float2) * (size_t)nt_max * (size_t)nt_max;  // the LJ table
@@ -2906,14 +2958,13 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
         return args<decltype(F)::value>(PA[i]);
       });
     };
-#define DYN_PAIRS(E, F64, ALCH) \
-  std::integral_constant<decltype(&k_eng_pairs<E, F64, ALCH>), &k_eng_pairs<E, F64, ALCH>> {}
-    if (f64 && energy_on) go(DYN_PAIRS(true, true, false), "k_eng_pairs<true, f64>");
-    else if (f64) go(DYN_PAIRS(false, true, false), "k_eng_pairs<false, f64>");
-    else if (alch && energy_on) go(DYN_PAIRS(true, false, true), "k_eng_pairs<true, alch>");
-    else if (alch) go(DYN_PAIRS(false, false, true), "k_eng_pairs<false, alch>");
-    else if (energy_on) go(DYN_PAIRS(true, false, false), "k_eng_pairs<true>");
-    else go(DYN_PAIRS(false, false, false), "k_eng_pairs<false>");
+#define DYN_PAIRS(...) std::integral_constant<decltype(&__VA_ARGS__), &__VA_ARGS__> {}
+    if (f64 && energy_on) go(DYN_PAIRS(k_eng_pairs64<true>), "k_eng_pairs64<true>");
+    else if (f64) go(DYN_PAIRS(k_eng_pairs64<false>), "k_eng_pairs64<false>");
+    else if (alch && energy_on) go(DYN_PAIRS(k_eng_pairs<true, true>), "k_eng_pairs<true, alch>");
+    else if (alch) go(DYN_PAIRS(k_eng_pairs<false, true>), "k_eng_pairs<false, alch>");
+    else if (energy_on) go(DYN_PAIRS(k_eng_pairs<true, false>), "k_eng_pairs<true>");
+    else go(DYN_PAIRS(k_eng_pairs<false, false>), "k_eng_pairs<false>");
 #undef DYN_PAIRS
   }
   if (any_staged && one_stream) set_build_lists(S, R, sgate, true);
@@ -2926,7 +2977,8 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
     std::memset(&P, 0, sizeof P);
     P.fx_site = e.fx_site.p;
     P.fx_recip = (pl.recip_on || pl.reuse) ? e.fx_recip.p : nullptr;
-    P.fx_pair = short_on ? e.fx_pair : nullptr;
+    // (FP64 pairs are in fx_site)
+    P.fx_pair = short_on && !(E[0]->prm.precision & DYN_PREC_PAIR_F64) ? e.fx_pair : nullptr;
     P.n_sites = e.n_sites;
     P.fl = e.dflags.p;
     P.forced = forced[i] ? 1 : 0;

@@ -90,3 +90,31 @@ def test_precision_errors(gpu, solvated):
     with pytest.raises(api.DynError):
         eng.set_alchemical(4, 12, 0.5)               # alchemical runs in f32 only
     eng.close()
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_md_f64_pairs_joined_steps(gpu, staged):
+    """FP64 pairs in MD with a list buffer: steps joined in one call (forces
+    summed from their parts, both copies of a staged list) and one step at a
+    time reach the same state bit for bit."""
+    s = systems.small_solvated()
+    ff = systems.chain_force_field(s)
+    eng = _engine(s, 0, (27, 27, 27))
+    pd, pw = api.relax(eng, ff, s.pos_dyn, systems.water_positions(s), steps=200)
+    eng.close()
+    v, vw = systems.initial_velocities(s, ff)
+    out = []
+    for calls in ([40], [1] * 40):
+        eng = api.Engine(s, cutoff=RC, beta=BETA, grid=(27, 27, 27), precision=api.PREC_PAIR_F64,
+                         list_buffer=0.6)
+        m = api.Md(eng, ff, seed=3, staged_builds=staged)
+        m.set_state(pd, v, pw, vw)
+        print(f"FP64 pairs, staged {staged}, calls {len(calls)}", flush=True)
+        for n in calls:
+            m.step(n)
+        out.append((m.state(), eng.energies()["list_builds"]))
+        m.close()
+        eng.close()
+    assert all(b > 2 for _, b in out)
+    for x, y in zip(out[0][0], out[1][0]):
+        assert np.array_equal(x, y)
