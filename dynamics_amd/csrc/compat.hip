@@ -261,9 +261,11 @@ struct NblGrid {
   double ext[3];
 };
 
-// The cell of a coordinate along one axis.  (Rows reach one cell further than
-// their list radius needs, so the wrap of a coordinate a few boxes out may
-// round; far ones are reduced exactly.)
+// The cell of a coordinate along one axis.  A cell is at least the list
+// radius and its margin (1e-5 of it and 1e-3 Å) wide, so the ±1 cells hold every
+// neighbour if a wrapped coordinate is off by less than half the margin: its
+// rounding is below 2e-10 box lengths for coordinates within 10⁶ boxes (1e-3 Å
+// in boxes of up to 10⁶ Å); farther ones are reduced exactly.
 __device__ __forceinline__ int nbl_cell_1d(float x, double ext, double cw, int nc) {
   double w = fabs((double)x) < 1e6 * ext ? (double)x - floor((double)x / ext) * ext : fmod((double)x, ext);
   if (w < 0) w += ext;
@@ -380,8 +382,13 @@ k_scan_u32(const uint32_t* __restrict__ in, uint32_t n, uint32_t* __restrict__ o
 }
 
 constexpr int kNblCap = 4096;  // max neighbors per row
-// Inner indices a row's bitmap holds (16 KB of LDS); more are taken in ranges.
-constexpr uint32_t kNblBits = 1u << 17;
+// Inner indices up to which a row is put in order by a bitmap over them (4 KB
+// of LDS), above by a sort of its hits.  The bitmap is cleared and read in
+// full by every row, and its LDS limits the waves in flight: rows of 30, 72 and 384
+// neighbours among 16,000 points 40, 44 and 88 µs (sorted 45, 54 and 158), among
+// 32,000 78, 82 and 149 (74, 87, 263), among 64,000 274, 289 and 526 (132, 159, 536),
+// among 130,000 1,579, 1,655 and 2,314 (253, 306, 974).
+constexpr uint32_t kNblBits = 1u << 15;
 
 struct NblRowArgs {
   const float* outer;
@@ -394,8 +401,7 @@ struct NblRowArgs {
   float lo, hi;  // an approximate r² below lo or above hi decides the test
   int symmetric;
   int use_nb[3];  // 1: the ±1 neighbour cells along the axis, 0: its one cell
-  uint32_t n_inner;
-  uint32_t range;  // indices per bitmap, a multiple of 2048 (64 words)
+  uint32_t words;  // of a row's bitmap (PASS 1)
 };
 
 // The reference's exact pair test (src/neighbors.rs:221-222).
@@ -409,22 +415,21 @@ __device__ __forceinline__ bool nbl_accept(const float* po, const float* pi, con
 
 // One wave per outer point, in a workgroup of its own.  PASS 0 counts the
 // accepted inner points; PASS 1 marks them in a bitmap over the inner indices
-// and writes the row from it in ascending order.
+// and writes the row from it in ascending order; PASS 2 collects them and sorts.
 //
 // Bound: the pair tests (27 cells of candidates, 11% accepted).  The
 // reference's test takes three correctly rounded divisions; here an approximate
 // r² by reciprocals decides all but those within its error of the threshold
 // (about one in 10⁴), which take the exact test.  The points lie in cell order,
 // so a wave reads the cells of a column (contiguous along z) as one run of
-// 16-byte loads, and the bitmap replaces a sort of the row: 64 words, a few
-// bits each, per step.  With a 256-thread workgroup per row that gathered points
+// 16-byte loads, and the bitmap replaces a sort of the row (see kNblBits).  With a 256-thread workgroup per row that gathered points
 // by index, tested exactly and sorted in LDS, 8,000 points (3.0 M neighbours)
 // took 124 µs (count) and 183 µs (rows); now 39 and 55.
 template <int PASS>
 __global__ void __launch_bounds__(64)
 k_nbl_rows(NblRowArgs A, uint32_t n_outer, uint32_t* __restrict__ row_count,
            const uint32_t* __restrict__ row_ptr, uint32_t* __restrict__ col) {
-  extern __shared__ uint32_t bits[];
+  extern __shared__ uint32_t bits[];  // PASS 2: the row's indices
   const uint32_t i = blockIdx.x, lane = threadIdx.x;
   if (i >= n_outer) return;
   const float po[3] = {A.outer[3 * (size_t)i], A.outer[3 * (size_t)i + 1], A.outer[3 * (size_t)i + 2]};
@@ -436,68 +441,92 @@ k_nbl_rows(NblRowArgs A, uint32_t n_outer, uint32_t* __restrict__ row_count,
   const int z0 = cz - A.use_nb[2], z1 = cz + A.use_nb[2] + 1;
   const int runs = z0 < 0 || z1 > nz ? 2 : 1;
   uint32_t found = 0;
-  uint32_t out = PASS == 1 ? row_ptr[i] : 0u;
-  for (uint64_t r0 = 0; r0 < A.n_inner; r0 += PASS == 1 ? A.range : A.n_inner) {
-    const uint32_t words = PASS == 1 ? (uint32_t)(min((uint64_t)A.range, A.n_inner - r0) + 31) / 32 : 0u;
-    if (PASS == 1) {
-      for (uint32_t k = lane; k < words; k += 64) bits[k] = 0u;
-      __syncthreads();
-    }
-    for (int ox = -A.use_nb[0]; ox <= A.use_nb[0]; ++ox)
-      for (int oy = -A.use_nb[1]; oy <= A.use_nb[1]; ++oy) {
-        const int x = (cc[0] + ox + A.G.nc[0]) % A.G.nc[0];
-        const int y = (cc[1] + oy + A.G.nc[1]) % A.G.nc[1];
-        const uint32_t c = (uint32_t)((x * A.G.nc[1] + y) * nz);
-        for (int r = 0; r < runs; ++r) {
-          // [z0, z1) within [0, nz), and what wraps
-          const int a = r == 0 ? max(z0, 0) : (z0 < 0 ? z0 + nz : 0);
-          const int b = r == 0 ? min(z1, nz) : (z0 < 0 ? nz : z1 - nz);
-          const uint32_t k1 = A.cell_start[c + b];
-          for (uint32_t k = A.cell_start[c + a] + lane; k < k1; k += 64) {
-            const float4 s = A.sorted[k];
-            const uint32_t j = __float_as_uint(s.w);
-            const float p[3] = {s.x, s.y, s.z};
-            float r2 = 0.f, far = 0.f;
-            for (int q = 0; q < 3; ++q) {
-              const float dv = po[q] - p[q];
-              const float n = rintf(dv * A.inv_ext[q]);
-              const float d = dyn_fmaf(-n, A.ext[q], dv);
-              r2 = dyn_fmaf(d, d, r2);
-              far = fmaxf(far, fabsf(n));
+  if (PASS == 1) {
+    for (uint32_t k = lane; k < A.words; k += 64) bits[k] = 0u;
+    __syncthreads();
+  }
+  for (int ox = -A.use_nb[0]; ox <= A.use_nb[0]; ++ox)
+    for (int oy = -A.use_nb[1]; oy <= A.use_nb[1]; ++oy) {
+      const int x = (cc[0] + ox + A.G.nc[0]) % A.G.nc[0];
+      const int y = (cc[1] + oy + A.G.nc[1]) % A.G.nc[1];
+      const uint32_t c = (uint32_t)((x * A.G.nc[1] + y) * nz);
+      for (int r = 0; r < runs; ++r) {
+        // [z0, z1) within [0, nz), and what wraps
+        const int a = r == 0 ? max(z0, 0) : (z0 < 0 ? z0 + nz : 0);
+        const int b = r == 0 ? min(z1, nz) : (z0 < 0 ? nz : z1 - nz);
+        const uint32_t k1 = A.cell_start[c + b];
+        for (uint32_t k = A.cell_start[c + a] + lane; k < k1; k += 64) {
+          const float4 s = A.sorted[k];
+          const uint32_t j = __float_as_uint(s.w);
+          const float p[3] = {s.x, s.y, s.z};
+          float r2 = 0.f, far = 0.f;
+          for (int q = 0; q < 3; ++q) {
+            const float dv = po[q] - p[q];
+            const float n = rintf(dv * A.inv_ext[q]);
+            const float d = dyn_fmaf(-n, A.ext[q], dv);
+            r2 = dyn_fmaf(d, d, r2);
+            far = fmaxf(far, fabsf(n));
+          }
+          bool ok = r2 < A.lo;
+          // (not a number: the exact test)
+          if (!(far <= 8.f && (r2 < A.lo || r2 > A.hi))) ok = nbl_accept(po, p, A.ext, A.thr);
+          if (A.symmetric && j == i) ok = false;
+          if (A.is_static && st_i && ok && A.is_static[j]) ok = false;
+          if (PASS == 1) {
+            if (ok) atomicOr(&bits[j >> 5], 1u << (j & 31u));
+          } else {
+            const unsigned long long m = __ballot(ok);
+            if (PASS == 2 && ok) {
+              const uint32_t at = found + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+              if (at < (uint32_t)kNblCap) bits[at] = j;
             }
-            bool ok = r2 < A.lo;
-            // (not a number: the exact test)
-            if (!(far <= 8.f && (r2 < A.lo || r2 > A.hi))) ok = nbl_accept(po, p, A.ext, A.thr);
-            if (A.symmetric && j == i) ok = false;
-            if (A.is_static && st_i && ok && A.is_static[j]) ok = false;
-            if (PASS == 0) {
-              found += (uint32_t)__popcll(__ballot(ok));
-            } else if (ok && j >= r0 && j - r0 < A.range) {
-              const uint32_t at = j - (uint32_t)r0;
-              atomicOr(&bits[at >> 5], 1u << (at & 31u));
-            }
+            found += (uint32_t)__popcll(m);
           }
         }
+        // (a lane counts the ballots of the loop trips it took part in: lane 0
+        // took part in all of them)
+        if (PASS != 1) found = (uint32_t)__builtin_amdgcn_readfirstlane((int)found);
       }
-    if (PASS == 1) {
-      __syncthreads();
-      for (uint32_t w0 = 0; w0 < words; w0 += 64) {
-        uint32_t v = w0 + lane < words ? bits[w0 + lane] : 0u;
-        const uint32_t c = (uint32_t)__popc(v), inc = wave_scan_u32(c);
-        uint32_t* __restrict__ o = col + out + (inc - c);
-        const uint32_t j0 = (uint32_t)r0 + 32 * (w0 + lane);
-        while (v) {
-          *o++ = j0 + (uint32_t)__ffs((int)v) - 1u;
-          v &= v - 1u;
+    }
+  if (PASS == 0) {
+    if (lane == 0) row_count[i] = found;
+    return;
+  }
+  __syncthreads();
+  uint32_t out = row_ptr[i];
+  if (PASS == 1) {
+    for (uint32_t w0 = 0; w0 < A.words; w0 += 64) {
+      uint32_t v = w0 + lane < A.words ? bits[w0 + lane] : 0u;
+      const uint32_t c = (uint32_t)__popc(v), inc = wave_scan_u32(c);
+      uint32_t* __restrict__ o = col + out + (inc - c);
+      const uint32_t j0 = 32 * (w0 + lane);
+      while (v) {
+        *o++ = j0 + (uint32_t)__ffs((int)v) - 1u;
+        v &= v - 1u;
+      }
+      out += __shfl(inc, 63, 64);
+    }
+    return;
+  }
+  // a bitonic sort by the wave, padded to a power of two
+  const uint32_t m = min(found, (uint32_t)kNblCap);
+  uint32_t np2 = 1;
+  while (np2 < m) np2 <<= 1;
+  for (uint32_t k = m + lane; k < np2; k += 64) bits[k] = 0xffffffffu;
+  __syncthreads();
+  for (uint32_t size = 2; size <= np2; size <<= 1)
+    for (uint32_t step = size >> 1; step > 0; step >>= 1) {
+      for (uint32_t t = lane; t < np2 / 2; t += 64) {
+        const uint32_t a = 2 * t - (t & (step - 1)), b = a + step;
+        const uint32_t u = bits[a], v = bits[b];
+        if ((u > v) == ((a & size) == 0)) {
+          bits[a] = v;
+          bits[b] = u;
         }
-        out += __shfl(inc, 63, 64);
       }
       __syncthreads();
     }
-  }
-  // (a lane counts the ballots of the loop trips it took part in: lane 0
-  // took part in all of them)
-  if (PASS == 0 && lane == 0) row_count[i] = found;
+  for (uint32_t k = lane; k < m; k += 64) col[out + k] = bits[k];
 }
 
 }  // namespace
@@ -1052,8 +1081,7 @@ extern "C" int dyn_nb_build_neighbors(dyn_nb_ctx* ctx, const float* posits_outer
     A.lo = (float)((double)A.thr - slack);
     A.hi = (float)((double)A.thr + slack);
     A.symmetric = symmetric ? 1 : 0;
-    A.n_inner = n_inner;
-    A.range = std::min(kNblBits, (n_inner + 2047u) & ~2047u);
+    A.words = (n_inner + 31u) / 32u;
     hipLaunchKernelGGL(k_nbl_rows<0>, dim3(n_outer), dim3(64), 0, ctx->stream, A,
                        n_outer, ctx->nb_row_count.p, (const uint32_t*)nullptr,
                        (uint32_t*)nullptr);
@@ -1076,9 +1104,13 @@ extern "C" int dyn_nb_build_neighbors(dyn_nb_ctx* ctx, const float* posits_outer
     if (total == 0) return DYN_OK;
     DYN_REQUIRE(col_idx, "col_idx is null");
     ctx->nb_col.reserve(total);
-    hipLaunchKernelGGL(k_nbl_rows<1>, dim3(n_outer), dim3(64), A.range / 8, ctx->stream, A,
-                       n_outer, (uint32_t*)nullptr, ctx->nb_row_ptr.p, ctx->nb_col.p);
-    DYN_CHECK_LAUNCH("k_nbl_rows<1>");
+    const bool sorts = n_inner > kNblBits;
+    uint32_t slots = 1;  // of the sort, the longest row's
+    while (slots < maxrow) slots <<= 1;
+    hipLaunchKernelGGL(sorts ? k_nbl_rows<2> : k_nbl_rows<1>, dim3(n_outer), dim3(64),
+                       sorts ? 4 * slots : 4 * A.words, ctx->stream, A, n_outer, (uint32_t*)nullptr,
+                       ctx->nb_row_ptr.p, ctx->nb_col.p);
+    DYN_CHECK_LAUNCH("k_nbl_rows");
     copy_out(ctx, col_idx, ctx->nb_col.p, total);
   });
 }

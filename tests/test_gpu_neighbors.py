@@ -93,3 +93,22 @@ def test_neighbor_rows_sizes(gpu, n_outer, n_inner, ext, radius, spread):
     ctx = api.ForcesPositsGpu(n_outer, 0, 10.0, 0.3)
     _check(ctx, po, pi, None, e, False, np.float32(radius * radius))
     _check(ctx, po, po, (np.arange(n_outer) % 3 == 0).astype(np.uint8), e, True, np.float32(radius * radius))
+
+
+@pytest.mark.parametrize("n_outer,n_inner,ext,radius", [
+    (70, 32_768, 60.0, 6.0), (70, 32_769, 60.0, 6.0),  # bitmap and sort
+    (40, 33_000, 30.0, 9.0),      # rows of nearly 4,096
+    (200, 40_000, 1500.0, 10.0),  # rows of none to a few
+    (64, 65_537, 120.0, 7.0),
+])
+def test_neighbor_rows_sorted(gpu, n_outer, n_inner, ext, radius):
+    """Rows of many inner points, put in order by a sort, equal the
+    brute-force lists; those of the bitmap's largest set too."""
+    rng = np.random.default_rng(n_inner)
+    po = rng.uniform(0, ext, (n_outer, 3)).astype(np.float32)
+    pi = rng.uniform(0, ext, (n_inner, 3)).astype(np.float32)
+    pi[:n_outer:3] = po[::3] + np.array([0, radius, 0], np.float32)
+    e = np.full(3, ext, np.float32)
+    print(f"neighbors: {n_outer} x {n_inner}, box {ext}, radius {radius}", flush=True)
+    ctx = api.ForcesPositsGpu(n_outer, 0, 10.0, 0.3)
+    _check(ctx, po, pi, None, e, False, np.float32(radius * radius))
