@@ -330,6 +330,13 @@ DYN_HD float dyn_rcpf(float x) {
 // 0.3123/Å) take φ(x) and erfc(x) over x = βr on [0, 4]: DYN_COUL_X_N cubic
 // Hermite pieces each (error ≤ h⁴/384·max|f⁗| ≈ 1e-10, h = 1/128).
 //
+// A small β would leave most pairs below the first octave (at 0.005/Å all
+// within 4.4 Å).  The tables are then over y = b²r² with b = 2ᵏβ, and hold
+// 2⁻³ᵏΨ(y/4ᵏ) and 2⁻ᵏΛ(y/4ᵏ): s = qq·b³·(entry), E = qq·b·(entry) as before.
+// k = dyn_coul_tab_shift(β, cutoff) is 0 from β·cutoff = 0.5 on and the least
+// that brings b·cutoff there below, so the first octave ends at 0.044 cutoffs at
+// most.
+//
 // Layout: two halves of DYN_COUL_TAB_N entries, the forces' (φ by x, then Ψ
 // by y) and the energies' (erfc by x, then Λ by y).
 #define DYN_COUL_X_N 512
@@ -353,7 +360,7 @@ DYN_HD float dyn_tab_cubic(const float4* tab, int entry_off, float x) {
   return dyn_tab_cubic_u(tab, entry_off, x * DYN_COUL_TAB_SCALE);
 }
 
-// An entry times a factor (β³ of the forces, β of the energies).
+// An entry times a factor (b³ of the forces, b of the energies).
 DYN_HD float4 dyn_tab_scale(float4 c, float f) {
   c.x *= f;
   c.y *= f;
@@ -383,10 +390,17 @@ DYN_HD float dyn_tab_y(const float4* ytab, float y, float f) {
   return dyn_fmaf(dyn_fmaf(dyn_fmaf(c.w, t, c.z), t, c.y), t, c.x);
 }
 
-// r² below which a pair's y = r²β² may lie below the y tables (with room for
+// r² below which a pair's y = r²b² may lie below the y tables (with room for
 // the product's rounding); never below the r² of coincident sites.
-DYN_HD float dyn_coul_r2_lo(float beta2) {
-  return dyn_maxf(1e-16f, 1.0001f * DYN_COUL_Y_MIN / beta2);
+DYN_HD float dyn_coul_r2_lo(float b2) {
+  return dyn_maxf(1e-16f, 1.0001f * DYN_COUL_Y_MIN / b2);
+}
+
+// The k of the y tables (see above; a host function), β > 0.
+static inline int dyn_coul_tab_shift(float beta, float cutoff) {
+  int k = 0;
+  while (ldexp((double)beta, k) * (double)cutoff < 0.5) ++k;
+  return k;
 }
 
 // The x tables' form, for pairs below the y tables.
@@ -398,23 +412,22 @@ DYN_HD void dyn_coul_erfc_close(float r2, float qq, float beta, const float4* ta
   *e = qq * rinv * dyn_tab_cubic_u(tab, 1, u);
 }
 
-// The tabulated pair at any r² (both forms; rinv = 1/r is not needed).
-DYN_HD void dyn_coul_erfc_tab(float r2, float rinv, float qq, float beta, const float4* tab,
-                              float* s, float* e) {
-  const float beta2 = beta * beta;
-  (void)rinv;
-  if (!(r2 > dyn_coul_r2_lo(beta2))) {
+// The tabulated pair at any r² (both forms; b = 2ᵏβ).
+DYN_HD void dyn_coul_erfc_tab(float r2, float qq, float beta, float b, const float4* tab, float* s,
+                              float* e) {
+  const float b2 = b * b;
+  if (!(r2 > dyn_coul_r2_lo(b2))) {
     dyn_coul_erfc_close(r2, qq, beta, tab, s, e);
     return;
   }
-  const float y = r2 * beta2;
-  *s = qq * dyn_tab_y<false>(tab + DYN_COUL_X_N, y, beta2 * beta);
-  *e = qq * dyn_tab_y<false>(tab + DYN_COUL_TAB_N + DYN_COUL_X_N, y, beta);
+  const float y = r2 * b2;
+  *s = qq * dyn_tab_y<false>(tab + DYN_COUL_X_N, y, b2 * b);
+  *e = qq * dyn_tab_y<false>(tab + DYN_COUL_TAB_N + DYN_COUL_X_N, y, b);
 }
 
-// The table (2·DYN_COUL_TAB_N float4 as 8·DYN_COUL_TAB_N floats), built on
-// the host in double from the closed forms (a host function).
-static inline void dyn_coul_tab_build(float* out) {
+// The table (2·DYN_COUL_TAB_N float4 as 8·DYN_COUL_TAB_N floats) of shift k,
+// built on the host in double from the closed forms (a host function).
+static inline void dyn_coul_tab_build(float* out, int shift) {
   const double k2 = 1.1283791670955126;  // 2/√π
   // the Hermite piece over an interval of width h, in t = argument − lower
   // end times sc
@@ -433,10 +446,11 @@ static inline void dyn_coul_tab_build(float* out) {
     const double er = erfc(x), ex = exp(-x * x);
     return Node{er + k2 * x * ex, -2.0 * k2 * x * x * ex, er, -k2 * ex};
   };
+  const double down3 = ldexp(1.0, -3 * shift);
   auto node_y = [&](double y) {
-    const double x = sqrt(y), er = erfc(x), ex = exp(-y);
-    const double psi = (er + k2 * x * ex) / (y * x);
-    return Node{psi, (-k2 * ex - 1.5 * psi) / y, er / x, -0.5 * psi};
+    const double w = sqrt(y), x = ldexp(w, -shift), er = erfc(x), ex = exp(-x * x);
+    const double psi = (er + k2 * x * ex) / (y * w);
+    return Node{psi, (-k2 * ex * down3 - 1.5 * psi) / y, er / w, -0.5 * psi};
   };
   auto put = [&](int at, const Node& a, const Node& b, double h, double sc) {
     piece(out + 4 * at, a.f, b.f, a.df, b.df, h, sc);

@@ -67,11 +67,12 @@ struct DynPairParams {
   int n_types;      // LJ type tables are (n_types × n_types) float2
   int alch_on;      // a decoupled molecule exists
   DynSchedule sch;  // staged decoupling schedule at the current λ
+  float tab_b, tab_b2;     // the b of its y tables, b²
   const float4* coul_tab;  // the erfc Coulomb table (dyn_coul_tab_build)
 };
 
-// The two Coulomb tables a lane reads (dyn_math.h): Ψ and Λ over y = β²r².
-// The pair kernel reads copies in LDS, multiplied by β³ and β (etab is not
+// The two Coulomb tables a lane reads (dyn_math.h): Ψ and Λ over y = b²r².
+// The pair kernel reads copies in LDS, multiplied by b³ and b (etab is not
 // read by a forces-only evaluation).
 struct DynCoulTabs {
   const float4 *ftab, *etab;
@@ -83,9 +84,9 @@ DYN_HD DynCoulTabs dyn_coul_tabs(const float4* coul_tab) {
 // The pair (i, j) of the given kind at squared distance r2: the scalar s
 // (F_i = s·d) and energies, zero for an inactive lane.  `active` already
 // includes the list mask; the cutoff test happens here.  r2_lo =
-// dyn_coul_r2_lo(β²).  No square root or reciprocal of r² is taken for
-// Coulomb pairs (tabulated over β²r²); LJ takes 1/r² directly.  SCALED: tabs
-// holds the tables multiplied by β³ and β.  Returns whether the pair interacts but lies below
+// dyn_coul_r2_lo(b²).  No square root or reciprocal of r² is taken for
+// Coulomb pairs (tabulated over b²r²); LJ takes 1/r² directly.  SCALED: tabs
+// holds the tables multiplied by b³ and b.  Returns whether the pair interacts but lies below
 // the Coulomb tables: then s and the energies are not set, and
 // dyn_tile_close gives them.
 template <int KIND, bool SCALED>
@@ -101,10 +102,10 @@ DYN_HD bool dyn_tile_eval(float r2, float qi, float qj, float c6, float c12, boo
   float s = 0.f, elj = 0.f, ec = 0.f;
   if (kLj) dyn_lj(dyn_rcpf(r2), c6, c12, &s, &elj);
   if (kCoul) {
-    const float y = r2 * P.beta2;
+    const float y = r2 * P.tab_b2;
     const float qq = qi * qj;
-    const float sc = qq * dyn_tab_y<SCALED>(tabs.ftab, y, P.beta2 * P.beta);
-    ec = qq * dyn_tab_y<SCALED>(tabs.etab, y, P.beta);
+    const float sc = qq * dyn_tab_y<SCALED>(tabs.ftab, y, P.tab_b2 * P.tab_b);
+    ec = qq * dyn_tab_y<SCALED>(tabs.etab, y, P.tab_b);
     s = kLj ? (r2 <= P.lj_rc2 ? sc + s : sc) : sc;
     *s_out = in ? s : 0.f;
     *e_lj = kLj && lj_in ? elj : 0.f;
@@ -154,7 +155,7 @@ DYN_HD void dyn_tile_pair(const float pi[4], int ti, const float pj[4], int tj, 
   for (int a = 0; a < 3; ++a) d[a] = dyn_min_image_rint(pi[a] - pj[a], P.ext[a], P.inv_ext[a]);
   const float r2 = dyn_fmaf(d[2], d[2], dyn_fmaf(d[1], d[1], d[0] * d[0]));
   const float2 c = dyn_tile_c<KIND>(ti, tj, P, lj_table);
-  if (dyn_tile_eval<KIND, false>(r2, pi[3], pj[3], c.x, c.y, active, dyn_coul_r2_lo(P.beta2), P,
+  if (dyn_tile_eval<KIND, false>(r2, pi[3], pj[3], c.x, c.y, active, dyn_coul_r2_lo(P.tab_b2), P,
                                  dyn_coul_tabs(P.coul_tab), s_out, e_lj, e_c, hit))
     dyn_tile_close<KIND>(r2, pi[3], pj[3], c.x, c.y, P, s_out, e_lj, e_c, hit);
   *r2_out = *hit ? r2 : 0.f;

@@ -1257,7 +1257,7 @@ __device__ __forceinline__ bool tile_fast(float r2, float qi, float qj, const fl
   float s = 0.f, elj = 0.f, ec = 0.f;
   if (kLj) dyn_lj(dyn_rcpf(r2), c.x, c.y, &s, &elj);
   if (kCoul) {
-    const float y = r2 * P.beta2, qq = qi * qj;
+    const float y = r2 * P.tab_b2, qq = qi * qj;
     const float sc = qq * dyn_tab_y<true>(tabs.ftab, y, 0.f);
     ec = qq * dyn_tab_y<true>(tabs.etab, y, 0.f);
     s = kLj ? (r2 <= P.lj_rc2 ? sc + s : sc) : sc;
@@ -1687,7 +1687,7 @@ __device__ __forceinline__ TileI tile_i(const PairArgs& A, uint32_t row, int ia)
   I.p[1] = p.y;
   I.p[2] = p.z;
   I.p[3] = p.w;
-  I.r2_lo = dyn_coul_r2_lo(A.P.beta2);
+  I.r2_lo = dyn_coul_r2_lo(A.P.tab_b2);
   I.t = A.slot_type[slot];
   I.g = A.slot_gid[slot];
   I.ci = A.cl_class[row];
@@ -1702,7 +1702,7 @@ __device__ __forceinline__ TileI tile_i(const PairArgs& A, uint32_t row, int ia)
 // Bound: VALU issue (85% of the cycles at 252,480 sites, 33 instructions a
 // group of 64 pairs in the forces variant; LDS and memory stay below half of
 // theirs).  So what a pair does was cut to the least: the Coulomb force is
-// one table value over β²r² (no square root, no reciprocal), 1/r² of LJ an
+// one table value over b²r² (no square root, no reciprocal), 1/r² of LJ an
 // integer guess and a Newton step, minimum images are taken per j site of a
 // batch instead of per pair, and the j site reaches the lanes as DPP operands
 // (tile_item).  Per-lane table reads from LDS are counted apart from the global
@@ -1722,7 +1722,7 @@ __device__ __forceinline__ TileI tile_i(const PairArgs& A, uint32_t row, int ia)
 template <bool ENERGY, bool ALCH>
 __device__ __forceinline__ void
 k_eng_pairs(PairArgs A) {
-  // the Coulomb tables over y (β³Ψ, and βΛ with energies; at offset 0, so a
+  // the Coulomb tables over y (b³Ψ, and bΛ with energies; at offset 0, so a
   // lane's table address is its entry's offset) and the row's forces (two
   // buffers); in FP32 the LJ (c6, c12) table of n_types² entries follows
   __shared__ float4 s_tab[(ENERGY ? 2 : 1) * DYN_COUL_Y_N];
@@ -1736,8 +1736,8 @@ k_eng_pairs(PairArgs A) {
   if (blockIdx.x >= n_cl) return;
   const DynCoulTabs src = dyn_coul_tabs(A.P.coul_tab);
   for (int k = threadIdx.x; k < DYN_COUL_Y_N; k += kPairBlock) {
-    s_tab[k] = dyn_tab_scale(src.ftab[k], A.P.beta2 * A.P.beta);
-    if (ENERGY) s_tab[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], A.P.beta);
+    s_tab[k] = dyn_tab_scale(src.ftab[k], A.P.tab_b2 * A.P.tab_b);
+    if (ENERGY) s_tab[DYN_COUL_Y_N + k] = dyn_tab_scale(src.etab[k], A.P.tab_b);
   }
   const int nt2 = A.P.n_types * A.P.n_types;
   for (int k = threadIdx.x; k < nt2; k += kPairBlock) s_lj[k] = A.lj_table[k];
@@ -2708,6 +2708,8 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
     P.alch_on = pl.alch_on ? 1 : 0;
     P.sch = dyn_schedule((float)e.lambda);
     P.coul_tab = e.coul_tab.p;
+    P.tab_b = (float)std::ldexp((double)e.prm.beta, dyn_coul_tab_shift(e.prm.beta, e.prm.cutoff));
+    P.tab_b2 = P.tab_b * P.tab_b;
     // the reference's SPME cadence: keep the last SPME forces, energy and
     // virial (reference mode, no decoupled molecule, same box)
     pl.reuse = e.pme_on && (flags & DYN_COMPUTE_RECIP_REUSE) && !(flags & DYN_COMPUTE_RECIP) &&
@@ -3311,7 +3313,7 @@ extern "C" int dyn_engine_create(dyn_engine** out, int device, const dyn_engine_
     }
     {
       std::vector<float4> tab(2 * DYN_COUL_TAB_N);
-      dyn_coul_tab_build(reinterpret_cast<float*>(tab.data()));
+      dyn_coul_tab_build(reinterpret_cast<float*>(tab.data()), dyn_coul_tab_shift(p.beta, p.cutoff));
       E->coul_tab.reserve(tab.size());
       DYN_HIP(hipMemcpyAsync(E->coul_tab.p, tab.data(), sizeof(float4) * tab.size(),
                              hipMemcpyHostToDevice, E->stream));

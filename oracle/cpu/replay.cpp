@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <vector>
 
 #include "dyn_math.h"
@@ -30,19 +31,26 @@ void orc_coul_erfc(float r2, float qq, float beta, float* s, float* e) {
   const float rinv = dyn_rsqrtf(r2);
   dyn_coul_erfc(r2, rinv, qq, beta, beta * beta, 2.0f * beta * DYN_INV_SQRT_PI, s, e);
 }
-// The pair tiles' tabulated erfc Coulomb (dyn_coul_erfc_tab) and its table.
-static const float4* coul_table() {
-  static std::vector<float> tab;
+// The pair tiles' tabulated erfc Coulomb (dyn_coul_erfc_tab) and its table
+// of shift k.
+static const float4* coul_table(int k = 0) {
+  static std::map<int, std::vector<float>> tabs;
+  std::vector<float>& tab = tabs[k];
   if (tab.empty()) {
     tab.resize(8 * DYN_COUL_TAB_N);
-    dyn_coul_tab_build(tab.data());
+    dyn_coul_tab_build(tab.data(), k);
   }
   return reinterpret_cast<const float4*>(tab.data());
 }
 void orc_coul_erfc_tab(float r2, float qq, float beta, float* s, float* e) {
-  const float rinv = dyn_rsqrtf(r2);
-  dyn_coul_erfc_tab(r2, rinv, qq, beta, coul_table(), s, e);
+  dyn_coul_erfc_tab(r2, qq, beta, beta, coul_table(), s, e);
 }
+// The same with the table an engine of this cutoff takes.
+void orc_coul_erfc_tab_cutoff(float r2, float qq, float beta, float cutoff, float* s, float* e) {
+  const int k = dyn_coul_tab_shift(beta, cutoff);
+  dyn_coul_erfc_tab(r2, qq, beta, (float)ldexp((double)beta, k), coul_table(k), s, e);
+}
+float orc_rcpf(float x) { return dyn_rcpf(x); }
 // The two tabulated functions at x: φ(x) and erfc(x).
 void orc_coul_tab_eval(float x, float* phi, float* erfc_x) {
   *phi = dyn_tab_cubic(coul_table(), 0, x);
@@ -201,12 +209,10 @@ void orc_engine_tiles(const float* xyzq, const int32_t* slot_type, const int32_t
   P.n_types = n_types;
   P.alch_on = alch_on;
   P.sch = dyn_schedule(lambda);
-  static std::vector<float> coul_tab;
-  if (coul_tab.empty()) {
-    coul_tab.resize(8 * DYN_COUL_TAB_N);
-    dyn_coul_tab_build(coul_tab.data());
-  }
-  P.coul_tab = reinterpret_cast<const float4*>(coul_tab.data());
+  const int k = dyn_coul_tab_shift(beta, cutoff);
+  P.tab_b = (float)ldexp((double)beta, k);
+  P.tab_b2 = P.tab_b * P.tab_b;
+  P.coul_tab = coul_table(k);
   const float2* lj = reinterpret_cast<const float2*>(lj_table);
   const float2* lse = reinterpret_cast<const float2*>(lj_se_table);
   memset(fx, 0, sizeof(int64_t) * 3 * n_slots);

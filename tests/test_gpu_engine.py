@@ -109,6 +109,24 @@ def test_pair_tile_images_and_remainders(gpu, cases, cutoff, close):
     eng.close()
 
 
+@pytest.mark.parametrize("beta", [0.049, 0.011, 1e-3, 1e-20])
+def test_small_beta(gpu, cases, beta):
+    """β down to a plain cutoff Coulomb sum: the tables reach the pairs
+    within the cutoff (their y range follows β), fixed-point sums equal the
+    replay's and forces the FP64 sum."""
+    s = cases["solvated"]
+    b = float(np.float32(beta))
+    print(f"small beta: {beta}", flush=True)
+    eng = _engine(s, beta=b)
+    eng.compute(api.COMPUTE_SHORT | api.COMPUTE_CORR)
+    assert rel_rms(eng.site_forces(), fp64.pair_sum_fp64(s, RC, RC, b)["forces"]) <= 1e-5
+    dbg = eng.debug_export()
+    fx, _, ie = replay_engine_tiles(dbg, s, RC, RC, b, per_item=True)
+    assert np.array_equal(fx, dbg["fx_slot"])
+    _check_item_sums(eng, dbg, ie)
+    eng.close()
+
+
 def _check_item_sums(eng, dbg, ie):
     """Per work item energies, virial and dH/dλ against the host replay: a
     sum the replay leaves at zero (e.g. a solute energy of a water-only item)

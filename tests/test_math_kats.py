@@ -206,6 +206,27 @@ def test_coulomb_table_accuracy():
     assert max(re) < 3e-7, max(re)
 
 
+@pytest.mark.parametrize("beta", [0.3123, 0.051, 0.049, 0.011, 1e-3, 1e-5, 1e-12, 1e-30])
+def test_coulomb_table_of_any_beta(beta):
+    """The table an engine with a 10 Å cutoff takes, from 0.5 Å (beyond the
+    closed form for close pairs at every β) to the cutoff."""
+    L = oracle_lib()
+    f = C.c_float
+    L.orc_coul_erfc_tab_cutoff.argtypes = [f, f, f, f, C.POINTER(f), C.POINTER(f)]
+    b = float(np.float32(beta))
+    s, e = f(), f()
+    for r in np.linspace(0.5, 9.99, 400):
+        r2 = float(np.float32(r * r))
+        r = math.sqrt(r2)
+        L.orc_coul_erfc_tab_cutoff(r2, -200.0, b, 10.0, C.byref(s), C.byref(e))
+        e_an = -200.0 * erfc(b * r) / r
+        s_an = e_an / r2 - 200.0 * 2 * b / math.sqrt(math.pi) * math.exp(-(b * r) ** 2) / r2
+        # f32 rounding of y (~1e-7) times |d ln s/d ln y| ≤ 1.5 + x² = 11, and
+        # half as much again for the cubic's own operations
+        assert abs(s.value - s_an) <= 2e-6 * abs(s_an), (beta, r)
+        assert abs(e.value - e_an) <= 2e-6 * abs(e_an), (beta, r)
+
+
 @pytest.mark.parametrize("form", COUL_FORMS)
 def test_coulomb_short_range_direction(form):
     """tests/forces.rs:428-462: like charges repel, opposite attract."""
