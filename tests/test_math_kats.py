@@ -206,6 +206,20 @@ def test_coulomb_table_accuracy():
     assert max(re) < 3e-7, max(re)
 
 
+def test_reciprocal_accuracy():
+    """dyn_rcpf (1/r² of the pair kernel's LJ): relative error at most 1.3e-7
+    over the pair distances, and over the r² a tile lane may hold, from
+    coincident sites to slots that pair with nothing."""
+    L = oracle_lib()
+    L.orc_rcpf.argtypes, L.orc_rcpf.restype = [C.c_float], C.c_float
+    rng = np.random.default_rng(1)
+    mant = np.concatenate([np.linspace(1.0, 2.0, 4001), 1.0 + rng.random(4000)])
+    xs = [np.float32(m * 2.0 ** k) for k in (-3, 0, 1, 4, 7) for m in mant]  # r up to 16 Å
+    xs += [np.float32(x) for x in np.geomspace(1e-16, 4.1e36, 4001)]
+    err = max(abs(float(L.orc_rcpf(x)) * float(x) - 1.0) for x in xs)
+    assert err <= 1.3e-7, err
+
+
 @pytest.mark.parametrize("beta", [0.3123, 0.051, 0.049, 0.011, 1e-3, 1e-5, 1e-12, 1e-30])
 def test_coulomb_table_of_any_beta(beta):
     """The table an engine with a 10 Å cutoff takes, from 0.5 Å (beyond the
