@@ -1899,21 +1899,18 @@ struct PrepArgs {
   uint32_t unused;    // no implicit padding: argument packs are compared byte for byte
 };
 
-// A pass of more than kPrepLate and at most kPrepEarly sites (of all its
-// systems) prepares its SPME charges by a launch of its own at the head of the
-// second stream, others by further workgroups of the evaluation's first launch.
-// Small passes wait for the second stream, which then starts with the spread: 20
-// MD steps of 2,000 sites 1564 -> 1464 µs, of 28,000 2334 -> 2195.  Medium ones
-// wait for the main stream, where the first launch takes 3.4 µs longer with the
-// charges: 37,000 sites, 140.4 µs a step with them, 136.2 without.  In large ones
-// the pair kernel has no room for a launch beside it: 252,480 sites 7860 µs a
-// run with the charges in the first launch, 8036 apart; 16 windows, 134,000 sites,
-// 9060 and 9200; 32 boxes, 126,000, 6645 and 6720.
-constexpr uint32_t kPrepLate = 32768, kPrepEarly = 65536;
-
 // The SPME charges of an evaluation that runs SPME: their wrapped positions
 // (and the second evaluation's charges), their listing under the grid
-// bricks, and the cleared SPME force sums.
+// bricks, and the cleared SPME force sums.  By further workgroups of the
+// evaluation's first launch: the second stream then starts with the spread.  20 MD
+// steps of 2,000 sites 1564 -> 1464 µs, of 28,000 2334 -> 2195 (with a launch of
+// their own at the head of the second stream before).  A step of a box of water,
+// 9 and 10 Å cutoff, in µs, a launch of their own and this: 16,384 sites 89.8 and
+// 92.3, 81.9 and 84.4; 35,200 110.4 and 114.2, 104.6 and 112.0; 50,688 129.5 and
+// 137.2, 127.5 and 137.6; 64,896 155 and 167, 148 and 161; 256,000 411 and 463,
+// 405 and 457; 5 boxes of 6,912 121.9, 120.4; 12 215, 210.  Of all systems measured
+// only the 37,000-site solvated chain, whose main stream is the longer one, is
+// slower (1,183 ns/day against 1,208).
 struct PmePrepArgs {
   const float4* pos;
   const float* q;
@@ -1950,8 +1947,6 @@ __device__ __forceinline__ void pme_prep(const PmePrepArgs& A, uint32_t block) {
   pme_bin_charge(A.bin, p, qv);
 }
 
-__device__ __forceinline__ void k_eng_pme_prep(const PmePrepArgs& Q) { pme_prep(Q, blockIdx.x); }
-
 // The exclusion and 1-4 corrections (n_corr blocks) and the bonded terms of an
 // evaluation without SPME on their stream (its spread launch takes them
 // otherwise).  Both are a few dependent memory latencies and little else, so
@@ -1985,7 +1980,7 @@ __device__ __forceinline__ void copy_grid(T* __restrict__ dst, const T* __restri
 // the taken staged list the current one for good.
 //
 // Its first A.blocks workgroups prepare the SPME charges beside this (see
-// kPrepLate): both are chains of a few memory latencies.
+// PmePrepArgs): both are chains of a few memory latencies.
 __device__ __forceinline__ void k_eng_prep(const PrepArgs& A, const PmePrepArgs& Q) {
   __shared__ unsigned int red[256 / kWave];
   if (blockIdx.x < A.blocks) {
@@ -2729,40 +2724,14 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
     any_b = any_b || pl.recip_b;
     any_corr = any_corr || pl.corr_on;
   }
-  // the SPME charges: in the first launch, or by one of their own (kPrepLate)
-  uint64_t all_sites = 0;
-  for (uint32_t i = 0; i < ns; ++i) all_sites += E[i]->n_sites;
-  const bool prep_late = all_sites > kPrepLate && all_sites <= kPrepEarly;
-  const unsigned n_prep = !any_recip ? 0u : max_grid(S, [](dyn_engine& e) {
+  const unsigned np = !any_recip ? 0u : max_grid(S, [](dyn_engine& e) {
     return std::max(grid_for(e.n_sites, 256), grid_for(e.n_q, 256));
   });
-  auto prep_args = [&](uint32_t i) {
-    dyn_engine& e = *E[i];
-    const Plan& pl = PL[i];
-    PmePrepArgs Q;
-    std::memset(&Q, 0, sizeof Q);
-    if (pl.recip_on) {  // (a system without SPME this evaluation: nothing to do)
-      Q.pos = e.pos_dev;
-      Q.q = e.q.p;
-      Q.g = e.geom;
-      Q.qsite = e.qsite.p;
-      Q.nq = e.n_q;
-      Q.alch0 = e.alch0;
-      Q.alch1 = e.alch1;
-      Q.pme_xyzq = e.pme_xyzq.p;
-      Q.pme_b = pl.recip_b ? e.pme_b.p : nullptr;
-      Q.fx_recip = e.fx_recip.p;
-      e.pme.ensure_cap(e.n_q);
-      Q.bin = e.pme.bin_args(e.status.p, kStPme);
-    }
-    return Q;
-  };
   {
     Profiler::Scope ps(prof, "prep");
     const unsigned gp = max_grid(S, [](dyn_engine& e) {
       return std::max(grid_for(e.n_sites, 256), grid_for(e.cap_slots, 256));
     });
-    const unsigned np = prep_late ? 0u : n_prep;
     launch<k_eng_prep>(R, "k_eng_prep", 0, np + gp, 256, 0, [&](uint32_t i) {
       dyn_engine& e = *E[i];
       const Plan& pl = PL[i];
@@ -2784,7 +2753,20 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
       A.stride = gp * 256u;
       PmePrepArgs Q;
       std::memset(&Q, 0, sizeof Q);
-      if (np) Q = prep_args(i);
+      if (pl.recip_on) {  // (a system without SPME this evaluation: nothing to do)
+        Q.pos = e.pos_dev;
+        Q.q = e.q.p;
+        Q.g = e.geom;
+        Q.qsite = e.qsite.p;
+        Q.nq = e.n_q;
+        Q.alch0 = e.alch0;
+        Q.alch1 = e.alch1;
+        Q.pme_xyzq = e.pme_xyzq.p;
+        Q.pme_b = pl.recip_b ? e.pme_b.p : nullptr;
+        Q.fx_recip = e.fx_recip.p;
+        e.pme.ensure_cap(e.n_q);
+        Q.bin = e.pme.bin_args(e.status.p, kStPme);
+      }
       return args<k_eng_prep>(A, Q);
     });
   }
@@ -2799,11 +2781,6 @@ void engine_set_enqueue(EngineSet& S, uint32_t flags, const SideWork* side) {
   // kernel at once and would take the compute units the FFT planes need —
   // before the pair kernel on the main stream
   const BatchRun& RP = staged_mode ? R : RS;
-  if (n_prep && prep_late) {
-    Profiler::Scope ps(prof, "pme_prep");
-    launch<k_eng_pme_prep>(RP, "k_eng_pme_prep", 0, n_prep, 256, 0,
-                           [&](uint32_t i) { return args<k_eng_pme_prep>(prep_args(i)); });
-  }
   // the exclusion and 1-4 corrections (site accumulators; finalize reads
   // them) and the caller's bonded terms ride in the spread launch of an SPME
   // sum on the same stream; without one they are a launch of their own
