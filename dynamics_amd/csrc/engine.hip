@@ -506,7 +506,7 @@ struct ListArgs {
   uint32_t* col_count;               // cleared by the walk for the next binning pass
   uint32_t n_cols;
   uint32_t unused;                   // no implicit padding: argument packs are compared byte for byte
-  uint32_t* tot;                     // groups, work items, longest row (from the scan)
+  uint32_t* tot;                     // groups, work items
 };
 
 // LDS of the row walk, per wave: I's slot positions, a batch of up to 64
@@ -937,8 +937,8 @@ __device__ __forceinline__ void k_eng_row_sums(const ListArgs& A, uint2* __restr
 // seg: the sums of k_eng_row_sums, or null.
 __device__ __forceinline__ void
 k_eng_list_fill(const ListArgs& A, const uint32_t* __restrict__ ent_tmp,
-                uint32_t* __restrict__ row_cnt, uint32_t* __restrict__ row_ptr,
-                uint32_t* __restrict__ chunk_ptr, const uint2* __restrict__ seg, ListCopies C) {
+                uint32_t* __restrict__ row_ptr, uint32_t* __restrict__ chunk_ptr,
+                const uint2* __restrict__ seg, ListCopies C) {
   __shared__ uint32_t s_m[kFillRows], s_g[kFillRows], s_i[kFillRows];
   __shared__ uint32_t s_red[2][kListWaves];
   if (!build_on(A.gate)) return;
@@ -1006,7 +1006,6 @@ k_eng_list_fill(const ListArgs& A, const uint32_t* __restrict__ ent_tmp,
     }
     __syncthreads();
     if (threadIdx.x < nr) {
-      row_cnt[r0 + threadIdx.x] = s_m[threadIdx.x];
       row_ptr[r0 + threadIdx.x] = s_g[threadIdx.x];
       chunk_ptr[r0 + threadIdx.x] = s_i[threadIdx.x];
     }
@@ -1874,11 +1873,11 @@ struct ListSlots {
   int32_t* slot_type;
   int32_t* slot_gid;
   uint8_t* cl_class;
-  uint32_t* slot_of;
+  uint32_t* slot_of;   // (read by the build's own walk only)
   float4* xyzq;
   uint32_t* row_ptr;
   uint32_t* chunk_ptr;
-  uint32_t* counters;  // [0] clusters, [1] groups, [2] work items, [3] longest row, [4] overflow
+  uint32_t* counters;  // [0] clusters, [1] groups, [2] work items, [4] overflow
 };
 
 struct PrepArgs {
@@ -2029,11 +2028,10 @@ __device__ __forceinline__ void k_eng_prep(const PrepArgs& A, const PmePrepArgs&
     copy_grid(A.cur.slot_type, A.stg.slot_type, ns, t, A.stride);
     copy_grid(A.cur.slot_gid, A.stg.slot_gid, ns, t, A.stride);
     copy_grid(A.cur.cl_class, A.stg.cl_class, n_cl, t, A.stride);
-    copy_grid(A.cur.slot_of, A.stg.slot_of, n, t, A.stride);
     copy_grid(A.cur.wpos_ref, A.stg.wpos_ref, n, t, A.stride);
     copy_grid(A.cur.row_ptr, A.stg.row_ptr, (size_t)n_cl + 1, t, A.stride);
     copy_grid(A.cur.chunk_ptr, A.stg.chunk_ptr, (size_t)n_cl + 1, t, A.stride);
-    copy_grid(A.cur.counters, A.stg.counters, 4, t, A.stride);
+    copy_grid(A.cur.counters, A.stg.counters, 3, t, A.stride);
   }
   for (int m = kWave / 2; m >= 1; m >>= 1) v = max(v, (unsigned int)__shfl_xor((int)v, m, kWave));
   if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = v;
@@ -2249,15 +2247,15 @@ struct dyn_engine {
   DevBuf<uint8_t> cl_class;
   DevBuf<uint32_t> slot_of;
   DevBuf<float4> xyzq, bb_c, bb_h;
-  DevBuf<uint32_t> row_cnt, row_ptr, chunk_ptr, cj, ent_tmp, unit_cnt;
+  DevBuf<uint32_t> row_ptr, chunk_ptr, cj, ent_tmp, unit_cnt;
   DevBuf<uint8_t> xb_tmp;  // exclusion byte of each ent_tmp entry
   DevBuf<uint2> seg_sum;   // groups and work items per kScanSeg rows
   DevBuf<unsigned long long> cmask;
   DevBuf<uint2> chunks;
   uint64_t cap_entries = 0, cap_chunks = 0;  // groups of 8 j entries, work items
   uint32_t row_cap = 0;                      // j entries per walk-unit slice of ent_tmp
-  // device counters: [0] n_cl, [1] n_groups, [2] n_items, [3] max row (groups),
-  // [4] longest row that overflowed its slice (entries)
+  // device counters: [0] n_cl, [1] n_groups, [2] n_items, [4] longest row that
+  // overflowed its slice (entries)
   View<uint32_t> counters;
   // the staging list of an asynchronous build (slot and row arrays, copied
   // into the ones above by the next evaluation's preparation kernel) and the
@@ -2422,7 +2420,6 @@ void dyn_engine::set_geometry() {
   xyzq.reserve(cap_slots + DYN_CL_SIZE);
   bb_c.reserve(cap_cl);
   bb_h.reserve(cap_cl);
-  row_cnt.reserve(cap_cl + 1);
   unit_cnt.reserve((size_t)cap_cl * kUnits);
   seg_sum.reserve((cap_cl + kScanSeg - 1) / kScanSeg);  // (a step call allocates nothing)
   row_ptr.reserve(cap_cl + 1);
@@ -2632,7 +2629,7 @@ static void set_build_lists(EngineSet& S, const BatchRun& R, const std::vector<B
     launch<k_eng_list_fill, kListBlock>(R, "k_eng_list_fill", 0, list_grid, kListBlock, 0,
                                         [&](uint32_t i) {
       dyn_engine& e = *E[i];
-      return args<k_eng_list_fill>(LA[i], e.ent_tmp.p, e.row_cnt.p, T[i].row_ptr, T[i].chunk_ptr,
+      return args<k_eng_list_fill>(LA[i], e.ent_tmp.p, T[i].row_ptr, T[i].chunk_ptr,
                                    scan ? (const uint2*)e.seg_sum.p : (const uint2*)nullptr,
                                    e.copies(staged));
     });
