@@ -127,6 +127,28 @@ def test_small_beta(gpu, cases, beta):
     eng.close()
 
 
+@pytest.mark.parametrize("n_types", [1, 40, 64])
+def test_many_lj_types(gpu, cases, n_types):
+    """Up to 64 LJ types (66 with water O and the types without LJ: with the
+    Coulomb tables of an evaluation with energies more than 64 KB of LDS):
+    fixed-point sums equal the replay's, forces the FP64 sum."""
+    s = copy.copy(cases["solvated"])
+    rng = np.random.default_rng(n_types)
+    s.lj_types = np.stack([rng.uniform(2.0, 3.6, n_types), rng.uniform(0.02, 0.2, n_types)], 1).astype(np.float32)
+    s.type_dyn = (np.arange(s.n_dyn) * 7 % n_types).astype(np.int32)
+    s.sigma_dyn, s.eps_dyn = (np.ascontiguousarray(s.lj_types[s.type_dyn, k]) for k in (0, 1))
+    print(f"LJ types: {n_types}", flush=True)
+    eng = _engine(s)
+    ref = fp64.pair_sum_fp64(s, RC, RC, BETA)
+    for flags in (api.COMPUTE_SHORT | api.COMPUTE_CORR, api.COMPUTE_SHORT | api.COMPUTE_CORR | api.COMPUTE_NO_ENERGY):
+        eng.compute(flags)
+        assert rel_rms(eng.site_forces(), ref["forces"]) <= 1e-5
+        dbg = eng.debug_export()
+        fx = replay_engine_tiles(dbg, s, RC, RC, BETA)
+        assert np.array_equal(fx, dbg["fx_slot"])
+    eng.close()
+
+
 def _check_item_sums(eng, dbg, ie):
     """Per work item energies, virial and dH/dλ against the host replay: a
     sum the replay leaves at zero (e.g. a solute energy of a water-only item)
