@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -124,6 +125,13 @@ struct ListSites {
   unsigned long long f[3][kListSites];
 };
 
+__device__ __forceinline__ void site_add(int64_t* __restrict__ fx, uint32_t site, int64_t q0, int64_t q1,
+                                         int64_t q2) {
+  atomic_add_fx(fx + 3u * (size_t)site + 0, q0);
+  atomic_add_fx(fx + 3u * (size_t)site + 1, q1);
+  atomic_add_fx(fx + 3u * (size_t)site + 2, q2);
+}
+
 __device__ __forceinline__ void list_site_add(ListSites& S, int64_t* __restrict__ fx, uint32_t site,
                                               int64_t q0, int64_t q1, int64_t q2) {
   uint32_t at = site & (kListSites - 1);
@@ -140,14 +148,20 @@ __device__ __forceinline__ void list_site_add(ListSites& S, int64_t* __restrict_
       return;
     }
   }
-  atomic_add_fx(fx + 3u * (size_t)site + 0, q0);
-  atomic_add_fx(fx + 3u * (size_t)site + 1, q1);
-  atomic_add_fx(fx + 3u * (size_t)site + 2, q2);
+  site_add(fx, site, q0, q1, q2);
 }
+
+// Up to kListDirect pairs, a pair per thread and its six atomics in memory:
+// the table's clearing and emptying take longer than so few additions.  A call,
+// 1,000 sites, 100, 3,000, 16,000 and 30,000 pairs: 43, 43, 47 and 51 µs, with the
+// table 46, 46, 46 and 48; 16,000 sites: 79, 79, 80 and 81, with it 83, 87, 85 and 86.
+constexpr uint32_t kListDirect = 16384;
+constexpr int kDirectBlock = 256;
 
 // Pairs of a run, a multiple of kListBlock: n pairs in as few rounds of
 // kListGroups equal runs as keep a run within kListRun.
-__host__ __device__ inline uint32_t list_run(uint32_t n) {
+inline uint32_t list_run(uint32_t n) {
+  if (n <= kListDirect) return kDirectBlock;
   const uint64_t per_round = (uint64_t)kListGroups * kListRun;
   const uint64_t rounds = (n + per_round - 1) / per_round;
   const uint64_t parts = (rounds ? rounds : 1) * kListGroups;
@@ -155,18 +169,22 @@ __host__ __device__ inline uint32_t list_run(uint32_t n) {
   return run ? (uint32_t)run : (uint32_t)kListBlock;
 }
 
-__global__ void __launch_bounds__(kListBlock)
+template <bool TABLE>
+__global__ void __launch_bounds__(TABLE ? kListBlock : kDirectBlock)
 k_ref_pairs(const DynPairRec* __restrict__ pairs, uint32_t n, uint32_t run,
             const float* __restrict__ pos, DynRefParams P, float r2_far, int energy_all,
             int64_t* __restrict__ fx, double* __restrict__ partials) {
-  __shared__ ListSites S;
-  __shared__ double sh[3][kListBlock / 64];
+  constexpr int kBlock = TABLE ? kListBlock : kDirectBlock;
+  __shared__ std::conditional_t<TABLE, ListSites, char> S;
+  __shared__ double sh[3][kBlock / 64];
   const uint32_t t = threadIdx.x;
-  for (uint32_t k = t; k < kListSites; k += kListBlock) {
-    S.key[k] = kNoSite;
-    for (int c = 0; c < 3; ++c) S.f[c][k] = 0ull;
+  if constexpr (TABLE) {
+    for (uint32_t k = t; k < kListSites; k += kBlock) {
+      S.key[k] = kNoSite;
+      for (int c = 0; c < 3; ++c) S.f[c][k] = 0ull;
+    }
+    __syncthreads();
   }
-  __syncthreads();
   double e_acc = 0.0, w_acc = 0.0, dh_acc = 0.0;
   for (uint64_t r0 = (uint64_t)blockIdx.x * run; r0 < n; r0 += (uint64_t)gridDim.x * run) {
     const DynPairRec* __restrict__ part = pairs + r0;
@@ -176,7 +194,7 @@ k_ref_pairs(const DynPairRec* __restrict__ pairs, uint32_t n, uint32_t run,
     if (i < len) next = part[i];
     while (i < len) {
       const DynPairRec p = next;
-      i += kListBlock;
+      i += kBlock;
       if (i < len) next = part[i];
       float f[3], e, dh;
       double vir;
@@ -186,20 +204,25 @@ k_ref_pairs(const DynPairRec* __restrict__ pairs, uint32_t n, uint32_t run,
       if (p.flags & DYN_PF_ALCH) dh_acc += (double)dh;
       const int64_t q0 = dyn_fx(f[0]), q1 = dyn_fx(f[1]), q2 = dyn_fx(f[2]);
       if ((q0 | q1 | q2) == 0) continue;
-      list_site_add(S, fx, p.tgt, q0, q1, q2);
-      if (p.flags & DYN_PF_SYMMETRIC) list_site_add(S, fx, p.src, -q0, -q1, -q2);
-    }
-    __syncthreads();
-    for (uint32_t k = t; k < kListSites; k += kListBlock) {
-      const uint32_t site = S.key[k];
-      if (site == kNoSite) continue;
-      for (int c = 0; c < 3; ++c) {
-        atomic_add_fx(fx + 3u * (size_t)site + c, (int64_t)S.f[c][k]);
-        S.f[c][k] = 0ull;
+      if constexpr (TABLE) {
+        list_site_add(S, fx, p.tgt, q0, q1, q2);
+        if (p.flags & DYN_PF_SYMMETRIC) list_site_add(S, fx, p.src, -q0, -q1, -q2);
+      } else {
+        site_add(fx, p.tgt, q0, q1, q2);
+        if (p.flags & DYN_PF_SYMMETRIC) site_add(fx, p.src, -q0, -q1, -q2);
       }
-      S.key[k] = kNoSite;
     }
-    __syncthreads();
+    if constexpr (TABLE) {
+      __syncthreads();
+      for (uint32_t k = t; k < kListSites; k += kBlock) {
+        const uint32_t site = S.key[k];
+        if (site == kNoSite) continue;
+        site_add(fx, site, (int64_t)S.f[0][k], (int64_t)S.f[1][k], (int64_t)S.f[2][k]);
+        for (int c = 0; c < 3; ++c) S.f[c][k] = 0ull;
+        S.key[k] = kNoSite;
+      }
+      __syncthreads();
+    }
   }
   for (int m = 1; m < 64; m <<= 1) {
     e_acc += __shfl_xor(e_acc, m, 64);
@@ -214,7 +237,7 @@ k_ref_pairs(const DynPairRec* __restrict__ pairs, uint32_t n, uint32_t run,
   __syncthreads();
   if (t < 3) {
     double x = 0.0;
-    for (int k = 0; k < kListBlock / 64; ++k) x += sh[t][k];
+    for (int k = 0; k < kBlock / 64; ++k) x += sh[t][k];
     partials[3 * blockIdx.x + t] = x;
   }
 }
@@ -819,8 +842,9 @@ extern "C" int dyn_nb_compute(dyn_nb_ctx* ctx, const float* pos_dyn, const float
     if (n) {
       // beyond this r² a pair's rounded r is beyond the Coulomb cutoff
       const float r2_far = ctx->cutoff * ctx->cutoff * 1.0001f;
-      hipLaunchKernelGGL(k_ref_pairs, dim3(grid), dim3(kListBlock), 0, ctx->stream,
-                         ctx->pairs.p, n, list_run(n), ctx->pos.p, P, r2_far,
+      const bool table = n > kListDirect;
+      hipLaunchKernelGGL(table ? k_ref_pairs<true> : k_ref_pairs<false>, dim3(grid),
+                         dim3(table ? kListBlock : kDirectBlock), 0, ctx->stream, ctx->pairs.p, n, list_run(n), ctx->pos.p, P, r2_far,
                          (int)ctx->opts.energy_all_pairs, ctx->fx.p, ctx->partials.p);
       DYN_CHECK_LAUNCH("k_ref_pairs");
       DYN_HIP(hipMemcpyAsync(ctx->h_part.p, ctx->partials.p, sizeof(double) * 3 * grid,

@@ -187,3 +187,29 @@ def test_compat_pair_runs(gpu, n):
     # sums of n double terms in another order: 1e-9 of the terms is ample
     assert abs(vir - w_r) <= 1e-9 * abs(w_r) + 1e-9
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [255, 257, 16384, 16385])
+def test_compat_short_lists(gpu, n):
+    """Lists at the edges of a pair per thread: fixed-point sums equal the
+    replay's exactly."""
+    s = systems.small_water()
+    rng = np.random.default_rng(n)
+    u8, f4 = np.uint8, np.float32
+    tgt = rng.integers(0, 512, n).astype(np.uint32)
+    one = np.ones(n, u8)
+    pairs = {"tgt": tgt, "src": ((tgt + rng.integers(1, 512, n)) % 512).astype(np.uint32),
+             "sigma": np.full(n, 3.1, f4), "eps": np.full(n, 0.2, f4), "q_tgt": np.full(n, -0.5, f4),
+             "q_src": np.full(n, 0.4, f4), "atom_type_tgt": one,
+             "water_site_tgt": rng.integers(1, 5, n).astype(u8), "atom_type_src": one,
+             "water_site_src": rng.integers(1, 5, n).astype(u8), "scale14": 0 * one,
+             "calc_lj": rng.integers(0, 2, n).astype(u8), "calc_coul": one,
+             "symmetric": rng.integers(0, 2, n).astype(u8)}
+    print(f"short lists: n={n}", flush=True)
+    ctx = _ctx(s)
+    ctx.set_pairs(pairs)
+    _, _, vir, _, _ = _compute(ctx, s)
+    fx_r, _, w_r, _ = replay_ref_pairs(s, pairs, RC, ALPHA)
+    assert np.array_equal(ctx.fixed_forces(), fx_r)
+    assert abs(vir - w_r) <= 1e-9 * abs(w_r) + 1e-9  # sums of n double terms in another order
+    ctx.close()
