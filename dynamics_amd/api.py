@@ -333,8 +333,9 @@ class ForcesPositsGpu:
         n_outer = po.shape[0]
         row_ptr = np.zeros(n_outer + 1, np.uint32)
         # room for a uniform density and a tenth more, so that dense sets are
-        # built once too (untouched pages of the array cost nothing)
-        cap = max(1024, n_outer * 64)
+        # built once too (untouched pages of the array cost nothing); where
+        # that much cannot be had, the first call tells the size
+        cap = least = max(1024, n_outer * 64)
         vol = float(np.prod(_c(extent, np.float32), dtype=np.float64))
         r2 = float(skin_sq_w_cutoff)
         if 0.0 < vol < 1e300 and 0.0 < r2 < 1e12:
@@ -342,7 +343,13 @@ class ForcesPositsGpu:
             cap = max(cap, int(n_outer * row))
         total = C.c_uint64()
         for _ in range(2):
-            col = np.zeros(cap, np.uint32)
+            try:
+                col = np.zeros(cap, np.uint32)
+            except MemoryError:
+                if total.value or cap == least:
+                    raise
+                cap = least
+                col = np.zeros(cap, np.uint32)
             rc = lib.dyn_nb_build_neighbors(self.h, _ptr(po), n_outer, _ptr(pi), pi.shape[0],
                                             _ptr(st), _c(extent, np.float32), int(symmetric),
                                             float(skin_sq_w_cutoff), row_ptr, _ptr(col), cap,

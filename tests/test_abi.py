@@ -57,3 +57,28 @@ def test_errors_are_status_codes_not_aborts():
     api.lib.dyn_nb_destroy(None)
     api.lib.dyn_engine_destroy(None)
     api.lib.dyn_pme_destroy(None)
+
+
+def test_neighbor_list_room_falls_back(monkeypatch):
+    """Where the memory for a uniform density's rows cannot be had, the
+    smaller first guess is taken, as for sparse sets."""
+    from dynamics_amd import api
+    zeros, sizes = np.zeros, []
+
+    def limited(shape, dtype=float):
+        if np.prod(shape) > 1_000_000:
+            raise MemoryError
+        return zeros(shape, dtype)
+
+    def build(h, po, n_outer, pi, n_inner, st, ext, sym, r2, row_ptr, col, cap, total):
+        sizes.append(cap)
+        total._obj.value = 3
+        return 0
+
+    ctx = object.__new__(api.ForcesPositsGpu)
+    ctx.h = None
+    monkeypatch.setattr(api.np, "zeros", limited)
+    monkeypatch.setattr(api.lib, "dyn_nb_build_neighbors", build)
+    p = np.ones((2000, 3), np.float32)
+    row_ptr, col = ctx.build_neighbors(p, p, None, np.full(3, 9.0), True, 81.0)
+    assert sizes == [2000 * 64] and col.size == 3 and row_ptr.size == 2001
