@@ -1118,23 +1118,18 @@ struct PairArgs {
   int64_t* fx_site;          // site sums the FP64 kernel's i forces are added to
 };
 
-// Whether the evaluation can go ahead (the same for every workgroup); A's
-// list pointers become those of the copy in use.
-__device__ __forceinline__ bool pairs_begin(PairArgs& A) {
-  if (*A.status) return false;
+// Which copy of the list the evaluation reads, or below 0: it is not to go
+// ahead (the same for every workgroup; −2: the list is stale).  By value, as
+// item_partials: an argument pack or a sum whose address is taken goes to scratch
+// memory (a 28,000-site MD step 4 % slower).
+__device__ __forceinline__ int pairs_copy(const unsigned int* status, const unsigned int* fl, int staged,
+                                          unsigned int hard_limit) {
+  if (*status) return -1;
   // in staged mode a site may have moved half the list buffer since the
   // current list's build: the list may then miss pairs, and the evaluation
   // is void
-  if (A.staged && A.fl[kFlDisp] >= A.hard_limit) {
-    if (threadIdx.x == 0) atomicOr(A.status, kStDisp);
-    return false;
-  }
-  if ((A.fl[kFlSel] ^ A.fl[kFlCommit]) != 0u) {
-    A.cj = A.cj2;
-    A.cmask = A.cmask2;
-    A.chunks = A.chunks2;
-  }
-  return true;
+  if (staged && fl[kFlDisp] >= hard_limit) return -2;
+  return (fl[kFlSel] ^ fl[kFlCommit]) != 0u ? 1 : 0;
 }
 
 __device__ __forceinline__ float xor_sum(float v, int m) { return v + __shfl_xor(v, m, kWave); }
@@ -1664,17 +1659,16 @@ __device__ __forceinline__ double row_sum(double v) {
 // the cost of two: a swap of half-waves leaves one value in each half, a swap
 // of rows one in each row of 16.
 template <class R>
-__device__ __forceinline__ void item_partials(const PairArgs& A, const TileAccT<R>& T, size_t item, int lane) {
+__device__ __forceinline__ void item_partials(double* out, size_t cap, TileAccT<R> T, int lane) {
   const double a0 = swap32_sum((double)T.e_lj_w, (double)T.e_c_w);
   const double a1 = swap32_sum((double)T.e_lj_s, (double)T.e_c_s);
   const double a2 = swap32_sum((double)T.vir, (double)T.dh);
   const double b0 = row_sum(swap16_sum(a0, a1)), b1 = row_sum(swap16_sum(a2, a2));
-  double* const out = A.partials + item;
   // rows of b0: LJ water, LJ solute, Coulomb water, Coulomb solute; of
   // b1: virial, virial, dH/dλ, dH/dλ
-  if ((lane & 15) == 0) out[(size_t)(lane >> 4) * A.cap_chunks] = b0;
-  if ((lane & 31) == 1) out[(size_t)(lane == 1 ? 4 : 8) * A.cap_chunks] = b1;
-  if (lane < 3) out[(size_t)(5 + lane) * A.cap_chunks] = (double)(lane == 0 ? T.n_ss : lane == 1 ? T.n_lj : T.n_c);
+  if ((lane & 15) == 0) out[(size_t)(lane >> 4) * cap] = b0;
+  if ((lane & 31) == 1) out[(size_t)(lane == 1 ? 4 : 8) * cap] = b1;
+  if (lane < 3) out[(size_t)(5 + lane) * cap] = (double)(lane == 0 ? T.n_ss : lane == 1 ? T.n_lj : T.n_c);
 }
 
 // The i side of a row for lane (ia, ·).
@@ -1730,7 +1724,13 @@ k_eng_pairs(PairArgs A) {
   const int lane = threadIdx.x & (kWave - 1);
   const int ia = lane & 7, jb = lane >> 3;
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  if (!pairs_begin(A)) return;
+  const int copy = pairs_copy(A.status, A.fl, A.staged, A.hard_limit);
+  if (copy == -2 && threadIdx.x == 0) atomicOr(A.status, kStDisp);
+  if (copy < 0) return;
+  if (copy == 1) {
+    A.cj = A.cj2;
+    A.cmask = A.cmask2;
+  }
   const uint32_t n_cl = *A.n_cl;
   if (blockIdx.x >= n_cl) return;
   const DynCoulTabs src = dyn_coul_tabs(A.P.coul_tab);
@@ -1772,7 +1772,7 @@ k_eng_pairs(PairArgs A) {
         acc[c] += q;
         if (A.keep_items && jb == 0) A.fitem[item * (3 * DYN_CL_SIZE) + c * DYN_CL_SIZE + ia] = q;
       }
-      if (ENERGY) item_partials(A, T, item, lane);
+      if (ENERGY) item_partials(A.partials + item, A.cap_chunks, T, lane);
     }
     // the row's forces: the waves' sums (integers: the order of the items
     // does not change them), stored by site.  Two buffers: the next row's
@@ -1801,7 +1801,14 @@ __device__ __forceinline__ void
 k_eng_pairs64(PairArgs A) {
   const int lane = threadIdx.x & (kWave - 1);
   const int ia = lane & 7, jb = lane >> 3;
-  if (!pairs_begin(A)) return;
+  const int copy = pairs_copy(A.status, A.fl, A.staged, A.hard_limit);
+  if (copy == -2 && threadIdx.x == 0) atomicOr(A.status, kStDisp);
+  if (copy < 0) return;
+  if (copy == 1) {
+    A.cj = A.cj2;
+    A.cmask = A.cmask2;
+    A.chunks = A.chunks2;
+  }
   const uint32_t n_items = (uint32_t)min((uint64_t)*A.n_chunks, A.cap_chunks);
   const uint32_t waves = gridDim.x * (kPairBlock / kWave);
   for (uint32_t item = blockIdx.x * (kPairBlock / kWave) + threadIdx.x / kWave; item < n_items; item += waves) {
@@ -1822,7 +1829,7 @@ k_eng_pairs64(PairArgs A) {
         atomicAdd(reinterpret_cast<unsigned long long*>(A.fx_site + (size_t)c * A.n_sites + site),
                   (unsigned long long)q);
     }
-    if (ENERGY) item_partials(A, T, item, lane);
+    if (ENERGY) item_partials(A.partials + item, A.cap_chunks, T, lane);
   }
 }
 
