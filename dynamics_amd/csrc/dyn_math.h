@@ -239,15 +239,6 @@ DYN_HD int64_t dyn_fx64(double f) {
   return dyn_fx_d(f, DYN_FX_SCALE);
 }
 
-// dyn_fx64, and what it rounds away in units of 2⁻⁶⁴ (for sums of many small
-// terms: integers, so the order of the additions changes neither sum).
-DYN_HD void dyn_fx128(double f, int64_t* hi, int64_t* lo) {
-  f = f < -(double)DYN_FX_CLAMP ? -(double)DYN_FX_CLAMP : (f > (double)DYN_FX_CLAMP ? (double)DYN_FX_CLAMP : f);
-  const double d = dyn_fma(f, DYN_FX_SCALE, 6755399441055744.0);
-  *hi = dyn_d2bits(d) - (int64_t)0x4338000000000000LL;
-  *lo = dyn_fx_d(dyn_fma(f, DYN_FX_SCALE, 6755399441055744.0 - d), DYN_FX_SCALE);
-}
-
 // ---------------------------------------------------------------------------
 // Minimum image.
 // ---------------------------------------------------------------------------

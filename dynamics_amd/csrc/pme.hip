@@ -530,6 +530,44 @@ k_fft_plane(float2* __restrict__ spec, const int64_t* __restrict__ grid_fx, floa
 
 // Energy and virial in units of 2⁻³², then what each leaves in units of 2⁻⁶⁴.
 constexpr int kConvSums = 4;
+// The wave's four sums, sum v in the lanes of row v (16 lanes): a swap of
+// half-waves leaves one value in each half, a swap of rows one in each row, four
+// rotations add a row.  (24 shuffles otherwise.)
+__device__ __forceinline__ long long wave_sums(const long long (&v)[kConvSums]) {
+  auto two = [](long long a) { return make_uint2((uint32_t)a, (uint32_t)((unsigned long long)a >> 32)); };
+  auto one = [](uint32_t lo, uint32_t hi) { return (long long)((unsigned long long)hi << 32 | lo); };
+  auto half = [&](long long a, long long b) {
+    const uint2 x = two(a), y = two(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+    return one(lo[0], hi[0]) + one(lo[1], hi[1]);
+  };
+  const uint2 x = two(half(v[0], v[2])), y = two(half(v[1], v[3]));
+  const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+  long long s = one(lo[0], hi[0]) + one(lo[1], hi[1]);
+  auto turn = [&](auto ctrl) {
+    const uint2 t = two(s);
+    s += one((uint32_t)__builtin_amdgcn_mov_dpp((int)t.x, decltype(ctrl)::value, 0xf, 0xf, true),
+             (uint32_t)__builtin_amdgcn_mov_dpp((int)t.y, decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  turn(std::integral_constant<int, 0x128>{});  // row_ror:8, 4, 2, 1
+  turn(std::integral_constant<int, 0x124>{});
+  turn(std::integral_constant<int, 0x122>{});
+  turn(std::integral_constant<int, 0x121>{});
+  return s;
+}
+// Adds x and what its rounding to 2⁻³² leaves to the two sums, in the same
+// units but each kFxBias too large (taken off once per workgroup; sums wrap).
+// x is clamped as every fixed-point value is.
+constexpr long long kFxBias = 0x4338000000000000LL;  // bits of 1.5·2⁵²
+__device__ __forceinline__ void add_fx128(double x, long long& hi, long long& lo) {
+  x = fmin(fmax(x, -(double)DYN_FX_CLAMP), (double)DYN_FX_CLAMP);
+  const double d = __builtin_fma(x, DYN_FX_SCALE, 0x1.8p52);
+  const double rest = __builtin_fma(x, DYN_FX_SCALE, 0x1.8p52 - d);
+  hi += __double_as_longlong(d);
+  lo += __double_as_longlong(__builtin_fma(rest, DYN_FX_SCALE, 0x1.8p52));
+}
 struct ConvArgs {
   float invL[3];
   double pi2_over_b2;  // π²/β²
@@ -542,7 +580,8 @@ struct ConvArgs {
 // fixed point, so the sums do not depend on the grouping of the lines; two
 // words (2⁻³² and what that rounds away, 2⁻⁶⁴), since most of a fine grid's points
 // are smaller than 2⁻³³ (with one word two charges of 0.1 on 64³ lost 1.8e-5 of
-// their energy; the second costs 0.6 µs of 8.8 on 64³, 1.0 of 18.6 on 128³).
+// their energy; with two and the sums over a wave by wave_sums 7.8 µs on 64³ and
+// 17.4 on 128³, with one word and shuffles 8.1 and 17.6).
 template <class C>
 __device__ __forceinline__ void
 k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
@@ -578,27 +617,19 @@ k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
     const double msq = fx * fx + fy * fy + fz * fz;
     const double wz = mz == 0 || 2 * mz == g.K[2] ? 0.5 : 1.0;
     const double en = wz * (double)gv * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
-    int64_t hi, lo;
-    dyn_fx128(en, &hi, &lo);
-    sum[0] += hi;
-    sum[2] += lo;
-    dyn_fx128(en * (1.0 - 2.0 * V.pi2_over_b2 * msq), &hi, &lo);
-    sum[1] += hi;
-    sum[3] += lo;
+    add_fx128(en, sum[0], sum[2]);
+    add_fx128(en * (1.0 - 2.0 * V.pi2_over_b2 * msq), sum[1], sum[3]);
     v.x *= gv;
     v.y *= gv;
     X[e] = v;
   });
-#pragma unroll
-  for (int v = 0; v < kConvSums; ++v) {
-    for (int m = 32; m >= 1; m >>= 1) sum[v] += __shfl_xor(sum[v], m, 64);
-    if ((threadIdx.x & 63) == 0) red[v][threadIdx.x / 64] = sum[v];
-  }
+  const long long w = wave_sums(sum);
+  if ((threadIdx.x & 15) == 0) red[(threadIdx.x >> 4) & 3][threadIdx.x / 64] = w;
   __syncthreads();
   if (threadIdx.x < kConvSums) {
     long long s = 0;
     for (int k = 0; k < kFftBlock / 64; ++k) s += red[threadIdx.x][k];
-    partials[kConvSums * blockIdx.x + threadIdx.x] = s;
+    partials[kConvSums * blockIdx.x + threadIdx.x] = s - (long long)(N * nl) * kFxBias;
   }
   const C* Z = lds_fft<+1>(X, X == A ? B : A, nl, nl, N, g.plan[0], s_tw);
   for (int e = threadIdx.x; e < N * nl; e += blockDim.x) {
@@ -829,11 +860,8 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
     long long sum[kConvSums] = {0, 0, 0, 0};
     for (int b = threadIdx.x; b < nbp; b += kGatherBlock)
       for (int v = 0; v < kConvSums; ++v) sum[v] += (long long)partials[kConvSums * b + v];
-#pragma unroll
-    for (int v = 0; v < kConvSums; ++v) {
-      for (int m = 32; m >= 1; m >>= 1) sum[v] += __shfl_xor(sum[v], m, 64);
-      if ((threadIdx.x & 63) == 0) red[v][threadIdx.x / 64] = sum[v];
-    }
+    const long long w = wave_sums(sum);
+    if ((threadIdx.x & 15) == 0) red[(threadIdx.x >> 4) & 3][threadIdx.x / 64] = w;
     __syncthreads();
     if (threadIdx.x < 2) {
       long long hi = 0, lo = 0;
