@@ -1118,20 +1118,6 @@ struct PairArgs {
   int64_t* fx_site;          // site sums the FP64 kernel's i forces are added to
 };
 
-// Which copy of the list the evaluation reads, or below 0: it is not to go
-// ahead (the same for every workgroup; −2: the list is stale).  By value, as
-// item_partials: an argument pack or a sum whose address is taken goes to scratch
-// memory (a 28,000-site MD step 4 % slower).
-__device__ __forceinline__ int pairs_copy(const unsigned int* status, const unsigned int* fl, int staged,
-                                          unsigned int hard_limit) {
-  if (*status) return -1;
-  // in staged mode a site may have moved half the list buffer since the
-  // current list's build: the list may then miss pairs, and the evaluation
-  // is void
-  if (staged && fl[kFlDisp] >= hard_limit) return -2;
-  return (fl[kFlSel] ^ fl[kFlCommit]) != 0u ? 1 : 0;
-}
-
 __device__ __forceinline__ float xor_sum(float v, int m) { return v + __shfl_xor(v, m, kWave); }
 __device__ __forceinline__ double xor_sum_d(double v, int m) { return v + __shfl_xor(v, m, kWave); }
 
@@ -1347,7 +1333,8 @@ __device__ __forceinline__ uint32_t ext8(uint32_t v) {
   v = f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true));
   return f(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, true));
 }
-__device__ __forceinline__ RowImage row_image(const DynPairParams& P, const float x[4]) {
+__device__ __forceinline__ RowImage row_image(const DynPairParams& P, const float4& p) {
+  const float x[3] = {p.x, p.y, p.z};
   RowImage r;
   const float rc = __builtin_amdgcn_sqrtf(P.rc2) * 1.0001f + 1e-3f;
   bool ok = true, in = true;
@@ -1657,7 +1644,9 @@ __device__ __forceinline__ double row_sum(double v) {
 
 // A work item's energies, virial and pair counts.  Six sums over the wave at
 // the cost of two: a swap of half-waves leaves one value in each half, a swap
-// of rows one in each row of 16.
+// of rows one in each row of 16.  (Everything by value: an argument pack or a sum
+// whose address is taken goes to scratch memory, and MD of 28,000 sites is 4 %
+// slower.)
 template <class R>
 __device__ __forceinline__ void item_partials(double* out, size_t cap, TileAccT<R> T, int lane) {
   const double a0 = swap32_sum((double)T.e_lj_w, (double)T.e_c_w);
@@ -1669,23 +1658,6 @@ __device__ __forceinline__ void item_partials(double* out, size_t cap, TileAccT<
   if ((lane & 15) == 0) out[(size_t)(lane >> 4) * cap] = b0;
   if ((lane & 31) == 1) out[(size_t)(lane == 1 ? 4 : 8) * cap] = b1;
   if (lane < 3) out[(size_t)(5 + lane) * cap] = (double)(lane == 0 ? T.n_ss : lane == 1 ? T.n_lj : T.n_c);
-}
-
-// The i side of a row for lane (ia, ·).
-__device__ __forceinline__ TileI tile_i(const PairArgs& A, uint32_t row, int ia) {
-  const uint32_t slot = row * DYN_CL_SIZE + ia;
-  const float4 p = A.xyzq[slot];
-  TileI I;
-  I.p[0] = p.x;
-  I.p[1] = p.y;
-  I.p[2] = p.z;
-  I.p[3] = p.w;
-  I.r2_lo = dyn_coul_r2_lo(A.P.tab_b2);
-  I.t = A.slot_type[slot];
-  I.g = A.slot_gid[slot];
-  I.ci = A.cl_class[row];
-  I.pad = I.g == DYN_GID_PAD;
-  return I;
 }
 
 // A workgroup per row (i cluster) at a time, a wave per work item (≤ A.chunk
@@ -1724,10 +1696,15 @@ k_eng_pairs(PairArgs A) {
   const int lane = threadIdx.x & (kWave - 1);
   const int ia = lane & 7, jb = lane >> 3;
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int copy = pairs_copy(A.status, A.fl, A.staged, A.hard_limit);
-  if (copy == -2 && threadIdx.x == 0) atomicOr(A.status, kStDisp);
-  if (copy < 0) return;
-  if (copy == 1) {
+  if (*A.status) return;
+  // in staged mode a site may have moved half the list buffer since the
+  // current list's build: the list may then miss pairs, and the evaluation
+  // is void (every workgroup reads the same words)
+  if (A.staged && A.fl[kFlDisp] >= A.hard_limit) {
+    if (threadIdx.x == 0) atomicOr(A.status, kStDisp);
+    return;
+  }
+  if ((A.fl[kFlSel] ^ A.fl[kFlCommit]) != 0u) {
     A.cj = A.cj2;
     A.cmask = A.cmask2;
   }
@@ -1745,14 +1722,24 @@ k_eng_pairs(PairArgs A) {
   int buf = 0;
   for (uint32_t row = blockIdx.x; row < n_cl; row += gridDim.x, buf ^= 1) {
     const uint32_t r0 = A.row_ptr[row], r1 = A.row_ptr[row + 1];
-    TileI I = tile_i(A, row, ia);
+    const float4 piv = A.xyzq[row * DYN_CL_SIZE + ia];
+    TileI I;
+    I.p[0] = piv.x;
+    I.p[1] = piv.y;
+    I.p[2] = piv.z;
+    I.p[3] = piv.w;
+    I.r2_lo = dyn_coul_r2_lo(A.P.tab_b2);
+    I.t = A.slot_type[row * DYN_CL_SIZE + ia];
+    I.g = A.slot_gid[row * DYN_CL_SIZE + ia];
+    I.ci = A.cl_class[row];
+    I.pad = I.g == DYN_GID_PAD;
     I.any_in = ALCH && lanes(!I.pad & ((I.t & DYN_TYPE_ALCH) != 0)) != 0ull;
     I.any_out = ALCH && lanes(!I.pad & ((I.t & DYN_TYPE_ALCH) == 0)) != 0ull;
     int64_t acc[3] = {0, 0, 0};
     uint32_t it = w, g0 = r0 + w * A.chunk;
     RowImage Im;
     if (g0 < r1) {
-      Im = row_image(A.P, I.p);
+      Im = row_image(A.P, piv);
       if (I.pad) I.p[0] = -kFarX;
     }
     for (; g0 < r1; it += kPairBlock / kWave, g0 += kPairBlock / kWave * A.chunk) {
@@ -1801,10 +1788,12 @@ __device__ __forceinline__ void
 k_eng_pairs64(PairArgs A) {
   const int lane = threadIdx.x & (kWave - 1);
   const int ia = lane & 7, jb = lane >> 3;
-  const int copy = pairs_copy(A.status, A.fl, A.staged, A.hard_limit);
-  if (copy == -2 && threadIdx.x == 0) atomicOr(A.status, kStDisp);
-  if (copy < 0) return;
-  if (copy == 1) {
+  if (*A.status) return;
+  if (A.staged && A.fl[kFlDisp] >= A.hard_limit) {  // (as k_eng_pairs)
+    if (threadIdx.x == 0) atomicOr(A.status, kStDisp);
+    return;
+  }
+  if ((A.fl[kFlSel] ^ A.fl[kFlCommit]) != 0u) {
     A.cj = A.cj2;
     A.cmask = A.cmask2;
     A.chunks = A.chunks2;
@@ -1816,7 +1805,15 @@ k_eng_pairs64(PairArgs A) {
     const uint32_t row = (uint32_t)__builtin_amdgcn_readfirstlane(ch.x);
     const uint32_t g0 = (uint32_t)__builtin_amdgcn_readfirstlane(ch.y);
     const uint32_t g1 = min(g0 + A.chunk, A.row_ptr[row + 1]);
-    const TileI I = tile_i(A, row, ia);
+    const float4 piv = A.xyzq[row * DYN_CL_SIZE + ia];
+    TileI I{};
+    I.p[0] = piv.x;
+    I.p[1] = piv.y;
+    I.p[2] = piv.z;
+    I.p[3] = piv.w;
+    I.t = A.slot_type[row * DYN_CL_SIZE + ia];
+    I.g = A.slot_gid[row * DYN_CL_SIZE + ia];
+    I.ci = A.cl_class[row];
     TileAccT<double> T;
     T.clear();
     tile_item64<ENERGY>(A, I, g0, g1, T);
