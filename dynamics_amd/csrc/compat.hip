@@ -359,16 +359,22 @@ __device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
 }
 
 // Single-workgroup exclusive scan of n uint32 values into out[0..n]
-// (out[n] = total), also writing the maximum element to *maxv.  A tile of
-// four values per thread at a time (in is padded to a multiple of 4).
+// (out[n] = total), also writing the maximum element and the total, which may
+// exceed 32 bits, to *top.  A tile of four values per thread at a time (in is
+// padded to a multiple of 4).
+struct ScanTop {
+  uint64_t total;
+  uint32_t max, unused;
+};
 constexpr int kScanBlock = 1024;
 __global__ void __launch_bounds__(kScanBlock)
 k_scan_u32(const uint32_t* __restrict__ in, uint32_t n, uint32_t* __restrict__ out,
-           uint32_t* __restrict__ maxv) {
+           ScanTop* __restrict__ top_out) {
   constexpr int kWaves = kScanBlock / 64;
   __shared__ uint32_t part[2][kWaves], top[kWaves];
   const uint32_t t = threadIdx.x, w = t / 64;
-  uint32_t carry = 0, m = 0;
+  uint64_t carry = 0;
+  uint32_t m = 0;
   int buf = 0;
   for (uint64_t b = 0; b < n; b += 4 * kScanBlock, buf ^= 1) {
     const uint64_t k = b + 4 * t;
@@ -382,7 +388,7 @@ k_scan_u32(const uint32_t* __restrict__ in, uint32_t n, uint32_t* __restrict__ o
     const uint32_t inc = wave_scan_u32(s);
     if ((t & 63u) == 63u) part[buf][w] = inc;
     __syncthreads();
-    uint32_t before = carry;
+    uint32_t before = (uint32_t)carry;
     for (int q = 0; q < kWaves; ++q) {
       const uint32_t x = part[buf][q];
       if ((uint32_t)q < w) before += x;
@@ -399,8 +405,8 @@ k_scan_u32(const uint32_t* __restrict__ in, uint32_t n, uint32_t* __restrict__ o
   __syncthreads();
   if (t == 0) {
     for (int q = 1; q < kWaves; ++q) m = max(m, top[q]);
-    *maxv = m;
-    out[n] = carry;
+    *top_out = ScanTop{carry, m, 0u};
+    out[n] = (uint32_t)carry;
   }
 }
 
@@ -608,7 +614,8 @@ struct dyn_nb_ctx {
   DevBuf<uint8_t> nb_static;
   DevBuf<float4> nb_sorted;
   DevBuf<uint2> nb_place;
-  DevBuf<uint32_t> nb_counts, nb_cell_start, nb_row_count, nb_row_ptr, nb_col, nb_max;
+  DevBuf<uint32_t> nb_counts, nb_cell_start, nb_row_count, nb_row_ptr, nb_col;
+  DevBuf<ScanTop> nb_top;
   PinnedBuf<uint32_t> nb_stage;
   hipEvent_t nb_ev[2] = {nullptr, nullptr};
   DevBuf<uint32_t> c14_i, c14_j;
@@ -1072,13 +1079,13 @@ extern "C" int dyn_nb_build_neighbors(dyn_nb_ctx* ctx, const float* posits_outer
     ctx->nb_sorted.reserve(n_inner);
     ctx->nb_row_count.reserve(((size_t)n_outer + 3) & ~(size_t)3);
     ctx->nb_row_ptr.reserve((size_t)n_outer + 1);
-    ctx->nb_max.reserve(2);
+    ctx->nb_top.reserve(1);
     DYN_HIP(hipMemsetAsync(ctx->nb_counts.p, 0, 4 * ncell4, ctx->stream));
     hipLaunchKernelGGL(k_nbl_cell_count, dim3(grid_for(n_inner, kNblCellBlock)), dim3(kNblCellBlock), 0,
                        ctx->stream, d_inner, n_inner, G, ncell, ctx->nb_place.p, ctx->nb_counts.p);
     DYN_CHECK_LAUNCH("k_nbl_cell_count");
     hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(kScanBlock), 0, ctx->stream, ctx->nb_counts.p,
-                       ncell, ctx->nb_cell_start.p, ctx->nb_max.p);
+                       ncell, ctx->nb_cell_start.p, ctx->nb_top.p);
     DYN_CHECK_LAUNCH("k_scan_u32");
     hipLaunchKernelGGL(k_nbl_cell_fill, dim3(grid_for(n_inner, 256)), dim3(256), 0,
                        ctx->stream, d_inner, n_inner, ctx->nb_place.p, ctx->nb_cell_start.p,
@@ -1111,16 +1118,20 @@ extern "C" int dyn_nb_build_neighbors(dyn_nb_ctx* ctx, const float* posits_outer
                        (uint32_t*)nullptr);
     DYN_CHECK_LAUNCH("k_nbl_rows<0>");
     hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(kScanBlock), 0, ctx->stream,
-                       ctx->nb_row_count.p, n_outer, ctx->nb_row_ptr.p, ctx->nb_max.p);
+                       ctx->nb_row_count.p, n_outer, ctx->nb_row_ptr.p, ctx->nb_top.p);
     DYN_CHECK_LAUNCH("k_scan_u32");
-    uint32_t maxrow = 0;
-    DYN_HIP(hipMemcpyAsync(&maxrow, ctx->nb_max.p, 4, hipMemcpyDeviceToHost, ctx->stream));
+    ScanTop top{};
+    DYN_HIP(hipMemcpyAsync(&top, ctx->nb_top.p, sizeof top, hipMemcpyDeviceToHost, ctx->stream));
     copy_out(ctx, row_ptr, ctx->nb_row_ptr.p, (size_t)n_outer + 1);
-    const uint64_t total = row_ptr[n_outer];
+    const uint32_t maxrow = top.max;
+    const uint64_t total = top.total;
     *n_total = total;
     if (maxrow > (uint32_t)kNblCap)
       throw Error(DYN_ERR_CAPACITY,
                   fmt("a row has %u neighbors; the build handles at most %d", maxrow, kNblCap));
+    if (total > 0xffffffffull)  // row_ptr's 32 bits
+      throw Error(DYN_ERR_ARG, fmt("%llu neighbors in all; row_ptr holds at most 4294967295",
+                                   (unsigned long long)total));
     if (total > col_capacity)
       throw Error(DYN_ERR_CAPACITY, fmt("col_idx needs %llu entries, capacity %llu",
                                         (unsigned long long)total,

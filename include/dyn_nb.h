@@ -134,7 +134,8 @@ int dyn_nb_correct_14_noalloc(dyn_nb_ctx* ctx, uint32_t n14, const uint32_t* i14
  * pairs skipped when is_static is non-NULL.  Output is CSR: row_ptr[n_outer+1]
  * and col_idx, each row ascending (the reference's order).  If col_capacity
  * is too small the call returns DYN_ERR_CAPACITY and *n_total holds the size
- * needed. */
+ * needed; more neighbors in all than row_ptr's 32 bits count are refused
+ * (DYN_ERR_ARG). */
 int dyn_nb_build_neighbors(dyn_nb_ctx* ctx, const float* posits_outer, uint32_t n_outer,
                            const float* posits_inner, uint32_t n_inner,
                            const uint8_t* is_static, const float cell_extent[3],

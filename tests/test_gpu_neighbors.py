@@ -112,3 +112,17 @@ def test_neighbor_rows_sorted(gpu, n_outer, n_inner, ext, radius):
     print(f"neighbors: {n_outer} x {n_inner}, box {ext}, radius {radius}", flush=True)
     ctx = api.ForcesPositsGpu(n_outer, 0, 10.0, 0.3)
     _check(ctx, po, pi, None, e, False, np.float32(radius * radius))
+
+
+def test_neighbor_total_beyond_32_bits(gpu):
+    """More neighbours than row_ptr can count (1.25 million rows of about
+    3,600) are refused."""
+    n = 1_250_000
+    rng = np.random.default_rng(3)
+    p = (rng.random((n, 3), np.float32) * np.float32(60.0)).astype(np.float32)
+    print("neighbors: total beyond 32 bits", flush=True)
+    ctx = api.ForcesPositsGpu(16, 0, 10.0, 0.3)
+    with pytest.raises(api.DynError):
+        ctx.build_neighbors(p, p, None, np.full(3, 60.0, np.float32), True, 5.3 ** 2)
+    row_ptr, col = ctx.build_neighbors(p[:100], p, None, np.full(3, 60.0, np.float32), False, 5.3 ** 2)
+    assert row_ptr[-1] == col.size > 100 * 3000
