@@ -1081,13 +1081,13 @@ extern "C" int dyn_nb_build_neighbors(dyn_nb_ctx* ctx, const float* posits_outer
     ctx->nb_row_ptr.reserve((size_t)n_outer + 1);
     ctx->nb_top.reserve(1);
     DYN_HIP(hipMemsetAsync(ctx->nb_counts.p, 0, 4 * ncell4, ctx->stream));
-    hipLaunchKernelGGL(k_nbl_cell_count, dim3(grid_for(n_inner, kNblCellBlock)), dim3(kNblCellBlock), 0,
+    hipLaunchKernelGGL(k_nbl_cell_count, dim3(grid_all(n_inner, kNblCellBlock)), dim3(kNblCellBlock), 0,
                        ctx->stream, d_inner, n_inner, G, ncell, ctx->nb_place.p, ctx->nb_counts.p);
     DYN_CHECK_LAUNCH("k_nbl_cell_count");
     hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(kScanBlock), 0, ctx->stream, ctx->nb_counts.p,
                        ncell, ctx->nb_cell_start.p, ctx->nb_top.p);
     DYN_CHECK_LAUNCH("k_scan_u32");
-    hipLaunchKernelGGL(k_nbl_cell_fill, dim3(grid_for(n_inner, 256)), dim3(256), 0,
+    hipLaunchKernelGGL(k_nbl_cell_fill, dim3(grid_all(n_inner, 256)), dim3(256), 0,
                        ctx->stream, d_inner, n_inner, ctx->nb_place.p, ctx->nb_cell_start.p,
                        ctx->nb_sorted.p);
     DYN_CHECK_LAUNCH("k_nbl_cell_fill");

@@ -126,3 +126,22 @@ def test_neighbor_total_beyond_32_bits(gpu):
         ctx.build_neighbors(p, p, None, np.full(3, 60.0, np.float32), True, 5.3 ** 2)
     row_ptr, col = ctx.build_neighbors(p[:100], p, None, np.full(3, 60.0, np.float32), False, 5.3 ** 2)
     assert row_ptr[-1] == col.size > 100 * 3000
+
+
+def test_neighbor_many_inner_points(gpu):
+    """Inner points beyond 2¹⁸ workgroups of 256 are sorted into cells too
+    (68 million points, the last few around the outer ones)."""
+    n, n_outer = 68_000_000, 64
+    rng = np.random.default_rng(5)
+    ext = np.full(3, 4000.0, np.float32)
+    pi = rng.random((n, 3), np.float32)
+    pi *= np.float32(4000.0)
+    po = (2000.0 + 20.0 * rng.random((n_outer, 3))).astype(np.float32)
+    pi[-200:] = (po[rng.integers(0, n_outer, 200)] + rng.normal(0, 1.0, (200, 3))).astype(np.float32)
+    print("neighbors: 68 million inner points", flush=True)
+    ctx = api.ForcesPositsGpu(n_outer, 0, 10.0, 0.3)
+    row_ptr, col = ctx.build_neighbors(po, pi, None, ext, False, 16.0)
+    near = np.flatnonzero((np.abs(pi - 2010.0) < 20.0).all(1))  # (far from the box faces)
+    rp_o, col_o = rp.build_neighbors(po, np.ascontiguousarray(pi[near]), None, ext, False, np.float32(16.0))
+    assert np.array_equal(row_ptr, rp_o) and np.array_equal(col, near[col_o])
+    assert (col >= n - 200).any()
