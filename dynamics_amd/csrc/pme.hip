@@ -1195,7 +1195,7 @@ void pme_run(const BatchRun& R, Profiler& prof, const PmeRun* runs, int tag, con
     gz[i] = pass_geom(c, 2, ns, el);
     gy[i] = pass_geom(c, 1, ns, el);
     gx[i] = pass_geom(c, 0, ns, el);
-    g_n = std::max(g_n, grid_for(r.n, 256));
+    g_n = std::max(g_n, grid_all(r.n, 256));
     g_b = std::max(g_b, c.nbk[0] * c.nbk[1] * c.nbk[2]);
     bz = std::max(bz, pass_groups(gz[i], 2));
     by = std::max(by, pass_groups(gy[i], 1));
@@ -1527,7 +1527,7 @@ extern "C" int dyn_pme_forces_and_virial(dyn_pme* pme, uint32_t n, const float* 
     for (int attempt = 0;; ++attempt) {
       core.ensure_cap(n);
       if (src)
-        launch<k_pme_take>(R, "k_pme_take", 0, grid_for(nn, 256), 256, 0, [&](uint32_t) {
+        launch<k_pme_take>(R, "k_pme_take", 0, grid_all(nn, 256), 256, 0, [&](uint32_t) {
           return args<k_pme_take>(src, n, pme->xyzq.p, core.bin_args(nullptr, 0));
         });
       else

@@ -88,11 +88,11 @@ def test_pme_energy_of_small_terms(gpu, n, scale, K):
     pme.close()
 
 
-def test_pme_very_many_charges(gpu):
-    """Forces of 22.5 million charges are all read back (beyond 2¹⁸
-    workgroups of the kernel that stores them): the last charge, at the first one's place
-    and with its value, has its force."""
-    n = 22_500_000
+@pytest.mark.parametrize("n", [22_500_000, 67_200_000])
+def test_pme_very_many_charges(gpu, n):
+    """Charges beyond 2¹⁸ workgroups of the kernels that store the forces
+    (22.5 million) and that list and gather them (67.2 million): the last one,
+    at the first one's place and with its value, has its force."""
     rng = np.random.default_rng(4)
     box = np.full(3, 60.0, np.float32)
     pos = rng.random((n, 3), np.float32) * box
