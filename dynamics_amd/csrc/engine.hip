@@ -1554,7 +1554,8 @@ __device__ __forceinline__ bool tile_item(const PairArgs& A, const TileI& I, con
 // option): a lane loads its own j entry.  Three or four waves a SIMD are too few
 // to hide the loads, so while a group is evaluated the j data of the next and
 // the entry of the one after it are in flight (the last loads repeat the last
-// group): 279,600 sites with energies 1.97 ms, without that 2.23.
+// group): with a workgroup per row, 279,600 sites with energies 1.97 ms, without
+// that 2.23.
 template <int KIND, bool ENERGY>
 __device__ __forceinline__ void tile_entry64(const PairArgs& A, const TileI& I, const float4& pjv, int tj,
                                              int gj, bool active, TileAccT<double>& T) {
@@ -1782,7 +1783,7 @@ k_eng_pairs(PairArgs A) {
 // Bound: FP64 issue with three or four waves a SIMD.  With so few a workgroup
 // per row, as in FP32, leaves waves idle at rows of one to three items and in the
 // last round of workgroups.  20 MD steps of 2,000, 28,000 and 252,480 sites, a
-// workgroup per row 1.96, 5.77 and 41.7 ms; a wave per item 1.70, 5.51 and 39.0.
+// workgroup per row 1.96, 5.77 and 41.7 ms; a wave per item 1.69, 5.42 and 38.7.
 template <bool ENERGY>
 __device__ __forceinline__ void
 k_eng_pairs64(PairArgs A) {

@@ -903,8 +903,7 @@ __device__ __forceinline__ void k_md_step_ba(StepArgs A, float4* __restrict__ x,
   if (g < A.water0 + A.G.n_water) step_group<true>(A, x, v, g, step_dev);
 }
 
-// After the force evaluation: kick ½ with the new forces, RATTLE; the step's
-// last launch advances the device step index.
+// After the force evaluation: kick ½ with the new forces, RATTLE.
 __device__ __forceinline__ void k_md_step_b(StepArgs A, float4* __restrict__ x,
                                             float4* __restrict__ v) {
   if (*A.status) return;

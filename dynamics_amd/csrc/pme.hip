@@ -292,7 +292,7 @@ __device__ __forceinline__ C* lds_fft(C* a, C* b, int nl, int S, int N, uint64_t
 // every element of its lines: whole cache lines, which with 4 consecutive
 // values were fetched by four workgroups on different XCDs.  Radix 8 and 9
 // stages halve the LDS exchanges of radix 4 and 3.  128³ alone: z pass 12 µs, y 14,
-// x with the convolution 19 (complex radix-4 passes of 4 lines: 12 to 28, and 37).
+// x with the convolution 17 (complex radix-4 passes of 4 lines: 12 to 28, and 37).
 struct FftGeom {
   int K[3];
   int nh;  // kz values of the spectrum: K[2]/2 + 1
