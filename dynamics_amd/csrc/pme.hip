@@ -533,10 +533,10 @@ constexpr int kConvSums = 4;
 // The wave's four sums, sum v in the lanes of row v (16 lanes): a swap of
 // half-waves leaves one value in each half, a swap of rows one in each row, four
 // rotations add a row.  (24 shuffles otherwise.)
-__device__ __forceinline__ long long wave_sums(const long long (&v)[kConvSums]) {
-  auto two = [](long long a) { return make_uint2((uint32_t)a, (uint32_t)((unsigned long long)a >> 32)); };
-  auto one = [](uint32_t lo, uint32_t hi) { return (long long)((unsigned long long)hi << 32 | lo); };
-  auto half = [&](long long a, long long b) {
+__device__ __forceinline__ uint64_t wave_sums(const uint64_t (&v)[kConvSums]) {
+  auto two = [](uint64_t a) { return make_uint2((uint32_t)a, (uint32_t)(a >> 32)); };
+  auto one = [](uint32_t lo, uint32_t hi) { return (uint64_t)hi << 32 | lo; };
+  auto half = [&](uint64_t a, uint64_t b) {
     const uint2 x = two(a), y = two(b);
     const auto lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
     const auto hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
@@ -545,7 +545,7 @@ __device__ __forceinline__ long long wave_sums(const long long (&v)[kConvSums]) 
   const uint2 x = two(half(v[0], v[2])), y = two(half(v[1], v[3]));
   const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
   const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
-  long long s = one(lo[0], hi[0]) + one(lo[1], hi[1]);
+  uint64_t s = one(lo[0], hi[0]) + one(lo[1], hi[1]);
   auto turn = [&](auto ctrl) {
     const uint2 t = two(s);
     s += one((uint32_t)__builtin_amdgcn_mov_dpp((int)t.x, decltype(ctrl)::value, 0xf, 0xf, true),
@@ -560,13 +560,13 @@ __device__ __forceinline__ long long wave_sums(const long long (&v)[kConvSums]) 
 // Adds x and what its rounding to 2⁻³² leaves to the two sums, in the same
 // units but each kFxBias too large (taken off once per workgroup; sums wrap).
 // x is clamped as every fixed-point value is.
-constexpr long long kFxBias = 0x4338000000000000LL;  // bits of 1.5·2⁵²
-__device__ __forceinline__ void add_fx128(double x, long long& hi, long long& lo) {
+constexpr uint64_t kFxBias = 0x4338000000000000LL;  // bits of 1.5·2⁵²
+__device__ __forceinline__ void add_fx128(double x, uint64_t& hi, uint64_t& lo) {
   x = fmin(fmax(x, -(double)DYN_FX_CLAMP), (double)DYN_FX_CLAMP);
   const double d = __builtin_fma(x, DYN_FX_SCALE, 0x1.8p52);
   const double rest = __builtin_fma(x, DYN_FX_SCALE, 0x1.8p52 - d);
-  hi += __double_as_longlong(d);
-  lo += __double_as_longlong(__builtin_fma(rest, DYN_FX_SCALE, 0x1.8p52));
+  hi += (uint64_t)__double_as_longlong(d);
+  lo += (uint64_t)__double_as_longlong(__builtin_fma(rest, DYN_FX_SCALE, 0x1.8p52));
 }
 struct ConvArgs {
   float invL[3];
@@ -588,7 +588,7 @@ k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
              const typename CxT<C>::R* __restrict__ G, ConvArgs V, int64_t* __restrict__ partials) {
   const FftGeom g = uni(geom);
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ long long red[kConvSums][kFftBlock / 64];
+  __shared__ uint64_t red[kConvSums][kFftBlock / 64];
   const int N = g.K[0], cols = g.K[1] * g.nh, c0 = blockIdx.x * g.L;
   if (c0 >= cols) return;  // beyond this system's lines
   const int nl = min(g.L, cols - c0);
@@ -603,7 +603,7 @@ k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
   }, [&](int e, C v) { A[e] = v; });
   __syncthreads();
   C* X = lds_fft<-1>(A, B, nl, nl, N, g.plan[0], s_tw);
-  long long sum[kConvSums] = {0, 0, 0, 0};
+  uint64_t sum[kConvSums] = {0, 0, 0, 0};
   for_loaded(N * nl, [&](int e) {
     const int n = fast_div(e, nl, rnl);
     return G[(size_t)n * cols + c0 + e - n * nl];
@@ -623,13 +623,13 @@ k_fft_conv_x(C* __restrict__ spec, FftGeom geom, const C* __restrict__ tw,
     v.y *= gv;
     X[e] = v;
   });
-  const long long w = wave_sums(sum);
+  const uint64_t w = wave_sums(sum);
   if ((threadIdx.x & 15) == 0) red[(threadIdx.x >> 4) & 3][threadIdx.x / 64] = w;
   __syncthreads();
   if (threadIdx.x < kConvSums) {
-    long long s = 0;
+    uint64_t s = 0;
     for (int k = 0; k < kFftBlock / 64; ++k) s += red[threadIdx.x][k];
-    partials[kConvSums * blockIdx.x + threadIdx.x] = s - (long long)(N * nl) * kFxBias;
+    partials[kConvSums * blockIdx.x + threadIdx.x] = (int64_t)(s - (uint64_t)(N * nl) * kFxBias);
   }
   const C* Z = lds_fft<+1>(X, X == A ? B : A, nl, nl, N, g.plan[0], s_tw);
   for (int e = threadIdx.x; e < N * nl; e += blockDim.x) {
@@ -856,20 +856,20 @@ __device__ __forceinline__ void k_pme_gather(const float4* __restrict__ xyzq, ui
   if (res && blockIdx.x == 0) {
     // the first workgroup also sums the convolution's energy and virial
     // partials
-    __shared__ long long red[kConvSums][kGatherBlock / 64];
-    long long sum[kConvSums] = {0, 0, 0, 0};
+    __shared__ uint64_t red[kConvSums][kGatherBlock / 64];
+    uint64_t sum[kConvSums] = {0, 0, 0, 0};
     for (int b = threadIdx.x; b < nbp; b += kGatherBlock)
-      for (int v = 0; v < kConvSums; ++v) sum[v] += (long long)partials[kConvSums * b + v];
-    const long long w = wave_sums(sum);
+      for (int v = 0; v < kConvSums; ++v) sum[v] += (uint64_t)partials[kConvSums * b + v];
+    const uint64_t w = wave_sums(sum);
     if ((threadIdx.x & 15) == 0) red[(threadIdx.x >> 4) & 3][threadIdx.x / 64] = w;
     __syncthreads();
     if (threadIdx.x < 2) {
-      long long hi = 0, lo = 0;
+      uint64_t hi = 0, lo = 0;
       for (int k = 0; k < kGatherBlock / 64; ++k) {
         hi += red[threadIdx.x][k];
         lo += red[threadIdx.x + 2][k];
       }
-      res[threadIdx.x] = ((double)hi + (double)lo * DYN_FX_INV_SCALE) * DYN_FX_INV_SCALE;
+      res[threadIdx.x] = ((double)(int64_t)hi + (double)(int64_t)lo * DYN_FX_INV_SCALE) * DYN_FX_INV_SCALE;
     }
   }
   constexpr int kLanes = gather_lanes(ORDER);
